@@ -21,6 +21,8 @@
 //              so its weight term vanishes; this kernel computes the exact one.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "pdfxc_device.hpp"
 #include "pdfxc_internal.hpp"
 #include "pdfxc_split.hpp"
@@ -357,110 +359,244 @@ __device__ inline void cell_step(int ss, double mu, double a, double& s, double&
     dsdmu = ds * (1.0 - 2.0 * a * mu);
 }
 
+// Sum or product over the GW lanes of a group (GW = 16, 32 or 64, groups
+// aligned): DPP within the rows of 16, a shuffle above; every lane gets it,
+// from the same tree in every lane.
+template <int CTRL>
+__device__ inline double dpp_f64(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppMirror = 0x140;
+template <int GW>
+__device__ inline double group_sum(double v) {
+    v += dpp_f64<kDppXor1>(v);
+    v += dpp_f64<kDppXor2>(v);
+    v += dpp_f64<kDppHalfMirror>(v);
+    v += dpp_f64<kDppMirror>(v);
+#pragma unroll
+    for (int off = 16; off < GW; off <<= 1) v += __shfl_xor(v, off);
+    return v;
+}
+template <int GW>
+__device__ inline double group_prod(double v) {
+    v *= dpp_f64<kDppXor1>(v);
+    v *= dpp_f64<kDppXor2>(v);
+    v *= dpp_f64<kDppHalfMirror>(v);
+    v *= dpp_f64<kDppMirror>(v);
+#pragma unroll
+    for (int off = 16; off < GW; off <<= 1) v *= __shfl_xor(v, off);
+    return v;
+}
+
+// ---------------------------------------------------------------------------
+// Weight term: for every point, K (grad_B P_A - omega grad_B Z) to every atom
+// B != A (K = e / P_A, e = w e_xc; omega = P_A / Z; Z = sum_i P_i; P_i = prod_j
+// s(mu_ij)) and the opposite sum to the point's own atom A.
+//
+// FP64 VALU bound.  With G_ij = (prod_{m != j} s_im) ds/dmu_ij / R_ij the two
+// terms are sums of f_i G_ij over cells i and their neighbours j, f_i = K
+// (delta_iA - omega), with grad_i mu_ij = (u_i - mu_ij e_ij) / R_ij and
+// grad_j mu_ij = (-u_j + mu_ij e_ij) / R_ij.  Only the few cells whose P_i is
+// not negligible contribute, so a group of GW lanes takes one point:
+//   1. a cell per lane against the kNear atoms nearest to A, which ends every
+//      cell with two zero factors (then P_i and every G_ij are 0) or a product
+//      below 1e-24 (s is 0 or above 5e-17, where ds/dmu is at most 4e4 s, so
+//      G_ij R_ij / Z stays below 1e-19; A's own cell, whose terms are divided
+//      by P_A, keeps any product).  16 near atoms leave 8 cells of 24 and 13 of
+//      59 on average, 8 atoms leave 10 and 18;
+//   2. a neighbour per lane for each cell left: P_i without its zero factors;
+//   3. the same again for G_ij: lane j adds the term of atom j, the group's
+//      sum of the rest goes to atom i.
+// The product without one factor is P_i / s_ij, or with one zero factor j the
+// product of the others for that j alone, so no product is formed again.  One
+// point per thread with all na^2 cell pairs and products repeated where a
+// factor vanished: 47.5 ms for a helix of 8 residues (59 atoms, 50 radial
+// shells of 200 points) and 1.90 ms for 8 waters; this form 3.37 and 0.76 ms
+// (of that 2.8 and 0.5 ms are kNear 8 -> 16 and the 1e-40 -> 1e-24 cut of 1.,
+// the short reciprocal and the unit vectors kept in LDS).
 // atoms: n x 4 (x, y, z, Z) | 1/R_mn [n][n] | a_mn [n][n] (the partition kernel's table);
-// ss: the grid's partition is Stratmann-Scuseria (else Becke)
-__global__ void k_grad_w(const double* __restrict__ atoms, int na, int64_t n_slots, const double* __restrict__ pts,
-                         const int* __restrict__ slot_atom, const double* __restrict__ ewf,
-                         double* __restrict__ gacc, int ss) {
-    extern __shared__ double s_buf[];  // r [blockDim][na] | P [blockDim][na] | sums [3 na]
+// nbr [n][kNear]: the atoms nearest to each atom, itself first, -1 past the last;
+// ss: the grid's partition is Stratmann-Scuseria (else Becke).
+// LDS: xyz [3 na] | per group: r, product [na], unit vectors, sums [3 na] | per group: cells [na]
+// ---------------------------------------------------------------------------
+constexpr double kCellMin = 1e-24;
+
+// 1 / x to the last bit or two, for x away from the ends of the exponent range:
+// the hardware's estimate and two Newton steps (a full division is twice that)
+__device__ inline double recip(double x) {
+    double y = __builtin_amdgcn_rcp(x);
+    y = __builtin_fma(__builtin_fma(-x, y, 1.0), y, y);
+    return __builtin_fma(__builtin_fma(-x, y, 1.0), y, y);
+}
+
+template <int GW>
+__global__ __launch_bounds__(256) void k_grad_w(const double* __restrict__ atoms, const int* __restrict__ nbr, int na,
+                                                int64_t n_slots, int per_group, const double* __restrict__ pts,
+                                                const int* __restrict__ slot_atom, const double* __restrict__ ewf,
+                                                double* __restrict__ gacc, int ss) {
+    extern __shared__ double s_buf[];
     const int tid = threadIdx.x;
-    const int nt = blockDim.x;
-    double* r = s_buf + (size_t)tid * na;
-    double* Pv = s_buf + (size_t)nt * na + (size_t)tid * na;
-    double* s_g = s_buf + 2 * (size_t)nt * na;
-    for (int i = tid; i < 3 * na; i += nt) s_g[i] = 0.0;
+    const int ng = blockDim.x / GW;  // groups of the workgroup
+    const int grp = tid / GW;
+    const int gl = tid & (GW - 1);
+    double* s_xyz = s_buf;
+    double* r = s_buf + 3 * (size_t)na + (size_t)grp * 8 * na;
+    double* Pv = r + na;
+    double* u = r + 2 * (size_t)na;    // [3][na], from the point to each atom
+    double* s_g = r + 5 * (size_t)na;  // [3][na], atom j only ever touched by lane j mod GW
+    int* cell = reinterpret_cast<int*>(s_buf + 3 * (size_t)na + (size_t)ng * 8 * na) + (size_t)grp * na;
+    for (int i = tid; i < 3 * na; i += blockDim.x) s_xyz[i] = atoms[4 * (i / 3) + i % 3];
+    for (int i = gl; i < 3 * na; i += GW) s_g[i] = 0.0;
     __syncthreads();
     const double* invd = atoms + 4 * na;
     const double* amat = invd + (size_t)na * na;
-    const int64_t slot = (int64_t)blockIdx.x * nt + tid;
-    const int A = (slot < n_slots) ? slot_atom[slot] : -1;
-    const double e = (A >= 0) ? ewf[slot] : 0.0;
-    if (A >= 0 && e != 0.0) {
-        const double x = pts[slot], y = pts[n_slots + slot], z = pts[2 * n_slots + slot];
-        for (int i = 0; i < na; ++i) {
-            const double dx = x - atoms[4 * i], dy = y - atoms[4 * i + 1], dz = z - atoms[4 * i + 2];
-            r[i] = sqrt(dx * dx + dy * dy + dz * dz);
+    // the lanes of this lane's group within its wave's ballot
+    const int gbase = (tid & 63) & ~(GW - 1);
+    const unsigned long long gmask = GW == 64 ? ~0ull : ((1ull << (GW & 63)) - 1ull) << gbase;
+    const unsigned long long below = ((1ull << (tid & 63)) - 1ull) & gmask;
+    for (int it = 0; it < per_group; ++it) {
+        // neighbouring slots go to the groups of one pass
+        const int64_t slot = ((int64_t)blockIdx.x * per_group + it) * ng + grp;
+        const int A = (slot < n_slots) ? slot_atom[slot] : -1;
+        const double e = (A >= 0) ? ewf[slot] : 0.0;
+        const bool valid = A >= 0 && e != 0.0;
+        // every lane keeps to the wave-wide barriers below: LDS written by one
+        // lane of a group is read by the others of the same wave only
+        if (valid) {
+            const double x = pts[slot], y = pts[n_slots + slot], z = pts[2 * n_slots + slot];
+            for (int j = gl; j < na; j += GW) {
+                const double dx = s_xyz[3 * j] - x, dy = s_xyz[3 * j + 1] - y, dz = s_xyz[3 * j + 2] - z;
+                const double rj = sqrt(dx * dx + dy * dy + dz * dz);
+                const double ir = 1.0 / rj;  // not used for A itself, where the point may sit
+                r[j] = rj;
+                u[j] = dx * ir;
+                u[na + j] = dy * ir;
+                u[2 * na + j] = dz * ir;
+            }
         }
-        double Zs = 0.0;
-        for (int i = 0; i < na; ++i) {
-            double p = 0.0;
-            if (atoms[4 * i + 3] > 0.0) {
-                p = 1.0;
-                for (int j = 0; j < na && p != 0.0; ++j) {
-                    if (j == i || atoms[4 * j + 3] <= 0.0) continue;
-                    const double mu = (r[i] - r[j]) * invd[(size_t)i * na + j];
+        __builtin_amdgcn_wave_barrier();
+        __threadfence_block();
+        // 1. cells that survive the nearest atoms of A
+        int ncell = 0;
+        for (int m0 = 0; m0 < na; m0 += GW) {
+            const int m = m0 + gl;
+            bool live = valid && m < na;
+            if (live) {
+                const double rm = r[m];
+                double p = 1.0;
+                int nz = 0;
+                for (int q = 0; q < kNear && live; ++q) {
+                    const int k = nbr[A * kNear + q];
+                    if (k < 0) break;
+                    if (k == m) continue;
+                    const double mu = (rm - r[k]) * invd[(size_t)m * na + k];
                     double s, ds;
-                    cell_step(ss, mu, amat[(size_t)i * na + j], s, ds);
-                    p *= s;
+                    cell_step(ss, mu, amat[(size_t)m * na + k], s, ds);
+                    if (s > 0.0)
+                        p *= s;
+                    else
+                        ++nz;
+                    live = nz < 2 && (p >= kCellMin || m == A);
                 }
             }
-            Pv[i] = p;
-            Zs += p;
+            const unsigned long long b = __ballot(live);
+            if (live) cell[ncell + __popcll(b & below)] = m;
+            ncell += __popcll(b & gmask);
         }
-        const double om = Pv[A] / Zs;
+        __builtin_amdgcn_wave_barrier();
+        __threadfence_block();
+        // 2. P_i of the cells left: the product of the factors that are not 0,
+        // negated when one is 0 (P_i = 0), 0 when more are
+        double Zs = 0.0, PA = 0.0;
+        for (int c = 0; c < ncell; ++c) {
+            const int i = cell[c];
+            const double ri = r[i];
+            double p = 1.0;
+            int nz = 0;
+            for (int j0 = 0; j0 < na; j0 += GW) {
+                const int j = j0 + gl;
+                bool zero = false;
+                if (j < na && j != i) {
+                    double s, ds;
+                    cell_step(ss, (ri - r[j]) * invd[(size_t)i * na + j], amat[(size_t)i * na + j], s, ds);
+                    zero = !(s > 0.0);
+                    if (!zero) p *= s;
+                }
+                nz += __popcll(__ballot(zero) & gmask);
+            }
+            p = group_prod<GW>(p);
+            if (nz == 0) {
+                Zs += p;
+                if (i == A) PA = p;
+            }
+            if (gl == 0) Pv[c] = (nz > 1 || (p < kCellMin && i != A)) ? 0.0 : nz == 1 ? -p : p;
+        }
+        __builtin_amdgcn_wave_barrier();
+        __threadfence_block();
+        // 3. the pair terms (none where omega = 0)
+        const double om = PA > 0.0 ? PA / Zs : 0.0;
         if (om > 0.0) {
             const double K = e / om / Zs;  // w_single e_xc / Z
-            // product of cell i's factors without the one of atom j
-            auto prod_ex = [&](int i, int j, double s_ij) {
-                if (s_ij > 1e-200) return Pv[i] / s_ij;
-                double q = 1.0;
-                for (int m = 0; m < na; ++m) {
-                    if (m == i || m == j || atoms[4 * m + 3] <= 0.0) continue;
-                    const double mu = (r[i] - r[m]) * invd[(size_t)i * na + m];
+            double t[3] = {0.0, 0.0, 0.0};  // this lane's part of the sum over B != A
+            for (int c = 0; c < ncell; ++c) {
+                const int i = cell[c];
+                const double Pc = Pv[c];
+                if (Pc == 0.0) continue;
+                const double f = K * ((i == A ? 1.0 : 0.0) - om) * fabs(Pc);
+                const double ri = r[i];
+                const double xi = s_xyz[3 * i], yi = s_xyz[3 * i + 1], zi = s_xyz[3 * i + 2];
+                double own[3] = {0.0, 0.0, 0.0}, gs = 0.0;
+                for (int j = gl; j < na; j += GW) {
+                    if (j == i) continue;
+                    const double id = invd[(size_t)i * na + j];
+                    const double mu = (ri - r[j]) * id;
                     double s, ds;
-                    cell_step(ss, mu, amat[(size_t)i * na + m], s, ds);
-                    q *= s;
-                }
-                return q;
-            };
-            double gA[3] = {0.0, 0.0, 0.0};
-            for (int Bt = 0; Bt < na; ++Bt) {
-                if (Bt == A || atoms[4 * Bt + 3] <= 0.0) continue;
-                const double uB[3] = {(atoms[4 * Bt] - x) / r[Bt], (atoms[4 * Bt + 1] - y) / r[Bt],
-                                      (atoms[4 * Bt + 2] - z) / r[Bt]};
-                double gZ[3] = {0.0, 0.0, 0.0}, gPA[3] = {0.0, 0.0, 0.0};
-                for (int i = 0; i < na; ++i) {
-                    if (i == Bt || atoms[4 * i + 3] <= 0.0) continue;
-                    const double id = invd[(size_t)Bt * na + i];
-                    const double Rv[3] = {(atoms[4 * Bt] - atoms[4 * i]) * id, (atoms[4 * Bt + 1] - atoms[4 * i + 1]) * id,
-                                          (atoms[4 * Bt + 2] - atoms[4 * i + 2]) * id};
-                    // cell B, factor of atom i: grad_B mu_Bi = (u_B - mu_Bi e_Bi) / R
-                    {
-                        const double mu = (r[Bt] - r[i]) * id;
-                        double s, ds;
-                        cell_step(ss, mu, amat[(size_t)Bt * na + i], s, ds);
-                        const double c = prod_ex(Bt, i, s) * ds * id;
+                    cell_step(ss, mu, amat[(size_t)i * na + j], s, ds);
+                    // with one zero factor, only that factor's own derivative is left
+                    const double g = Pc > 0.0 ? f * ds * id * recip(s) : (s > 0.0 ? 0.0 : f * ds * id);
+                    const double gm = g * mu * id;
+                    const double e3[3] = {gm * (xi - s_xyz[3 * j]), gm * (yi - s_xyz[3 * j + 1]),
+                                          gm * (zi - s_xyz[3 * j + 2])};
+                    gs += g;
 #pragma unroll
-                        for (int d = 0; d < 3; ++d) gZ[d] += c * (uB[d] - mu * Rv[d]);
-                    }
-                    // cell i, factor of atom B: grad_B mu_iB = (-u_B - mu_iB e_Bi) / R
-                    {
-                        const double mu = (r[i] - r[Bt]) * id;
-                        double s, ds;
-                        cell_step(ss, mu, amat[(size_t)i * na + Bt], s, ds);
-                        const double c = prod_ex(i, Bt, s) * ds * id;
-#pragma unroll
-                        for (int d = 0; d < 3; ++d) {
-                            const double gm = c * (-uB[d] - mu * Rv[d]);
-                            gZ[d] += gm;
-                            if (i == A) gPA[d] += gm;
+                    for (int d = 0; d < 3; ++d) {
+                        own[d] -= e3[d];
+                        if (j != A) {
+                            const double v = e3[d] - g * u[d * na + j];
+                            s_g[d * na + j] += v;
+                            t[d] += v;
                         }
                     }
                 }
+                if (i == A) continue;
 #pragma unroll
                 for (int d = 0; d < 3; ++d) {
-                    const double c = K * (gPA[d] - om * gZ[d]);
-                    atomicAdd(&s_g[3 * Bt + d], c);
-                    gA[d] -= c;
+                    const double v = group_sum<GW>(own[d] + gs * u[d * na + i]);
+                    if (gl == (i & (GW - 1))) {
+                        s_g[d * na + i] += v;
+                        t[d] += v;
+                    }
                 }
             }
 #pragma unroll
-            for (int d = 0; d < 3; ++d) atomicAdd(&s_g[3 * A + d], gA[d]);
+            for (int d = 0; d < 3; ++d) {
+                const double v = group_sum<GW>(t[d]);
+                if (gl == (A & (GW - 1))) s_g[d * na + A] -= v;
+            }
         }
+        __builtin_amdgcn_wave_barrier();
+        __threadfence_block();
     }
     __syncthreads();
-    for (int i = tid; i < 3 * na; i += nt)
-        if (s_g[i] != 0.0) atomicAdd(gacc + i, s_g[i]);
+    for (int k = tid; k < 3 * na; k += blockDim.x) {
+        const int d = k / na, j = k - d * na;
+        double v = 0.0;
+        for (int q = 0; q < ng; ++q) v += s_buf[3 * (size_t)na + (size_t)q * 8 * na + 5 * (size_t)na + k];
+        if (v != 0.0) atomicAdd(gacc + 3 * j + d, v);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -506,19 +642,38 @@ int launch_grad_fn(Context& c, const LaunchRange& r, const int* d_shell_atom, co
     }
 }
 
-int launch_grad_w(Context& c, const double* d_atoms, int n_atoms, const int* d_slot_atom, const double* d_ewf,
-                  double* d_gacc, int partition) {
-    int threads = 64;
-    while (threads > 1 && (size_t)threads * 2 * n_atoms * sizeof(double) + 3 * n_atoms * sizeof(double) > 65536)
-        threads >>= 1;
-    const size_t lds = ((size_t)threads * 2 * n_atoms + 3 * (size_t)n_atoms) * sizeof(double);
-    if (lds > 65536) {
+int launch_grad_w(Context& c, const double* d_atoms, const int* d_near, int n_atoms, const int* d_slot_atom,
+                  const double* d_ewf, double* d_gacc, int partition) {
+    // the atoms whose distances and sums one point needs at least (5 n_atoms doubles) keep to 64 KiB
+    if (5 * (size_t)n_atoms * sizeof(double) > 65536) {
         set_error("gradient: too many atoms for the weight-derivative kernel's LDS");
         return PDFXC_ERR_UNSUPPORTED;
     }
-    const int64_t g = (c.n_slots + threads - 1) / threads;
-    hipLaunchKernelGGL(k_grad_w, dim3((unsigned)g), dim3(threads), lds, c.stream, d_atoms, n_atoms, c.n_slots,
-                       c.d_pts, d_slot_atom, d_ewf, d_gacc + 3 * n_atoms, partition == PDFXC_PARTITION_SS ? 1 : 0);
+    // lanes per point: as many as there are atoms, within a row of 16 lanes and a wave
+    const int gw = n_atoms <= 16 ? 16 : n_atoms <= 32 ? 32 : 64;
+    auto lds_of = [&](int threads) {
+        const size_t ng = threads / gw;
+        return sizeof(double) * (3 + 8 * ng) * (size_t)n_atoms + sizeof(int) * ng * (size_t)n_atoms;
+    };
+    // four waves share the atom table while two such workgroups fit on a CU
+    const int threads = lds_of(256) <= 80 * 1024 ? 256 : 64;
+    const size_t lds = lds_of(threads);  // at most 147 KiB (one wave, 1638 atoms)
+    const int ng = threads / gw;
+    // up to 16 points per group between two flushes of the sums, fewer while
+    // that leaves less than 2048 workgroups
+    const int64_t per = std::min<int64_t>(16, std::max<int64_t>(1, c.n_slots / ((int64_t)ng * 2048)));
+    const int64_t g = (c.n_slots + per * ng - 1) / (per * ng);
+    const int ss = partition == PDFXC_PARTITION_SS ? 1 : 0;
+    double* out = d_gacc + 3 * n_atoms;
+#define PDFXC_GRAD_W(GW)                                                                                     \
+    hipLaunchKernelGGL(k_grad_w<GW>, dim3((unsigned)g), dim3(threads), lds, c.stream, d_atoms, d_near, n_atoms, \
+                       c.n_slots, (int)per, c.d_pts, d_slot_atom, d_ewf, out, ss)
+    switch (gw) {
+        case 16: PDFXC_GRAD_W(16); break;
+        case 32: PDFXC_GRAD_W(32); break;
+        default: PDFXC_GRAD_W(64); break;
+    }
+#undef PDFXC_GRAD_W
     return check("k_grad_w");
 }
 

@@ -1280,6 +1280,23 @@ static void orientation(int na, const int* Z, const double* xyz, double O[9]) {
     }
 }
 
+// [n][kNear]: each atom's nearest atoms by distance, itself first; -1 past the last
+static std::vector<int> near_atoms(int n, const double* xyz) {
+    std::vector<int> out((size_t)n * kNear, -1);
+    std::vector<std::pair<double, int>> d(n);
+    const int k = std::min(n, kNear);
+    for (int a = 0; a < n; ++a) {
+        for (int b = 0; b < n; ++b) {
+            double r2 = 0.0;
+            for (int q = 0; q < 3; ++q) r2 += (xyz[3 * a + q] - xyz[3 * b + q]) * (xyz[3 * a + q] - xyz[3 * b + q]);
+            d[b] = {b == a ? -1.0 : r2, b};
+        }
+        std::partial_sort(d.begin(), d.begin() + k, d.end());
+        for (int q = 0; q < k; ++q) out[(size_t)a * kNear + q] = d[q].second;
+    }
+    return out;
+}
+
 int ensure_beta_buffers(Context* c) {
     const size_t n = 4 * (size_t)c->n_slots;
     if (!c->d_rho_b) {
@@ -1950,10 +1967,12 @@ int pdfxc_gradient_rks(pdfxc_ctx* ctx, int functional, int n_atoms, const int* Z
         }
         gl.push_back(g);
     }
-    int *d_shat = nullptr, *d_slat = nullptr;
+    const std::vector<int> near = near_atoms(na, xyz);
+    int *d_shat = nullptr, *d_slat = nullptr, *d_near = nullptr;
     double *d_at = nullptr, *d_ewf = nullptr, *d_g = nullptr;
     int rc = dalloc(&d_shat, shell_atom.size());
     if (rc == PDFXC_OK) rc = dalloc(&d_slat, slot_atom.size());
+    if (rc == PDFXC_OK) rc = dalloc(&d_near, near.size());
     if (rc == PDFXC_OK) rc = dalloc(&d_at, at.size());
     if (rc == PDFXC_OK) rc = dalloc(&d_ewf, (size_t)c->n_slots);
     if (rc == PDFXC_OK) rc = dalloc(&d_g, 6 * (size_t)na);
@@ -1961,6 +1980,7 @@ int pdfxc_gradient_rks(pdfxc_ctx* ctx, int functional, int n_atoms, const int* Z
     if (rc == PDFXC_OK) {
         e = hipMemcpy(d_shat, shell_atom.data(), sizeof(int) * shell_atom.size(), hipMemcpyHostToDevice);
         if (e == hipSuccess) e = hipMemcpy(d_slat, slot_atom.data(), sizeof(int) * slot_atom.size(), hipMemcpyHostToDevice);
+        if (e == hipSuccess) e = hipMemcpy(d_near, near.data(), sizeof(int) * near.size(), hipMemcpyHostToDevice);
         if (e == hipSuccess) e = hipMemcpy(d_at, at.data(), sizeof(double) * at.size(), hipMemcpyHostToDevice);
         if (e == hipSuccess) e = hipMemset(d_g, 0, sizeof(double) * 6 * (size_t)na);
         if (e != hipSuccess) rc = hip_fail(e, "pdfxc_gradient_rks: upload");
@@ -1983,7 +2003,7 @@ int pdfxc_gradient_rks(pdfxc_ctx* ctx, int functional, int n_atoms, const int* Z
     if (rc == PDFXC_OK) rc = launch_xc_points(*c, functional, d_ewf);
     for (const LaunchRange& r : gl)
         if (rc == PDFXC_OK) rc = launch_grad_fn(*c, r, d_shat, d_slat, na, d_g);
-    if (rc == PDFXC_OK) rc = launch_grad_w(*c, d_at, na, d_slat, d_ewf, d_g, c->grid_partition);
+    if (rc == PDFXC_OK) rc = launch_grad_w(*c, d_at, d_near, na, d_slat, d_ewf, d_g, c->grid_partition);
     if (rc == PDFXC_OK) rc = launch_energy_sum(*c, c->d_E);
     std::vector<double> g(6 * (size_t)na);
     double E = 0.0;
@@ -1995,6 +2015,7 @@ int pdfxc_gradient_rks(pdfxc_ctx* ctx, int functional, int n_atoms, const int* Z
     }
     dfree(d_shat);
     dfree(d_slat);
+    dfree(d_near);
     dfree(d_at);
     dfree(d_ewf);
     dfree(d_g);

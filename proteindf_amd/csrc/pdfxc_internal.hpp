@@ -295,11 +295,13 @@ int launch_split_rho(Context& c);   // P slices + k_rho_split
 int launch_split_kmat(Context& c);  // k_kmat_split
 int split_kmat_max_dyn_lds(int S, size_t* out);
 int launch_mfma_split_selftest(float* d_out, hipStream_t s);
+constexpr int kNear = 16;  // entries per atom of a near-atom table
 // XC nuclear gradient (pdfxc_grad.hip); d_gacc: functional term [3 n_atoms] then weight term [3 n_atoms]
 int launch_grad_fn(Context& c, const LaunchRange& r, const int* d_shell_atom, const int* d_slot_atom,
                    int n_atoms, double* d_gacc);
-int launch_grad_w(Context& c, const double* d_atoms, int n_atoms, const int* d_slot_atom, const double* d_ewf,
-                  double* d_gacc, int partition);
+// d_near: near_atoms() of the molecule
+int launch_grad_w(Context& c, const double* d_atoms, const int* d_near, int n_atoms, const int* d_slot_atom,
+                  const double* d_ewf, double* d_gacc, int partition);
 int launch_copy(const double* src, double* dst, int64_t n, hipStream_t s);
 
 }  // namespace pdfxc

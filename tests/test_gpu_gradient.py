@@ -114,3 +114,48 @@ def test_split_gradient_matches_oracle(prec):
     np.testing.assert_allclose(gf, gf_ref, rtol=0, atol=g_tol)
     np.testing.assert_allclose(gw, gw_ref, rtol=0, atol=g_tol)
     np.testing.assert_allclose(gf.sum(0), 0.0, atol=10 * g_tol)
+
+
+# the weight term takes 16, 32 or 64 lanes per point (and more atoms than
+# lanes past 64), workgroups of four waves up to 409 atoms and of one beyond
+@pytest.mark.parametrize("n,ss", [(1, 0), (5, 0), (6, 1), (10, 0), (11, 0), (21, 1), (22, 0), (22, 1)])
+def test_weight_term_at_the_edges_of_its_lane_groups(n, ss):
+    mol = molecules.water_cluster(n, 11)
+    info = calc_grid.orbital_info(mol)
+    PA = 0.5 * guess.density_guess(mol, info, seed=11, eps=0.05)
+    say(f"[gpu-case] weight term, {mol.n_atoms} atoms, ss {ss}")
+    o = dict(n_rad=6, n_ang=26, pruning=0, partitioning=ss)
+    grid, atom = oracle.generate_grid_ex(mol.Z, mol.xyz, oracle.grid_opts(**o))
+    ctx = engine.XcContext(info)
+    opts = oracle.grid_opts(**o)
+    ctx.generate_grid_ex(mol.Z, mol.xyz, engine.GridOpts(**{f: getattr(opts, f) for f, _ in engine.GridOpts._fields_}))
+    E, gf, gw = ctx.gradient_rks(mol.Z, mol.xyz, guess.pack_lower(PA))
+    ctx.close()
+    e_ref, gf_ref, gw_ref = oracle.xc_gradient_rks(oracle.AoTable.from_basis(info), info.ao_atom, grid, atom,
+                                                   mol.Z, mol.xyz, PA, partition=2 * ss)
+    assert abs(E - e_ref) <= 1e-9
+    np.testing.assert_allclose(gw, gw_ref, rtol=0, atol=1e-9)
+    np.testing.assert_allclose(gw.sum(0), 0.0, atol=1e-10)
+
+
+def test_weight_term_of_many_atoms():
+    # a chain of 420 hydrogen atoms: one wave per workgroup; 600 points against the oracle
+    rng = np.random.default_rng(5)
+    xyz = np.zeros((420, 3))
+    xyz[:, 0] = 2.1 * np.arange(420)
+    mol = molecules.Molecule(["H"] * len(xyz), xyz + rng.uniform(-0.2, 0.2, xyz.shape), "H420")
+    info = calc_grid.orbital_info(mol)
+    PA = np.diag(np.full(info.n_aos, 0.2))
+    atom = np.sort(rng.integers(0, len(xyz), 600)).astype(np.int32)
+    pts = mol.xyz[atom] + rng.normal(0.0, 0.6, (600, 3))
+    grid = np.concatenate([pts, rng.uniform(0.1, 1.0, (600, 1))], 1)
+    say("[gpu-case] weight term, 420 atoms")
+    ctx = engine.XcContext(info)
+    ctx.set_grid(grid)
+    E, gf, gw = ctx.gradient_rks(mol.Z, mol.xyz, guess.pack_lower(PA), point_atom=atom)
+    ctx.close()
+    e_ref, gf_ref, gw_ref = oracle.xc_gradient_rks(oracle.AoTable.from_basis(info), info.ao_atom, grid, atom,
+                                                   mol.Z, mol.xyz, PA)
+    scale = np.abs(gw_ref).max()
+    assert abs(E - e_ref) <= 1e-10 * abs(e_ref)
+    np.testing.assert_allclose(gw, gw_ref, rtol=0, atol=1e-10 * scale)
