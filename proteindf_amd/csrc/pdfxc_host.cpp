@@ -333,6 +333,7 @@ int pdfxc_ctx_create(pdfxc_ctx** out, int n_aos, const double* ao_center, const 
 
 static void free_grid_buffers(Context* c) {
     dfree(c->d_pts);
+    dfree(c->d_slot_of_point);
     dfree(c->d_blocks);
     dfree(c->d_block_shells);
     dfree(c->d_block_cols);
@@ -344,6 +345,8 @@ static void free_grid_buffers(Context* c) {
     dfree(c->d_rho);
     dfree(c->d_coef_b);
     dfree(c->d_rho_b);
+    dfree(c->d_rho_out);
+    c->n_rho_out = 0;
     dfree(c->d_eblock);
     dfree(c->d_sblocks);
     dfree(c->d_chunks);
@@ -364,6 +367,7 @@ int pdfxc_ctx_destroy(pdfxc_ctx* ctx) {
     if (!c) return PDFXC_OK;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     free_grid_buffers(c);
+    dfree(c->d_grid);
     dfree(c->d_shells);
     dfree(c->d_shrec);
     dfree(c->d_P);
@@ -392,12 +396,16 @@ void* pdfxc_stream(pdfxc_ctx* ctx) {
 namespace pdfxc {
 
 // ---------------------------------------------------------------------------
-// Grid blocks: recursive bisection of the point set along its widest extent,
-// cutting at a multiple of 128 so that every block but the last is full.
+// Grid blocks of the split precision modes: recursive bisection of the point
+// set along its widest extent, cutting at a multiple of 128 so that every block
+// but the last is full.  The device's bisection makes the same cuts (12 times
+// as fast at 1.5 million points) but leaves the points of a block in another
+// order, and the FP32 sums of the split kernels, taken over runs of 16 points,
+// round to other values (4e-9 of K, as much as their error): these modes keep
+// the order, and so the results, that std::nth_element leaves.
 // ---------------------------------------------------------------------------
-static void partition_points(const Context& c, std::vector<int64_t>& order,
-                             std::vector<std::pair<int64_t, int64_t>>& leaves) {
-    order.resize(c.n_pts);
+static void partition_points(const Context& c, std::vector<int>& order) {
+    order.resize((size_t)c.n_pts);
     std::iota(order.begin(), order.end(), 0);
     std::vector<std::pair<int64_t, int64_t>> stack;
     stack.push_back({0, c.n_pts});
@@ -406,10 +414,7 @@ static void partition_points(const Context& c, std::vector<int64_t>& order,
         const auto [lo, hi] = stack.back();
         stack.pop_back();
         const int64_t n = hi - lo;
-        if (n <= kBlockPts) {
-            leaves.push_back({lo, hi});
-            continue;
-        }
+        if (n <= kBlockPts) continue;
         double mn[3] = {1e300, 1e300, 1e300}, mx[3] = {-1e300, -1e300, -1e300};
         for (int64_t k = lo; k < hi; ++k)
             for (int d = 0; d < 3; ++d) {
@@ -424,7 +429,7 @@ static void partition_points(const Context& c, std::vector<int64_t>& order,
         const int64_t mid = lo + (nch / 2) * kBlockPts;
         const double* v = X[dim];
         std::nth_element(order.begin() + lo, order.begin() + mid, order.begin() + hi,
-                         [v](int64_t a, int64_t b) { return v[a] < v[b] || (v[a] == v[b] && a < b); });
+                         [v](int a, int b) { return v[a] < v[b] || (v[a] == v[b] && a < b); });
         // right first so that leaves come out left to right
         stack.push_back({mid, hi});
         stack.push_back({lo, mid});
@@ -448,10 +453,29 @@ static double shell_bound(const Shell& s, double d) {
     return b;
 }
 
+// The distance past which shell_bound < screen: shell_bound does not grow with
+// d, so the test of every block comes down to one comparison with the largest
+// double that still passes it (0 <= cut; negative when none does).
+static double shell_cut(const Shell& s, double screen) {
+    if (!(screen > 0.0)) return HUGE_VAL;
+    if (shell_bound(s, 0.0) < screen) return -1.0;
+    double lo = 0.0, hi = 1.0;
+    while (shell_bound(s, hi) >= screen) {
+        lo = hi;
+        hi *= 2.0;
+    }
+    for (;;) {
+        const double mid = 0.5 * (lo + hi);
+        if (mid <= lo || mid >= hi) return lo;
+        (shell_bound(s, mid) < screen ? hi : lo) = mid;
+    }
+}
+
 // Drop every grid-dependent host list and device buffer: a context left like
 // this refuses builds with PDFXC_ERR_NO_GRID.
 static void reset_grid(Context& c) {
     free_grid_buffers(&c);
+    dfree(c.d_grid);
     c.n_pts = 0;
     c.n_slots = 0;
     c.gx.clear();
@@ -504,80 +528,122 @@ static int build_blocks(Context& c) {
     return rc;
 }
 
-static int build_blocks_impl(Context& c) {
-    std::vector<int64_t> order;
-    std::vector<std::pair<int64_t, int64_t>> leaves;
-    partition_points(c, order, leaves);
-    const int nb = (int)leaves.size();
-    const int nsh = (int)c.shells.size();
-    struct Tmp {
-        int64_t lo, hi;
-        std::vector<int> sh;
-        int nao;
-        double cost;
-    };
-    std::vector<Tmp> tmp(nb);
-    const double screen = c.opts.ao_screen;
-    for (int b = 0; b < nb; ++b) {
-        Tmp& t = tmp[b];
-        t.lo = leaves[b].first;
-        t.hi = leaves[b].second;
-        double mn[3] = {1e300, 1e300, 1e300}, mx[3] = {-1e300, -1e300, -1e300};
-        for (int64_t k = t.lo; k < t.hi; ++k) {
-            const int64_t p = order[k];
-            const double v[3] = {c.gx[p], c.gy[p], c.gz[p]};
-            for (int d = 0; d < 3; ++d) {
-                mn[d] = std::min(mn[d], v[d]);
-                mx[d] = std::max(mx[d], v[d]);
-            }
-        }
-        t.nao = 0;
-        for (int s = 0; s < nsh; ++s) {
-            const Shell& S = c.shells[s];
-            // distance from the shell's centre to the block's bounding box: no
-            // point of the block is nearer (shrunk by a relative 1e-12 for rounding)
-            double d2 = 0.0;
-            for (int d = 0; d < 3; ++d) {
-                const double e = std::max(0.0, std::max(mn[d] - S.center[d], S.center[d] - mx[d]));
-                d2 += e * e;
-            }
-            const double dmin = std::sqrt(d2) * (1.0 - 1e-12);
-            // the reference skips a primitive with a r^2 > 30: a shell whose most
-            // diffuse primitive is cut at the nearest point is exactly zero here
-            if (S.exps[0] * dmin * dmin > 30.0) continue;
-            if (screen > 0.0 && shell_bound(S, dmin) < screen) continue;
-            t.sh.push_back(s);
-            t.nao += 2 * S.l + 1;
-        }
-        const int ldn = std::max(kColPad, (t.nao + kColPad - 1) / kColPad * kColPad);
-        t.cost = (double)(t.hi - t.lo) * ldn * ldn + 1.0;
+// workspace freed at the end of its scope
+struct DeviceBuf {
+    void* p = nullptr;
+    ~DeviceBuf() {
+        if (p) (void)hipFree(p);
     }
-    // launch order: descending cost (longest blocks first)
-    std::vector<int> lorder(nb);
-    std::iota(lorder.begin(), lorder.end(), 0);
-    std::stable_sort(lorder.begin(), lorder.end(),
-                     [&](int a, int b) { return tmp[a].cost > tmp[b].cost; });
-    c.blocks.assign(nb, BlockDesc());
+    template <typename T>
+    T* as() const {
+        return reinterpret_cast<T*>(p);
+    }
+    int alloc(size_t bytes) {
+        char* q = nullptr;
+        const int rc = dalloc(&q, bytes);
+        p = q;
+        return rc;
+    }
+};
+
+static int build_blocks_impl(Context& c) {
+    const int64_t n = c.n_pts;
+    const int nb = (int)((n + kBlockPts - 1) / kBlockPts);
+    const int nsh = (int)c.shells.size();
     c.block_shells.clear();
     c.block_cols.clear();
     c.block_shell_col.clear();
     c.block_sorder.clear();
+    c.slot_of_point.clear();
+    free_grid_buffers(&c);
+
+    // shell table of the screening; cls: rank of (l, nprim), the blocks' evaluation order
+    const int nw = (nsh + 63) / 64;
+    std::vector<ScreenShell> sc(nsh);
+    int ncls = 0;
+    {
+        std::vector<std::pair<int, int>> cls;
+        for (const Shell& S : c.shells) cls.push_back({S.l, S.nprim});
+        std::sort(cls.begin(), cls.end());
+        cls.erase(std::unique(cls.begin(), cls.end()), cls.end());
+        ncls = (int)cls.size();
+        for (int k = 0; k < nsh; ++k) {
+            const Shell& S = c.shells[k];
+            for (int d = 0; d < 3; ++d) sc[k].center[d] = S.center[d];
+            sc[k].exp0 = S.exps[0];
+            // shells of one kind (an element's) share their primitives
+            const Shell* like = nullptr;
+            for (int j = k - 1; j >= std::max(0, k - 64) && !like; --j) {
+                const Shell& T = c.shells[j];
+                if (T.l == S.l && T.nprim == S.nprim && std::equal(T.exps, T.exps + T.nprim, S.exps) &&
+                    std::equal(T.coefs, T.coefs + T.nprim, S.coefs)) {
+                    like = &T;
+                    sc[k].cut = sc[j].cut;
+                }
+            }
+            if (!like) sc[k].cut = shell_cut(S, c.opts.ao_screen);
+            sc[k].l = S.l;
+            sc[k].first_ao = S.first_ao;
+            sc[k].cls = (int)(std::lower_bound(cls.begin(), cls.end(), std::make_pair(S.l, S.nprim)) - cls.begin());
+            sc[k].pad = 0;
+        }
+    }
+    // workspace: order | masks | counts | leaf of every block | shell table
+    auto align = [](size_t b) { return (b + 255) / 256 * 256; };
+    const size_t b_order = align(sizeof(int) * (size_t)n), b_mask = align(sizeof(unsigned long long) * (size_t)nb * nw),
+                 b_cnt = align(2 * sizeof(int) * (size_t)nb), b_leaf = align(sizeof(int) * (size_t)nb),
+                 b_sc = align(sizeof(ScreenShell) * (size_t)nsh);
+    DeviceBuf ws;
+    int rc = ws.alloc(b_order + b_mask + b_cnt + b_leaf + b_sc);
+    if (rc) return rc;
+    int* d_order = ws.as<int>();
+    unsigned long long* d_masks = reinterpret_cast<unsigned long long*>(ws.as<char>() + b_order);
+    int* d_counts = reinterpret_cast<int*>(ws.as<char>() + b_order + b_mask);
+    int* d_leaf = reinterpret_cast<int*>(ws.as<char>() + b_order + b_mask + b_cnt);
+    ScreenShell* d_sc = reinterpret_cast<ScreenShell*>(ws.as<char>() + b_order + b_mask + b_cnt + b_leaf);
+    std::vector<int> order;
+    if (c.opts.precision == PDFXC_FP64) {
+        rc = device_partition(n, c.d_grid, d_order, c.stream);
+        if (rc) return rc;
+    } else {
+        if (int e = ensure_host_grid(c)) return e;
+        partition_points(c, order);
+        PDFXC_HIP(hipMemcpyAsync(d_order, order.data(), sizeof(int) * (size_t)n, hipMemcpyHostToDevice, c.stream));
+    }
+    PDFXC_HIP(hipMemcpyAsync(d_sc, sc.data(), sizeof(ScreenShell) * (size_t)nsh, hipMemcpyHostToDevice, c.stream));
+    rc = launch_screen_blocks(nb, n, c.d_grid, d_order, nsh, d_sc, nw, d_masks, d_counts, c.stream);
+    if (rc) return rc;
+    std::vector<int> counts(2 * (size_t)nb);
+    PDFXC_HIP(hipMemcpyAsync(counts.data(), d_counts, 2 * sizeof(int) * (size_t)nb, hipMemcpyDeviceToHost, c.stream));
+    PDFXC_HIP(hipStreamSynchronize(c.stream));
+
+    // launch order: descending cost (longest blocks first)
+    auto padded = [](int nao) { return std::max(kColPad, (nao + kColPad - 1) / kColPad * kColPad); };
+    auto npts_of = [&](int leaf) { return (int)std::min<int64_t>(kBlockPts, n - (int64_t)leaf * kBlockPts); };
+    std::vector<int> lorder(nb);
+    std::vector<int64_t> cost(nb);
+    for (int b = 0; b < nb; ++b) {
+        const int64_t ldn = padded(counts[2 * b + 1]);
+        cost[b] = npts_of(b) * ldn * ldn;
+    }
+    std::iota(lorder.begin(), lorder.end(), 0);
+    std::stable_sort(lorder.begin(), lorder.end(), [&](int a, int b) { return cost[a] > cost[b]; });
+    c.blocks.assign(nb, BlockDesc());
     c.n_slots = (int64_t)nb * kBlockPts;
-    c.slot_of_point.assign(c.n_pts, -1);
-    std::vector<double> pts(4 * (size_t)c.n_slots, 0.0);
     c.flops = 0.0;
     double sum_nao = 0.0;
     c.max_nao = 0;
+    int64_t sh0 = 0, col0 = 0;
     for (int li = 0; li < nb; ++li) {
-        const Tmp& t = tmp[lorder[li]];
+        const int leaf = lorder[li];
         BlockDesc& B = c.blocks[li];
         B.pt_begin = li * kBlockPts;
-        B.npts = (int)(t.hi - t.lo);
-        B.shell_begin = (int)c.block_shells.size();
-        B.nshell = (int)t.sh.size();
-        B.col_begin = (int)c.block_cols.size();
-        B.nao = t.nao;
-        B.ldn = std::max(kColPad, (t.nao + kColPad - 1) / kColPad * kColPad);
+        B.npts = npts_of(leaf);
+        B.shell_begin = (int)sh0;
+        B.nshell = counts[2 * leaf];
+        B.col_begin = (int)col0;
+        B.nao = counts[2 * leaf + 1];
+        B.ldn = padded(B.nao);
         B.ldp = c.n_aos;  // one molecule: P and K start at 0
         B.poff = 0;
         B.psoff = 0;
@@ -586,40 +652,28 @@ static int build_blocks_impl(Context& c) {
                       " AOs; more than 1024 per block is not supported (raise ao_screen)");
             return PDFXC_ERR_UNSUPPORTED;
         }
-        int col = 0;
-        for (int s : t.sh) {
-            c.block_shells.push_back(s);
-            c.block_shell_col.push_back(col);
-            const Shell& S = c.shells[s];
-            for (int m = 0; m < 2 * S.l + 1; ++m) c.block_cols.push_back(S.first_ao + m);
-            col += 2 * S.l + 1;
-        }
-        // evaluation order: shells of equal (l, nprim) side by side, so that a
-        // wave's lanes mostly run the same code path
-        {
-            std::vector<int> so(B.nshell);
-            std::iota(so.begin(), so.end(), 0);
-            std::stable_sort(so.begin(), so.end(), [&](int a, int b) {
-                const Shell& A = c.shells[t.sh[a]];
-                const Shell& Bs = c.shells[t.sh[b]];
-                return A.l != Bs.l ? A.l < Bs.l : A.nprim < Bs.nprim;
-            });
-            c.block_sorder.insert(c.block_sorder.end(), so.begin(), so.end());
-        }
-        for (int k = 0; k < kBlockPts; ++k) {
-            const int64_t slot = (int64_t)li * kBlockPts + k;
-            const int64_t p = order[t.lo + std::min<int64_t>(k, B.npts - 1)];
-            pts[slot] = c.gx[p];
-            pts[c.n_slots + slot] = c.gy[p];
-            pts[2 * c.n_slots + slot] = c.gz[p];
-            pts[3 * c.n_slots + slot] = (k < B.npts) ? c.gw[p] : 0.0;
-            if (k < B.npts) c.slot_of_point[p] = slot;
-        }
+        sh0 += B.nshell;
+        col0 += B.nao;
         c.flops += 4.0 * B.npts * (double)B.nao * B.nao;
         sum_nao += B.nao;
         c.max_nao = std::max(c.max_nao, B.nao);
     }
     c.mean_nao = nb ? sum_nao / nb : 0.0;
+    c.n_block_shells = sh0;
+    c.n_block_cols = col0;
+    rc = dalloc(&c.d_pts, 4 * (size_t)c.n_slots);
+    if (rc == PDFXC_OK) rc = dalloc(&c.d_slot_of_point, (size_t)n);
+    if (rc == PDFXC_OK) rc = dalloc(&c.d_blocks, c.blocks.size());
+    if (rc == PDFXC_OK) rc = dalloc(&c.d_block_shells, (size_t)sh0);
+    if (rc == PDFXC_OK) rc = dalloc(&c.d_block_cols, (size_t)col0);
+    if (rc == PDFXC_OK) rc = dalloc(&c.d_block_shell_col, (size_t)sh0);
+    if (rc == PDFXC_OK) rc = dalloc(&c.d_block_sorder, (size_t)sh0);
+    if (rc) return rc;
+    PDFXC_HIP(hipMemcpyAsync(c.d_blocks, c.blocks.data(), sizeof(BlockDesc) * (size_t)nb, hipMemcpyHostToDevice, c.stream));
+    PDFXC_HIP(hipMemcpyAsync(d_leaf, lorder.data(), sizeof(int) * (size_t)nb, hipMemcpyHostToDevice, c.stream));
+    rc = launch_fill_blocks(c, d_order, d_leaf, nw, ncls, d_sc, d_masks);
+    if (rc) return rc;
+    PDFXC_HIP(hipStreamSynchronize(c.stream));
 
     // k_rho work lists by template class: ldn <= 128 (64 points per
     // workgroup), <= 256 (64 when the plane fits in LDS: class 4, else 32),
@@ -680,15 +734,36 @@ static int build_blocks_impl(Context& c) {
             int I = 0;
             while ((I + 1) * (I + 2) / 2 <= w.t1 - 1) ++I;
             w.ncols = 16 * (I + 1);
-            int nsh = 0;
-            while (nsh < B.nshell && c.block_shell_col[B.shell_begin + nsh] < w.ncols) ++nsh;
-            w.nsh = nsh;
+            w.nsh = w.ps = 0;
+            kw[cls].push_back(w);
+        }
+    }
+    // the shells of every item, counted where the block lists are
+    const size_t n_items = kw[0].size() + kw[1].size();
+    std::vector<int> item_nsh(n_items);
+    {
+        DeviceBuf items;
+        if (int e = items.alloc((sizeof(KWork) + sizeof(int)) * n_items)) return e;
+        KWork* d_items = items.as<KWork>();
+        int* d_nsh = reinterpret_cast<int*>(d_items + n_items);
+        for (int cls = 0, at = 0; cls < 2; at += (int)kw[cls].size(), ++cls)
+            if (!kw[cls].empty())
+                PDFXC_HIP(hipMemcpyAsync(d_items + at, kw[cls].data(), sizeof(KWork) * kw[cls].size(),
+                                         hipMemcpyHostToDevice, c.stream));
+        if (int e = launch_item_shells(c, (int)n_items, d_items, d_nsh)) return e;
+        PDFXC_HIP(hipMemcpyAsync(item_nsh.data(), d_nsh, sizeof(int) * n_items, hipMemcpyDeviceToHost, c.stream));
+        PDFXC_HIP(hipStreamSynchronize(c.stream));
+    }
+    for (int cls = 0, at = 0; cls < 2; ++cls)
+        for (KWork& w : kw[cls]) {
+            const int nsh_item = item_nsh[at++];
+            w.nsh = nsh_item;
             size_t lds = 0;
             const int LD = (w.ncols & 31) ? w.ncols : w.ncols + 16;
             for (int ps = 16; ps >= 4; ps /= 2) {
                 w.ps = ps;
-                lds = sizeof(double) * (4 * (size_t)ps * LD + (size_t)nsh * RS) +
-                      sizeof(int) * (size_t)(w.ncols + 2 * nsh);
+                lds = sizeof(double) * (4 * (size_t)ps * LD + (size_t)nsh_item * RS) +
+                      sizeof(int) * (size_t)(w.ncols + 2 * nsh_item);
                 if (lds <= (size_t)kMaxDynLds) break;
             }
             if (lds > (size_t)kMaxDynLds) {
@@ -696,9 +771,7 @@ static int build_blocks_impl(Context& c) {
                 return PDFXC_ERR_UNSUPPORTED;
             }
             klds[cls] = std::max(klds[cls], lds);
-            kw[cls].push_back(w);
         }
-    }
     std::vector<KWork> kall;
     c.kmat_launches.clear();
     for (int cls = 0; cls < 2; ++cls) {
@@ -728,6 +801,7 @@ static int build_blocks_impl(Context& c) {
     c.kg_masks.clear();
     if (c.opts.precision != PDFXC_FP64) {
         const int S = prec_slices(c.opts.precision);
+        if (int e = ensure_host_lists(c)) return e;
         c.sblocks.resize(nb);
         std::vector<int> ipos(c.n_aos);
         for (int q = 0; q < c.n_aos; ++q) ipos[c.split_perm[q]] = q;
@@ -998,13 +1072,6 @@ static int build_blocks_impl(Context& c) {
     }
 
     // device buffers
-    free_grid_buffers(&c);
-    int rc = dalloc(&c.d_pts, pts.size());
-    if (rc == PDFXC_OK) rc = dalloc(&c.d_blocks, c.blocks.size());
-    if (rc == PDFXC_OK) rc = dalloc(&c.d_block_shells, c.block_shells.size());
-    if (rc == PDFXC_OK) rc = dalloc(&c.d_block_cols, c.block_cols.size());
-    if (rc == PDFXC_OK) rc = dalloc(&c.d_block_shell_col, c.block_shell_col.size());
-    if (rc == PDFXC_OK) rc = dalloc(&c.d_block_sorder, c.block_sorder.size());
     if (rc == PDFXC_OK) rc = dalloc(&c.d_rho_work, rho_work.size());
     if (rc == PDFXC_OK) rc = dalloc(reinterpret_cast<char**>(&c.d_k_work), kall.size() * sizeof(KWork));
     if (rc == PDFXC_OK) rc = dalloc(&c.d_coef, 4 * (size_t)c.n_slots);
@@ -1026,16 +1093,8 @@ static int build_blocks_impl(Context& c) {
     }
     if (rc != PDFXC_OK) return rc;
     auto up = [](void* d, const void* h, size_t n) { return hipMemcpy(d, h, n, hipMemcpyHostToDevice); };
-    PDFXC_HIP(up(c.d_pts, pts.data(), pts.size() * sizeof(double)));
-    PDFXC_HIP(up(c.d_blocks, c.blocks.data(), c.blocks.size() * sizeof(BlockDesc)));
     PDFXC_HIP(up(c.d_rho_work, rho_work.data(), rho_work.size() * sizeof(int)));
     PDFXC_HIP(up(c.d_k_work, kall.data(), kall.size() * sizeof(KWork)));
-    if (!c.block_shells.empty()) {
-        PDFXC_HIP(up(c.d_block_shells, c.block_shells.data(), c.block_shells.size() * sizeof(int)));
-        PDFXC_HIP(up(c.d_block_shell_col, c.block_shell_col.data(), c.block_shell_col.size() * sizeof(int)));
-        PDFXC_HIP(up(c.d_block_cols, c.block_cols.data(), c.block_cols.size() * sizeof(int)));
-        PDFXC_HIP(up(c.d_block_sorder, c.block_sorder.data(), c.block_sorder.size() * sizeof(int)));
-    }
     if (c.opts.precision != PDFXC_FP64) {
         PDFXC_HIP(up(c.d_sblocks, c.sblocks.data(), c.sblocks.size() * sizeof(SplitBlock)));
         PDFXC_HIP(up(c.d_chunks, c.chunks.data(), c.chunks.size() * sizeof(int)));
@@ -1052,9 +1111,10 @@ static int build_blocks_impl(Context& c) {
             PDFXC_HIP(up(c.d_kg_masks, c.kg_masks.data(), c.kg_masks.size() * sizeof(unsigned)));
         }
     }
-    PDFXC_HIP(hipMemset(c.d_coef, 0, 4 * (size_t)c.n_slots * sizeof(double)));
-    PDFXC_HIP(hipMemset(c.d_rho, 0, 4 * (size_t)c.n_slots * sizeof(double)));
-    PDFXC_HIP(hipMemset(c.d_eblock, 0, (size_t)(c.n_slots + 255) / 256 * sizeof(double)));
+    PDFXC_HIP(hipMemsetAsync(c.d_coef, 0, 4 * (size_t)c.n_slots * sizeof(double), c.stream));
+    PDFXC_HIP(hipMemsetAsync(c.d_rho, 0, 4 * (size_t)c.n_slots * sizeof(double), c.stream));
+    PDFXC_HIP(hipMemsetAsync(c.d_eblock, 0, (size_t)(c.n_slots + 255) / 256 * sizeof(double), c.stream));
+    PDFXC_HIP(hipStreamSynchronize(c.stream));
     // host copies of the work lists (a batch concatenates them)
     c.h_rho_work = std::move(rho_work);
     c.h_k_work = std::move(kall);
@@ -1280,6 +1340,87 @@ static void orientation(int na, const int* Z, const double* xyz, double O[9]) {
     }
 }
 
+int ensure_host_grid(Context& c) {
+    if ((int64_t)c.gx.size() == c.n_pts) return PDFXC_OK;
+    std::vector<double>* g[4] = {&c.gx, &c.gy, &c.gz, &c.gw};
+    for (int q = 3; q >= 0; --q) {
+        g[q]->resize((size_t)c.n_pts);
+        PDFXC_HIP(hipMemcpyAsync(g[q]->data(), c.d_grid + q * c.n_pts, sizeof(double) * (size_t)c.n_pts,
+                                 hipMemcpyDeviceToHost, c.stream));
+    }
+    PDFXC_HIP(hipStreamSynchronize(c.stream));
+    return PDFXC_OK;
+}
+
+int ensure_host_lists(Context& c) {
+    if ((int64_t)c.block_cols.size() == c.n_block_cols && (int64_t)c.block_shells.size() == c.n_block_shells)
+        return PDFXC_OK;
+    auto get = [&](std::vector<int>& v, const int* d, int64_t n) {
+        v.resize((size_t)n);
+        return n ? hipMemcpyAsync(v.data(), d, sizeof(int) * (size_t)n, hipMemcpyDeviceToHost, c.stream) : hipSuccess;
+    };
+    PDFXC_HIP(get(c.block_shell_col, c.d_block_shell_col, c.n_block_shells));
+    PDFXC_HIP(get(c.block_sorder, c.d_block_sorder, c.n_block_shells));
+    PDFXC_HIP(get(c.block_shells, c.d_block_shells, c.n_block_shells));
+    PDFXC_HIP(get(c.block_cols, c.d_block_cols, c.n_block_cols));
+    PDFXC_HIP(hipStreamSynchronize(c.stream));
+    return PDFXC_OK;
+}
+
+int ensure_host_slots(Context& c) {
+    if ((int64_t)c.slot_of_point.size() == c.n_pts) return PDFXC_OK;
+    std::vector<int> s((size_t)c.n_pts);
+    PDFXC_HIP(hipMemcpyAsync(s.data(), c.d_slot_of_point, sizeof(int) * (size_t)c.n_pts, hipMemcpyDeviceToHost, c.stream));
+    PDFXC_HIP(hipStreamSynchronize(c.stream));
+    c.slot_of_point.assign(s.begin(), s.end());
+    return PDFXC_OK;
+}
+
+// A buffer for a new grid's columns; the old grid and its buffers go first.
+static int alloc_grid(Context& c, int64_t n, double** d_grid) {
+    reset_grid(c);
+    return dalloc(d_grid, 4 * (size_t)n);
+}
+
+// Takes over d_grid (n x 4 columns, written on c.stream) as the context's grid
+// and builds its blocks; a grid with a value that is not finite is refused and
+// leaves the context without one.
+static int set_device_grid(Context& c, int64_t n, double* d_grid, const char* who) {
+    dfree(c.d_grid);
+    c.d_grid = d_grid;
+    c.gx.clear();
+    c.gy.clear();
+    c.gz.clear();
+    c.gw.clear();
+    c.n_pts = n;
+    c.gen_atom.clear();
+    c.grid_partition = PDFXC_PARTITION_BECKE;
+    c.grid_size_adjust = 1;
+    unsigned long long first = (unsigned long long)n;
+    {
+        // the energy accumulator's 8 bytes hold the answer
+        unsigned long long* d_first = reinterpret_cast<unsigned long long*>(c.d_E);
+        hipError_t e = hipMemcpyAsync(d_first, &first, sizeof(first), hipMemcpyHostToDevice, c.stream);
+        int rc = e == hipSuccess ? device_check_finite(n, d_grid, d_first, c.stream) : hip_fail(e, who);
+        if (rc == PDFXC_OK) {
+            e = hipMemcpyAsync(&first, d_first, sizeof(first), hipMemcpyDeviceToHost, c.stream);
+            if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
+            if (e != hipSuccess) rc = hip_fail(e, who);
+        }
+        if (rc != PDFXC_OK) {
+            const std::string msg = g_last_error;
+            reset_grid(c);
+            set_error(msg);
+            return rc;
+        }
+    }
+    if (first < (unsigned long long)n) {
+        reset_grid(c);
+        return arg_error(std::string(who) + ": non-finite grid value at point " + std::to_string(first));
+    }
+    return build_blocks(c);
+}
+
 // [n][kNear]: each atom's nearest atoms by distance, itself first; -1 past the last
 static std::vector<int> near_atoms(int n, const double* xyz) {
     std::vector<int> out((size_t)n * kNear, -1);
@@ -1325,20 +1466,18 @@ int pdfxc_set_grid(pdfxc_ctx* ctx, int64_t n_pts, const double* x, const double*
         reset_grid(*c);
         return arg_error("pdfxc_set_grid: more than 2^31 points");
     }
-    for (int64_t i = 0; i < n_pts; ++i)
-        if (!std::isfinite(x[i]) || !std::isfinite(y[i]) || !std::isfinite(z[i]) || !std::isfinite(w[i])) {
-            reset_grid(*c);
-            return arg_error("pdfxc_set_grid: non-finite grid value at point " + std::to_string(i));
+    double* d_grid = nullptr;
+    if (int rc = alloc_grid(*c, n_pts, &d_grid)) return rc;
+    const double* col[4] = {x, y, z, w};
+    for (int q = 0; q < 4; ++q) {
+        const hipError_t e = hipMemcpyAsync(d_grid + q * n_pts, col[q], sizeof(double) * (size_t)n_pts,
+                                            hipMemcpyHostToDevice, c->stream);
+        if (e != hipSuccess) {
+            dfree(d_grid);
+            return hip_fail(e, "pdfxc_set_grid: upload");
         }
-    c->n_pts = n_pts;
-    c->gen_atom.clear();
-    c->grid_partition = PDFXC_PARTITION_BECKE;
-    c->grid_size_adjust = 1;
-    c->gx.assign(x, x + n_pts);
-    c->gy.assign(y, y + n_pts);
-    c->gz.assign(z, z + n_pts);
-    c->gw.assign(w, w + n_pts);
-    return build_blocks(*c);
+    }
+    return set_device_grid(*c, n_pts, d_grid, "pdfxc_set_grid");
 }
 
 int pdfxc_get_grid(pdfxc_ctx* ctx, double* x, double* y, double* z, double* w) {
@@ -1348,10 +1487,12 @@ int pdfxc_get_grid(pdfxc_ctx* ctx, double* x, double* y, double* z, double* w) {
         set_error("pdfxc_get_grid: no grid");
         return PDFXC_ERR_NO_GRID;
     }
-    if (x) std::copy(c->gx.begin(), c->gx.end(), x);
-    if (y) std::copy(c->gy.begin(), c->gy.end(), y);
-    if (z) std::copy(c->gz.begin(), c->gz.end(), z);
-    if (w) std::copy(c->gw.begin(), c->gw.end(), w);
+    double* col[4] = {x, y, z, w};
+    for (int q = 0; q < 4; ++q)
+        if (col[q])
+            PDFXC_HIP(hipMemcpyAsync(col[q], c->d_grid + q * c->n_pts, sizeof(double) * (size_t)c->n_pts,
+                                     hipMemcpyDeviceToHost, c->stream));
+    PDFXC_HIP(hipStreamSynchronize(c->stream));
     return PDFXC_OK;
 }
 
@@ -1770,15 +1911,17 @@ static int build_host(Context* c, int xc, int nspin, const double* const* P_pack
     *E_xc = E;
     if (rho_out) {
         const int stride = 4 * nspin;
-        std::vector<double> rs(4 * (size_t)c->n_slots);
-        for (int sp = 0; sp < nspin; ++sp) {
-            PDFXC_HIP(hipMemcpy(rs.data(), sp ? c->d_rho_b : c->d_rho, rs.size() * sizeof(double),
-                                hipMemcpyDeviceToHost));
-            for (int64_t p = 0; p < c->n_pts; ++p) {
-                const int64_t sl = c->slot_of_point[p];
-                for (int q = 0; q < 4; ++q) rho_out[stride * p + 4 * sp + q] = rs[4 * sl + q];
-            }
+        const size_t n_out = (size_t)stride * (size_t)c->n_pts;
+        if (c->n_rho_out < n_out) {  // kept with the grid: rho is asked for again with every iteration
+            dfree(c->d_rho_out);
+            c->n_rho_out = 0;
+            if (int e = dalloc(&c->d_rho_out, n_out)) return e;
+            c->n_rho_out = n_out;
         }
+        for (int sp = 0; sp < nspin; ++sp)
+            if (int e = launch_gather_points(*c, sp ? c->d_rho_b : c->d_rho, c->d_rho_out, stride, 4 * sp)) return e;
+        PDFXC_HIP(hipMemcpyAsync(rho_out, c->d_rho_out, sizeof(double) * n_out, hipMemcpyDeviceToHost, c->stream));
+        PDFXC_HIP(hipStreamSynchronize(c->stream));
     }
     return PDFXC_OK;
 }
@@ -1906,13 +2049,10 @@ int pdfxc_gradient_rks(pdfxc_ctx* ctx, int functional, int n_atoms, const int* Z
             return arg_error("pdfxc_gradient_rks: the centre of AO " + std::to_string(c->shells[k].first_ao) +
                              " is not at any atom");
     }
-    std::vector<int> slot_atom((size_t)c->n_slots, -1);
-    for (int64_t p = 0; p < c->n_pts; ++p) {
-        const int a = point_atom ? point_atom[p] : c->gen_atom[p];
-        if (a < 0 || a >= na || Z[a] <= 0)
+    const int* pt_atom = point_atom ? point_atom : c->gen_atom.data();
+    for (int64_t p = 0; p < c->n_pts; ++p)
+        if (pt_atom[p] < 0 || pt_atom[p] >= na)
             return arg_error("pdfxc_gradient_rks: point " + std::to_string(p) + " has no valid atom");
-        slot_atom[c->slot_of_point[p]] = a;
-    }
     // Becke table (x, y, z, Z | 1/R_mn | a_mn) as the grid generator builds it
     std::vector<double> at(4 * (size_t)na + 2 * (size_t)na * na, 0.0);
     for (int m = 0; m < na; ++m) {
@@ -1952,10 +2092,8 @@ int pdfxc_gradient_rks(pdfxc_ctx* ctx, int functional, int n_atoms, const int* Z
         LaunchRange g = r;
         g.lds = 0;
         if (g.cls == 4) g.cls = 1;  // the 64-point rho class of ldn <= 256 blocks: the gradient's ldn <= 256 kernel
-        std::vector<int> ids(r.count);
-        PDFXC_HIP(hipMemcpy(ids.data(), c->d_rho_work + r.offset, sizeof(int) * r.count, hipMemcpyDeviceToHost));
-        for (int b : ids) {
-            const BlockDesc& B = c->blocks[b];
+        for (int k = 0; k < r.count; ++k) {
+            const BlockDesc& B = c->blocks[c->h_rho_work[r.offset + k]];
             const size_t lds = sizeof(double) * (2 * (size_t)B.ldn * 16 + (size_t)B.nshell * RS + 3 * (size_t)na) +
                                sizeof(int) * (size_t)(B.ldn + 3 * B.nshell);
             if (g.cls > 2 || lds > (size_t)kMaxDynLds) {
@@ -1968,10 +2106,11 @@ int pdfxc_gradient_rks(pdfxc_ctx* ctx, int functional, int n_atoms, const int* Z
         gl.push_back(g);
     }
     const std::vector<int> near = near_atoms(na, xyz);
-    int *d_shat = nullptr, *d_slat = nullptr, *d_near = nullptr;
+    int *d_shat = nullptr, *d_slat = nullptr, *d_near = nullptr, *d_ptat = nullptr;
     double *d_at = nullptr, *d_ewf = nullptr, *d_g = nullptr;
     int rc = dalloc(&d_shat, shell_atom.size());
-    if (rc == PDFXC_OK) rc = dalloc(&d_slat, slot_atom.size());
+    if (rc == PDFXC_OK) rc = dalloc(&d_slat, (size_t)c->n_slots);
+    if (rc == PDFXC_OK) rc = dalloc(&d_ptat, (size_t)c->n_pts);
     if (rc == PDFXC_OK) rc = dalloc(&d_near, near.size());
     if (rc == PDFXC_OK) rc = dalloc(&d_at, at.size());
     if (rc == PDFXC_OK) rc = dalloc(&d_ewf, (size_t)c->n_slots);
@@ -1979,11 +2118,15 @@ int pdfxc_gradient_rks(pdfxc_ctx* ctx, int functional, int n_atoms, const int* Z
     hipError_t e = hipSuccess;
     if (rc == PDFXC_OK) {
         e = hipMemcpy(d_shat, shell_atom.data(), sizeof(int) * shell_atom.size(), hipMemcpyHostToDevice);
-        if (e == hipSuccess) e = hipMemcpy(d_slat, slot_atom.data(), sizeof(int) * slot_atom.size(), hipMemcpyHostToDevice);
+        // atoms to the slots (-1, all bits, in the repeated points of a partial block)
+        if (e == hipSuccess) e = hipMemsetAsync(d_slat, 0xff, sizeof(int) * (size_t)c->n_slots, c->stream);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(d_ptat, pt_atom, sizeof(int) * (size_t)c->n_pts, hipMemcpyHostToDevice, c->stream);
         if (e == hipSuccess) e = hipMemcpy(d_near, near.data(), sizeof(int) * near.size(), hipMemcpyHostToDevice);
         if (e == hipSuccess) e = hipMemcpy(d_at, at.data(), sizeof(double) * at.size(), hipMemcpyHostToDevice);
-        if (e == hipSuccess) e = hipMemset(d_g, 0, sizeof(double) * 6 * (size_t)na);
+        if (e == hipSuccess) e = hipMemsetAsync(d_g, 0, sizeof(double) * 6 * (size_t)na, c->stream);
         if (e != hipSuccess) rc = hip_fail(e, "pdfxc_gradient_rks: upload");
+        if (rc == PDFXC_OK) rc = launch_scatter_atoms(*c, d_ptat, d_slat);
     }
     if (rc == PDFXC_OK) {
         double* H = c->h_pinned;
@@ -2015,6 +2158,7 @@ int pdfxc_gradient_rks(pdfxc_ctx* ctx, int functional, int n_atoms, const int* Z
     }
     dfree(d_shat);
     dfree(d_slat);
+    dfree(d_ptat);
     dfree(d_near);
     dfree(d_at);
     dfree(d_ewf);
@@ -2041,22 +2185,13 @@ int pdfxc_set_tuning(pdfxc_ctx* ctx, const pdfxc_tuning* t) {
         t->split_k_patches == prev.split_k_patches && t->split_k_group == prev.split_k_group)
         return PDFXC_OK;  // same blocks and work lists (the launch mode is chosen per launch)
     PDFXC_HIP(hipStreamSynchronize(c->stream));
-    // a shape the grid's blocks do not fit drops the grid (build_blocks): put
-    // the grid back with the previous shape and report the failure
-    const std::vector<double> gx = c->gx, gy = c->gy, gz = c->gz, gw = c->gw;
-    const std::vector<int> gen_atom = c->gen_atom;
-    const int64_t n_pts = c->n_pts;
-    const int rc = build_blocks(*c);
+    // a shape the grid's blocks do not fit: build them with the previous shape
+    // again and report the failure
+    const int rc = build_blocks_impl(*c);
     if (rc == PDFXC_OK) return rc;
     const std::string msg = g_last_error;
     c->tune = prev;
-    c->n_pts = n_pts;
-    c->gx = gx;
-    c->gy = gy;
-    c->gz = gz;
-    c->gw = gw;
-    c->gen_atom = gen_atom;
-    if (build_blocks(*c) != PDFXC_OK) c->tune = prev;
+    (void)build_blocks(*c);
     set_error(msg);
     return rc;
 }
@@ -2147,13 +2282,21 @@ int pdfxc_density_at_points(pdfxc_ctx* ctx, const double* P_packed, int64_t n, c
                               &o);
     if (rc) return rc;
     Context* t = reinterpret_cast<Context*>(th);
-    std::vector<double> X(n), Y(n), Zc(n), W(n, 1.0);
-    for (int64_t i = 0; i < n; ++i) {
-        X[i] = xyz[3 * i];
-        Y[i] = xyz[3 * i + 1];
-        Zc[i] = xyz[3 * i + 2];
+    if (n > ((int64_t)1 << 31) - kBlockPts) {
+        rc = arg_error("pdfxc_set_grid: more than 2^31 points");
     }
-    rc = pdfxc_set_grid(th, n, X.data(), Y.data(), Zc.data(), W.data());
+    // one buffer for the points on their way in and for (rho, grad rho) on its way out
+    DeviceBuf io;
+    if (rc == PDFXC_OK) rc = io.alloc(sizeof(double) * 4 * (size_t)n);
+    double* d_grid = nullptr;
+    if (rc == PDFXC_OK) rc = alloc_grid(*t, n, &d_grid);
+    if (rc == PDFXC_OK) {
+        const hipError_t e = hipMemcpyAsync(io.p, xyz, sizeof(double) * 3 * (size_t)n, hipMemcpyHostToDevice, t->stream);
+        rc = e == hipSuccess ? launch_points_to_grid(n, io.as<double>(), d_grid, t->stream)
+                             : hip_fail(e, "pdfxc_density_at_points: points upload");
+        if (rc == PDFXC_OK) rc = set_device_grid(*t, n, d_grid, "pdfxc_set_grid");
+        else dfree(d_grid);
+    }
     if (rc == PDFXC_OK) {
         double* H = t->h_pinned;
         for (int r = 0, k = 0; r < N; ++r)
@@ -2166,16 +2309,16 @@ int pdfxc_density_at_points(pdfxc_ctx* ctx, const double* P_packed, int64_t n, c
     }
     if (rc == PDFXC_OK) rc = run_rho(t, t->d_P, t->d_rho);
     if (rc == PDFXC_OK) {
-        std::vector<double> rs(4 * (size_t)t->n_slots);
-        hipError_t e = hipStreamSynchronize(t->stream);
-        if (e == hipSuccess) e = hipMemcpy(rs.data(), t->d_rho, rs.size() * sizeof(double), hipMemcpyDeviceToHost);
+        // columns rho | grad rho x 3: the first alone unless the gradient is asked for
+        rc = launch_gather_density(*t, t->d_rho, io.as<double>(), grad_rho != nullptr);
+        hipError_t e = hipSuccess;
+        if (rc == PDFXC_OK)
+            e = hipMemcpyAsync(rho, io.p, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost, t->stream);
+        if (rc == PDFXC_OK && e == hipSuccess && grad_rho)
+            e = hipMemcpyAsync(grad_rho, io.as<double>() + n, sizeof(double) * 3 * (size_t)n, hipMemcpyDeviceToHost,
+                               t->stream);
+        if (rc == PDFXC_OK && e == hipSuccess) e = hipStreamSynchronize(t->stream);
         if (e != hipSuccess) rc = hip_fail(e, "pdfxc_density_at_points: download");
-        for (int64_t i = 0; rc == PDFXC_OK && i < n; ++i) {
-            const int64_t sl = t->slot_of_point[i];
-            rho[i] = rs[4 * sl];
-            if (grad_rho)
-                for (int d = 0; d < 3; ++d) grad_rho[3 * i + d] = rs[4 * sl + 1 + d];
-        }
     }
     pdfxc_ctx_destroy(th);
     return rc;
@@ -2369,6 +2512,13 @@ int pdfxc_batch_create(pdfxc_batch** out, int n_mol, pdfxc_ctx* const* ctxs) {
         const Context* c0 = reinterpret_cast<const Context*>(ctxs[0]);
         if (c->opts.precision != c0->opts.precision || c->opts.density_cutoff != c0->opts.density_cutoff)
             return arg_error("pdfxc_batch_create: contexts differ in precision or density cut-off");
+    }
+    // the batch concatenates host copies of the contexts' grids, lists and slots
+    for (int i = 0; i < n_mol; ++i) {
+        Context& c = *reinterpret_cast<Context*>(ctxs[i]);
+        if (int rc = ensure_host_grid(c)) return rc;
+        if (int rc = ensure_host_lists(c)) return rc;
+        if (int rc = ensure_host_slots(c)) return rc;
     }
     Batch* b = new Batch();
     Context& m = b->m;

@@ -110,6 +110,14 @@ struct KGWork {
     int group, q0, q1, c0, c1, k0, nbuf, pad;
 };
 
+// What block screening needs of a shell: it is dropped from a block whose
+// box lies further than cut, or where exp0 d^2 > 30 (cls: rank of (l, nprim)).
+struct ScreenShell {
+    double center[3];
+    double exp0, cut;
+    int l, first_ao, cls, pad;
+};
+
 struct DeviceShell {
     double cx, cy, cz;
     int l, nprim;
@@ -128,8 +136,10 @@ struct Context {
     hipStream_t stream = nullptr;
     hipEvent_t ev[6] = {};
 
-    // grid (host copies in caller order)
+    // grid in caller order: x, y, z, w columns on the device; host copies only
+    // where a caller needs them (ensure_host_grid)
     int64_t n_pts = 0;
+    double* d_grid = nullptr;
     std::vector<double> gx, gy, gz, gw;
     std::vector<int> gen_atom;  // atom of each point when pdfxc_generate_grid made the grid
     int grid_partition = 0;     // partition weights of a generated grid (PDFXC_PARTITION_*)
@@ -137,6 +147,9 @@ struct Context {
 
     // blocks
     std::vector<BlockDesc> blocks;     // launch order (descending cost)
+    // host copies of the block lists and slots, made by ensure_host_lists and
+    // ensure_host_slots (a batch's are its own)
+    int64_t n_block_shells = 0, n_block_cols = 0;
     std::vector<int> block_shells;     // global shell ids per block
     std::vector<int> block_cols;       // global AO index per block column
     std::vector<int> block_shell_col;  // local first column of each block shell
@@ -153,6 +166,7 @@ struct Context {
     int rec_stride = 0;
     double* d_pts = nullptr;  // 4 x n_slots SoA: x, y, z, w
     int64_t n_slots = 0;
+    int* d_slot_of_point = nullptr;
     BlockDesc* d_blocks = nullptr;
     int* d_block_shells = nullptr;
     int* d_block_cols = nullptr;
@@ -164,6 +178,8 @@ struct Context {
     double* d_rho = nullptr;      // per slot: rho, grad rho (4)
     double* d_rho_b = nullptr;    // UKS: beta rho, grad rho per slot (allocated by the first UKS build)
     double* d_coef_b = nullptr;   // UKS: beta point terms
+    double* d_rho_out = nullptr;  // rho in the caller's order (allocated by the first build that returns it)
+    size_t n_rho_out = 0;
     double* d_eblock = nullptr;   // per 256 slots: energy (k_xc_points partial sums)
     double* d_P = nullptr;        // dense N x N
     double* d_K = nullptr;        // dense N x N
@@ -237,6 +253,29 @@ int hip_fail(hipError_t e, const char* what);
         hipError_t e_ = (call);                                  \
         if (e_ != hipSuccess) return ::pdfxc::hip_fail(e_, #call); \
     } while (0)
+
+// host copies of a context's grid, block lists and slots (no-ops once made)
+int ensure_host_grid(Context& c);
+int ensure_host_lists(Context& c);
+int ensure_host_slots(Context& c);
+
+// grid blocks (pdfxc_blocks.hip)
+// d_order: the points of block b are d_order[128 b ..); synchronises s
+int device_partition(int64_t n, const double* d_grid, int* d_order, hipStream_t s);
+// lowers *d_first to the first point with a non-finite value
+int device_check_finite(int64_t n, const double* d_grid, unsigned long long* d_first, hipStream_t s);
+int launch_screen_blocks(int nb, int64_t n, const double* d_grid, const int* d_order, int nsh,
+                         const ScreenShell* d_shells, int nw, unsigned long long* d_masks, int* d_counts,
+                         hipStream_t s);
+int launch_fill_blocks(Context& c, const int* d_order, const int* d_leaf, int nw, int ncls,
+                       const ScreenShell* d_shells, const unsigned long long* d_masks);
+int launch_item_shells(Context& c, int n, const KWork* d_work, int* d_nsh);
+// four values per point between the slots and the caller's order (row stride and offset of the latter)
+int launch_gather_points(Context& c, const double* d_slots, double* d_pts, int stride, int off);
+int launch_gather_density(Context& c, const double* d_slots, double* d_out, bool grad);  // rho [n] | grad [n][3]
+int launch_scatter_points(Context& c, const double* d_pts, double* d_slots);
+int launch_scatter_atoms(Context& c, const int* d_atom, int* d_slot_atom);
+int launch_points_to_grid(int64_t n, const double* d_xyz, double* d_grid, hipStream_t s);
 
 // kernel launchers (pdfxc_kernels.hip)
 int launch_rho(Context& c, const LaunchRange& r);

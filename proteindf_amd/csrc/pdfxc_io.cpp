@@ -119,21 +119,27 @@ static int write_matrix(const char* path, int type, int64_t rows, int64_t cols, 
 
 // caller-order rho (n_pts x 4) <-> the context's slots
 static int download_rho(Context* c, double* rho, const double* d_src) {
-    std::vector<double> rs(4 * (size_t)c->n_slots);
-    PDFXC_HIP(hipStreamSynchronize(c->stream));
-    PDFXC_HIP(hipMemcpy(rs.data(), d_src, rs.size() * sizeof(double), hipMemcpyDeviceToHost));
-    for (int64_t p = 0; p < c->n_pts; ++p)
-        for (int q = 0; q < 4; ++q) rho[4 * p + q] = rs[4 * c->slot_of_point[p] + q];
-    return PDFXC_OK;
+    const size_t bytes = sizeof(double) * 4 * (size_t)c->n_pts;
+    double* d = nullptr;
+    PDFXC_HIP(hipMalloc(reinterpret_cast<void**>(&d), bytes));
+    int rc = launch_gather_points(*c, d_src, d, 4, 0);
+    hipError_t e = rc == PDFXC_OK ? hipMemcpyAsync(rho, d, bytes, hipMemcpyDeviceToHost, c->stream) : hipSuccess;
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    (void)hipFree(d);
+    return rc != PDFXC_OK ? rc : e == hipSuccess ? PDFXC_OK : hip_fail(e, "rho download");
 }
 
 static int upload_rho(Context* c, const double* rho, double* d_dst) {
-    std::vector<double> rs(4 * (size_t)c->n_slots, 0.0);
-    for (int64_t p = 0; p < c->n_pts; ++p)
-        for (int q = 0; q < 4; ++q) rs[4 * c->slot_of_point[p] + q] = rho[4 * p + q];
-    PDFXC_HIP(hipStreamSynchronize(c->stream));
-    PDFXC_HIP(hipMemcpy(d_dst, rs.data(), rs.size() * sizeof(double), hipMemcpyHostToDevice));
-    return PDFXC_OK;
+    const size_t bytes = sizeof(double) * 4 * (size_t)c->n_pts;
+    double* d = nullptr;
+    PDFXC_HIP(hipMalloc(reinterpret_cast<void**>(&d), bytes));
+    int rc = PDFXC_OK;
+    hipError_t e = hipMemsetAsync(d_dst, 0, sizeof(double) * 4 * (size_t)c->n_slots, c->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(d, rho, bytes, hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess) rc = launch_scatter_points(*c, d, d_dst);
+    if (e == hipSuccess && rc == PDFXC_OK) e = hipStreamSynchronize(c->stream);
+    (void)hipFree(d);
+    return rc != PDFXC_OK ? rc : e == hipSuccess ? PDFXC_OK : hip_fail(e, "rho upload");
 }
 
 }  // namespace pdfxc
@@ -268,10 +274,7 @@ int pdfxc_save_grid_matrix(pdfxc_ctx* ctx, const char* path, int n_rho_cols) {
     }
     const int64_t n = c->n_pts, nc = 5 + n_rho_cols;
     std::vector<double> m((size_t)(n * nc));
-    std::copy(c->gx.begin(), c->gx.end(), m.begin());
-    std::copy(c->gy.begin(), c->gy.end(), m.begin() + n);
-    std::copy(c->gz.begin(), c->gz.end(), m.begin() + 2 * n);
-    std::copy(c->gw.begin(), c->gw.end(), m.begin() + 3 * n);
+    if (int rc = pdfxc_get_grid(ctx, m.data(), m.data() + n, m.data() + 2 * n, m.data() + 3 * n)) return rc;
     for (int64_t p = 0; p < n; ++p) m[4 * n + p] = c->gen_atom.size() == (size_t)n ? c->gen_atom[p] : -1.0;
     const int nspin = (n_rho_cols == 2 || n_rho_cols == 8) ? 2 : 1;
     const int per_spin = n_rho_cols / nspin;
