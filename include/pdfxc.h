@@ -218,6 +218,11 @@ int pdfxc_generate_grid_oriented(pdfxc_ctx* ctx, int n_atoms, const int* Z, cons
  * columns, n_pts each). */
 int pdfxc_get_grid(pdfxc_ctx* ctx, double* x, double* y, double* z, double* w);
 
+/* getWholeDensity (DfCalcGridX.cpp:2502-2537): the integrated rho_alpha (and,
+ * after a UKS build, rho_beta; n_beta may be null) of the context's last build
+ * through a host entry point. */
+int pdfxc_whole_density(pdfxc_ctx* ctx, double* n_alpha, double* n_beta);
+
 /* calcXCIntegForFockAndEnergy, RKS (DfCalcGridX.cpp:2280-2289 LDA, :2305-2315 GGA):
  * P_alpha_packed: N(N+1)/2 doubles, row r, column c <= r (RLHD order).
  * K_alpha_packed: same layout, ACCUMULATED into (the caller zeroes it).

@@ -140,7 +140,7 @@ class DfCalcGridX:
             self.ctx.load_grid_matrix(grid)
         else:
             self.ctx.set_grid(grid)
-        self._rho = None
+        self._whole_density = None
 
     @classmethod
     def from_pdfparam(cls, param, grid=None, ao_screen=0.0, precision=engine.PDFXC_FP64):
@@ -171,12 +171,12 @@ class DfCalcGridX:
         fid = functional.functional_id
         if len(args) == 3:
             build = self.ctx.build_rks_update if update else self.ctx.build_rks
-            E, _, rho = build(P_A, F_A, want_rho=keep_rho, functional=fid)
+            E, _, _ = build(P_A, F_A, functional=fid)
         else:
             build = self.ctx.build_uks_update if update else self.ctx.build_uks
-            E, _, _, rho = build(P_A, P_B, F_A, F_B, want_rho=keep_rho, functional=fid)
-        if keep_rho:
-            self._rho = rho
+            E, _, _, _ = build(P_A, P_B, F_A, F_B, functional=fid)
+        if keep_rho:  # the density stays on the device, its integral is summed by the build
+            self._whole_density = self.ctx.whole_density(1 if len(args) == 3 else 2)
         return E
 
     def saveGridMatrix(self, path, functional, uks=False):
@@ -187,12 +187,9 @@ class DfCalcGridX:
     def getWholeDensity(self):
         """Integrated rho_alpha (RKS), or (rho_alpha, rho_beta) after a UKS build
         (DfCalcGridX.cpp:2502-2537)."""
-        if self._rho is None:
+        if self._whole_density is None:
             raise RuntimeError("no density kept: call calcXCIntegForFockAndEnergy(..., keep_rho=True)")
-        w = self.grid[:, 3]
-        if self._rho.shape[1] == 8:
-            return float((w * self._rho[:, 0]).sum()), float((w * self._rho[:, 4]).sum())
-        return float((w * self._rho[:, 0]).sum())
+        return self._whole_density
 
 
 class TlDensField:

@@ -278,6 +278,7 @@ int pdfxc_ctx_create(pdfxc_ctx** out, int n_aos, const double* ao_center, const 
     if (rc == PDFXC_OK) rc = dalloc(&c->d_P, (size_t)n_aos * n_aos);
     if (rc == PDFXC_OK) rc = dalloc(&c->d_K, (size_t)n_aos * n_aos);
     if (rc == PDFXC_OK) rc = dalloc(&c->d_E, 1);
+    if (rc == PDFXC_OK) rc = dalloc(&c->d_packed, packed_doubles(n_aos));
     if (rc == PDFXC_OK) rc = dalloc(&c->d_queue, kMaxQueues);
     if (rc == PDFXC_OK) {
         e = hipDeviceGetAttribute(&c->n_cu, hipDeviceAttributeMultiprocessorCount, c->device);
@@ -320,7 +321,7 @@ int pdfxc_ctx_create(pdfxc_ctx** out, int n_aos, const double* ao_center, const 
     }
     if (rc == PDFXC_OK) {
         e = hipHostMalloc(reinterpret_cast<void**>(&c->h_pinned),
-                          sizeof(double) * (size_t)n_aos * n_aos, hipHostMallocDefault);
+                          sizeof(double) * packed_doubles(n_aos), hipHostMallocDefault);
         if (e != hipSuccess) rc = hip_fail(e, "pdfxc_ctx_create: pinned staging");
     }
     if (rc != PDFXC_OK) {
@@ -376,6 +377,7 @@ int pdfxc_ctx_destroy(pdfxc_ctx* ctx) {
     dfree(c->d_P2);
     dfree(c->d_K2);
     dfree(c->d_E);
+    dfree(c->d_packed);
     dfree(c->d_Ps);
     dfree(c->d_perm);
     if (c->h_pinned) (void)hipHostFree(c->h_pinned);
@@ -1076,7 +1078,7 @@ static int build_blocks_impl(Context& c) {
     if (rc == PDFXC_OK) rc = dalloc(reinterpret_cast<char**>(&c.d_k_work), kall.size() * sizeof(KWork));
     if (rc == PDFXC_OK) rc = dalloc(&c.d_coef, 4 * (size_t)c.n_slots);
     if (rc == PDFXC_OK) rc = dalloc(&c.d_rho, 4 * (size_t)c.n_slots);
-    if (rc == PDFXC_OK) rc = dalloc(&c.d_eblock, (size_t)(c.n_slots + 255) / 256);
+    if (rc == PDFXC_OK) rc = dalloc(&c.d_eblock, 3 * (size_t)((c.n_slots + 255) / 256));
     if (rc == PDFXC_OK && c.opts.precision != PDFXC_FP64) {
         rc = dalloc(&c.d_sblocks, c.sblocks.size());
         if (rc == PDFXC_OK) rc = dalloc(&c.d_chunks, c.chunks.size());
@@ -1113,7 +1115,7 @@ static int build_blocks_impl(Context& c) {
     }
     PDFXC_HIP(hipMemsetAsync(c.d_coef, 0, 4 * (size_t)c.n_slots * sizeof(double), c.stream));
     PDFXC_HIP(hipMemsetAsync(c.d_rho, 0, 4 * (size_t)c.n_slots * sizeof(double), c.stream));
-    PDFXC_HIP(hipMemsetAsync(c.d_eblock, 0, (size_t)(c.n_slots + 255) / 256 * sizeof(double), c.stream));
+    PDFXC_HIP(hipMemsetAsync(c.d_eblock, 0, 3 * (size_t)((c.n_slots + 255) / 256) * sizeof(double), c.stream));
     PDFXC_HIP(hipStreamSynchronize(c.stream));
     // host copies of the work lists (a batch concatenates them)
     c.h_rho_work = std::move(rho_work);
@@ -1774,10 +1776,14 @@ struct QueueScope {
     ~QueueScope() { c->queue_open = false; }
 };
 
+static int build_times(Context* c);
+
 // One RKS (nspin 1) or UKS (nspin 2) build on device buffers: the rho pass of
-// each spin, the point terms, the K pass of each spin, the energy sum.
+// each spin, the point terms, the K pass of each spin, the energy sum; put on
+// the stream only when wait is false (build_times then follows the caller's
+// own synchronisation).
 static int build_device(Context* c, int xc, int nspin, const double* const* dP, double* const* dK, double* dE,
-                        int accumulate_rho) {
+                        int accumulate_rho, bool wait = true) {
     if (c->n_pts == 0 || c->blocks.empty()) {
         set_error("build: no grid set");
         return PDFXC_ERR_NO_GRID;
@@ -1808,7 +1814,12 @@ static int build_device(Context* c, int xc, int nspin, const double* const* dP, 
     PDFXC_HIP(hipEventRecord(c->ev[3], c->stream));
     c->rho_accumulate = 0;
     if (rc) return rc;
+    if (!wait) return PDFXC_OK;
     PDFXC_HIP(hipEventSynchronize(c->ev[3]));
+    return build_times(c);
+}
+
+static int build_times(Context* c) {
     float t1, t2, t3;
     PDFXC_HIP(hipEventElapsedTime(&t1, c->ev[0], c->ev[1]));
     PDFXC_HIP(hipEventElapsedTime(&t2, c->ev[1], c->ev[2]));
@@ -1845,9 +1856,6 @@ int pdfxc_build_rks_update_device(pdfxc_ctx* ctx, int functional, const double* 
 
 static int build_host(Context* c, int xc, const double* P_packed, double* K_packed, double* E_xc,
                       double* rho_out, int accumulate_rho);
-static int build_device(Context* c, int xc, int nspin, const double* const* dP, double* const* dK, double* dE,
-                        int accumulate_rho);
-
 int pdfxc_build_rks_update(pdfxc_ctx* ctx, int functional, const double* dP_packed, double* K_packed,
                            double* E_xc, double* rho_out) {
     Context* c = reinterpret_cast<Context*>(ctx);
@@ -1888,27 +1896,24 @@ static int build_host(Context* c, int xc, int nspin, const double* const* P_pack
     double* dP[2] = {c->d_P, c->d_P2};
     double* dK[2] = {c->d_K, c->d_K2};
     double* H = c->h_pinned;
-    for (int sp = 0; sp < nspin; ++sp) {
-        for (int r = 0, k = 0; r < N; ++r)
-            for (int q = 0; q <= r; ++q, ++k) {
-                H[(size_t)r * N + q] = P_packed[sp][k];
-                H[(size_t)q * N + r] = P_packed[sp][k];
-            }
-        PDFXC_HIP(hipMemcpyAsync(dP[sp], H, sizeof(double) * NN, hipMemcpyHostToDevice, c->stream));
-        PDFXC_HIP(hipMemsetAsync(dK[sp], 0, sizeof(double) * NN, c->stream));
-        PDFXC_HIP(hipStreamSynchronize(c->stream));  // H is reused
-    }
-    int rc = build_device(c, xc, nspin, dP, dK, c->d_E, accumulate_rho);
+    const size_t NP = (size_t)N * (N + 1) / 2;
+    double* d_sums = c->d_packed + nspin * NP;  // E_xc, integrated densities: behind the packed K
+    for (int sp = 0; sp < nspin; ++sp) std::copy(P_packed[sp], P_packed[sp] + NP, H + sp * NP);
+    PDFXC_HIP(hipMemcpyAsync(c->d_packed, H, sizeof(double) * nspin * NP, hipMemcpyHostToDevice, c->stream));
+    for (int sp = 0; sp < nspin; ++sp)
+        if (int rc = launch_unpack(N, c->d_packed + sp * NP, dP[sp], dK[sp], c->stream)) return rc;
+    c->whole_density = nspin;
+    int rc = build_device(c, xc, nspin, dP, dK, d_sums, accumulate_rho, false);
+    c->whole_density = 0;
+    for (int sp = 0; sp < nspin && rc == PDFXC_OK; ++sp) rc = launch_pack(N, dK[sp], c->d_packed + sp * NP, c->stream);
     if (rc) return rc;
-    double E = 0.0;
-    PDFXC_HIP(hipMemcpyAsync(&E, c->d_E, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    for (int sp = 0; sp < nspin; ++sp) {
-        PDFXC_HIP(hipMemcpyAsync(H, dK[sp], sizeof(double) * NN, hipMemcpyDeviceToHost, c->stream));
-        PDFXC_HIP(hipStreamSynchronize(c->stream));
-        for (int r = 0, k = 0; r < N; ++r)
-            for (int q = 0; q <= r; ++q, ++k) K_packed[sp][k] += H[(size_t)r * N + q];
-    }
-    *E_xc = E;
+    PDFXC_HIP(hipMemcpyAsync(H, c->d_packed, sizeof(double) * (nspin * NP + 1 + nspin), hipMemcpyDeviceToHost, c->stream));
+    PDFXC_HIP(hipStreamSynchronize(c->stream));
+    if ((rc = build_times(c))) return rc;
+    for (int sp = 0; sp < nspin; ++sp)
+        for (size_t k = 0; k < NP; ++k) K_packed[sp][k] += H[sp * NP + k];
+    *E_xc = H[nspin * NP];
+    for (int sp = 0; sp < nspin; ++sp) c->n_whole[sp] = H[nspin * NP + 1 + sp];
     if (rho_out) {
         const int stride = 4 * nspin;
         const size_t n_out = (size_t)stride * (size_t)c->n_pts;
@@ -1939,6 +1944,14 @@ static int uks_args(Context* c, int functional, const void* a, const void* b, co
     if (!c) return arg_error(std::string(who) + ": null context");
     if (int rc = check_functional(functional, who)) return rc;
     if (!a || !b || !ka || !kb || !e) return arg_error(std::string(who) + ": null buffer");
+    return PDFXC_OK;
+}
+
+int pdfxc_whole_density(pdfxc_ctx* ctx, double* n_alpha, double* n_beta) {
+    Context* c = reinterpret_cast<Context*>(ctx);
+    if (!c || !n_alpha) return arg_error("pdfxc_whole_density: bad arguments");
+    *n_alpha = c->n_whole[0];
+    if (n_beta) *n_beta = c->n_whole[1];
     return PDFXC_OK;
 }
 
@@ -2129,14 +2142,11 @@ int pdfxc_gradient_rks(pdfxc_ctx* ctx, int functional, int n_atoms, const int* Z
         if (rc == PDFXC_OK) rc = launch_scatter_atoms(*c, d_ptat, d_slat);
     }
     if (rc == PDFXC_OK) {
-        double* H = c->h_pinned;
-        for (int r = 0, k = 0; r < N; ++r)
-            for (int q = 0; q <= r; ++q, ++k) {
-                H[(size_t)r * N + q] = P_packed[k];
-                H[(size_t)q * N + r] = P_packed[k];
-            }
-        e = hipMemcpyAsync(c->d_P, H, sizeof(double) * (size_t)N * N, hipMemcpyHostToDevice, c->stream);
-        if (e != hipSuccess) rc = hip_fail(e, "pdfxc_gradient_rks: P upload");
+        const size_t NP = (size_t)N * (N + 1) / 2;
+        std::copy(P_packed, P_packed + NP, c->h_pinned);
+        e = hipMemcpyAsync(c->d_packed, c->h_pinned, sizeof(double) * NP, hipMemcpyHostToDevice, c->stream);
+        rc = e == hipSuccess ? launch_unpack(N, c->d_packed, c->d_P, nullptr, c->stream)
+                             : hip_fail(e, "pdfxc_gradient_rks: P upload");
     }
     // rho (the build's rho pass: FP64, or split when the context's precision
     // splits it), the point terms (with w e_xc per slot), the two gradient
@@ -2298,14 +2308,11 @@ int pdfxc_density_at_points(pdfxc_ctx* ctx, const double* P_packed, int64_t n, c
         else dfree(d_grid);
     }
     if (rc == PDFXC_OK) {
-        double* H = t->h_pinned;
-        for (int r = 0, k = 0; r < N; ++r)
-            for (int q = 0; q <= r; ++q, ++k) {
-                H[(size_t)r * N + q] = P_packed[k];
-                H[(size_t)q * N + r] = P_packed[k];
-            }
-        hipError_t e = hipMemcpyAsync(t->d_P, H, sizeof(double) * (size_t)N * N, hipMemcpyHostToDevice, t->stream);
-        if (e != hipSuccess) rc = hip_fail(e, "pdfxc_density_at_points: P upload");
+        const size_t NP = (size_t)N * (N + 1) / 2;
+        std::copy(P_packed, P_packed + NP, t->h_pinned);
+        const hipError_t e = hipMemcpyAsync(t->d_packed, t->h_pinned, sizeof(double) * NP, hipMemcpyHostToDevice, t->stream);
+        rc = e == hipSuccess ? launch_unpack(N, t->d_packed, t->d_P, nullptr, t->stream)
+                             : hip_fail(e, "pdfxc_density_at_points: P upload");
     }
     if (rc == PDFXC_OK) rc = run_rho(t, t->d_P, t->d_rho);
     if (rc == PDFXC_OK) {

@@ -180,13 +180,16 @@ struct Context {
     double* d_coef_b = nullptr;   // UKS: beta point terms
     double* d_rho_out = nullptr;  // rho in the caller's order (allocated by the first build that returns it)
     size_t n_rho_out = 0;
-    double* d_eblock = nullptr;   // per 256 slots: energy (k_xc_points partial sums)
+    double* d_eblock = nullptr;   // per 256 slots: energy, then w rho of each spin (k_xc_points partial sums)
     double* d_P = nullptr;        // dense N x N
     double* d_K = nullptr;        // dense N x N
     double* d_P2 = nullptr;       // UKS host entry points: beta P and K (allocated on first use)
     double* d_K2 = nullptr;
     double* d_E = nullptr;        // 1 double
-    double* h_pinned = nullptr;   // packed staging (pinned)
+    double* d_packed = nullptr;   // host entry points: packed P in, packed K and E, integrated densities out
+    double* h_pinned = nullptr;   // its pinned staging (packed_doubles(N) values)
+    int whole_density = 0;        // spins whose integrated density the running build sums (0: none)
+    double n_whole[2] = {0.0, 0.0};  // integrated rho_alpha (and rho_beta) of the last host build
 
     // split precision (opts.precision != PDFXC_FP64)
     int split_nc = 0;                   // N rounded up to 8: row length of the P slices
@@ -244,6 +247,9 @@ struct Context {
 
 constexpr int kMaxQueues = 64;  // persistent launches per build sequence
 
+// packed P or K of two spins, then E_xc and the two integrated densities
+inline size_t packed_doubles(int n) { return (size_t)n * (n + 1) + 3; }
+
 // error helpers
 void set_error(const std::string& msg);
 int hip_fail(hipError_t e, const char* what);
@@ -287,6 +293,9 @@ int launch_xc_points(Context& c, int xc_type, double* d_ewf = nullptr);
 int launch_kmat(Context& c, const LaunchRange& r);
 int configure_kernels();
 int launch_energy_sum(Context& c, double* dE);
+// packed lower triangle -> dense symmetric dP, dK (if given) cleared; lower triangle of dK -> packed
+int launch_unpack(int N, const double* d_packed, double* dP, double* dK, hipStream_t s);
+int launch_pack(int N, const double* dK, double* d_packed, hipStream_t s);
 int launch_zero(double* d, int64_t n, hipStream_t s);
 // start a build sequence's persistent launches: zero the counters on the stream
 int begin_queues(Context& c);

@@ -562,23 +562,35 @@ __global__ __launch_bounds__(512) void k_rho(const int* __restrict__ work, const
 // Functional point terms for every slot (buildVxc, DfCalcGridX.cpp:2137-2193
 // for GGA and :2056-2091 for LDA, and the coefficients of build_XC_Matrix,
 // :2353-2368 and :2455-2500): coef = (w vrho / 2, w (2 vgAA + vgAB) grad rho),
-// zero where rho <= the density cut-off or w = 0 (padding slots).  For the
+// zero where rho <= the density cut-off or w = 0 (padding slots).  npart
+// (builds that return the electron count, getWholeDensity) receives the same
+// sums of w rho.  For the
 // LDA functionals vgAA = vgAB = 0, so the gradient part of coef is exactly
 // zero and K = sum_g w vrho phi phi, the LDA matrix.  Per-workgroup sums of
 // w e_xc in a fixed order, and w e_xc per slot when ewf is given.
 // ---------------------------------------------------------------------------
+// Sum of v over the 256 threads of a workgroup in a fixed order, valid in thread 0.
+__device__ inline double block_sum256(double v, double* s4) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+    if ((threadIdx.x & 63) == 0) s4[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return (s4[0] + s4[1]) + (s4[2] + s4[3]);
+}
+
 template <int XC>
 __global__ __launch_bounds__(256) void k_xc_points(int64_t n_slots, const double* __restrict__ pts,
                                                    const double* __restrict__ rho, double* __restrict__ coef,
                                                    double* __restrict__ epart, double* __restrict__ ewf,
-                                                   double dens_cut) {
-    __shared__ double s_e[256];
+                                                   double* __restrict__ npart, double dens_cut) {
+    __shared__ double s_sum[2][4];
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    double e = 0.0;
+    double e = 0.0, nw = 0.0;
     if (i < n_slots) {
         const double w = pts[3 * n_slots + i];
         const double r = rho[4 * i], gx = rho[4 * i + 1], gy = rho[4 * i + 2], gz = rho[4 * i + 3];
         double a = 0.0, cx = 0.0, cy = 0.0, cz = 0.0;
+        nw = w * r;
         if (w != 0.0 && r > dens_cut) {
             const double gamma = gx * gx + gy * gy + gz * gz;
             const XcPoint f = eval_rks(XC, r, gamma);
@@ -595,13 +607,12 @@ __global__ __launch_bounds__(256) void k_xc_points(int64_t n_slots, const double
         coef[4 * i + 3] = cz;
         if (ewf) ewf[i] = e;
     }
-    s_e[threadIdx.x] = e;
-    __syncthreads();
-    for (int k = 128; k > 0; k >>= 1) {
-        if (threadIdx.x < k) s_e[threadIdx.x] += s_e[threadIdx.x + k];
-        __syncthreads();
+    const double es = block_sum256(e, s_sum[0]);
+    if (threadIdx.x == 0) epart[blockIdx.x] = es;
+    if (npart) {
+        const double ns = block_sum256(nw, s_sum[1]);
+        if (threadIdx.x == 0) npart[blockIdx.x] = ns;
     }
-    if (threadIdx.x == 0) epart[blockIdx.x] = s_e[0];
 }
 
 // UKS point terms (buildVxc UKS, DfCalcGridX.cpp:2093-2135 LDA, :2195-2278
@@ -614,15 +625,18 @@ __global__ __launch_bounds__(256) void k_xc_points_uks(int64_t n_slots, const do
                                                        const double* __restrict__ rho_a,
                                                        const double* __restrict__ rho_b,
                                                        double* __restrict__ coef_a, double* __restrict__ coef_b,
-                                                       double* __restrict__ epart, double dens_cut) {
-    __shared__ double s_e[256];
+                                                       double* __restrict__ epart, double* __restrict__ npart,
+                                                       double dens_cut) {
+    __shared__ double s_sum[3][4];
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    double e = 0.0;
+    double e = 0.0, nwa = 0.0, nwb = 0.0;
     if (i < n_slots) {
         const double w = pts[3 * n_slots + i];
         const double ra = rho_a[4 * i], ax = rho_a[4 * i + 1], ay = rho_a[4 * i + 2], az = rho_a[4 * i + 3];
         const double rb = rho_b[4 * i], bx = rho_b[4 * i + 1], by = rho_b[4 * i + 2], bz = rho_b[4 * i + 3];
         double ca[4] = {0.0, 0.0, 0.0, 0.0}, cb[4] = {0.0, 0.0, 0.0, 0.0};
+        nwa = w * ra;
+        nwb = w * rb;
         if (w != 0.0 && (ra > dens_cut || rb > dens_cut)) {
             const double gaa = ax * ax + ay * ay + az * az;
             const double gab = ax * bx + ay * by + az * bz;
@@ -644,13 +658,15 @@ __global__ __launch_bounds__(256) void k_xc_points_uks(int64_t n_slots, const do
             coef_b[4 * i + q] = cb[q];
         }
     }
-    s_e[threadIdx.x] = e;
-    __syncthreads();
-    for (int k = 128; k > 0; k >>= 1) {
-        if (threadIdx.x < k) s_e[threadIdx.x] += s_e[threadIdx.x + k];
-        __syncthreads();
+    const double es = block_sum256(e, s_sum[0]);
+    if (threadIdx.x == 0) epart[blockIdx.x] = es;
+    if (npart) {
+        const double na = block_sum256(nwa, s_sum[1]), nb = block_sum256(nwb, s_sum[2]);
+        if (threadIdx.x == 0) {
+            npart[blockIdx.x] = na;
+            npart[gridDim.x + blockIdx.x] = nb;
+        }
     }
-    if (threadIdx.x == 0) epart[blockIdx.x] = s_e[0];
 }
 
 // ---------------------------------------------------------------------------
@@ -881,11 +897,13 @@ __global__ __launch_bounds__(768) void k_kmat(const KWork* __restrict__ work, co
 
 // deterministic sum of the per-block energies (one workgroup)
 // E_xc of molecule blockIdx.x: the partial sums [bounds[m], bounds[m + 1]) in a
-// fixed order (one molecule: bounds = {0, n})
+// fixed order; without bounds, quantity blockIdx.x (E_xc, then the integrated
+// densities) of one molecule: the run of n partial sums from n blockIdx.x
 __global__ __launch_bounds__(256) void k_energy_sum(const double* __restrict__ eb, const int* __restrict__ bounds,
                                                     int n, double* __restrict__ out) {
     __shared__ double s[256];
-    const int lo = bounds ? bounds[blockIdx.x] : 0, hi = bounds ? bounds[blockIdx.x + 1] : n;
+    const int lo = bounds ? bounds[blockIdx.x] : n * (int)blockIdx.x;
+    const int hi = bounds ? bounds[blockIdx.x + 1] : lo + n;
     double v = 0.0;
     for (int i = lo + threadIdx.x; i < hi; i += 256) v += eb[i];
     s[threadIdx.x] = v;
@@ -1092,7 +1110,8 @@ template <int XC>
 static void xc_points_one(Context& c, double* d_ewf) {
     const int64_t g = (c.n_slots + 255) / 256;
     hipLaunchKernelGGL(k_xc_points<XC>, dim3((unsigned)g), dim3(256), 0, c.stream, c.n_slots, c.d_pts,
-                       c.d_rho, c.d_coef, c.d_eblock, d_ewf, c.opts.density_cutoff);
+                       c.d_rho, c.d_coef, c.d_eblock, d_ewf, c.whole_density ? c.d_eblock + g : nullptr,
+                       c.opts.density_cutoff);
 }
 
 int launch_xc_points(Context& c, int xc_type, double* d_ewf) {
@@ -1111,7 +1130,8 @@ template <int XC>
 static void xc_points_uks_one(Context& c) {
     const int64_t g = (c.n_slots + 255) / 256;
     hipLaunchKernelGGL(k_xc_points_uks<XC>, dim3((unsigned)g), dim3(256), 0, c.stream, c.n_slots, c.d_pts,
-                       c.d_rho, c.d_rho_b, c.d_coef, c.d_coef_b, c.d_eblock, c.opts.density_cutoff);
+                       c.d_rho, c.d_rho_b, c.d_coef, c.d_coef_b, c.d_eblock, c.whole_density ? c.d_eblock + g : nullptr,
+                       c.opts.density_cutoff);
 }
 
 int launch_xc_points_uks(Context& c, int xc_type) {
@@ -1166,9 +1186,39 @@ int configure_kernels() {
 }
 
 int launch_energy_sum(Context& c, double* dE) {
-    hipLaunchKernelGGL(k_energy_sum, dim3(1), dim3(256), 0, c.stream, c.d_eblock, (const int*)nullptr,
+    hipLaunchKernelGGL(k_energy_sum, dim3(1 + c.whole_density), dim3(256), 0, c.stream, c.d_eblock, (const int*)nullptr,
                        (int)((c.n_slots + 255) / 256), dE);
     return check_launch("k_energy_sum");
+}
+
+// Packed lower triangle (row r, column c <= r) to the dense symmetric P, and
+// K cleared in the same pass; the lower triangle of K back to packed order.
+// One workgroup row per matrix row keeps every access on contiguous runs but
+// the mirrored half of P.  N = 152 with both copies in one: the two host loops
+// they replace took 140 us of an 8-water build.
+__global__ __launch_bounds__(256) void k_unpack(int N, const double* __restrict__ packed, double* __restrict__ P,
+                                                double* __restrict__ K) {
+    const int r = blockIdx.x;
+    const double* row = packed + (int64_t)r * (r + 1) / 2;
+    for (int c = threadIdx.x; c < N; c += 256) {
+        const double v = c <= r ? row[c] : packed[(int64_t)c * (c + 1) / 2 + r];
+        P[(int64_t)r * N + c] = v;
+        if (K) K[(int64_t)r * N + c] = 0.0;
+    }
+}
+__global__ __launch_bounds__(256) void k_pack(int N, const double* __restrict__ K, double* __restrict__ packed) {
+    const int r = blockIdx.x;
+    for (int c = threadIdx.x; c <= r; c += 256) packed[(int64_t)r * (r + 1) / 2 + c] = K[(int64_t)r * N + c];
+}
+
+int launch_unpack(int N, const double* d_packed, double* dP, double* dK, hipStream_t s) {
+    hipLaunchKernelGGL(k_unpack, dim3(N), dim3(256), 0, s, N, d_packed, dP, dK);
+    return check_launch("k_unpack");
+}
+
+int launch_pack(int N, const double* dK, double* d_packed, hipStream_t s) {
+    hipLaunchKernelGGL(k_pack, dim3(N), dim3(256), 0, s, N, dK, d_packed);
+    return check_launch("k_pack");
 }
 
 int launch_zero(double* d, int64_t n, hipStream_t s) {

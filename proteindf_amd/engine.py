@@ -36,7 +36,7 @@ ERROR_CODES = {v: k for k, v in ERROR_NAMES.items()}
 # every symbol declared in include/pdfxc.h
 EXPORTED = [
     "pdfxc_default_opts", "pdfxc_normalize_cgto", "pdfxc_ctx_create", "pdfxc_ctx_destroy",
-    "pdfxc_set_grid", "pdfxc_generate_grid", "pdfxc_get_grid", "pdfxc_build_rks",
+    "pdfxc_set_grid", "pdfxc_generate_grid", "pdfxc_get_grid", "pdfxc_whole_density", "pdfxc_build_rks",
     "pdfxc_build_rks_device", "pdfxc_eval_functional", "pdfxc_eval_aos", "pdfxc_get_stats",
     "pdfxc_stream", "pdfxc_last_error", "pdfxc_gradient_rks", "pdfxc_build_rks_update",
     "pdfxc_build_rks_update_device", "pdfxc_selftest_mfma", "pdfxc_selftest_mfma_split",
@@ -131,6 +131,7 @@ def lib():
         L.pdfxc_generate_grid_ex.argtypes = [P, i32, P, P, P, P]
         L.pdfxc_generate_grid_oriented.argtypes = [P, i32, P, P, P, P, P]
         L.pdfxc_get_grid.argtypes = [P, P, P, P, P]
+        L.pdfxc_whole_density.argtypes = [P, P, P]
         L.pdfxc_build_rks.argtypes = [P, i32, P, P, P, P]
         L.pdfxc_build_rks_device.argtypes = [P, i32, P, P, P]
         L.pdfxc_eval_functional.argtypes = [i32, i64, P, P]
@@ -401,6 +402,12 @@ class XcContext:
         rho = np.zeros((self.n_pts, 4)) if want_rho else None
         check(lib().pdfxc_build_rks(self.h, functional, _p(P), _p(K), ctypes.byref(E), _p(rho)))
         return E.value, K, rho
+
+    def whole_density(self, nspin=1):
+        """Integrated rho_alpha (nspin 1) or (rho_alpha, rho_beta) of the last host build."""
+        n = (ctypes.c_double(), ctypes.c_double())
+        check(lib().pdfxc_whole_density(self.h, ctypes.byref(n[0]), ctypes.byref(n[1])))
+        return n[0].value if nspin == 1 else (n[0].value, n[1].value)
 
     def gradient_rks(self, Z, xyz, P_alpha_packed, point_atom=None, functional=PDFXC_B3LYP):
         """(E_xc, grad_functional (n_atoms, 3), grad_weight (n_atoms, 3)); dE/dR."""
