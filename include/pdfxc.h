@@ -105,8 +105,9 @@ typedef struct pdfxc_stats {
  * takes 64 points per workgroup when they fit in LDS, else 32; in the block
  * floating point rho pass a block takes the first of the 64-, 32- and
  * 16-point classes from split_rho_shift on that holds its columns and fits
- * in LDS); k_tiles (8..96): FP64 K pass work item size in lower
- * 16 x 16 tiles for blocks of more than 32 tiles; split_k_patches (4..32):
+ * in LDS); k_tiles (8..96): FP64 K pass work item size for blocks of more
+ * than 10 tiles of 16 columns a side, 96 standing for the largest, 36 lower
+ * 2 x 2 tile patches (16 tiles a side); split_k_patches (4..32):
  * split K pass work item size in 2 x 2 tile patches (up to 16: workgroups of
  * 16 waves, one patch each; up to 24: 12 waves of two; up to 32: 8 waves of
  * four); split_k_group (1, 2, 4 or 8): grid blocks (128 points each,

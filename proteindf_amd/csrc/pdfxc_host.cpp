@@ -718,37 +718,40 @@ static int build_blocks_impl(Context& c) {
         r.lds = maxdyn;
         if (r.count) c.rho_launches.push_back(r);
     }
-    // k_kmat work: lower tiles split into items of at most 96 tiles
-    std::vector<KWork> kw[2];
-    size_t klds[2] = {0, 0};
+    // k_kmat work: the lower 2 x 2 tile patches of a block, row-major, in one
+    // item where a workgroup shape holds them (10 of 12, 15 of 16 or 36
+    // patches: at most 8, 10 or 16 tiles a side), else in items of at most 36
+    // (k_tiles = 96; the tuning may cut those smaller)
+    std::vector<KWork> kw[kKmatClasses];
+    size_t klds[kKmatClasses] = {};
     for (int b = 0; b < nb; ++b) {
         const BlockDesc& B = c.blocks[b];
-        const int T = B.ldn / 16;
-        const int nt = T * (T + 1) / 2;
-        const int cls = (nt <= 32) ? 0 : 1;
-        // at most 8 x 12 tiles (the kernel's consumer limit); the tuning may cut items smaller
-        const int per = (cls == 0) ? 32 : c.tune.k_tiles;
-        for (int t0 = 0; t0 < nt; t0 += per) {
+        const int T = B.ldn / 16, Tp = (T + 1) / 2;
+        const int np = Tp * (Tp + 1) / 2;
+        const int cls = T <= 8 ? 0 : T <= 10 ? 1 : 2;
+        const int per = cls < 2 ? np : c.tune.k_tiles * 36 / 96;
+        for (int t0 = 0; t0 < np; t0 += per) {
             KWork w;
             w.block = b;
             w.t0 = t0;
-            w.t1 = std::min(nt, t0 + per);
-            int I = 0;
-            while ((I + 1) * (I + 2) / 2 <= w.t1 - 1) ++I;
-            w.ncols = 16 * (I + 1);
+            w.t1 = std::min(np, t0 + per);
+            int P = 0;
+            while ((P + 1) * (P + 2) / 2 <= w.t1 - 1) ++P;
+            w.ncols = std::min(B.ldn, 32 * (P + 1));
             w.nsh = w.ps = 0;
             kw[cls].push_back(w);
         }
     }
     // the shells of every item, counted where the block lists are
-    const size_t n_items = kw[0].size() + kw[1].size();
+    size_t n_items = 0;
+    for (const auto& w : kw) n_items += w.size();
     std::vector<int> item_nsh(n_items);
     {
         DeviceBuf items;
         if (int e = items.alloc((sizeof(KWork) + sizeof(int)) * n_items)) return e;
         KWork* d_items = items.as<KWork>();
         int* d_nsh = reinterpret_cast<int*>(d_items + n_items);
-        for (int cls = 0, at = 0; cls < 2; at += (int)kw[cls].size(), ++cls)
+        for (int cls = 0, at = 0; cls < kKmatClasses; at += (int)kw[cls].size(), ++cls)
             if (!kw[cls].empty())
                 PDFXC_HIP(hipMemcpyAsync(d_items + at, kw[cls].data(), sizeof(KWork) * kw[cls].size(),
                                          hipMemcpyHostToDevice, c.stream));
@@ -756,19 +759,19 @@ static int build_blocks_impl(Context& c) {
         PDFXC_HIP(hipMemcpyAsync(item_nsh.data(), d_nsh, sizeof(int) * n_items, hipMemcpyDeviceToHost, c.stream));
         PDFXC_HIP(hipStreamSynchronize(c.stream));
     }
-    for (int cls = 0, at = 0; cls < 2; ++cls)
+    // points per slab: 16, or 8 where 16 would cost the class its workgroups
+    // per CU (3, 2 and 1 by its registers), or what one workgroup can have
+    for (int cls = 0, at = 0; cls < kKmatClasses; ++cls)
         for (KWork& w : kw[cls]) {
-            const int nsh_item = item_nsh[at++];
-            w.nsh = nsh_item;
-            size_t lds = 0;
-            const int LD = (w.ncols & 31) ? w.ncols : w.ncols + 16;
-            for (int ps = 16; ps >= 4; ps /= 2) {
-                w.ps = ps;
-                lds = sizeof(double) * (4 * (size_t)ps * LD + (size_t)nsh_item * RS) +
-                      sizeof(int) * (size_t)(w.ncols + 2 * nsh_item);
-                if (lds <= (size_t)kMaxDynLds) break;
-            }
-            if (lds > (size_t)kMaxDynLds) {
+            w.nsh = item_nsh[at++];
+            auto lds_of = [&](int ps) {
+                return sizeof(double) * (4 * (size_t)ps * w.ncols + (size_t)w.nsh * RS) +
+                       sizeof(int) * (size_t)(w.ncols + 2 * w.nsh);
+            };
+            w.ps = 16;
+            if (lds_of(16) > kKmatLds[cls]) w.ps = lds_of(8) <= kKmatLds[kKmatClasses - 1] ? 8 : 4;
+            const size_t lds = lds_of(w.ps);
+            if (lds > kKmatLds[kKmatClasses - 1]) {
                 set_error("set_grid: block too wide for the K kernel's LDS");
                 return PDFXC_ERR_UNSUPPORTED;
             }
@@ -776,7 +779,7 @@ static int build_blocks_impl(Context& c) {
         }
     std::vector<KWork> kall;
     c.kmat_launches.clear();
-    for (int cls = 0; cls < 2; ++cls) {
+    for (int cls = 0; cls < kKmatClasses; ++cls) {
         if (kw[cls].empty()) continue;
         c.kmat_launches.push_back(LaunchRange{cls, (int)kall.size(), (int)kw[cls].size(), klds[cls]});
         kall.insert(kall.end(), kw[cls].begin(), kw[cls].end());
@@ -1064,7 +1067,7 @@ static int build_blocks_impl(Context& c) {
         const int kshape = c.tune.split_k_patches <= 16 ? 0 : c.tune.split_k_patches <= 24 ? 1 : 2;
         if (!skw.empty()) c.sk_launches.push_back(LaunchRange{kshape, 0, (int)skw.size(), sk_lds});
         // FP64 K items of those blocks, appended to the FP64 work list
-        for (int cls = 0; cls < 2; ++cls) {
+        for (int cls = 0; cls < kKmatClasses; ++cls) {
             LaunchRange r{cls, (int)kall.size(), 0, klds[cls]};
             for (const KWork& w : kw[cls])
                 if (k_fp64_block[w.block]) kall.push_back(w);

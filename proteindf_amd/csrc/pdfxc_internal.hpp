@@ -69,11 +69,16 @@ struct SplitBlock {
     int chunk_begin, nchunk, ldnp, pad;
 };
 
-// One k_kmat work item: lower 16 x 16 tiles [t0, t1) of a block (k_kmat_split:
-// lower 2 x 2 tile patches [t0, t1), ps = slab buffers).
+// One k_kmat work item: lower 2 x 2 tile patches [t0, t1) of a block, row-major,
+// on its first ncols columns and nsh shells, in slabs of ps points.
 struct KWork {
     int block, t0, t1, ncols, nsh, ps;
 };
+// k_kmat workgroup shapes (4, 8 and 12 waves) and the dynamic LDS with which
+// 3, 2 and 1 of them share a CU's 160 KiB (7184 bytes of static LDS each,
+// granules of 1280)
+constexpr int kKmatClasses = 3;
+constexpr size_t kKmatLds[kKmatClasses] = {45 * 1024, 72 * 1024, 152 * 1024};
 
 // A launch of one kernel instantiation over a contiguous range of a work list.
 struct LaunchRange {

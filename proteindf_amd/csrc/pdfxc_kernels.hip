@@ -7,10 +7,10 @@
 //           16-column slabs through LDS; then rho = sum_j X_pj phi_pj and
 //           grad rho = 2 sum_j X_pj grad phi_pj with phi, grad phi
 //           re-evaluated per 64-column chunk, then the B3LYP point terms.
-//   k_kmat  for a range of lower 16 x 16 tiles of K_bb (held in
-//           accumulators): Phi_b^T V_b + V_b^T Phi_b over the block's points
-//           in 16-point slabs, phi / grad phi / V evaluated into LDS, then
-//           scattered into the dense lower triangle of K.
+//   k_kmat  for a range of lower 2 x 2 patches of 16 x 16 tiles of K_bb (held
+//           in accumulators): Phi_b^T V_b + V_b^T Phi_b over the block's points
+//           in slabs of 16 or 8, phi and V evaluated into LDS, then scattered
+//           into the dense lower triangle of K.
 // The reference runs the same quantities point by point
 // (DfCalcGridX.cpp:1923-1962, :2137-2193, :2455-2500).
 #include <hip/hip_runtime.h>
@@ -670,117 +670,70 @@ __global__ __launch_bounds__(256) void k_xc_points_uks(int64_t n_slots, const do
 }
 
 // ---------------------------------------------------------------------------
-// K pass consumer: NT accumulator tiles of K_bb (a contiguous run [tb, te)
-// of lower tiles, t = I (I + 1) / 2 + J, rounded up to a multiple of 4 with
-// repeats of the last tile that are not scattered) over the point slabs the
-// producer waves fill.  Slab element (point p, column c) sits at
-// p LD + (c ^ (p & 15)): the XOR keeps the 16 lanes of an operand read on
-// one 128-byte run while spreading a producer's column writes over the banks.
+// K pass: K_bb += Phi^T V + V^T Phi for a run [t0, t1) of lower 2 x 2 patches
+// of 16 x 16 tiles of one block, row-major (patch (P, Q), Q <= P, is number
+// P (P + 1) / 2 + Q).  Patch t0 + wave + NW m belongs to wave `wave`: NPW of
+// them at most, four accumulator tiles each (a diagonal patch runs three, the
+// last row of an odd tile count two or one; wave-uniform branches skip the
+// rest).  phi and V of a point and column sit side by side in LDS, so four
+// 16-byte reads per lane feed the eight MFMAs of a patch and K step.
+// All waves produce the next point slab and multiply the current one; one
+// wave per SIMD (waves 0-3) produces first and multiplies last, the others
+// the other way round, so VALU and matrix cores work at the same time.
+// Production goes in chunks of 64 (shell, point) pairs from an LDS counter.
+//
+// Measured (MI355X): before, 8 consumer and 4 producer waves ran over a linear
+// list of tiles, two operand reads per MFMA, and either half alone took 85 %
+// of the pass.  K pass of 8 waters 0.47 -> 0.22 ms, of a 10-residue helix
+// 4.6 -> 4.0 ms, of a 30-residue helix 43.1 -> 36.9 ms; what is left of the
+// wide ones are the scatter's atomics (26.6 ms without them).
+// Slab element (point p, column c) is at p LD + (c ^ (p & 15)): the 16 lanes
+// of an operand read stay on one 256-byte run, and a producer's 16 points of
+// one column fall on 16 different 16-byte slots.
+// Tiles go into the dense lower triangle of K with FP64 atomics
+// (build_XC_Matrix GGA, DfCalcGridX.cpp:2455-2500).
 // ---------------------------------------------------------------------------
-template <int NT>
-__device__ inline void kmat_consume(int tb, int te, int nslab, int PS, int LD, int SLAB, int lane,
-                                    const double* s_buf, const int* s_cols, double* __restrict__ K, int N) {
-    const int li = lane & 15, lq = lane >> 4;
-    int offI[NT], offJ[NT];
-    {
-        int I = 0;
-        while ((I + 1) * (I + 2) / 2 <= tb) ++I;
-        int J = tb - I * (I + 1) / 2;
-#pragma unroll
-        for (int m = 0; m < NT; ++m) {
-            offI[m] = I * 16;
-            offJ[m] = J * 16;
-            if (tb + m + 1 < te) {  // advance along the run; padding repeats the last tile
-                if (J == I) {
-                    ++I;
-                    J = 0;
-                } else {
-                    ++J;
-                }
-            }
-        }
-    }
-    v4d acc[NT];
-#pragma unroll
-    for (int m = 0; m < NT; ++m) acc[m] = v4d{0.0, 0.0, 0.0, 0.0};
-    __syncthreads();
-    for (int s = 0; s < nslab; ++s) {
-        const double* cur = s_buf + (s & 1) * 2 * SLAB;
-        for (int ks = 0; ks < PS / 4; ++ks) {
-            const int p = 4 * ks + lq;
-            const double* fr = cur + p * LD + (li ^ (p & 15));
-            const double* vr = fr + SLAB;
-            // groups of 4 tiles: bounded operand lookahead keeps the
-            // accumulators and operands within the register budget
-#pragma unroll
-            for (int m0 = 0; m0 < NT; m0 += 4) {
-#pragma unroll
-                for (int m = m0; m < m0 + 4; ++m) {
-                    const double a1 = fr[offI[m]], b1 = vr[offJ[m]];
-                    const double a2 = vr[offI[m]], b2 = fr[offJ[m]];
-                    acc[m] = mfma16x16x4(a1, b1, acc[m]);
-                    acc[m] = mfma16x16x4(a2, b2, acc[m]);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        __syncthreads();
-    }
-    // scatter: tile element (4 r + lq, li) -> K[cols[I 16 + 4 r + lq]][cols[J 16 + li]]
-#pragma unroll
-    for (int m = 0; m < NT; ++m) {
-        if (tb + m < te) {
-            const int lc = offJ[m] + li;
-            const int gj = s_cols[lc];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int lr = offI[m] + 4 * r + lq;
-                const int gi = s_cols[lr];
-                if (gi >= 0 && gj >= 0 && lr >= lc) atomicAdd(K + (int64_t)gi * N + gj, acc[m][r]);
-            }
-        }
-    }
-}
+struct KOperands {
+    double2 i0, i1, j0, j1;  // (phi, V) of the patch's two row and two column tiles
+};
 
-// ---------------------------------------------------------------------------
-// K pass: K_bb += Phi^T V + V^T Phi for the lower 16 x 16 tiles t0 <= t < t1
-// (at most 96) of one block.  Twelve waves: waves 0-7 (consumers, two per
-// SIMD) each hold a contiguous eighth of the tiles in accumulators and run
-// the MFMAs on point slab s while waves 8-11 (producers) evaluate slab s + 1
-// into the other
-// half of a double-buffered LDS area: phi and grad phi of the needed columns
-// from the LDS shell records, and V = (w vrho / 2) phi + c . grad phi with
-// the per-point coefficients (build_XC_Matrix GGA, DfCalcGridX.cpp:2455-2500).
-// Tiles go into the dense lower triangle of K with FP64 atomics.
-// ---------------------------------------------------------------------------
+template <int NW, int NPW, bool PERSIST>
 __device__ __forceinline__ void k_kmat_item(int item, const KWork* __restrict__ work, const BlockDesc* __restrict__ blocks,
                                               const double* __restrict__ pts, int64_t n_slots,
                                               const double* __restrict__ shrec, int RS,
                                               const int* __restrict__ bshells, const int* __restrict__ bshell_col,
                                               const int* __restrict__ bcols, const int* __restrict__ bsorder,
-                                              const double* __restrict__ coef, double* __restrict__ K, int N,
-        double (*s_pt)[3], double (*s_cf)[4], double* s_dynd) {
+                                              const double* __restrict__ coef, double* __restrict__ K,
+        int* __restrict__ queue, double (*s_pt)[3], double (*s_cf)[4], int* s_pcount, int* s_item, double* s_dynd) {
+    constexpr int NT = NW * 64;
     const KWork W = work[item];
     const BlockDesc B = blocks[W.block];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
+    const int li = lane & 15, lq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const bool producer = wave >= 8;
     const int ncols = W.ncols;  // multiple of 16, <= ldn
-    const int LD = (ncols & 31) ? ncols : ncols + 16;
-    const int PS = W.ps;
+    const int LD = ncols;
+    const int PS = W.ps;  // 16, 8 or 4
     const int ps_log = 31 - __builtin_clz(PS);
     const int nsh = W.nsh;
-    const int SLAB = PS * LD;  // doubles per array per buffer
-    // LDS: [2 buffers][phi, V][PS][LD] | records [nsh][RS] | cols [ncols] | shcol [nsh] | shid [nsh]
-    double* s_buf = s_dynd;
-    double* s_rec = s_buf + 4 * SLAB;
+    const int SLAB = PS * LD;
+    const int T = B.ldn >> 4;
+    // LDS: [2 buffers][PS][LD] of (phi, V) | records [nsh][RS] | cols [ncols] | shcol [nsh] | shid [nsh]
+    double2* s_buf = reinterpret_cast<double2*>(s_dynd);
+    double* s_rec = s_dynd + 4 * SLAB;
     int* s_cols = reinterpret_cast<int*>(s_rec + (size_t)nsh * RS);
     int* s_shcol = s_cols + ncols;
     int* s_shid = s_shcol + nsh;
-    for (int c = tid; c < ncols; c += 768) s_cols[c] = (c < B.nao) ? bcols[B.col_begin + c] : -1;
-    // shells this item needs (local index < nsh), in (l, nprim) order, compacted by wave 8
-    if (wave == 8) {
+    for (int c = tid; c < ncols; c += NT) s_cols[c] = (c < B.nao) ? bcols[B.col_begin + c] : -1;
+    if (tid < 2) s_pcount[tid] = 0;
+    // the next item is asked for now and published with the first slab: by the
+    // end of this one every wave has scatter atomics in flight, which the
+    // answer would wait for
+    int nxt = 0;
+    if (PERSIST && tid == NT - 64) nxt = atomicAdd(queue, 1);
+    // shells this item needs (local index < nsh), in (l, nprim) order, compacted by the last wave
+    if (wave == NW - 1) {
         int base = 0;
         for (int i0 = 0; i0 < B.nshell; i0 += 64) {
             const int i = i0 + lane;
@@ -795,7 +748,7 @@ __device__ __forceinline__ void k_kmat_item(int item, const KWork* __restrict__ 
             base += __popcll(m);
         }
     }
-    for (int p = tid; p < kBlockPts; p += 768) {
+    for (int p = tid; p < kBlockPts; p += NT) {
         const int64_t slot = B.pt_begin + p;
         s_pt[p][0] = pts[slot];
         s_pt[p][1] = pts[n_slots + slot];
@@ -805,93 +758,169 @@ __device__ __forceinline__ void k_kmat_item(int item, const KWork* __restrict__ 
         s_cf[p][2] = coef[4 * slot + 2];
         s_cf[p][3] = coef[4 * slot + 3];
     }
+    {
+        // columns past the block's AOs stay zero in both buffers: the swizzle
+        // maps the last 16 columns of a row onto themselves, so clear those
+        const int z0 = min(ncols, B.nao) & ~15;
+        const int nz = ncols - z0;  // 16, or 0 when the AOs fill the columns
+        for (int it = tid; it < 2 * PS * nz; it += NT) s_buf[(it / nz) * LD + z0 + it % nz] = double2{0.0, 0.0};
+    }
     __syncthreads();
-    for (int idx = tid; idx < nsh * RS; idx += 768) {
+    for (int idx = tid; idx < nsh * RS; idx += NT) {
         const int k = idx / RS;
         s_rec[idx] = shrec[(int64_t)s_shid[k] * RS + (idx - k * RS)];
     }
     __syncthreads();
 
-    const int ptid = tid - 512;  // producer thread index
-    auto produce = [&](int pb, double* phi, double* vv) {
-        for (int it = ptid; it < nsh * PS; it += 256) {
-            const int p = it & (PS - 1);  // PS is a power of two (16, 8 or 4)
-            const int k = it >> ps_log;
+    auto produce = [&](int s) {
+        double2* buf = s_buf + (s & 1) * SLAB;
+        const int pb = s * PS;
+        int* pc = s_pcount + (s & 1);
+        for (;;) {
+            int chunk = 0;
+            if (lane == 0) chunk = atomicAdd(pc, 1);
+            const int r0 = __builtin_amdgcn_readfirstlane(chunk) * 64;
+            if (r0 >= nsh * PS) break;
+            const int it = r0 + lane;
+            if (it >= nsh * PS) continue;
+            const int p = it & (PS - 1);
+            const int k = nsh - 1 - (it >> ps_log);  // the costliest (l, nprim) first
             const int pp = pb + p;
             const double* rec = s_rec + k * RS;
             const double x = s_pt[pp][0] - rec[0], y = s_pt[pp][1] - rec[1], z = s_pt[pp][2] - rec[2];
             double R0, R1;
             rec_radial01(rec, x, y, z, R0, R1);
             const int c0 = s_shcol[k];
+            double2* row = buf + p * LD;
             const int sw = p & 15;
             shell_phi_v(((int)rec[3]) & 3, x, y, z, R0, R1, s_cf[pp][0], s_cf[pp][1], s_cf[pp][2], s_cf[pp][3],
                         [&](int m, double v, double V) {
                             const int c = c0 + m;
-                            if (c < ncols) {
-                                phi[p * LD + (c ^ sw)] = v;
-                                vv[p * LD + (c ^ sw)] = V;
-                            }
+                            if (c < ncols) row[c ^ sw] = double2{v, V};
                         });
-        }
-        for (int it = ptid; it < (ncols - min(ncols, B.nao)) * PS; it += 256) {
-            const int c = B.nao + (it >> ps_log);
-            const int p = it & (PS - 1);
-            phi[p * LD + (c ^ (p & 15))] = 0.0;
-            vv[p * LD + (c ^ (p & 15))] = 0.0;
         }
     };
 
-    const int nslab = (B.npts + PS - 1) / PS;
-    if (producer) {
-        // producers: slab s + 1 while the consumers multiply slab s; the
-        // number of barriers matches the consumer branch
-        produce(0, s_buf, s_buf + SLAB);
-        __syncthreads();
-        for (int s = 0; s < nslab; ++s) {
-            if (s + 1 < nslab) {
-                double* nxt = s_buf + ((s + 1) & 1) * 2 * SLAB;
-                produce((s + 1) * PS, nxt, nxt + SLAB);
-            }
-            __syncthreads();
+    // the wave's patches: element offsets of their tiles in a slab row, and
+    // which of the four tiles run (second row: 2 P + 1 < T; tile (0, 1): P > Q)
+    int i0[NPW], i1[NPW], j0[NPW], j1[NPW];
+    bool has[NPW], two[NPW], off[NPW];
+    {
+        int P = 0, q = W.t0 + wave, base = 0;  // base = P (P + 1) / 2
+#pragma unroll
+        for (int m = 0; m < NPW; ++m, q += NW) {
+            has[m] = q < W.t1;
+            const int qq = has[m] ? q : W.t0;  // a wave without a patch keeps valid offsets
+            if (!has[m]) P = base = 0;
+            while (base + P + 1 <= qq) base += ++P;
+            const int Q = qq - base;
+            two[m] = 2 * P + 1 < T;
+            off[m] = P > Q;
+            i0[m] = 32 * P;
+            i1[m] = two[m] ? 32 * P + 16 : 32 * P;
+            j0[m] = 32 * Q;
+            j1[m] = off[m] ? 32 * Q + 16 : i1[m];
         }
-        return;  // to the next item's barrier, which the consumers reach after their scatter
     }
-    // consumers: a contiguous run [tb, te) of the item's tiles, dispatched on
-    // the run length rounded up to 4 (one barrier before the slab loop, one per slab)
-    const int q8 = (W.t1 - W.t0 + 7) >> 3;
-    const int tstart = W.t0 + wave * q8;
-    const int tend = min(W.t1, tstart + q8);
-    const bool has = tstart < tend;
-    const int tb = has ? tstart : W.t1 - 1;  // a wave without tiles keeps valid offsets
-    const int te = has ? tend : tb;          // and scatters nothing
-    const int ngrp = has ? (tend - tstart + 3) >> 2 : 1;
-    switch (ngrp) {
-        case 1: kmat_consume<4>(tb, te, nslab, PS, LD, SLAB, lane, s_buf, s_cols, K + B.poff, B.ldp); break;
-        case 2: kmat_consume<8>(tb, te, nslab, PS, LD, SLAB, lane, s_buf, s_cols, K + B.poff, B.ldp); break;
-        default: kmat_consume<12>(tb, te, nslab, PS, LD, SLAB, lane, s_buf, s_cols, K + B.poff, B.ldp); break;
+    v4d acc[NPW][4];  // tiles (0, 0), (1, 0), (0, 1), (1, 1)
+#pragma unroll
+    for (int m = 0; m < NPW; ++m)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) acc[m][t] = v4d{0.0, 0.0, 0.0, 0.0};
+
+    auto consume = [&](int s) {
+        const double2* cur = s_buf + (s & 1) * SLAB + lq * LD;
+        const int nks = PS >> 2;
+        auto load = [&](int m, int ks) {
+            const double2* row = cur + 4 * ks * LD + (li ^ (4 * ks + lq));
+            return KOperands{row[i0[m]], row[i1[m]], row[j0[m]], row[j1[m]]};
+        };
+        for (int ks = 0; ks < nks; ++ks) {
+#pragma unroll
+            for (int m = 0; m < NPW; ++m) {
+                if (!has[m]) continue;
+                const KOperands o = load(m, ks);
+                acc[m][0] = mfma16x16x4(o.i0.x, o.j0.y, acc[m][0]);
+                acc[m][0] = mfma16x16x4(o.i0.y, o.j0.x, acc[m][0]);
+                if (two[m]) {
+                    acc[m][1] = mfma16x16x4(o.i1.x, o.j0.y, acc[m][1]);
+                    acc[m][3] = mfma16x16x4(o.i1.x, o.j1.y, acc[m][3]);
+                    acc[m][1] = mfma16x16x4(o.i1.y, o.j0.x, acc[m][1]);
+                    acc[m][3] = mfma16x16x4(o.i1.y, o.j1.x, acc[m][3]);
+                }
+                if (off[m]) {
+                    acc[m][2] = mfma16x16x4(o.i0.x, o.j1.y, acc[m][2]);
+                    acc[m][2] = mfma16x16x4(o.i0.y, o.j1.x, acc[m][2]);
+                }
+            }
+        }
+    };
+
+    // step s multiplies slab s and produces slab s + 1 (one copy of either
+    // body: two of them spill)
+    const int nslab = (B.npts + PS - 1) >> ps_log;
+    const bool first = wave < (NW > 4 ? 4 : 2);
+#pragma unroll 1
+    for (int s = -1; s < nslab; ++s) {
+        if (s >= 0 && tid == 0) s_pcount[s & 1] = 0;  // slab s is in; its counter serves slab s + 2
+#pragma unroll 1
+        for (int ph = 0; ph < 2; ++ph) {
+            if ((ph == 0) == first) {
+                if (s + 1 < nslab) produce(s + 1);
+            } else if (s >= 0) {
+                consume(s);
+            }
+        }
+        if (PERSIST && s < 0 && tid == NT - 64) *s_item = nxt;
+        __syncthreads();
+    }
+    // scatter: tile element (4 r + lq, li) -> K[cols[I 16 + 4 r + lq]][cols[J 16 + li]]
+    double* Km = K + B.poff;
+    const int64_t N = B.ldp;
+#pragma unroll
+    for (int m = 0; m < NPW; ++m) {
+        if (!has[m]) continue;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            if (((t & 1) && !two[m]) || (t == 2 && !off[m])) continue;
+            const int lc = ((t >> 1) ? j1[m] : j0[m]) + li;
+            const int gj = s_cols[lc];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int lr = ((t & 1) ? i1[m] : i0[m]) + 4 * r + lq;
+                const int gi = s_cols[lr];
+                if (gi >= 0 && gj >= 0 && lr >= lc) atomicAdd(Km + (int64_t)gi * N + gj, acc[m][t][r]);
+            }
+        }
     }
 }
 
-template <bool PERSIST>
-__global__ __launch_bounds__(768) void k_kmat(const KWork* __restrict__ work, const BlockDesc* __restrict__ blocks,
+// Workgroup shapes by the block's tile count T: up to 8 tiles (10
+// patches) 4 waves, up to 10 (15 patches) 8, wider 12 (36 patches are T = 16).
+template <int NW, int NPW, bool PERSIST>
+__global__ __launch_bounds__(NW * 64, NW == 8 ? 4 : 3) void k_kmat(const KWork* __restrict__ work, const BlockDesc* __restrict__ blocks,
                                               const double* __restrict__ pts, int64_t n_slots,
                                               const double* __restrict__ shrec, int RS,
                                               const int* __restrict__ bshells, const int* __restrict__ bshell_col,
                                               const int* __restrict__ bcols, const int* __restrict__ bsorder,
-                                              const double* __restrict__ coef, double* __restrict__ K, int N,
+                                              const double* __restrict__ coef, double* __restrict__ K,
                                               int* __restrict__ queue, int n_items) {
     __shared__ double s_pt[kBlockPts][3];
     __shared__ double s_cf[kBlockPts][4];
-    extern __shared__ double s_dynd[];
+    __shared__ int s_pcount[2];
+    extern __shared__ __attribute__((aligned(16))) double s_dynd[];
     if constexpr (PERSIST) {
         __shared__ int s_item;
-        for (int iter = 0;; ++iter) {
-            const int item = next_item(queue, n_items, iter, &s_item);
-            if (item >= n_items) break;
-            k_kmat_item(item, work, blocks, pts, n_slots, shrec, RS, bshells, bshell_col, bcols, bsorder, coef, K, N, s_pt, s_cf, s_dynd);
+        int item = __builtin_amdgcn_readfirstlane(next_item(queue, n_items, 0, &s_item));
+        while (item < n_items) {
+            k_kmat_item<NW, NPW, true>(item, work, blocks, pts, n_slots, shrec, RS, bshells, bshell_col, bcols, bsorder,
+                                       coef, K, queue, s_pt, s_cf, s_pcount, &s_item, s_dynd);
+            __syncthreads();  // the item's LDS is no longer read
+            item = __builtin_amdgcn_readfirstlane(s_item);
         }
     } else {
-        k_kmat_item((int)blockIdx.x, work, blocks, pts, n_slots, shrec, RS, bshells, bshell_col, bcols, bsorder, coef, K, N, s_pt, s_cf, s_dynd);
+        k_kmat_item<NW, NPW, false>((int)blockIdx.x, work, blocks, pts, n_slots, shrec, RS, bshells, bshell_col, bcols,
+                                    bsorder, coef, K, nullptr, s_pt, s_cf, s_pcount, nullptr, s_dynd);
     }
 }
 
@@ -1146,27 +1175,27 @@ int launch_xc_points_uks(Context& c, int xc_type) {
     return check_launch("k_xc_points_uks");
 }
 
+template <int NW, int NPW>
 static int kmat_one(Context& c, const LaunchRange& r) {
     unsigned grid = 0;
-    int* q = launch_queue(c, kQueueK, r.count, resident_per_cu(&k_kmat<true>, 768, r.lds), &grid);
-    if (q)
-        hipLaunchKernelGGL(k_kmat<true>, dim3(grid), dim3(768), r.lds, c.stream,
+    int* q = launch_queue(c, kQueueK, r.count, resident_per_cu(&k_kmat<NW, NPW, true>, NW * 64, r.lds), &grid);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(NW * 64), r.lds, c.stream,
                            reinterpret_cast<const KWork*>(c.d_k_work) + r.offset, c.d_blocks, c.d_pts,
                            c.n_slots, c.d_shrec, c.rec_stride, c.d_block_shells, c.d_block_shell_col,
-                           c.d_block_cols, c.d_block_sorder, c.d_coef, c.d_K, c.n_aos, q, r.count);
-    else
-        hipLaunchKernelGGL(k_kmat<false>, dim3(grid), dim3(768), r.lds, c.stream,
-                           reinterpret_cast<const KWork*>(c.d_k_work) + r.offset, c.d_blocks, c.d_pts,
-                           c.n_slots, c.d_shrec, c.rec_stride, c.d_block_shells, c.d_block_shell_col,
-                           c.d_block_cols, c.d_block_sorder, c.d_coef, c.d_K, c.n_aos, q, r.count);
+                           c.d_block_cols, c.d_block_sorder, c.d_coef, c.d_K, q, r.count);
+    };
+    if (q) launch(k_kmat<NW, NPW, true>);
+    else launch(k_kmat<NW, NPW, false>);
     return check_launch("k_kmat");
 }
 
 int launch_kmat(Context& c, const LaunchRange& r) {
     if (r.count <= 0) return PDFXC_OK;
     switch (r.cls) {
-        case 0:
-        case 1: return kmat_one(c, r);
+        case 0: return kmat_one<4, 3>(c, r);
+        case 1: return kmat_one<8, 2>(c, r);
+        case 2: return kmat_one<12, 3>(c, r);
         default: set_error("k_kmat: bad class"); return PDFXC_ERR_ARGUMENT;
     }
 }
