@@ -440,23 +440,14 @@ __global__ __launch_bounds__(256) void k_screen_blocks(int nb, int64_t n, const 
     }
 }
 
-// The lists and slots of every block (one wave per block, in launch order):
-// kept shells in ascending order with their columns, the order by (l, nprim)
-// class, the points (a partial block repeats its last one with weight 0).
-__global__ __launch_bounds__(256) void k_fill_blocks(int nb, int64_t n, int64_t n_slots, const double* __restrict__ grid,
-                                                     const int* __restrict__ order, const int* __restrict__ leaf,
-                                                     const BlockDesc* __restrict__ blocks, int nw, int ncls,
-                                                     const ScreenShell* __restrict__ shells,
-                                                     const unsigned long long* __restrict__ masks,
-                                                     int* __restrict__ bshells, int* __restrict__ bshell_col,
-                                                     int* __restrict__ bcols, int* __restrict__ bsorder,
-                                                     double* __restrict__ pts, int* __restrict__ slot_of_point) {
-    const int b = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (b >= nb) return;
-    const BlockDesc B = blocks[b];
-    const int lf = leaf[b];
+// Lists of one shell mask (by one wave): kept shells in ascending order with
+// their columns, and their order by (l, nprim) class.
+__device__ __forceinline__ void fill_lists(const unsigned long long* mask, int shell_begin, int col_begin, int nw, int ncls,
+                                           const ScreenShell* __restrict__ shells, int* __restrict__ bshells,
+                                           int* __restrict__ bshell_col, int* __restrict__ bcols,
+                                           int* __restrict__ bsorder) {
+    const int lane = threadIdx.x & 63;
     const unsigned long long below = (1ull << lane) - 1ull;
-    const unsigned long long* mask = masks + (int64_t)lf * nw;
     int pos0 = 0, col0 = 0;
     for (int w = 0; w < nw; ++w) {
         const unsigned long long m = mask[w];
@@ -471,9 +462,9 @@ __global__ __launch_bounds__(256) void k_fill_blocks(int nb, int64_t n, int64_t 
         if (keep) {
             const int pos = pos0 + __popcll(m & below);
             const int col = col0 + __popcll(m & below) + 2 * __popcll(m1 & below) + 4 * __popcll(m2 & below);
-            bshells[B.shell_begin + pos] = s;
-            bshell_col[B.shell_begin + pos] = col;
-            for (int q = 0; q < 2 * l + 1; ++q) bcols[B.col_begin + col + q] = first + q;
+            bshells[shell_begin + pos] = s;
+            bshell_col[shell_begin + pos] = col;
+            for (int q = 0; q < 2 * l + 1; ++q) bcols[col_begin + col + q] = first + q;
         }
         pos0 += __popcll(m);
         col0 += __popcll(m) + 2 * __popcll(m1) + 4 * __popcll(m2);
@@ -485,11 +476,29 @@ __global__ __launch_bounds__(256) void k_fill_blocks(int nb, int64_t n, int64_t 
             const unsigned long long m = mask[w];
             const bool keep = ((m >> lane) & 1ull) && shells[w * 64 + lane].cls == c;
             const unsigned long long mc = __ballot(keep);
-            if (keep) bsorder[B.shell_begin + out + __popcll(mc & below)] = pos0 + __popcll(m & below);
+            if (keep) bsorder[shell_begin + out + __popcll(mc & below)] = pos0 + __popcll(m & below);
             out += __popcll(mc);
             pos0 += __popcll(m);
         }
     }
+}
+
+// The lists and slots of every block (one wave per block, in launch order; a
+// partial block repeats its last point with weight 0).
+__global__ __launch_bounds__(256) void k_fill_blocks(int nb, int64_t n, int64_t n_slots, const double* __restrict__ grid,
+                                                     const int* __restrict__ order, const int* __restrict__ leaf,
+                                                     const BlockDesc* __restrict__ blocks, int nw, int ncls,
+                                                     const ScreenShell* __restrict__ shells,
+                                                     const unsigned long long* __restrict__ masks,
+                                                     int* __restrict__ bshells, int* __restrict__ bshell_col,
+                                                     int* __restrict__ bcols, int* __restrict__ bsorder,
+                                                     double* __restrict__ pts, int* __restrict__ slot_of_point) {
+    const int b = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (b >= nb) return;
+    const BlockDesc B = blocks[b];
+    const int lf = leaf[b];
+    fill_lists(masks + (int64_t)lf * nw, B.shell_begin, B.col_begin, nw, ncls, shells, bshells, bshell_col, bcols,
+               bsorder);
     for (int k = lane; k < kBlockPts; k += 64) {
         const int p = order[lf * kBlockPts + min(k, B.npts - 1)];
         const int64_t slot = (int64_t)b * kBlockPts + k;
@@ -501,13 +510,52 @@ __global__ __launch_bounds__(256) void k_fill_blocks(int nb, int64_t n, int64_t 
     }
 }
 
+// Shells of `per` neighbouring leaves together (one wave per group): the union
+// of their masks and its shell and AO counts.
+__global__ __launch_bounds__(256) void k_group_masks(int nb, int per, int nsh, const ScreenShell* __restrict__ shells,
+                                                     int nw, const unsigned long long* __restrict__ masks,
+                                                     unsigned long long* __restrict__ gmasks, int* __restrict__ counts) {
+    const int g = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int l0 = g * per, l1 = min(nb, l0 + per);
+    if (l0 >= nb) return;
+    int nshell = 0, nao = 0;
+    for (int w = 0; w < nw; ++w) {
+        unsigned long long m = 0;
+        for (int lf = l0; lf < l1; ++lf) m |= masks[(int64_t)lf * nw + w];
+        const int s = w * 64 + lane;
+        const bool keep = s < nsh && ((m >> lane) & 1ull);
+        const int l = keep ? shells[s].l : 0;
+        nshell += __popcll(m);
+        nao += __popcll(m) + 2 * __popcll(__ballot(keep && l == 1)) + 4 * __popcll(__ballot(keep && l == 2));
+        if (lane == 0) gmasks[(int64_t)g * nw + w] = m;
+    }
+    if (lane == 0) {
+        counts[2 * g] = nshell;
+        counts[2 * g + 1] = nao;
+    }
+}
+
+// The lists of the K units that hold several blocks: group[u] >= 0 is the mask
+// of unit u (one wave per unit; the others have the lists of their block).
+__global__ __launch_bounds__(256) void k_fill_groups(int n, const int* __restrict__ group,
+                                                     const KBlock* __restrict__ units, int nw, int ncls,
+                                                     const ScreenShell* __restrict__ shells,
+                                                     const unsigned long long* __restrict__ gmasks,
+                                                     int* __restrict__ bshells, int* __restrict__ bshell_col,
+                                                     int* __restrict__ bcols, int* __restrict__ bsorder) {
+    const int u = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (u >= n || group[u] < 0) return;
+    fill_lists(gmasks + (int64_t)group[u] * nw, units[u].shell_begin, units[u].col_begin, nw, ncls, shells, bshells,
+               bshell_col, bcols, bsorder);
+}
+
 // shells of each K item: those whose first column lies below the item's columns
 __global__ __launch_bounds__(256) void k_item_shells(int n, const KWork* __restrict__ work,
-                                                     const BlockDesc* __restrict__ blocks,
+                                                     const KBlock* __restrict__ units,
                                                      const int* __restrict__ bshell_col, int* __restrict__ nsh) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
-    const BlockDesc B = blocks[work[i].block];
+    const KBlock& B = units[work[i].block];
     int lo = 0, hi = B.nshell;
     while (lo < hi) {
         const int m = (lo + hi) / 2;
@@ -680,9 +728,24 @@ int launch_fill_blocks(Context& c, const int* d_order, const int* d_leaf, int nw
     return check("k_fill_blocks");
 }
 
+int launch_group_masks(int nb, int per, int nsh, const ScreenShell* d_shells, int nw,
+                       const unsigned long long* d_masks, unsigned long long* d_gmasks, int* d_gcounts, hipStream_t s) {
+    const int ng = (nb + per - 1) / per;
+    hipLaunchKernelGGL(k_group_masks, dim3((ng + 3) / 4), dim3(256), 0, s, nb, per, nsh, d_shells, nw, d_masks, d_gmasks,
+                       d_gcounts);
+    return check("k_group_masks");
+}
+
+int launch_fill_groups(Context& c, int n, const int* d_group, int nw, int ncls, const ScreenShell* d_shells,
+                       const unsigned long long* d_gmasks) {
+    hipLaunchKernelGGL(k_fill_groups, dim3((n + 3) / 4), dim3(256), 0, c.stream, n, d_group, c.d_kblocks, nw, ncls,
+                       d_shells, d_gmasks, c.d_block_shells, c.d_block_shell_col, c.d_block_cols, c.d_block_sorder);
+    return check("k_fill_groups");
+}
+
 int launch_item_shells(Context& c, int n, const KWork* d_work, int* d_nsh) {
     if (n <= 0) return PDFXC_OK;
-    hipLaunchKernelGGL(k_item_shells, dim3(blocks256(n)), dim3(256), 0, c.stream, n, d_work, c.d_blocks,
+    hipLaunchKernelGGL(k_item_shells, dim3(blocks256(n)), dim3(256), 0, c.stream, n, d_work, c.d_kblocks,
                        c.d_block_shell_col, d_nsh);
     return check("k_item_shells");
 }

@@ -336,6 +336,7 @@ static void free_grid_buffers(Context* c) {
     dfree(c->d_pts);
     dfree(c->d_slot_of_point);
     dfree(c->d_blocks);
+    dfree(c->d_kblocks);
     dfree(c->d_block_shells);
     dfree(c->d_block_cols);
     dfree(c->d_block_shell_col);
@@ -486,6 +487,7 @@ static void reset_grid(Context& c) {
     c.gw.clear();
     c.gen_atom.clear();
     c.blocks.clear();
+    c.kblocks.clear();
     c.block_shells.clear();
     c.block_cols.clear();
     c.block_shell_col.clear();
@@ -517,6 +519,11 @@ static void reset_grid(Context& c) {
 }
 
 static int build_blocks_impl(Context& c);
+
+// dynamic LDS of a k_kmat item
+static size_t kmat_lds(int ps, int ncols, int nsh, int rec_stride) {
+    return sizeof(double) * (4 * (size_t)ps * ncols + (size_t)nsh * rec_stride) + sizeof(int) * (size_t)(ncols + 2 * nsh);
+}
 
 // Blocks, work lists and device buffers of the context's grid; on failure the
 // context is left with no grid (nothing half-built stays reachable).
@@ -590,19 +597,30 @@ static int build_blocks_impl(Context& c) {
             sc[k].pad = 0;
         }
     }
-    // workspace: order | masks | counts | leaf of every block | shell table
+    // Blocks per K unit: the FP64 K pass adds N_b^2 / 2 values to K by atomics
+    // per unit, at 53 G/s a longer time than its matrix products, and the
+    // union of two neighbours is only 2 % wider than either
+    int kper = c.opts.precision == PDFXC_FP64 ? std::min(kKGroupMax, c.tune.split_k_group) : 1;
+    while (kper > 1 && nb / kper < kKUnitsPerCu * c.n_cu) kper /= 2;
+    const int ng = kper > 1 ? (nb + kper - 1) / kper : 0;
+    // workspace: order | masks | counts | leaf of every block | shell table | masks and unit list of the groups
     auto align = [](size_t b) { return (b + 255) / 256 * 256; };
     const size_t b_order = align(sizeof(int) * (size_t)n), b_mask = align(sizeof(unsigned long long) * (size_t)nb * nw),
                  b_cnt = align(2 * sizeof(int) * (size_t)nb), b_leaf = align(sizeof(int) * (size_t)nb),
-                 b_sc = align(sizeof(ScreenShell) * (size_t)nsh);
+                 b_sc = align(sizeof(ScreenShell) * (size_t)nsh),
+                 b_gmask = align(sizeof(unsigned long long) * (size_t)ng * nw),
+                 b_gcnt = align(2 * sizeof(int) * (size_t)ng);
     DeviceBuf ws;
-    int rc = ws.alloc(b_order + b_mask + b_cnt + b_leaf + b_sc);
+    int rc = ws.alloc(b_order + b_mask + b_cnt + b_leaf + b_sc + b_gmask + b_gcnt + (ng ? b_leaf : 0));
     if (rc) return rc;
     int* d_order = ws.as<int>();
     unsigned long long* d_masks = reinterpret_cast<unsigned long long*>(ws.as<char>() + b_order);
     int* d_counts = reinterpret_cast<int*>(ws.as<char>() + b_order + b_mask);
     int* d_leaf = reinterpret_cast<int*>(ws.as<char>() + b_order + b_mask + b_cnt);
     ScreenShell* d_sc = reinterpret_cast<ScreenShell*>(ws.as<char>() + b_order + b_mask + b_cnt + b_leaf);
+    unsigned long long* d_gmasks = reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(d_sc) + b_sc);
+    int* d_gcounts = reinterpret_cast<int*>(reinterpret_cast<char*>(d_gmasks) + b_gmask);
+    int* d_group = reinterpret_cast<int*>(reinterpret_cast<char*>(d_gcounts) + b_gcnt);
     std::vector<int> order;
     if (c.opts.precision == PDFXC_FP64) {
         rc = device_partition(n, c.d_grid, d_order, c.stream);
@@ -615,7 +633,12 @@ static int build_blocks_impl(Context& c) {
     PDFXC_HIP(hipMemcpyAsync(d_sc, sc.data(), sizeof(ScreenShell) * (size_t)nsh, hipMemcpyHostToDevice, c.stream));
     rc = launch_screen_blocks(nb, n, c.d_grid, d_order, nsh, d_sc, nw, d_masks, d_counts, c.stream);
     if (rc) return rc;
-    std::vector<int> counts(2 * (size_t)nb);
+    std::vector<int> counts(2 * (size_t)nb), gcounts(2 * (size_t)ng);
+    if (ng) {
+        rc = launch_group_masks(nb, kper, nsh, d_sc, nw, d_masks, d_gmasks, d_gcounts, c.stream);
+        if (rc) return rc;
+        PDFXC_HIP(hipMemcpyAsync(gcounts.data(), d_gcounts, 2 * sizeof(int) * (size_t)ng, hipMemcpyDeviceToHost, c.stream));
+    }
     PDFXC_HIP(hipMemcpyAsync(counts.data(), d_counts, 2 * sizeof(int) * (size_t)nb, hipMemcpyDeviceToHost, c.stream));
     PDFXC_HIP(hipStreamSynchronize(c.stream));
 
@@ -661,11 +684,66 @@ static int build_blocks_impl(Context& c) {
         c.max_nao = std::max(c.max_nao, B.nao);
     }
     c.mean_nao = nb ? sum_nao / nb : 0.0;
+    // units of k_kmat: the groups, or the blocks of a group whose union would
+    // not fit a workgroup's LDS, in descending order of cost
+    const int RS = c.rec_stride;
+    c.kblocks.clear();
+    auto unit_of = [&](int li) {
+        const BlockDesc& B = c.blocks[li];
+        return KBlock{{B.pt_begin}, B.npts, B.shell_begin, B.nshell, B.nao, B.ldn, B.col_begin, B.ldp, 0, B.poff};
+    };
+    std::vector<int> unit_group;  // mask of a unit of several blocks, else -1
+    if (!ng) {
+        for (int li = 0; li < nb; ++li) c.kblocks.push_back(unit_of(li));
+    } else {
+        std::vector<int> block_of_leaf(nb);
+        for (int li = 0; li < nb; ++li) block_of_leaf[lorder[li]] = li;
+        std::vector<KBlock> units;
+        std::vector<int> ugroup;
+        for (int g = 0; g < ng; ++g) {
+            const int l0 = g * kper, l1 = std::min(nb, l0 + kper);
+            KBlock U{};
+            U.nshell = gcounts[2 * g];
+            U.nao = gcounts[2 * g + 1];
+            U.ldn = padded(U.nao);
+            U.ldp = c.n_aos;
+            if (l1 - l0 == 1 || kmat_lds(8, U.ldn, U.nshell, RS) > kKmatLds[kKmatClasses - 1]) {
+                for (int lf = l0; lf < l1; ++lf) {
+                    units.push_back(unit_of(block_of_leaf[lf]));
+                    ugroup.push_back(-1);
+                }
+                continue;
+            }
+            for (int lf = l0; lf < l1; ++lf) {
+                const BlockDesc& B = c.blocks[block_of_leaf[lf]];
+                U.slot[lf - l0] = B.pt_begin;
+                U.npts += B.npts;  // only the grid's last leaf is partial
+            }
+            units.push_back(U);
+            ugroup.push_back(g);
+        }
+        std::vector<int> uorder(units.size());
+        std::iota(uorder.begin(), uorder.end(), 0);
+        auto ucost = [&](int u) { return (int64_t)units[u].npts * units[u].ldn * units[u].ldn; };
+        std::stable_sort(uorder.begin(), uorder.end(), [&](int x, int y) { return ucost(x) > ucost(y); });
+        for (int u : uorder) {
+            if (ugroup[u] >= 0) {
+                units[u].shell_begin = (int)sh0;
+                units[u].col_begin = (int)col0;
+                sh0 += units[u].nshell;
+                col0 += units[u].nao;
+            }
+            c.kblocks.push_back(units[u]);
+            unit_group.push_back(ugroup[u]);
+        }
+    }
+    const int nu = (int)c.kblocks.size();
     c.n_block_shells = sh0;
     c.n_block_cols = col0;
     rc = dalloc(&c.d_pts, 4 * (size_t)c.n_slots);
     if (rc == PDFXC_OK) rc = dalloc(&c.d_slot_of_point, (size_t)n);
     if (rc == PDFXC_OK) rc = dalloc(&c.d_blocks, c.blocks.size());
+    if (rc == PDFXC_OK) rc = dalloc(&c.d_kblocks, c.kblocks.size());
     if (rc == PDFXC_OK) rc = dalloc(&c.d_block_shells, (size_t)sh0);
     if (rc == PDFXC_OK) rc = dalloc(&c.d_block_cols, (size_t)col0);
     if (rc == PDFXC_OK) rc = dalloc(&c.d_block_shell_col, (size_t)sh0);
@@ -673,8 +751,14 @@ static int build_blocks_impl(Context& c) {
     if (rc) return rc;
     PDFXC_HIP(hipMemcpyAsync(c.d_blocks, c.blocks.data(), sizeof(BlockDesc) * (size_t)nb, hipMemcpyHostToDevice, c.stream));
     PDFXC_HIP(hipMemcpyAsync(d_leaf, lorder.data(), sizeof(int) * (size_t)nb, hipMemcpyHostToDevice, c.stream));
+    PDFXC_HIP(hipMemcpyAsync(c.d_kblocks, c.kblocks.data(), sizeof(KBlock) * (size_t)nu, hipMemcpyHostToDevice, c.stream));
     rc = launch_fill_blocks(c, d_order, d_leaf, nw, ncls, d_sc, d_masks);
     if (rc) return rc;
+    if (ng) {
+        PDFXC_HIP(hipMemcpyAsync(d_group, unit_group.data(), sizeof(int) * (size_t)nu, hipMemcpyHostToDevice, c.stream));
+        rc = launch_fill_groups(c, nu, d_group, nw, ncls, d_sc, d_gmasks);
+        if (rc) return rc;
+    }
     PDFXC_HIP(hipStreamSynchronize(c.stream));
 
     // k_rho work lists by template class: ldn <= 128 (64 points per
@@ -683,7 +767,6 @@ static int build_blocks_impl(Context& c) {
     // classes (fewer points per workgroup; ldn <= 256 then takes 16)
     std::vector<int> rho_work;
     c.rho_launches.clear();
-    const int RS = c.rec_stride;
     auto rho_lds = [&](const BlockDesc& B, size_t pb) {
         return sizeof(double) * (std::max<size_t>((size_t)B.ldn * pb, 4 * 512) + (size_t)B.nshell * RS) +
                sizeof(int) * (size_t)(B.ldn + 2 * B.nshell);
@@ -718,14 +801,14 @@ static int build_blocks_impl(Context& c) {
         r.lds = maxdyn;
         if (r.count) c.rho_launches.push_back(r);
     }
-    // k_kmat work: the lower 2 x 2 tile patches of a block, row-major, in one
+    // k_kmat work: the lower 2 x 2 tile patches of a unit, row-major, in one
     // item where a workgroup shape holds them (10 of 12, 15 of 16 or 36
     // patches: at most 8, 10 or 16 tiles a side), else in items of at most 36
     // (k_tiles = 96; the tuning may cut those smaller)
     std::vector<KWork> kw[kKmatClasses];
     size_t klds[kKmatClasses] = {};
-    for (int b = 0; b < nb; ++b) {
-        const BlockDesc& B = c.blocks[b];
+    for (int b = 0; b < nu; ++b) {
+        const KBlock& B = c.kblocks[b];
         const int T = B.ldn / 16, Tp = (T + 1) / 2;
         const int np = Tp * (Tp + 1) / 2;
         const int cls = T <= 8 ? 0 : T <= 10 ? 1 : 2;
@@ -764,10 +847,7 @@ static int build_blocks_impl(Context& c) {
     for (int cls = 0, at = 0; cls < kKmatClasses; ++cls)
         for (KWork& w : kw[cls]) {
             w.nsh = item_nsh[at++];
-            auto lds_of = [&](int ps) {
-                return sizeof(double) * (4 * (size_t)ps * w.ncols + (size_t)w.nsh * RS) +
-                       sizeof(int) * (size_t)(w.ncols + 2 * w.nsh);
-            };
+            auto lds_of = [&](int ps) { return kmat_lds(ps, w.ncols, w.nsh, RS); };
             w.ps = 16;
             if (lds_of(16) > kKmatLds[cls]) w.ps = lds_of(8) <= kKmatLds[kKmatClasses - 1] ? 8 : 4;
             const size_t lds = lds_of(w.ps);
@@ -2549,7 +2629,7 @@ int pdfxc_batch_create(pdfxc_batch** out, int n_mol, pdfxc_ctx* const* ctxs) {
     int64_t psoff = 0;
     int shell_base = 0, nblocks = 0;
     int64_t slot_base = 0;
-    std::vector<int> block_base(n_mol), slot_first(n_mol), group_base(n_mol, 0);
+    std::vector<int> block_base(n_mol), kblock_base(n_mol), slot_first(n_mol), group_base(n_mol, 0);
     for (int i = 0; i < n_mol; ++i) {
         const Context& c = *reinterpret_cast<const Context*>(ctxs[i]);
         const int N = c.n_aos;
@@ -2588,6 +2668,15 @@ int pdfxc_batch_create(pdfxc_batch** out, int n_mol, pdfxc_ctx* const* ctxs) {
                 SB.chunk_begin += chunk_list;
                 m.sblocks.push_back(SB);
             }
+        }
+        kblock_base[i] = (int)m.kblocks.size();
+        for (KBlock U : c.kblocks) {
+            for (int& s : U.slot) s += (int)slot_base;
+            U.shell_begin += sh_list;
+            U.col_begin += col_list;
+            U.ldp = N;
+            U.poff = b->doff.back();
+            m.kblocks.push_back(U);
         }
         for (int s : c.block_shells) m.block_shells.push_back(s + shell_base);
         m.block_shell_col.insert(m.block_shell_col.end(), c.block_shell_col.begin(), c.block_shell_col.end());
@@ -2683,7 +2772,7 @@ int pdfxc_batch_create(pdfxc_batch** out, int n_mol, pdfxc_ctx* const* ctxs) {
                     const std::vector<KWork>& L = get_list(c);
                     for (int k = 0; k < q.count; ++k) {
                         KWork w = L[q.offset + k];
-                        w.block += block_base[i];
+                        w.block += kblock_base[i];
                         out_list.push_back(w);
                     }
                     r.lds = std::max(r.lds, q.lds);
@@ -2740,6 +2829,7 @@ int pdfxc_batch_create(pdfxc_batch** out, int n_mol, pdfxc_ctx* const* ctxs) {
     if (rc == PDFXC_OK) rc = dalloc(&m.d_queue, kMaxQueues);
     if (rc == PDFXC_OK) rc = dalloc(&m.d_pts, soa.size());
     if (rc == PDFXC_OK) rc = dalloc(&m.d_blocks, m.blocks.size());
+    if (rc == PDFXC_OK) rc = dalloc(&m.d_kblocks, m.kblocks.size());
     if (rc == PDFXC_OK) rc = dalloc(&m.d_block_shells, std::max<size_t>(1, m.block_shells.size()));
     if (rc == PDFXC_OK) rc = dalloc(&m.d_block_cols, std::max<size_t>(1, m.block_cols.size()));
     if (rc == PDFXC_OK) rc = dalloc(&m.d_block_shell_col, std::max<size_t>(1, m.block_shell_col.size()));
@@ -2769,6 +2859,7 @@ int pdfxc_batch_create(pdfxc_batch** out, int n_mol, pdfxc_ctx* const* ctxs) {
     up(m.d_shrec, rec);
     up(m.d_pts, soa);
     up(m.d_blocks, m.blocks);
+    up(m.d_kblocks, m.kblocks);
     up(m.d_block_shells, m.block_shells);
     up(m.d_block_cols, m.block_cols);
     up(m.d_block_shell_col, m.block_shell_col);

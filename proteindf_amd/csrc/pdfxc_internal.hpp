@@ -69,16 +69,33 @@ struct SplitBlock {
     int chunk_begin, nchunk, ldnp, pad;
 };
 
-// One k_kmat work item: lower 2 x 2 tile patches [t0, t1) of a block, row-major,
+// K pass work unit of k_kmat: 1 to kKGroupMax blocks, neighbours in the point
+// bisection, on the union of their shells; all of them but the last full.
+constexpr int kKGroupMax = 2;
+// Units of two blocks where that leaves this many per CU.  K pass with one and
+// two blocks a unit: 37.0 and 28.1 ms (79,000 blocks, a 30-residue helix), 4.0
+// and 3.4 ms (10,600 blocks, 10 residues), but 0.234 and 0.240 ms (3,200
+// blocks, 8 waters) and 0.42 and 0.75 ms (2,800 blocks, UKS, 12 waters), whose
+// last round of workgroups is then nearly empty.
+constexpr int kKUnitsPerCu = 10;
+struct KBlock {
+    int slot[kKGroupMax];  // first slot of every block
+    int npts;              // real points of all of them
+    int shell_begin, nshell, nao, ldn, col_begin;  // as in BlockDesc
+    int ldp, pad;
+    int64_t poff;
+};
+
+// One k_kmat work item: lower 2 x 2 tile patches [t0, t1) of a KBlock, row-major,
 // on its first ncols columns and nsh shells, in slabs of ps points.
 struct KWork {
     int block, t0, t1, ncols, nsh, ps;
 };
 // k_kmat workgroup shapes (4, 8 and 12 waves) and the dynamic LDS with which
-// 3, 2 and 1 of them share a CU's 160 KiB (7184 bytes of static LDS each,
+// 3, 2 and 1 of them share a CU's 160 KiB (under 2 KiB of static LDS each,
 // granules of 1280)
 constexpr int kKmatClasses = 3;
-constexpr size_t kKmatLds[kKmatClasses] = {45 * 1024, 72 * 1024, 152 * 1024};
+constexpr size_t kKmatLds[kKmatClasses] = {50 * 1024, 77 * 1024, 157 * 1024};
 
 // A launch of one kernel instantiation over a contiguous range of a work list.
 struct LaunchRange {
@@ -154,7 +171,8 @@ struct Context {
     std::vector<BlockDesc> blocks;     // launch order (descending cost)
     // host copies of the block lists and slots, made by ensure_host_lists and
     // ensure_host_slots (a batch's are its own)
-    int64_t n_block_shells = 0, n_block_cols = 0;
+    int64_t n_block_shells = 0, n_block_cols = 0;  // those of the K units of several blocks included
+    std::vector<KBlock> kblocks;       // units of k_kmat, in launch order
     std::vector<int> block_shells;     // global shell ids per block
     std::vector<int> block_cols;       // global AO index per block column
     std::vector<int> block_shell_col;  // local first column of each block shell
@@ -173,6 +191,7 @@ struct Context {
     int64_t n_slots = 0;
     int* d_slot_of_point = nullptr;
     BlockDesc* d_blocks = nullptr;
+    KBlock* d_kblocks = nullptr;
     int* d_block_shells = nullptr;
     int* d_block_cols = nullptr;
     int* d_block_shell_col = nullptr;
@@ -280,6 +299,11 @@ int launch_screen_blocks(int nb, int64_t n, const double* d_grid, const int* d_o
                          hipStream_t s);
 int launch_fill_blocks(Context& c, const int* d_order, const int* d_leaf, int nw, int ncls,
                        const ScreenShell* d_shells, const unsigned long long* d_masks);
+// shells of blocks [g per, (g + 1) per) together: masks, (shells, AOs) counts, lists of c.kblocks
+int launch_group_masks(int nb, int per, int nsh, const ScreenShell* d_shells, int nw,
+                       const unsigned long long* d_masks, unsigned long long* d_gmasks, int* d_gcounts, hipStream_t s);
+int launch_fill_groups(Context& c, int n, const int* d_group, int nw, int ncls, const ScreenShell* d_shells,
+                       const unsigned long long* d_gmasks);
 int launch_item_shells(Context& c, int n, const KWork* d_work, int* d_nsh);
 // four values per point between the slots and the caller's order (row stride and offset of the latter)
 int launch_gather_points(Context& c, const double* d_slots, double* d_pts, int stride, int off);

@@ -670,8 +670,9 @@ __global__ __launch_bounds__(256) void k_xc_points_uks(int64_t n_slots, const do
 }
 
 // ---------------------------------------------------------------------------
-// K pass: K_bb += Phi^T V + V^T Phi for a run [t0, t1) of lower 2 x 2 patches
-// of 16 x 16 tiles of one block, row-major (patch (P, Q), Q <= P, is number
+// K pass: K_uu += Phi^T V + V^T Phi for a run [t0, t1) of lower 2 x 2 patches
+// of 16 x 16 tiles of one unit (1 to kKGroupMax neighbouring blocks on the
+// union of their AO columns), row-major (patch (P, Q), Q <= P, is number
 // P (P + 1) / 2 + Q).  Patch t0 + wave + NW m belongs to wave `wave`: NPW of
 // them at most, four accumulator tiles each (a diagonal patch runs three, the
 // last row of an odd tile count two or one; wave-uniform branches skip the
@@ -685,8 +686,10 @@ __global__ __launch_bounds__(256) void k_xc_points_uks(int64_t n_slots, const do
 // Measured (MI355X): before, 8 consumer and 4 producer waves ran over a linear
 // list of tiles, two operand reads per MFMA, and either half alone took 85 %
 // of the pass.  K pass of 8 waters 0.47 -> 0.22 ms, of a 10-residue helix
-// 4.6 -> 4.0 ms, of a 30-residue helix 43.1 -> 36.9 ms; what is left of the
-// wide ones are the scatter's atomics (26.6 ms without them).
+// 4.6 -> 4.0 ms, of a 30-residue helix 43.1 -> 36.9 ms, there bound by the
+// scatter's atomics (26.6 ms without them); with two blocks a unit 3.4 and
+// 28.1 ms, 26.9 without the scatter, 22.5 without the production and 18.4
+// without the products, whose MFMAs alone take 17.
 // Slab element (point p, column c) is at p LD + (c ^ (p & 15)): the 16 lanes
 // of an operand read stay on one 256-byte run, and a producer's 16 points of
 // one column fall on 16 different 16-byte slots.
@@ -698,16 +701,16 @@ struct KOperands {
 };
 
 template <int NW, int NPW, bool PERSIST>
-__device__ __forceinline__ void k_kmat_item(int item, const KWork* __restrict__ work, const BlockDesc* __restrict__ blocks,
+__device__ __forceinline__ void k_kmat_item(int item, const KWork* __restrict__ work, const KBlock* __restrict__ units,
                                               const double* __restrict__ pts, int64_t n_slots,
                                               const double* __restrict__ shrec, int RS,
                                               const int* __restrict__ bshells, const int* __restrict__ bshell_col,
                                               const int* __restrict__ bcols, const int* __restrict__ bsorder,
                                               const double* __restrict__ coef, double* __restrict__ K,
-        int* __restrict__ queue, double (*s_pt)[3], double (*s_cf)[4], int* s_pcount, int* s_item, double* s_dynd) {
+        int* __restrict__ queue, double (*s_pt)[7][16], int* s_pcount, int* s_item, double* s_dynd) {
     constexpr int NT = NW * 64;
     const KWork W = work[item];
-    const BlockDesc B = blocks[W.block];
+    const KBlock& B = units[W.block];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int li = lane & 15, lq = lane >> 4;
@@ -727,9 +730,8 @@ __device__ __forceinline__ void k_kmat_item(int item, const KWork* __restrict__ 
     int* s_shid = s_shcol + nsh;
     for (int c = tid; c < ncols; c += NT) s_cols[c] = (c < B.nao) ? bcols[B.col_begin + c] : -1;
     if (tid < 2) s_pcount[tid] = 0;
-    // the next item is asked for now and published with the first slab: by the
-    // end of this one every wave has scatter atomics in flight, which the
-    // answer would wait for
+    // the next item is asked for now: by the end of this one every wave has
+    // scatter atomics in flight, which the answer would wait for
     int nxt = 0;
     if (PERSIST && tid == NT - 64) nxt = atomicAdd(queue, 1);
     // shells this item needs (local index < nsh), in (l, nprim) order, compacted by the last wave
@@ -748,24 +750,26 @@ __device__ __forceinline__ void k_kmat_item(int item, const KWork* __restrict__ 
             base += __popcll(m);
         }
     }
-    for (int p = tid; p < kBlockPts; p += NT) {
-        const int64_t slot = B.pt_begin + p;
-        s_pt[p][0] = pts[slot];
-        s_pt[p][1] = pts[n_slots + slot];
-        s_pt[p][2] = pts[2 * n_slots + slot];
-        s_cf[p][0] = coef[4 * slot + 0];
-        s_cf[p][1] = coef[4 * slot + 1];
-        s_cf[p][2] = coef[4 * slot + 2];
-        s_cf[p][3] = coef[4 * slot + 3];
-    }
+    // x, y, z and the four point terms of slab s: a value per thread, fetched a
+    // step before the slab is produced
+    const int nslab = (B.npts + PS - 1) >> ps_log;
+    const bool stage = tid < 7 * PS;
+    const int sf = tid >> ps_log, sp = tid & (PS - 1);
+    auto fetch = [&](int s) {
+        const int at = s << ps_log;
+        const int64_t slot = B.slot[at / kBlockPts] + (at & (kBlockPts - 1)) + sp;
+        return sf < 3 ? pts[sf * n_slots + slot] : coef[4 * slot + sf - 3];
+    };
+    if (stage) s_pt[0][sf][sp] = fetch(0);
     {
-        // columns past the block's AOs stay zero in both buffers: the swizzle
+        // columns past the unit's AOs stay zero in both buffers: the swizzle
         // maps the last 16 columns of a row onto themselves, so clear those
         const int z0 = min(ncols, B.nao) & ~15;
         const int nz = ncols - z0;  // 16, or 0 when the AOs fill the columns
         for (int it = tid; it < 2 * PS * nz; it += NT) s_buf[(it / nz) * LD + z0 + it % nz] = double2{0.0, 0.0};
     }
     __syncthreads();
+    if (PERSIST && tid == NT - 64) *s_item = nxt;  // every wave has read the last one
     for (int idx = tid; idx < nsh * RS; idx += NT) {
         const int k = idx / RS;
         s_rec[idx] = shrec[(int64_t)s_shid[k] * RS + (idx - k * RS)];
@@ -774,7 +778,7 @@ __device__ __forceinline__ void k_kmat_item(int item, const KWork* __restrict__ 
 
     auto produce = [&](int s) {
         double2* buf = s_buf + (s & 1) * SLAB;
-        const int pb = s * PS;
+        const auto& pt = s_pt[s & 1];
         int* pc = s_pcount + (s & 1);
         for (;;) {
             int chunk = 0;
@@ -785,15 +789,14 @@ __device__ __forceinline__ void k_kmat_item(int item, const KWork* __restrict__ 
             if (it >= nsh * PS) continue;
             const int p = it & (PS - 1);
             const int k = nsh - 1 - (it >> ps_log);  // the costliest (l, nprim) first
-            const int pp = pb + p;
             const double* rec = s_rec + k * RS;
-            const double x = s_pt[pp][0] - rec[0], y = s_pt[pp][1] - rec[1], z = s_pt[pp][2] - rec[2];
+            const double x = pt[0][p] - rec[0], y = pt[1][p] - rec[1], z = pt[2][p] - rec[2];
             double R0, R1;
             rec_radial01(rec, x, y, z, R0, R1);
             const int c0 = s_shcol[k];
             double2* row = buf + p * LD;
             const int sw = p & 15;
-            shell_phi_v(((int)rec[3]) & 3, x, y, z, R0, R1, s_cf[pp][0], s_cf[pp][1], s_cf[pp][2], s_cf[pp][3],
+            shell_phi_v(((int)rec[3]) & 3, x, y, z, R0, R1, pt[3][p], pt[4][p], pt[5][p], pt[6][p],
                         [&](int m, double v, double V) {
                             const int c = c0 + m;
                             if (c < ncols) row[c ^ sw] = double2{v, V};
@@ -858,11 +861,12 @@ __device__ __forceinline__ void k_kmat_item(int item, const KWork* __restrict__ 
 
     // step s multiplies slab s and produces slab s + 1 (one copy of either
     // body: two of them spill)
-    const int nslab = (B.npts + PS - 1) >> ps_log;
     const bool first = wave < (NW > 4 ? 4 : 2);
 #pragma unroll 1
     for (int s = -1; s < nslab; ++s) {
         if (s >= 0 && tid == 0) s_pcount[s & 1] = 0;  // slab s is in; its counter serves slab s + 2
+        const bool ahead = stage && s + 2 < nslab;
+        const double pv = ahead ? fetch(s + 2) : 0.0;
 #pragma unroll 1
         for (int ph = 0; ph < 2; ++ph) {
             if ((ph == 0) == first) {
@@ -871,7 +875,7 @@ __device__ __forceinline__ void k_kmat_item(int item, const KWork* __restrict__ 
                 consume(s);
             }
         }
-        if (PERSIST && s < 0 && tid == NT - 64) *s_item = nxt;
+        if (ahead) s_pt[s & 1][sf][sp] = pv;
         __syncthreads();
     }
     // scatter: tile element (4 r + lq, li) -> K[cols[I 16 + 4 r + lq]][cols[J 16 + li]]
@@ -895,32 +899,31 @@ __device__ __forceinline__ void k_kmat_item(int item, const KWork* __restrict__ 
     }
 }
 
-// Workgroup shapes by the block's tile count T: up to 8 tiles (10
+// Workgroup shapes by the unit's tile count T: up to 8 tiles (10
 // patches) 4 waves, up to 10 (15 patches) 8, wider 12 (36 patches are T = 16).
 template <int NW, int NPW, bool PERSIST>
-__global__ __launch_bounds__(NW * 64, NW == 8 ? 4 : 3) void k_kmat(const KWork* __restrict__ work, const BlockDesc* __restrict__ blocks,
+__global__ __launch_bounds__(NW * 64, NW == 8 ? 4 : 3) void k_kmat(const KWork* __restrict__ work, const KBlock* __restrict__ units,
                                               const double* __restrict__ pts, int64_t n_slots,
                                               const double* __restrict__ shrec, int RS,
                                               const int* __restrict__ bshells, const int* __restrict__ bshell_col,
                                               const int* __restrict__ bcols, const int* __restrict__ bsorder,
                                               const double* __restrict__ coef, double* __restrict__ K,
                                               int* __restrict__ queue, int n_items) {
-    __shared__ double s_pt[kBlockPts][3];
-    __shared__ double s_cf[kBlockPts][4];
+    __shared__ double s_pt[2][7][16];
     __shared__ int s_pcount[2];
     extern __shared__ __attribute__((aligned(16))) double s_dynd[];
     if constexpr (PERSIST) {
         __shared__ int s_item;
         int item = __builtin_amdgcn_readfirstlane(next_item(queue, n_items, 0, &s_item));
         while (item < n_items) {
-            k_kmat_item<NW, NPW, true>(item, work, blocks, pts, n_slots, shrec, RS, bshells, bshell_col, bcols, bsorder,
-                                       coef, K, queue, s_pt, s_cf, s_pcount, &s_item, s_dynd);
+            k_kmat_item<NW, NPW, true>(item, work, units, pts, n_slots, shrec, RS, bshells, bshell_col, bcols, bsorder,
+                                       coef, K, queue, s_pt, s_pcount, &s_item, s_dynd);
             __syncthreads();  // the item's LDS is no longer read
             item = __builtin_amdgcn_readfirstlane(s_item);
         }
     } else {
-        k_kmat_item<NW, NPW, false>((int)blockIdx.x, work, blocks, pts, n_slots, shrec, RS, bshells, bshell_col, bcols,
-                                    bsorder, coef, K, nullptr, s_pt, s_cf, s_pcount, nullptr, s_dynd);
+        k_kmat_item<NW, NPW, false>((int)blockIdx.x, work, units, pts, n_slots, shrec, RS, bshells, bshell_col, bcols,
+                                    bsorder, coef, K, nullptr, s_pt, s_pcount, nullptr, s_dynd);
     }
 }
 
@@ -1181,7 +1184,7 @@ static int kmat_one(Context& c, const LaunchRange& r) {
     int* q = launch_queue(c, kQueueK, r.count, resident_per_cu(&k_kmat<NW, NPW, true>, NW * 64, r.lds), &grid);
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(grid), dim3(NW * 64), r.lds, c.stream,
-                           reinterpret_cast<const KWork*>(c.d_k_work) + r.offset, c.d_blocks, c.d_pts,
+                           reinterpret_cast<const KWork*>(c.d_k_work) + r.offset, c.d_kblocks, c.d_pts,
                            c.n_slots, c.d_shrec, c.rec_stride, c.d_block_shells, c.d_block_shell_col,
                            c.d_block_cols, c.d_block_sorder, c.d_coef, c.d_K, q, r.count);
     };

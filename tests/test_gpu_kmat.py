@@ -5,6 +5,7 @@ FP64 build; one grid in another order or other items changes the summation
 order alone."""
 import numpy as np
 import pytest
+import torch
 
 from oracle import oracle
 from proteindf_amd import calc_grid, engine, guess, molecules
@@ -37,3 +38,23 @@ def test_k_of_every_tile_count(waters, n_pts):
     K8 = ctx.build_rks(guess.pack_lower(PA))[1]
     ctx.close()
     np.testing.assert_allclose(K8, K, rtol=0, atol=1e-12)
+
+
+@pytest.mark.parametrize("waters", [3, 11])
+def test_pairs_of_blocks_give_the_sum_of_two_grids(waters):
+    # 10 units of two blocks per CU and a ragged rest; its halves run block by block
+    half = 10 * torch.cuda.get_device_properties(0).multi_processor_count * 128
+    mol = molecules.water_cluster(waters, 5)
+    info = calc_grid.orbital_info(mol)
+    P = guess.pack_lower(0.5 * guess.density_guess(mol, info, seed=5, eps=0.05))
+    grid = _points(mol, 2 * half + 77, 5)
+    print(f"[gpu-case] pairs of blocks, {len(grid)} points, {info.n_aos} AOs", flush=True)
+    ctx = engine.XcContext(info)
+    got = []
+    for part in (grid, grid[:half], grid[half:]):
+        ctx.set_grid(part)
+        got.append(ctx.build_rks(P))
+    ctx.close()
+    # 1e-12 of the sums: the order of about 10^6 terms
+    assert abs(got[0][0] - got[1][0] - got[2][0]) <= 1e-12 * abs(got[0][0])
+    np.testing.assert_allclose(got[0][1], got[1][1] + got[2][1], rtol=0, atol=1e-12 * np.abs(got[0][1]).max())
