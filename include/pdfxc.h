@@ -219,6 +219,8 @@ int pdfxc_generate_grid_oriented(pdfxc_ctx* ctx, int n_atoms, const int* Z, cons
 /* Copy the context's grid back in the caller's point order (x, y, z, w
  * columns, n_pts each). */
 int pdfxc_get_grid(pdfxc_ctx* ctx, double* x, double* y, double* z, double* w);
+/* The same as rows (x, y, z, w), 4 n_pts values. */
+int pdfxc_get_grid_rows(pdfxc_ctx* ctx, double* xyzw);
 
 /* getWholeDensity (DfCalcGridX.cpp:2502-2537): the integrated rho_alpha (and,
  * after a UKS build, rho_beta; n_beta may be null) of the context's last build

@@ -371,6 +371,97 @@ __global__ __launch_bounds__(1024) void k_part_leaf(const LeafNode* __restrict__
     for (int i = t; i < n; i += 1024) order[L.lo + i] = s_idx[s_ord[i]];
 }
 
+// Raw points of a generated grid, one workgroup per radial shell: the rotated
+// directions of its rule times its radius, around its atom.  Plain products
+// and sums, as a host compiler forms them.
+__global__ __launch_bounds__(256) void k_raw_points(const RawShell* __restrict__ shells, const double* __restrict__ dirs,
+                                                    double* __restrict__ pts, double* __restrict__ w,
+                                                    int* __restrict__ atom) {
+#pragma clang fp contract(off)
+    const RawShell S = shells[blockIdx.x];
+    for (int k = threadIdx.x; k < S.n; k += 256) {
+        const double* d = dirs + 4 * (int64_t)(S.dir_begin + k);
+        const int64_t i = S.first + k;
+        for (int q = 0; q < 3; ++q) pts[3 * i + q] = d[q] * S.r + S.center[q];
+        w[i] = d[3] * S.w;
+        atom[i] = S.atom;
+    }
+}
+
+// Points of every shell whose weight passes the screen.
+__global__ __launch_bounds__(256) void k_keep_count(const RawShell* __restrict__ shells, const double* __restrict__ w,
+                                                    double cutoff, long long* __restrict__ counts) {
+    __shared__ int s_n[4];
+    const RawShell S = shells[blockIdx.x];
+    int n = 0;
+    for (int k = threadIdx.x; k < S.n; k += 256) n += fabs(w[S.first + k]) > cutoff;
+    for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off);
+    if ((threadIdx.x & 63) == 0) s_n[threadIdx.x >> 6] = n;
+    __syncthreads();
+    if (threadIdx.x == 0) counts[blockIdx.x] = s_n[0] + s_n[1] + s_n[2] + s_n[3];
+}
+
+// v[0 .. n] to its exclusive prefix sums, v[n] the total (one workgroup)
+__global__ __launch_bounds__(1024) void k_scan(int n, long long* __restrict__ v) {
+    __shared__ long long s_part[1024];
+    const int t = threadIdx.x, per = (n + 1023) / 1024;
+    const int b = min(n, t * per), e = min(n, b + per);
+    long long sum = 0;
+    for (int i = b; i < e; ++i) sum += v[i];
+    s_part[t] = sum;
+    __syncthreads();
+    for (int off = 1; off < 1024; off <<= 1) {
+        const long long a = t >= off ? s_part[t - off] : 0;
+        __syncthreads();
+        s_part[t] += a;
+        __syncthreads();
+    }
+    long long run = s_part[t] - sum;
+    for (int i = b; i < e; ++i) {
+        const long long c = v[i];
+        v[i] = run;
+        run += c;
+    }
+    if (t == 1023) v[n] = s_part[t];
+}
+
+// The kept points in their order, as grid columns (n of them).
+__global__ __launch_bounds__(256) void k_keep_write(const RawShell* __restrict__ shells, const double* __restrict__ pts,
+                                                    const double* __restrict__ w, double cutoff,
+                                                    const long long* __restrict__ first, int64_t n,
+                                                    double* __restrict__ grid) {
+    __shared__ int s_n[4];
+    const RawShell S = shells[blockIdx.x];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int64_t at = first[blockIdx.x];
+    for (int k0 = 0; k0 < S.n; k0 += 256) {
+        const int k = k0 + threadIdx.x;
+        const int64_t i = S.first + k;
+        const double wi = k < S.n ? w[i] : 0.0;
+        const bool keep = k < S.n && fabs(wi) > cutoff;
+        const unsigned long long m = __ballot(keep);
+        if (lane == 0) s_n[wave] = __popcll(m);
+        __syncthreads();
+        int64_t to = at + __popcll(m & ((1ull << lane) - 1ull));
+        for (int q = 0; q < 4; ++q) {
+            if (q < wave) to += s_n[q];
+            at += s_n[q];
+        }
+        if (keep) {
+            for (int q = 0; q < 3; ++q) grid[q * n + to] = pts[3 * i + q];
+            grid[3 * n + to] = wi;
+        }
+        __syncthreads();
+    }
+}
+
+// points [first, first + n) of the grid columns (stride apart) to rows (x, y, z, w)
+__global__ __launch_bounds__(256) void k_grid_rows(int64_t first, int64_t n, int64_t stride,
+                                                   const double* __restrict__ grid, double* __restrict__ rows) {
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (t < 4 * n) rows[t] = grid[(t & 3) * stride + first + (t >> 2)];
+}
+
 // First point with a value that is not finite (n when there is none).
 __global__ __launch_bounds__(256) void k_check_finite(int64_t n, const double* __restrict__ grid,
                                                       unsigned long long* __restrict__ first) {
@@ -704,6 +795,30 @@ int device_partition(int64_t n64, const double* d_grid, int* d_order, hipStream_
     (void)hipFree(ws);
     if (rc == PDFXC_OK && e != hipSuccess) rc = hip_fail(e, "block partition");
     return rc;
+}
+
+int launch_raw_points(int ns, const RawShell* d_shells, const double* d_dirs, double* d_pts, double* d_w, int* d_atom,
+                      hipStream_t s) {
+    hipLaunchKernelGGL(k_raw_points, dim3(ns), dim3(256), 0, s, d_shells, d_dirs, d_pts, d_w, d_atom);
+    return check("k_raw_points");
+}
+
+int launch_keep_count(int ns, const RawShell* d_shells, const double* d_w, double cutoff, long long* d_first,
+                      hipStream_t s) {
+    hipLaunchKernelGGL(k_keep_count, dim3(ns), dim3(256), 0, s, d_shells, d_w, cutoff, d_first);
+    hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, ns, d_first);
+    return check("k_keep_count");
+}
+
+int launch_keep_write(int ns, const RawShell* d_shells, const double* d_pts, const double* d_w, double cutoff,
+                      const long long* d_first, int64_t n, double* d_grid, hipStream_t s) {
+    hipLaunchKernelGGL(k_keep_write, dim3(ns), dim3(256), 0, s, d_shells, d_pts, d_w, cutoff, d_first, n, d_grid);
+    return check("k_keep_write");
+}
+
+int launch_grid_rows(int64_t first, int64_t n, int64_t stride, const double* d_grid, double* d_rows, hipStream_t s) {
+    hipLaunchKernelGGL(k_grid_rows, dim3(blocks256(4 * n)), dim3(256), 0, s, first, n, stride, d_grid, d_rows);
+    return check("k_grid_rows");
 }
 
 int device_check_finite(int64_t n, const double* d_grid, unsigned long long* d_first, hipStream_t s) {

@@ -1581,6 +1581,25 @@ int pdfxc_get_grid(pdfxc_ctx* ctx, double* x, double* y, double* z, double* w) {
     return PDFXC_OK;
 }
 
+int pdfxc_get_grid_rows(pdfxc_ctx* ctx, double* xyzw) {
+    Context* c = reinterpret_cast<Context*>(ctx);
+    if (!c || !xyzw) return arg_error("pdfxc_get_grid_rows: bad arguments");
+    if (c->n_pts == 0) {
+        set_error("pdfxc_get_grid_rows: no grid");
+        return PDFXC_ERR_NO_GRID;
+    }
+    const int64_t per = std::min<int64_t>(c->n_pts, 1 << 22);  // 128 MiB of rows at a time
+    DeviceBuf rows;
+    if (int rc = rows.alloc(4 * sizeof(double) * (size_t)per)) return rc;
+    for (int64_t at = 0; at < c->n_pts; at += per) {
+        const int64_t n = std::min(per, c->n_pts - at);
+        if (int rc = launch_grid_rows(at, n, c->n_pts, c->d_grid, rows.as<double>(), c->stream)) return rc;
+        PDFXC_HIP(hipMemcpyAsync(xyzw + 4 * at, rows.p, 4 * sizeof(double) * (size_t)n, hipMemcpyDeviceToHost, c->stream));
+        PDFXC_HIP(hipStreamSynchronize(c->stream));
+    }
+    return PDFXC_OK;
+}
+
 int pdfxc_grid_opts_preset(const char* grid_type, pdfxc_grid_opts* out) {
     if (!grid_type || !out) return arg_error("pdfxc_grid_opts_preset: bad arguments");
     std::string t(grid_type);
@@ -1674,9 +1693,12 @@ static int generate_grid_impl(pdfxc_ctx* ctx, int n_atoms, const int* Z, const d
         std::copy(O_given, O_given + 9, O);
     else
         orientation(n_atoms, Z, xyz, O);
-    // single-centre points and weights, atom by atom, radial shell by shell
-    std::vector<double> pts, w;
-    std::vector<int> atom;
+    // radial shells, atom by atom; their points are made on the device, from
+    // the directions of every rule turned by O
+    std::vector<RawShell> shells;
+    std::vector<double> dirs;
+    std::vector<int> dir_begin(leb.size(), -1);
+    int64_t n = 0;
     for (int a = 0; a < n_atoms; ++a) {
         if (Z[a] <= 0) continue;
         const double R = (o.radii == PDFXC_RADII_SG1) ? sg1_radius(Z[a]) : bragg_slater(Z[a]);
@@ -1690,17 +1712,18 @@ static int generate_grid_impl(pdfxc_ctx* ctx, int n_atoms, const int* Z, const d
             const int q = rule_index(pruned_order(o.pruning, Z[a], ri, R, o.n_ang));
             const std::vector<double>& L = leb[q];
             const int nq = (int)lebw[q].size();
-            for (int k = 0; k < nq; ++k) {
-                for (int d = 0; d < 3; ++d) {
-                    const double v = O[3 * d] * L[3 * k] + O[3 * d + 1] * L[3 * k + 1] + O[3 * d + 2] * L[3 * k + 2];
-                    pts.push_back(v * ri + xyz[3 * a + d]);
+            if (dir_begin[q] < 0) {
+                dir_begin[q] = (int)(dirs.size() / 4);
+                for (int k = 0; k < nq; ++k) {
+                    for (int d = 0; d < 3; ++d)
+                        dirs.push_back(O[3 * d] * L[3 * k] + O[3 * d + 1] * L[3 * k + 1] + O[3 * d + 2] * L[3 * k + 2]);
+                    dirs.push_back(lebw[q][k]);
                 }
-                w.push_back(lebw[q][k] * wr);
-                atom.push_back(a);
             }
+            shells.push_back(RawShell{ri, wr, {xyz[3 * a], xyz[3 * a + 1], xyz[3 * a + 2]}, n, dir_begin[q], nq, a, 0});
+            n += nq;
         }
     }
-    const int64_t n = (int64_t)w.size();
     // atom table for the partition kernel: (x, y, z, Z), 1/R_mn, Becke size
     // adjustments a_mn (getCovalentRadiiForBecke: H 0.35, else Bragg-Slater,
     // a dummy 0; |a| <= 1/2; zero when the adjustments are off)
@@ -1732,50 +1755,64 @@ static int generate_grid_impl(pdfxc_ctx* ctx, int n_atoms, const int* Z, const d
                 amat[(size_t)k * n_atoms + m] = aa;  // a_mk at [k][m]: the kernel's lanes run over m
             }
         }
-    double *d_at = nullptr, *d_p = nullptr, *d_w = nullptr;
-    int* d_a = nullptr;
-    int rc = dalloc(&d_at, at.size());
-    if (rc == PDFXC_OK && n > 0) rc = dalloc(&d_p, pts.size());
-    if (rc == PDFXC_OK && n > 0) rc = dalloc(&d_w, w.size());
-    if (rc == PDFXC_OK && n > 0) rc = dalloc(&d_a, atom.size());
-    hipError_t e = hipSuccess;
-    if (rc == PDFXC_OK && n > 0) {
-        e = hipMemcpyAsync(d_at, at.data(), at.size() * sizeof(double), hipMemcpyHostToDevice, c->stream);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(d_p, pts.data(), pts.size() * sizeof(double), hipMemcpyHostToDevice, c->stream);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(d_w, w.data(), w.size() * sizeof(double), hipMemcpyHostToDevice, c->stream);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(d_a, atom.data(), atom.size() * sizeof(int), hipMemcpyHostToDevice, c->stream);
-        if (e != hipSuccess) rc = hip_fail(e, "pdfxc_generate_grid_ex: upload");
+    // weights and the weight screen (screeningGridsByWeight0,
+    // DfGenerateGrid.cpp:1979-2004), all of it on the device
+    const int ns = (int)shells.size();
+    std::vector<long long> first(ns + 1, 0);  // first kept point of every shell, and their number
+    DeviceBuf tab, raw;
+    auto align = [](size_t b) { return (b + 255) / 256 * 256; };
+    const size_t b_at = align(at.size() * sizeof(double)), b_sh = align(shells.size() * sizeof(RawShell)),
+                 b_dir = align(dirs.size() * sizeof(double)), b_first = align(first.size() * sizeof(long long));
+    int rc = PDFXC_OK;
+    if (n > 0) {
+        rc = tab.alloc(b_at + b_sh + b_dir + b_first);
+        if (rc == PDFXC_OK) rc = raw.alloc((4 * sizeof(double) + sizeof(int)) * (size_t)n);
+        if (rc) return rc;
+    }
+    double* d_at = tab.as<double>();
+    RawShell* d_sh = reinterpret_cast<RawShell*>(tab.as<char>() + b_at);
+    double* d_dir = reinterpret_cast<double*>(tab.as<char>() + b_at + b_sh);
+    long long* d_first = reinterpret_cast<long long*>(tab.as<char>() + b_at + b_sh + b_dir);
+    double* d_p = raw.as<double>();
+    double* d_w = d_p + 3 * n;
+    int* d_a = reinterpret_cast<int*>(d_w + n);
+    if (n > 0) {
+        PDFXC_HIP(hipMemcpyAsync(d_at, at.data(), at.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
+        PDFXC_HIP(hipMemcpyAsync(d_sh, shells.data(), shells.size() * sizeof(RawShell), hipMemcpyHostToDevice, c->stream));
+        PDFXC_HIP(hipMemcpyAsync(d_dir, dirs.data(), dirs.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
+        rc = launch_raw_points(ns, d_sh, d_dir, d_p, d_w, d_a, c->stream);
         if (rc == PDFXC_OK) rc = launch_becke(d_at, n_atoms, n, d_p, d_a, d_w, o.partitioning, c->stream);
+        if (rc == PDFXC_OK) rc = launch_keep_count(ns, d_sh, d_w, o.weight_cutoff, d_first, c->stream);
         if (rc == PDFXC_OK) {
-            e = hipMemcpyAsync(w.data(), d_w, w.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream);
-            if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+            const hipError_t e = hipMemcpyAsync(first.data(), d_first, first.size() * sizeof(long long),
+                                                hipMemcpyDeviceToHost, c->stream);
             if (e != hipSuccess) rc = hip_fail(e, "pdfxc_generate_grid_ex: partition weights");
         }
+        // also on failure: the tables go with this scope
+        const hipError_t e = hipStreamSynchronize(c->stream);
+        if (rc == PDFXC_OK && e != hipSuccess) rc = hip_fail(e, "pdfxc_generate_grid_ex: partition weights");
+        if (rc) return rc;
     }
-    dfree(d_at);
-    dfree(d_p);
-    dfree(d_w);
-    dfree(d_a);
-    if (rc != PDFXC_OK) return rc;
-    // weight screening (screeningGridsByWeight0, DfGenerateGrid.cpp:1979-2004)
-    std::vector<double> X, Y, Zc, W;
-    std::vector<int> kept_atom;
-    for (int64_t i = 0; i < n; ++i)
-        if (std::fabs(w[i]) > o.weight_cutoff) {
-            X.push_back(pts[3 * i]);
-            Y.push_back(pts[3 * i + 1]);
-            Zc.push_back(pts[3 * i + 2]);
-            W.push_back(w[i]);
-            kept_atom.push_back(atom[i]);
-        }
-    if (W.empty()) return arg_error("pdfxc_generate_grid_ex: no grid point survives the weight screen");
-    if (n_out) *n_out = (int64_t)W.size();
-    rc = pdfxc_set_grid(ctx, (int64_t)W.size(), X.data(), Y.data(), Zc.data(), W.data());
+    const int64_t n_kept = first[ns];
+    if (n_kept == 0) return arg_error("pdfxc_generate_grid_ex: no grid point survives the weight screen");
+    if (n_out) *n_out = n_kept;
+    if (n_kept > ((int64_t)1 << 31) - kBlockPts) {
+        reset_grid(*c);
+        return arg_error("pdfxc_set_grid: more than 2^31 points");
+    }
+    double* d_grid = nullptr;
+    rc = alloc_grid(*c, n_kept, &d_grid);
+    if (rc) return rc;
+    rc = launch_keep_write(ns, d_sh, d_p, d_w, o.weight_cutoff, d_first, n_kept, d_grid, c->stream);
+    if (rc) {
+        dfree(d_grid);
+        return rc;
+    }
+    rc = set_device_grid(*c, n_kept, d_grid, "pdfxc_set_grid");
     if (rc == PDFXC_OK) {
-        c->gen_atom = std::move(kept_atom);
+        c->gen_atom.resize((size_t)n_kept);
+        for (int s = 0; s < ns; ++s)
+            std::fill(c->gen_atom.begin() + first[s], c->gen_atom.begin() + first[s + 1], shells[s].atom);
         c->grid_partition = o.partitioning;
         c->grid_size_adjust = o.size_adjust ? 1 : 0;
     }

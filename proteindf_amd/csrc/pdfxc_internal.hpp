@@ -132,6 +132,14 @@ struct KGWork {
     int group, q0, q1, c0, c1, k0, nbuf, pad;
 };
 
+// A radial shell of a generated grid: n raw points from `first` on, directions
+// (x, y, z, weight) from dir_begin on.
+struct RawShell {
+    double r, w, center[3];
+    int64_t first;
+    int dir_begin, n, atom, pad;
+};
+
 // What block screening needs of a shell: it is dropped from a block whose
 // box lies further than cut, or where exp0 d^2 > 30 (cls: rank of (l, nprim)).
 struct ScreenShell {
@@ -294,6 +302,14 @@ int ensure_host_slots(Context& c);
 int device_partition(int64_t n, const double* d_grid, int* d_order, hipStream_t s);
 // lowers *d_first to the first point with a non-finite value
 int device_check_finite(int64_t n, const double* d_grid, unsigned long long* d_first, hipStream_t s);
+// generated grids: raw points, first kept point of every shell (d_first[ns]: their number), kept points
+int launch_raw_points(int ns, const RawShell* d_shells, const double* d_dirs, double* d_pts, double* d_w, int* d_atom,
+                      hipStream_t s);
+int launch_keep_count(int ns, const RawShell* d_shells, const double* d_w, double cutoff, long long* d_first,
+                      hipStream_t s);
+int launch_keep_write(int ns, const RawShell* d_shells, const double* d_pts, const double* d_w, double cutoff,
+                      const long long* d_first, int64_t n, double* d_grid, hipStream_t s);
+int launch_grid_rows(int64_t first, int64_t n, int64_t stride, const double* d_grid, double* d_rows, hipStream_t s);
 int launch_screen_blocks(int nb, int64_t n, const double* d_grid, const int* d_order, int nsh,
                          const ScreenShell* d_shells, int nw, unsigned long long* d_masks, int* d_counts,
                          hipStream_t s);

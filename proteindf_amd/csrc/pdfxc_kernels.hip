@@ -1011,11 +1011,12 @@ __global__ __launch_bounds__(256) void k_eval_aos_points(int64_t n, const double
 // dummy neighbours k, the SS product does not.  One wave per point: the
 // point's atom distances in LDS, lanes over the cells m (so the [k][m] reads
 // of a neighbour k are contiguous), the sums over cells in a fixed butterfly.
+// (k_becke; k_ss is the Stratmann-Scuseria form.)
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_becke(const double* __restrict__ atoms, int na,
                                               int64_t n, const double* __restrict__ pts,
                                               const int* __restrict__ atom_of_pt,
-                                              double* __restrict__ w, int ss) {
+                                              double* __restrict__ w) {
     extern __shared__ double s_r[];  // [waves][na]
     const int lane = threadIdx.x & 63;
     const int wv = threadIdx.x >> 6;
@@ -1033,8 +1034,8 @@ __global__ __launch_bounds__(256) void k_becke(const double* __restrict__ atoms,
     __syncthreads();
     const int A = atom_of_pt[i];
     // the point's own atom is the first neighbour of every cell: it is (near)
-    // the nearest, so a far cell's product reaches zero (Stratmann-Scuseria:
-    // exactly, u > 0.64) or underflows after few factors and the loop ends
+    // the nearest, so a far cell's product underflows after few factors and the
+    // loop ends
     const int A0 = (A >= 0 && A < na) ? A : 0;
     double total = 0.0, mine = 0.0;
     for (int m = lane; m < na; m += 64) {
@@ -1044,25 +1045,12 @@ __global__ __launch_bounds__(256) void k_becke(const double* __restrict__ atoms,
             const int k = (j == 0) ? A0 : (j <= A0 ? j - 1 : j);  // A0, then the others in index order
             if (k == m) continue;
             double u = (rm - r[k]) * inv_d[(int64_t)k * na + m];
-            double g;
-            if (ss) {
-                // Stratmann-Scuseria g(u), a = 0.64
-                if (u < -0.64) {
-                    g = -1.0;
-                } else if (u > 0.64) {
-                    g = 1.0;
-                } else {
-                    const double q = u / 0.64, q2 = q * q, q3 = q2 * q, q5 = q2 * q3;
-                    g = (1.0 / 16.0) * (35.0 * q - 35.0 * q3 + 21.0 * q5 - 5.0 * q5 * q2);
-                }
-            } else {
-                if (atoms[4 * k + 3] <= 0.0) continue;  // Becke: dummy neighbours do not cut
-                const double a = amat_t[(int64_t)k * na + m];
-                u = u + a * (1.0 - u * u);
-                g = 0.5 * u * (3.0 - u * u);
-                g = 0.5 * g * (3.0 - g * g);
-                g = 0.5 * g * (3.0 - g * g);
-            }
+            if (atoms[4 * k + 3] <= 0.0) continue;  // dummy neighbours do not cut
+            const double a = amat_t[(int64_t)k * na + m];
+            u = u + a * (1.0 - u * u);
+            double g = 0.5 * u * (3.0 - u * u);
+            g = 0.5 * g * (3.0 - g * g);
+            g = 0.5 * g * (3.0 - g * g);
             ps *= 0.5 * (1.0 - g);
         }
         if (m == A) mine = ps;
@@ -1073,6 +1061,101 @@ __global__ __launch_bounds__(256) void k_becke(const double* __restrict__ atoms,
         total += __shfl_xor(total, off);
         mine += __shfl_xor(mine, off);
     }
+    if (valid && lane == 0) w[i] *= (mine / total);
+}
+
+// The Stratmann-Scuseria form of the same weight.  g(u), a = 0.64, is exactly
+// 1 above u = 0.64 (the factor (1 - g) / 2 is 0) and exactly -1 below -0.64
+// (the factor is 1): a cell whose factor against the point's own or nearest
+// atom is 0 leaves with one test, and of a cell that stays the lanes take the
+// neighbours, only the factors that are not 1 being multiplied (own atom
+// first, then in index order).  One lane per cell with all neighbours in turn
+// (k_becke) took 23.2 ms for the 2.6 million points of a 142-atom helix,
+// bound by the few lanes whose cells stay; this takes 8.1 ms.
+__device__ __forceinline__ double ss_factor(double rm, double rk, double inv) {
+    const double u = (rm - rk) * inv;
+    double g;
+    if (u < -0.64) {
+        g = -1.0;
+    } else if (u > 0.64) {
+        g = 1.0;
+    } else {
+        const double q = u / 0.64, q2 = q * q, q3 = q2 * q, q5 = q2 * q3;
+        g = (1.0 / 16.0) * (35.0 * q - 35.0 * q3 + 21.0 * q5 - 5.0 * q5 * q2);
+    }
+    return 0.5 * (1.0 - g);
+}
+
+__global__ __launch_bounds__(256) void k_ss(const double* __restrict__ atoms, int na, int64_t n,
+                                            const double* __restrict__ pts, const int* __restrict__ atom_of_pt,
+                                            double* __restrict__ w) {
+    extern __shared__ double s_r[];  // [waves][na]
+    const int lane = threadIdx.x & 63;
+    const int wv = threadIdx.x >> 6;
+    const int64_t i0 = (int64_t)blockIdx.x * (blockDim.x >> 6) + wv;
+    const bool valid = i0 < n;
+    const int64_t i = valid ? i0 : n - 1;  // a spare wave repeats the last point and writes nothing
+    const double* inv_d = atoms + 4 * na;
+    double* r = s_r + (int64_t)wv * na;
+    const double x = pts[3 * i], y = pts[3 * i + 1], z = pts[3 * i + 2];
+    double best = 1e300;
+    int near = 0;
+    for (int m = lane; m < na; m += 64) {
+        const double dx = x - atoms[4 * m], dy = y - atoms[4 * m + 1], dz = z - atoms[4 * m + 2];
+        const double d = sqrt(dx * dx + dy * dy + dz * dz);
+        r[m] = d;
+        if (d < best) {
+            best = d;
+            near = m;
+        }
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const double ob = __shfl_xor(best, off);
+        const int on = __shfl_xor(near, off);
+        if (ob < best || (ob == best && on < near)) {
+            best = ob;
+            near = on;
+        }
+    }
+    near = __builtin_amdgcn_readfirstlane(near);
+    __syncthreads();
+    const int A = __builtin_amdgcn_readfirstlane(atom_of_pt[i]);
+    const int A0 = (A >= 0 && A < na) ? A : 0;
+    const double rA = r[A0], rN = r[near];
+    double total = 0.0, mine = 0.0;
+    for (int m0 = 0; m0 < na; m0 += 64) {
+        const int mm = m0 + lane;
+        bool stays = false;
+        if (mm < na) {
+            const double rm = r[mm];
+            stays = !(mm != A0 && (rm - rA) * inv_d[(int64_t)A0 * na + mm] > 0.64) &&
+                    !(mm != near && (rm - rN) * inv_d[(int64_t)near * na + mm] > 0.64);
+        }
+        for (unsigned long long cells = __ballot(stays); cells; cells &= cells - 1) {
+            const int c = __builtin_ctzll(cells);
+            const int m = m0 + c;
+            const double rm = r[m];
+            const double* inv = inv_d + (int64_t)m * na;
+            bool cut = false;  // some neighbour's factor is 0
+            for (int k = lane; k < na; k += 64) cut = cut || (k != m && (rm - r[k]) * inv[k] > 0.64);
+            if (__ballot(cut)) continue;
+            double ps = m == A0 ? 1.0 : ss_factor(rm, rA, inv[A0]);
+            for (int k0 = 0; k0 < na; k0 += 64) {
+                const int k = k0 + lane;
+                const double f = (k < na && k != m && k != A0) ? ss_factor(rm, r[k], inv[k]) : 1.0;
+                for (unsigned long long q = __ballot(f != 1.0); q; q &= q - 1) {
+                    const int from = __builtin_ctzll(q);
+                    ps *= __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(f), from),
+                                           __builtin_amdgcn_readlane(__double2loint(f), from));
+                }
+            }
+            if (lane == c) total += ps;
+            if (m == A) mine = ps;
+        }
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) total += __shfl_xor(total, off);
     if (valid && lane == 0) w[i] *= (mine / total);
 }
 
@@ -1399,9 +1482,9 @@ int launch_becke(const double* d_atoms, int n_atoms, int64_t n, const double* d_
     const int waves = ((size_t)4 * n_atoms * sizeof(double) <= 65536) ? 4 : 1;
     const int64_t g = (n + waves - 1) / waves;
     const size_t lds = sizeof(double) * (size_t)waves * (size_t)n_atoms;
-    hipLaunchKernelGGL(k_becke, dim3((unsigned)g), dim3(64 * waves), lds, s, d_atoms, n_atoms, n,
-                       d_pts, d_atom_of_pt, d_w, partition == 1 ? 1 : 0);
-    return check_launch("k_becke");
+    hipLaunchKernelGGL(partition == PDFXC_PARTITION_SS ? k_ss : k_becke, dim3((unsigned)g), dim3(64 * waves), lds, s,
+                       d_atoms, n_atoms, n, d_pts, d_atom_of_pt, d_w);
+    return check_launch("partition weights");
 }
 
 // MFMA layout self test: A[i][k] = i + 100 k, B[k][j] = j - 7 k; D = A B

@@ -36,7 +36,7 @@ ERROR_CODES = {v: k for k, v in ERROR_NAMES.items()}
 # every symbol declared in include/pdfxc.h
 EXPORTED = [
     "pdfxc_default_opts", "pdfxc_normalize_cgto", "pdfxc_ctx_create", "pdfxc_ctx_destroy",
-    "pdfxc_set_grid", "pdfxc_generate_grid", "pdfxc_get_grid", "pdfxc_whole_density", "pdfxc_build_rks",
+    "pdfxc_set_grid", "pdfxc_generate_grid", "pdfxc_get_grid", "pdfxc_get_grid_rows", "pdfxc_whole_density", "pdfxc_build_rks",
     "pdfxc_build_rks_device", "pdfxc_eval_functional", "pdfxc_eval_aos", "pdfxc_get_stats",
     "pdfxc_stream", "pdfxc_last_error", "pdfxc_gradient_rks", "pdfxc_build_rks_update",
     "pdfxc_build_rks_update_device", "pdfxc_selftest_mfma", "pdfxc_selftest_mfma_split",
@@ -131,6 +131,7 @@ def lib():
         L.pdfxc_generate_grid_ex.argtypes = [P, i32, P, P, P, P]
         L.pdfxc_generate_grid_oriented.argtypes = [P, i32, P, P, P, P, P]
         L.pdfxc_get_grid.argtypes = [P, P, P, P, P]
+        L.pdfxc_get_grid_rows.argtypes = [P, P]
         L.pdfxc_whole_density.argtypes = [P, P, P]
         L.pdfxc_build_rks.argtypes = [P, i32, P, P, P, P]
         L.pdfxc_build_rks_device.argtypes = [P, i32, P, P, P]
@@ -385,9 +386,9 @@ class XcContext:
         return (rho, grad) if want_grad else rho
 
     def get_grid(self):
-        cols = [np.zeros(self.n_pts) for _ in range(4)]
-        check(lib().pdfxc_get_grid(self.h, *[_p(c) for c in cols]))
-        return np.stack(cols, 1)
+        rows = np.empty((self.n_pts, 4))
+        check(lib().pdfxc_get_grid_rows(self.h, _p(rows)))
+        return rows
 
     def build_rks(self, P_alpha_packed, K_alpha_packed=None, want_rho=False,
                   functional=PDFXC_B3LYP):
