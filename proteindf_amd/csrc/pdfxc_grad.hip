@@ -11,8 +11,9 @@
 // the opposite sum (:1372-1377); the factor 4 is the reference's -2 w times
 // its RKS doubling (:1234).
 //   k_grad_fn  per 16 points of a block: phi and W into LDS, X^T = P_bb phi^T
-//              and Z^T = P_bb W^T on v_mfma_f64_16x16x4, then grad phi and the
-//              AO second derivatives per (point, shell), summed per atom in LDS
+//              and Z^T = P_bb W^T on v_mfma_f64_16x16x4, then the sums with
+//              grad phi and the AO second derivatives per (point, shell),
+//              summed per atom in LDS
 //   k_grad_w   per point: grad_B omega_A of the grid's partition (Becke with
 //              or without size adjustments, or Stratmann-Scuseria)
 //              for every atom B (point fixed), times w_single e_xc, to B and
@@ -28,6 +29,21 @@
 #include "pdfxc_split.hpp"
 
 namespace pdfxc {
+
+// Sum of v over a row of 16 lanes (all of them active), in every lane: four
+// rotations within the row (DPP row_ror).
+template <int N>
+__device__ inline double row_ror(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x120 + N, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x120 + N, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+__device__ inline double row_sum16(double v) {
+    v += row_ror<8>(v);
+    v += row_ror<4>(v);
+    v += row_ror<2>(v);
+    return v + row_ror<1>(v);
+}
 
 template <int NI>
 __device__ inline void grad_tiles(int wave, int lane, int T, const int* s_cols, double* s_phi, double* s_w,
@@ -55,7 +71,14 @@ __device__ inline void grad_tiles(int wave, int lane, int T, const int* s_cols, 
             for (int i = 0; i < NI; ++i) a[d][i] = prow[gi[i]];
         }
     };
-    load_a(0, aC);
+    // the first group through aN as well, and the copy held behind the MFMAs:
+    // else every group waits for the loads of the next one
+    load_a(0, aN);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int d = 0; d < G; ++d)
+#pragma unroll
+        for (int i = 0; i < NI; ++i) aC[d][i] = aN[d][i];
     for (int g = 0; g < ngroups; ++g) {
         if (g + 1 < ngroups) load_a(g + 1, aN);
 #pragma unroll
@@ -71,6 +94,7 @@ __device__ inline void grad_tiles(int wave, int lane, int T, const int* s_cols, 
                 }
             }
         }
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int d = 0; d < G; ++d)
 #pragma unroll
@@ -242,17 +266,36 @@ __global__ __launch_bounds__(512) void k_grad_fn(const int* __restrict__ work, c
     const double px = s_pt[p][0], py = s_pt[p][1], pz = s_pt[p][2];
     const double a2 = 2.0 * s_cf[p][0];
     const double cd[3] = {s_cf[p][1], s_cf[p][2], s_cf[p][3]};
-    // 1. phi and W = c . grad phi
-    for (int j = kk; j < nsh; j += NSL) {
-        const int k = s_sord[j];
-        double v[5], vx[5], vy[5], vz[5];
-        rec_values(s_rec + k * RS, px, py, pz, v, vx, vy, vz);
+    // 1. phi and W = c . grad phi; the radial sums of a thread's first NC shells
+    // stay in registers for step 3 (most of a thread's share, within the
+    // registers that leave two workgroups per CU where the planes do)
+    constexpr int NC = S > 0 ? 0 : NIMAX == 4 ? 6 : 3;
+    double cR[NC > 0 ? NC : 1][3];
+    auto put_values = [&](int k, double x, double y, double z, double R0, double R1) {
         const int c0 = s_shcol[k];
-        const int nc = 2 * (((int)s_rec[k * RS + 3]) & 3) + 1;
-        for (int m = 0; m < nc; ++m) {
-            s_phi[(c0 + m) * PB + p] = v[m];
-            s_w[(c0 + m) * PB + p] = cd[0] * vx[m] + cd[1] * vy[m] + cd[2] * vz[m];
+        shell_phi_v(((int)s_rec[k * RS + 3]) & 3, x, y, z, R0, R1, 0.0, cd[0], cd[1], cd[2],
+                    [&](int m, double v, double V) {
+                        s_phi[(c0 + m) * PB + p] = v;
+                        s_w[(c0 + m) * PB + p] = V;
+                    });
+    };
+#pragma unroll
+    for (int jj = 0; jj < NC; ++jj) {
+        const int j = kk + jj * NSL;
+        if (j < nsh) {
+            const int k = s_sord[j];
+            double r3[3];
+            rec_radial2(s_rec + k * RS, px, py, pz, r3, cR[jj][0], cR[jj][1], cR[jj][2]);
+            put_values(k, r3[0], r3[1], r3[2], cR[jj][0], cR[jj][1]);
         }
+    }
+    for (int j = kk + NC * NSL; j < nsh; j += NSL) {
+        const int k = s_sord[j];
+        const double* rec = s_rec + k * RS;
+        const double x = px - rec[0], y = py - rec[1], z = pz - rec[2];
+        double R0, R1;
+        rec_radial01(rec, x, y, z, R0, R1);
+        put_values(k, x, y, z, R0, R1);
     }
     for (int it = tid; it < (ldn - nao) * PB; it += 512) {
         s_phi[nao * PB + it] = 0.0;
@@ -282,43 +325,81 @@ __global__ __launch_bounds__(512) void k_grad_fn(const int* __restrict__ work, c
     }
     __syncthreads();
 
-    // 3. grad phi and second derivatives per (point, shell), summed per atom
+    // 3. the sums over a shell's components in closed form, with T = a2 X + Z,
+    // S_A = sum_m A_m f_m, G_A = sum_m A_m grad f_m and H = sum_m X_m
+    // grad grad f_m over the angular polynomials f_m:
+    //   sum_m T_m grad phi_m + X_m (c . grad) grad phi_m = R0 (G_T + H c)
+    //     + R1 (r (S_T + c . G_X) + (c . r) G_X + c S_X) + R2 (c . r) S_X r
+    // A row of 16 lanes holds the 16 points of one shell: its sum goes to the
+    // atom with one atomic per component.
     double gp[3] = {0.0, 0.0, 0.0};
-    for (int j = kk; j < nsh; j += NSL) {
+    auto add_shell = [&](int k, double x, double y, double z, double R0, double R1, double R2) {
+        const int c0 = s_shcol[k];
+        const int l = ((int)s_rec[k * RS + 3]) & 3;
+        double X[5], Tm[5];
+        auto get = [&](int m) {
+            X[m] = s_phi[(c0 + m) * PB + p];
+            Tm[m] = a2 * X[m] + s_w[(c0 + m) * PB + p];
+        };
+        double ST, SX, GT[3] = {0.0, 0.0, 0.0}, GX[3] = {0.0, 0.0, 0.0};
+        get(0);
+        if (l == 0) {
+            ST = Tm[0];
+            SX = X[0];
+        } else if (l == 1) {
+            get(1);
+            get(2);
+            ST = Tm[0] * x + Tm[1] * y + Tm[2] * z;
+            SX = X[0] * x + X[1] * y + X[2] * z;
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                GT[a] = Tm[a];
+                GX[a] = X[a];
+            }
+        } else {
+            get(1);
+            get(2);
+            get(3);
+            get(4);
+            const double fd = 0.5 * (x * x - y * y), fe = kInvSqrt3 * (z * z - 0.5 * (x * x + y * y));
+            const double X4 = kInvSqrt3 * X[4], T4 = kInvSqrt3 * Tm[4];
+            ST = Tm[0] * (x * y) + Tm[1] * (z * x) + Tm[2] * (y * z) + Tm[3] * fd + Tm[4] * fe;
+            SX = X[0] * (x * y) + X[1] * (z * x) + X[2] * (y * z) + X[3] * fd + X[4] * fe;
+            GX[0] = X[0] * y + X[1] * z + (X[3] - X4) * x;
+            GX[1] = X[0] * x + X[2] * z - (X[3] + X4) * y;
+            GX[2] = X[1] * x + X[2] * y + 2.0 * X4 * z;
+            // G_T and H c in one sum: both take the factor R0
+            GT[0] = Tm[0] * y + Tm[1] * z + (Tm[3] - T4) * x + X[0] * cd[1] + X[1] * cd[2] + (X[3] - X4) * cd[0];
+            GT[1] = Tm[0] * x + Tm[2] * z - (Tm[3] + T4) * y + X[0] * cd[0] + X[2] * cd[2] - (X[3] + X4) * cd[1];
+            GT[2] = Tm[1] * x + Tm[2] * y + 2.0 * T4 * z + X[1] * cd[0] + X[2] * cd[1] + 2.0 * X4 * cd[2];
+        }
+        const double cr = cd[0] * x + cd[1] * y + cd[2] * z;
+        const double cG = cd[0] * GX[0] + cd[1] * GX[1] + cd[2] * GX[2];
+        const double radial = R1 * (ST + cG) + R2 * cr * SX;
+        const double r3[3] = {x, y, z};
+        const int at = s_shat[k];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const double g = R0 * GT[a] + radial * r3[a] + R1 * (cr * GX[a] + cd[a] * SX);
+            gp[a] += g;
+            const double sum = row_sum16(g);
+            if ((lane & 15) == a && sum != 0.0) atomicAdd(&s_g[3 * at + a], sum);
+        }
+    };
+#pragma unroll
+    for (int jj = 0; jj < NC; ++jj) {
+        const int j = kk + jj * NSL;
+        if (j < nsh) {
+            const int k = s_sord[j];
+            const double* rec = s_rec + k * RS;
+            add_shell(k, px - rec[0], py - rec[1], pz - rec[2], cR[jj][0], cR[jj][1], cR[jj][2]);
+        }
+    }
+    for (int j = kk + NC * NSL; j < nsh; j += NSL) {
         const int k = s_sord[j];
         double r3[3], R0, R1, R2;
-        const int l = rec_radial2(s_rec + k * RS, px, py, pz, r3, R0, R1, R2);
-        const int c0 = s_shcol[k];
-        double g[3] = {0.0, 0.0, 0.0};
-        for (int m = 0; m < 2 * l + 1; ++m) {
-            double f, fg[3], fh[6];
-            angular2(l, m, r3, f, fg, fh);
-            const double X = s_phi[(c0 + m) * PB + p];
-            const double Zv = s_w[(c0 + m) * PB + p];
-            const double t = a2 * X + Zv;
-            // H[a][b] = fh_ab R0 + (fg_a r_b + fg_b r_a) R1 + f (delta_ab R1 + r_a r_b R2)
-            double H[3][3];
-            const int hix[3][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, 5}};
-#pragma unroll
-            for (int a = 0; a < 3; ++a)
-#pragma unroll
-                for (int b = 0; b < 3; ++b)
-                    H[a][b] = fh[hix[a][b]] * R0 + (fg[a] * r3[b] + fg[b] * r3[a]) * R1 +
-                              f * ((a == b ? R1 : 0.0) + r3[a] * r3[b] * R2);
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                const double dphi = fg[a] * R0 + f * r3[a] * R1;
-                g[a] += dphi * t + X * (cd[0] * H[a][0] + cd[1] * H[a][1] + cd[2] * H[a][2]);
-            }
-        }
-        if (g[0] != 0.0 || g[1] != 0.0 || g[2] != 0.0) {
-            const int at = s_shat[k];
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                atomicAdd(&s_g[3 * at + a], g[a]);
-                gp[a] += g[a];
-            }
-        }
+        rec_radial2(s_rec + k * RS, px, py, pz, r3, R0, R1, R2);
+        add_shell(k, r3[0], r3[1], r3[2], R0, R1, R2);
     }
     if (s_pa[p] >= 0 && (gp[0] != 0.0 || gp[1] != 0.0 || gp[2] != 0.0)) {
 #pragma unroll
