@@ -1051,6 +1051,9 @@ __global__ __launch_bounds__(256) void k_becke(const double* __restrict__ atoms,
             double g = 0.5 * u * (3.0 - u * u);
             g = 0.5 * g * (3.0 - g * g);
             g = 0.5 * g * (3.0 - g * g);
+            // 1 - g of the rounded g: fused into the product above it moves the
+            // small weights, and with them points across the weight screen
+            __asm__ volatile("" : "+v"(g));
             ps *= 0.5 * (1.0 - g);
         }
         if (m == A) mine = ps;
