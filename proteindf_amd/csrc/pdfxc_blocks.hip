@@ -706,7 +706,7 @@ unsigned blocks256(int64_t n) { return (unsigned)((n + 255) / 256); }
 
 }  // namespace
 
-int device_partition(int64_t n64, const double* d_grid, int* d_order, hipStream_t s) {
+int device_partition(int64_t n64, const double* d_grid, int* d_order, hipStream_t s, DevicePool& pool) {
     const int n = (int)n64;
     // the tree: every level's large nodes and their chunks, and the nodes left to k_part_leaf
     std::vector<PartNode> nodes;
@@ -744,9 +744,10 @@ int device_partition(int64_t n64, const double* d_grid, int* d_order, hipStream_
     const size_t b_n = up(sizeof(PartNode) * nodes.size()), b_c = up(sizeof(PartChunk) * chunks.size());
     const size_t b_l = up(sizeof(LeafNode) * leaves.size());
     const int nbuf = levels > 0 ? 2 : 1;
-    char* ws = nullptr;
+    void* taken = nullptr;
     const size_t total = nbuf * (3 * b_v + b_i) + b_st + b_h + b_n + b_c + b_l;
-    hipError_t e = hipMalloc(reinterpret_cast<void**>(&ws), total);
+    hipError_t e = pool.take(&taken, total);
+    char* ws = static_cast<char*>(taken);
     if (e != hipSuccess) {
         set_error("block partition: hipMalloc of " + std::to_string(total) + " bytes: " + hipGetErrorString(e));
         return PDFXC_ERR_MEMORY;
@@ -792,7 +793,7 @@ int device_partition(int64_t n64, const double* d_grid, int* d_order, hipStream_
         rc = check("block partition");
     }
     e = hipStreamSynchronize(s);  // the workspace and the host tables end here
-    (void)hipFree(ws);
+    pool.give(ws);
     if (rc == PDFXC_OK && e != hipSuccess) rc = hip_fail(e, "block partition");
     return rc;
 }

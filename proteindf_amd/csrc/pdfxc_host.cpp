@@ -49,6 +49,28 @@ static void dfree(T*& p) {
     p = nullptr;
 }
 
+// the same from a context's pool
+template <typename T>
+static int galloc(Context& c, T** p, size_t count) {
+    void* q = nullptr;
+    *p = nullptr;
+    if (count == 0) count = 1;
+    const hipError_t e = c.pool.take(&q, count * sizeof(T));
+    if (e != hipSuccess) {
+        set_error(std::string("hipMalloc of ") + std::to_string(count * sizeof(T)) +
+                  " bytes: " + hipGetErrorString(e));
+        return PDFXC_ERR_MEMORY;
+    }
+    *p = static_cast<T*>(q);
+    return PDFXC_OK;
+}
+
+template <typename T>
+static void gfree(Context& c, T*& p) {
+    if (p && !c.pool.give(p)) (void)hipFree(reinterpret_cast<void*>(p));
+    p = nullptr;
+}
+
 // ---------------------------------------------------------------------------
 // Contracted-GTO normalisation, as TlOrbitalInfoObject::setCGTO forms the
 // coefficients (TlOrbitalInfoObject.cpp:38-106): c_k = d_k N(a_k) N_c with the
@@ -333,43 +355,44 @@ int pdfxc_ctx_create(pdfxc_ctx** out, int n_aos, const double* ao_center, const 
 }
 
 static void free_grid_buffers(Context* c) {
-    dfree(c->d_pts);
-    dfree(c->d_slot_of_point);
-    dfree(c->d_blocks);
-    dfree(c->d_kblocks);
-    dfree(c->d_block_shells);
-    dfree(c->d_block_cols);
-    dfree(c->d_block_shell_col);
-    dfree(c->d_block_sorder);
-    dfree(c->d_rho_work);
-    dfree(c->d_k_work);
-    dfree(c->d_coef);
-    dfree(c->d_rho);
-    dfree(c->d_coef_b);
-    dfree(c->d_rho_b);
-    dfree(c->d_rho_out);
+    gfree(*c, c->d_pts);
+    gfree(*c, c->d_slot_of_point);
+    gfree(*c, c->d_blocks);
+    gfree(*c, c->d_kblocks);
+    gfree(*c, c->d_block_shells);
+    gfree(*c, c->d_block_cols);
+    gfree(*c, c->d_block_shell_col);
+    gfree(*c, c->d_block_sorder);
+    gfree(*c, c->d_rho_work);
+    gfree(*c, c->d_k_work);
+    gfree(*c, c->d_coef);
+    gfree(*c, c->d_rho);
+    gfree(*c, c->d_coef_b);
+    gfree(*c, c->d_rho_b);
+    gfree(*c, c->d_rho_out);
     c->n_rho_out = 0;
-    dfree(c->d_eblock);
-    dfree(c->d_sblocks);
-    dfree(c->d_chunks);
-    dfree(c->d_sshell_col);
-    dfree(c->d_srho_work);
-    dfree(c->d_kg_work);
-    dfree(c->d_kgroups);
-    dfree(c->d_kg_blocks);
-    dfree(c->d_kg_shells);
-    dfree(c->d_kg_shell_col);
-    dfree(c->d_kg_sorder);
-    dfree(c->d_kg_cols);
-    dfree(c->d_kg_masks);
+    gfree(*c, c->d_eblock);
+    gfree(*c, c->d_sblocks);
+    gfree(*c, c->d_chunks);
+    gfree(*c, c->d_sshell_col);
+    gfree(*c, c->d_srho_work);
+    gfree(*c, c->d_kg_work);
+    gfree(*c, c->d_kgroups);
+    gfree(*c, c->d_kg_blocks);
+    gfree(*c, c->d_kg_shells);
+    gfree(*c, c->d_kg_shell_col);
+    gfree(*c, c->d_kg_sorder);
+    gfree(*c, c->d_kg_cols);
+    gfree(*c, c->d_kg_masks);
 }
 
 int pdfxc_ctx_destroy(pdfxc_ctx* ctx) {
     Context* c = reinterpret_cast<Context*>(ctx);
     if (!c) return PDFXC_OK;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
+    if (c->probe) pdfxc_ctx_destroy(reinterpret_cast<pdfxc_ctx*>(c->probe));
     free_grid_buffers(c);
-    dfree(c->d_grid);
+    gfree(*c, c->d_grid);
     dfree(c->d_shells);
     dfree(c->d_shrec);
     dfree(c->d_P);
@@ -478,7 +501,8 @@ static double shell_cut(const Shell& s, double screen) {
 // this refuses builds with PDFXC_ERR_NO_GRID.
 static void reset_grid(Context& c) {
     free_grid_buffers(&c);
-    dfree(c.d_grid);
+    gfree(c, c.d_grid);
+    c.pool.trim(kPoolKeep);
     c.n_pts = 0;
     c.n_slots = 0;
     c.gx.clear();
@@ -539,17 +563,17 @@ static int build_blocks(Context& c) {
 
 // workspace freed at the end of its scope
 struct DeviceBuf {
+    Context& c;  // from its pool
     void* p = nullptr;
-    ~DeviceBuf() {
-        if (p) (void)hipFree(p);
-    }
+    explicit DeviceBuf(Context& ctx) : c(ctx) {}
+    ~DeviceBuf() { gfree(c, p); }
     template <typename T>
     T* as() const {
         return reinterpret_cast<T*>(p);
     }
     int alloc(size_t bytes) {
         char* q = nullptr;
-        const int rc = dalloc(&q, bytes);
+        const int rc = galloc(c, &q, bytes);
         p = q;
         return rc;
     }
@@ -600,7 +624,7 @@ static int build_blocks_impl(Context& c) {
     // Blocks per K unit: the FP64 K pass adds N_b^2 / 2 values to K by atomics
     // per unit, at 53 G/s a longer time than its matrix products, and the
     // union of two neighbours is only 2 % wider than either
-    int kper = c.opts.precision == PDFXC_FP64 ? std::min(kKGroupMax, c.tune.split_k_group) : 1;
+    int kper = c.opts.precision == PDFXC_FP64 && !c.rho_only ? std::min(kKGroupMax, c.tune.split_k_group) : 1;
     while (kper > 1 && nb / kper < kKUnitsPerCu * c.n_cu) kper /= 2;
     const int ng = kper > 1 ? (nb + kper - 1) / kper : 0;
     // workspace: order | masks | counts | leaf of every block | shell table | masks and unit list of the groups
@@ -610,7 +634,7 @@ static int build_blocks_impl(Context& c) {
                  b_sc = align(sizeof(ScreenShell) * (size_t)nsh),
                  b_gmask = align(sizeof(unsigned long long) * (size_t)ng * nw),
                  b_gcnt = align(2 * sizeof(int) * (size_t)ng);
-    DeviceBuf ws;
+    DeviceBuf ws(c);
     int rc = ws.alloc(b_order + b_mask + b_cnt + b_leaf + b_sc + b_gmask + b_gcnt + (ng ? b_leaf : 0));
     if (rc) return rc;
     int* d_order = ws.as<int>();
@@ -623,7 +647,7 @@ static int build_blocks_impl(Context& c) {
     int* d_group = reinterpret_cast<int*>(reinterpret_cast<char*>(d_gcounts) + b_gcnt);
     std::vector<int> order;
     if (c.opts.precision == PDFXC_FP64) {
-        rc = device_partition(n, c.d_grid, d_order, c.stream);
+        rc = device_partition(n, c.d_grid, d_order, c.stream, c.pool);
         if (rc) return rc;
     } else {
         if (int e = ensure_host_grid(c)) return e;
@@ -740,14 +764,14 @@ static int build_blocks_impl(Context& c) {
     const int nu = (int)c.kblocks.size();
     c.n_block_shells = sh0;
     c.n_block_cols = col0;
-    rc = dalloc(&c.d_pts, 4 * (size_t)c.n_slots);
-    if (rc == PDFXC_OK) rc = dalloc(&c.d_slot_of_point, (size_t)n);
-    if (rc == PDFXC_OK) rc = dalloc(&c.d_blocks, c.blocks.size());
-    if (rc == PDFXC_OK) rc = dalloc(&c.d_kblocks, c.kblocks.size());
-    if (rc == PDFXC_OK) rc = dalloc(&c.d_block_shells, (size_t)sh0);
-    if (rc == PDFXC_OK) rc = dalloc(&c.d_block_cols, (size_t)col0);
-    if (rc == PDFXC_OK) rc = dalloc(&c.d_block_shell_col, (size_t)sh0);
-    if (rc == PDFXC_OK) rc = dalloc(&c.d_block_sorder, (size_t)sh0);
+    rc = galloc(c, &c.d_pts, 4 * (size_t)c.n_slots);
+    if (rc == PDFXC_OK) rc = galloc(c, &c.d_slot_of_point, (size_t)n);
+    if (rc == PDFXC_OK) rc = galloc(c, &c.d_blocks, c.blocks.size());
+    if (rc == PDFXC_OK) rc = galloc(c, &c.d_kblocks, c.kblocks.size());
+    if (rc == PDFXC_OK) rc = galloc(c, &c.d_block_shells, (size_t)sh0);
+    if (rc == PDFXC_OK) rc = galloc(c, &c.d_block_cols, (size_t)col0);
+    if (rc == PDFXC_OK) rc = galloc(c, &c.d_block_shell_col, (size_t)sh0);
+    if (rc == PDFXC_OK) rc = galloc(c, &c.d_block_sorder, (size_t)sh0);
     if (rc) return rc;
     PDFXC_HIP(hipMemcpyAsync(c.d_blocks, c.blocks.data(), sizeof(BlockDesc) * (size_t)nb, hipMemcpyHostToDevice, c.stream));
     PDFXC_HIP(hipMemcpyAsync(d_leaf, lorder.data(), sizeof(int) * (size_t)nb, hipMemcpyHostToDevice, c.stream));
@@ -807,7 +831,7 @@ static int build_blocks_impl(Context& c) {
     // (k_tiles = 96; the tuning may cut those smaller)
     std::vector<KWork> kw[kKmatClasses];
     size_t klds[kKmatClasses] = {};
-    for (int b = 0; b < nu; ++b) {
+    for (int b = 0; b < nu && !c.rho_only; ++b) {
         const KBlock& B = c.kblocks[b];
         const int T = B.ldn / 16, Tp = (T + 1) / 2;
         const int np = Tp * (Tp + 1) / 2;
@@ -829,8 +853,8 @@ static int build_blocks_impl(Context& c) {
     size_t n_items = 0;
     for (const auto& w : kw) n_items += w.size();
     std::vector<int> item_nsh(n_items);
-    {
-        DeviceBuf items;
+    if (n_items > 0) {
+        DeviceBuf items(c);
         if (int e = items.alloc((sizeof(KWork) + sizeof(int)) * n_items)) return e;
         KWork* d_items = items.as<KWork>();
         int* d_nsh = reinterpret_cast<int*>(d_items + n_items);
@@ -1157,29 +1181,29 @@ static int build_blocks_impl(Context& c) {
     }
 
     // device buffers
-    if (rc == PDFXC_OK) rc = dalloc(&c.d_rho_work, rho_work.size());
-    if (rc == PDFXC_OK) rc = dalloc(reinterpret_cast<char**>(&c.d_k_work), kall.size() * sizeof(KWork));
-    if (rc == PDFXC_OK) rc = dalloc(&c.d_coef, 4 * (size_t)c.n_slots);
-    if (rc == PDFXC_OK) rc = dalloc(&c.d_rho, 4 * (size_t)c.n_slots);
-    if (rc == PDFXC_OK) rc = dalloc(&c.d_eblock, 3 * (size_t)((c.n_slots + 255) / 256));
+    if (rc == PDFXC_OK) rc = galloc(c, &c.d_rho_work, rho_work.size());
+    if (rc == PDFXC_OK) rc = galloc(c, reinterpret_cast<char**>(&c.d_k_work), kall.size() * sizeof(KWork));
+    if (rc == PDFXC_OK && !c.rho_only) rc = galloc(c, &c.d_coef, 4 * (size_t)c.n_slots);
+    if (rc == PDFXC_OK) rc = galloc(c, &c.d_rho, 4 * (size_t)c.n_slots);
+    if (rc == PDFXC_OK) rc = galloc(c, &c.d_eblock, 3 * (size_t)((c.n_slots + 255) / 256));
     if (rc == PDFXC_OK && c.opts.precision != PDFXC_FP64) {
-        rc = dalloc(&c.d_sblocks, c.sblocks.size());
-        if (rc == PDFXC_OK) rc = dalloc(&c.d_chunks, c.chunks.size());
-        if (rc == PDFXC_OK) rc = dalloc(&c.d_sshell_col, c.sshell_col.size());
-        if (rc == PDFXC_OK) rc = dalloc(&c.d_srho_work, srho_work.size());
-        if (rc == PDFXC_OK) rc = dalloc(&c.d_kg_work, skw.size());
-        if (rc == PDFXC_OK) rc = dalloc(&c.d_kgroups, c.kgroups.size());
-        if (rc == PDFXC_OK) rc = dalloc(&c.d_kg_blocks, c.kg_blocks.size());
-        if (rc == PDFXC_OK) rc = dalloc(&c.d_kg_shells, c.kg_shells.size());
-        if (rc == PDFXC_OK) rc = dalloc(&c.d_kg_shell_col, c.kg_shell_col.size());
-        if (rc == PDFXC_OK) rc = dalloc(&c.d_kg_sorder, c.kg_sorder.size());
-        if (rc == PDFXC_OK) rc = dalloc(&c.d_kg_cols, c.kg_cols.size());
-        if (rc == PDFXC_OK) rc = dalloc(&c.d_kg_masks, c.kg_masks.size());
+        rc = galloc(c, &c.d_sblocks, c.sblocks.size());
+        if (rc == PDFXC_OK) rc = galloc(c, &c.d_chunks, c.chunks.size());
+        if (rc == PDFXC_OK) rc = galloc(c, &c.d_sshell_col, c.sshell_col.size());
+        if (rc == PDFXC_OK) rc = galloc(c, &c.d_srho_work, srho_work.size());
+        if (rc == PDFXC_OK) rc = galloc(c, &c.d_kg_work, skw.size());
+        if (rc == PDFXC_OK) rc = galloc(c, &c.d_kgroups, c.kgroups.size());
+        if (rc == PDFXC_OK) rc = galloc(c, &c.d_kg_blocks, c.kg_blocks.size());
+        if (rc == PDFXC_OK) rc = galloc(c, &c.d_kg_shells, c.kg_shells.size());
+        if (rc == PDFXC_OK) rc = galloc(c, &c.d_kg_shell_col, c.kg_shell_col.size());
+        if (rc == PDFXC_OK) rc = galloc(c, &c.d_kg_sorder, c.kg_sorder.size());
+        if (rc == PDFXC_OK) rc = galloc(c, &c.d_kg_cols, c.kg_cols.size());
+        if (rc == PDFXC_OK) rc = galloc(c, &c.d_kg_masks, c.kg_masks.size());
     }
     if (rc != PDFXC_OK) return rc;
     auto up = [](void* d, const void* h, size_t n) { return hipMemcpy(d, h, n, hipMemcpyHostToDevice); };
     PDFXC_HIP(up(c.d_rho_work, rho_work.data(), rho_work.size() * sizeof(int)));
-    PDFXC_HIP(up(c.d_k_work, kall.data(), kall.size() * sizeof(KWork)));
+    if (!kall.empty()) PDFXC_HIP(up(c.d_k_work, kall.data(), kall.size() * sizeof(KWork)));
     if (c.opts.precision != PDFXC_FP64) {
         PDFXC_HIP(up(c.d_sblocks, c.sblocks.data(), c.sblocks.size() * sizeof(SplitBlock)));
         PDFXC_HIP(up(c.d_chunks, c.chunks.data(), c.chunks.size() * sizeof(int)));
@@ -1196,7 +1220,7 @@ static int build_blocks_impl(Context& c) {
             PDFXC_HIP(up(c.d_kg_masks, c.kg_masks.data(), c.kg_masks.size() * sizeof(unsigned)));
         }
     }
-    PDFXC_HIP(hipMemsetAsync(c.d_coef, 0, 4 * (size_t)c.n_slots * sizeof(double), c.stream));
+    if (!c.rho_only) PDFXC_HIP(hipMemsetAsync(c.d_coef, 0, 4 * (size_t)c.n_slots * sizeof(double), c.stream));
     PDFXC_HIP(hipMemsetAsync(c.d_rho, 0, 4 * (size_t)c.n_slots * sizeof(double), c.stream));
     PDFXC_HIP(hipMemsetAsync(c.d_eblock, 0, 3 * (size_t)((c.n_slots + 255) / 256) * sizeof(double), c.stream));
     PDFXC_HIP(hipStreamSynchronize(c.stream));
@@ -1464,14 +1488,14 @@ int ensure_host_slots(Context& c) {
 // A buffer for a new grid's columns; the old grid and its buffers go first.
 static int alloc_grid(Context& c, int64_t n, double** d_grid) {
     reset_grid(c);
-    return dalloc(d_grid, 4 * (size_t)n);
+    return galloc(c, d_grid, 4 * (size_t)n);
 }
 
 // Takes over d_grid (n x 4 columns, written on c.stream) as the context's grid
 // and builds its blocks; a grid with a value that is not finite is refused and
 // leaves the context without one.
 static int set_device_grid(Context& c, int64_t n, double* d_grid, const char* who) {
-    dfree(c.d_grid);
+    gfree(c, c.d_grid);
     c.d_grid = d_grid;
     c.gx.clear();
     c.gy.clear();
@@ -1558,7 +1582,7 @@ int pdfxc_set_grid(pdfxc_ctx* ctx, int64_t n_pts, const double* x, const double*
         const hipError_t e = hipMemcpyAsync(d_grid + q * n_pts, col[q], sizeof(double) * (size_t)n_pts,
                                             hipMemcpyHostToDevice, c->stream);
         if (e != hipSuccess) {
-            dfree(d_grid);
+            gfree(*c, d_grid);
             return hip_fail(e, "pdfxc_set_grid: upload");
         }
     }
@@ -1589,7 +1613,7 @@ int pdfxc_get_grid_rows(pdfxc_ctx* ctx, double* xyzw) {
         return PDFXC_ERR_NO_GRID;
     }
     const int64_t per = std::min<int64_t>(c->n_pts, 1 << 22);  // 128 MiB of rows at a time
-    DeviceBuf rows;
+    DeviceBuf rows(*c);
     if (int rc = rows.alloc(4 * sizeof(double) * (size_t)per)) return rc;
     for (int64_t at = 0; at < c->n_pts; at += per) {
         const int64_t n = std::min(per, c->n_pts - at);
@@ -1759,7 +1783,7 @@ static int generate_grid_impl(pdfxc_ctx* ctx, int n_atoms, const int* Z, const d
     // DfGenerateGrid.cpp:1979-2004), all of it on the device
     const int ns = (int)shells.size();
     std::vector<long long> first(ns + 1, 0);  // first kept point of every shell, and their number
-    DeviceBuf tab, raw;
+    DeviceBuf tab(*c), raw(*c);
     auto align = [](size_t b) { return (b + 255) / 256 * 256; };
     const size_t b_at = align(at.size() * sizeof(double)), b_sh = align(shells.size() * sizeof(RawShell)),
                  b_dir = align(dirs.size() * sizeof(double)), b_first = align(first.size() * sizeof(long long));
@@ -1805,7 +1829,7 @@ static int generate_grid_impl(pdfxc_ctx* ctx, int n_atoms, const int* Z, const d
     if (rc) return rc;
     rc = launch_keep_write(ns, d_sh, d_p, d_w, o.weight_cutoff, d_first, n_kept, d_grid, c->stream);
     if (rc) {
-        dfree(d_grid);
+        gfree(*c, d_grid);
         return rc;
     }
     rc = set_device_grid(*c, n_kept, d_grid, "pdfxc_set_grid");
@@ -2241,13 +2265,13 @@ int pdfxc_gradient_rks(pdfxc_ctx* ctx, int functional, int n_atoms, const int* Z
     const std::vector<int> near = near_atoms(na, xyz);
     int *d_shat = nullptr, *d_slat = nullptr, *d_near = nullptr, *d_ptat = nullptr;
     double *d_at = nullptr, *d_ewf = nullptr, *d_g = nullptr;
-    int rc = dalloc(&d_shat, shell_atom.size());
-    if (rc == PDFXC_OK) rc = dalloc(&d_slat, (size_t)c->n_slots);
-    if (rc == PDFXC_OK) rc = dalloc(&d_ptat, (size_t)c->n_pts);
-    if (rc == PDFXC_OK) rc = dalloc(&d_near, near.size());
-    if (rc == PDFXC_OK) rc = dalloc(&d_at, at.size());
-    if (rc == PDFXC_OK) rc = dalloc(&d_ewf, (size_t)c->n_slots);
-    if (rc == PDFXC_OK) rc = dalloc(&d_g, 6 * (size_t)na);
+    int rc = galloc(*c, &d_shat, shell_atom.size());
+    if (rc == PDFXC_OK) rc = galloc(*c, &d_slat, (size_t)c->n_slots);
+    if (rc == PDFXC_OK) rc = galloc(*c, &d_ptat, (size_t)c->n_pts);
+    if (rc == PDFXC_OK) rc = galloc(*c, &d_near, near.size());
+    if (rc == PDFXC_OK) rc = galloc(*c, &d_at, at.size());
+    if (rc == PDFXC_OK) rc = galloc(*c, &d_ewf, (size_t)c->n_slots);
+    if (rc == PDFXC_OK) rc = galloc(*c, &d_g, 6 * (size_t)na);
     hipError_t e = hipSuccess;
     if (rc == PDFXC_OK) {
         e = hipMemcpy(d_shat, shell_atom.data(), sizeof(int) * shell_atom.size(), hipMemcpyHostToDevice);
@@ -2286,13 +2310,14 @@ int pdfxc_gradient_rks(pdfxc_ctx* ctx, int functional, int n_atoms, const int* Z
         if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
         if (e != hipSuccess) rc = hip_fail(e, "pdfxc_gradient_rks: results");
     }
-    dfree(d_shat);
-    dfree(d_slat);
-    dfree(d_ptat);
-    dfree(d_near);
-    dfree(d_at);
-    dfree(d_ewf);
-    dfree(d_g);
+    if (rc != PDFXC_OK) (void)hipStreamSynchronize(c->stream);  // before the buffers change hands
+    gfree(*c, d_shat);
+    gfree(*c, d_slat);
+    gfree(*c, d_ptat);
+    gfree(*c, d_near);
+    gfree(*c, d_at);
+    gfree(*c, d_ewf);
+    gfree(*c, d_g);
     if (rc != PDFXC_OK) return rc;
     std::copy(g.begin(), g.begin() + 3 * na, grad_functional);
     std::copy(g.begin() + 3 * na, g.end(), grad_weight);
@@ -2391,41 +2416,51 @@ int pdfxc_density_at_points(pdfxc_ctx* ctx, const double* P_packed, int64_t n, c
     if (n < 0 || (n > 0 && (!P_packed || !xyz || !rho))) return arg_error("pdfxc_density_at_points: bad arguments");
     if (n == 0) return PDFXC_OK;
     const int N = c->n_aos;
-    std::vector<double> center(3 * (size_t)N), exps((size_t)N * kMaxPrim, 0.0), coefs((size_t)N * kMaxPrim, 0.0);
-    std::vector<int> type(N), nprim(N);
-    static const int first_type[3] = {0, 1, 4};
-    for (const Shell& sh : c->shells)
-        for (int m = 0; m < 2 * sh.l + 1; ++m) {
-            const int a = sh.first_ao + m;
-            type[a] = first_type[sh.l] + m;
-            nprim[a] = sh.nprim;
-            for (int d = 0; d < 3; ++d) center[3 * a + d] = sh.center[d];
-            for (int k = 0; k < sh.nprim; ++k) {
-                exps[(size_t)a * kMaxPrim + k] = sh.exps[k];
-                coefs[(size_t)a * kMaxPrim + k] = sh.coefs[k];
+    // the points' own context is kept for the next call; a second call at the
+    // same time, or on another device, makes one for itself
+    int dev = 0;
+    PDFXC_HIP(hipGetDevice(&dev));
+    std::unique_lock<std::mutex> lock(c->probe_mu, std::try_to_lock);
+    const bool keep = lock.owns_lock() && dev == c->device;
+    pdfxc_ctx* th = keep ? reinterpret_cast<pdfxc_ctx*>(c->probe) : nullptr;
+    if (keep) c->probe = nullptr;  // back once the call has succeeded
+    int rc = PDFXC_OK;
+    if (!th) {
+        std::vector<double> center(3 * (size_t)N), exps((size_t)N * kMaxPrim, 0.0), coefs((size_t)N * kMaxPrim, 0.0);
+        std::vector<int> type(N), nprim(N);
+        static const int first_type[3] = {0, 1, 4};
+        for (const Shell& sh : c->shells)
+            for (int m = 0; m < 2 * sh.l + 1; ++m) {
+                const int a = sh.first_ao + m;
+                type[a] = first_type[sh.l] + m;
+                nprim[a] = sh.nprim;
+                for (int d = 0; d < 3; ++d) center[3 * a + d] = sh.center[d];
+                for (int k = 0; k < sh.nprim; ++k) {
+                    exps[(size_t)a * kMaxPrim + k] = sh.exps[k];
+                    coefs[(size_t)a * kMaxPrim + k] = sh.coefs[k];
+                }
             }
-        }
-    pdfxc_opts o = c->opts;
-    o.precision = PDFXC_FP64;
-    pdfxc_ctx* th = nullptr;
-    int rc = pdfxc_ctx_create(&th, N, center.data(), type.data(), nprim.data(), exps.data(), coefs.data(), kMaxPrim,
-                              &o);
-    if (rc) return rc;
+        pdfxc_opts o = c->opts;
+        o.precision = PDFXC_FP64;
+        rc = pdfxc_ctx_create(&th, N, center.data(), type.data(), nprim.data(), exps.data(), coefs.data(), kMaxPrim, &o);
+        if (rc) return rc;
+        reinterpret_cast<Context*>(th)->rho_only = true;
+    }
     Context* t = reinterpret_cast<Context*>(th);
     if (n > ((int64_t)1 << 31) - kBlockPts) {
         rc = arg_error("pdfxc_set_grid: more than 2^31 points");
     }
     // one buffer for the points on their way in and for (rho, grad rho) on its way out
-    DeviceBuf io;
-    if (rc == PDFXC_OK) rc = io.alloc(sizeof(double) * 4 * (size_t)n);
+    double* d_io = nullptr;
+    if (rc == PDFXC_OK) rc = galloc(*t, &d_io, 4 * (size_t)n);
     double* d_grid = nullptr;
     if (rc == PDFXC_OK) rc = alloc_grid(*t, n, &d_grid);
     if (rc == PDFXC_OK) {
-        const hipError_t e = hipMemcpyAsync(io.p, xyz, sizeof(double) * 3 * (size_t)n, hipMemcpyHostToDevice, t->stream);
-        rc = e == hipSuccess ? launch_points_to_grid(n, io.as<double>(), d_grid, t->stream)
+        const hipError_t e = hipMemcpyAsync(d_io, xyz, sizeof(double) * 3 * (size_t)n, hipMemcpyHostToDevice, t->stream);
+        rc = e == hipSuccess ? launch_points_to_grid(n, d_io, d_grid, t->stream)
                              : hip_fail(e, "pdfxc_density_at_points: points upload");
         if (rc == PDFXC_OK) rc = set_device_grid(*t, n, d_grid, "pdfxc_set_grid");
-        else dfree(d_grid);
+        else gfree(*t, d_grid);
     }
     if (rc == PDFXC_OK) {
         const size_t NP = (size_t)N * (N + 1) / 2;
@@ -2437,17 +2472,27 @@ int pdfxc_density_at_points(pdfxc_ctx* ctx, const double* P_packed, int64_t n, c
     if (rc == PDFXC_OK) rc = run_rho(t, t->d_P, t->d_rho);
     if (rc == PDFXC_OK) {
         // columns rho | grad rho x 3: the first alone unless the gradient is asked for
-        rc = launch_gather_density(*t, t->d_rho, io.as<double>(), grad_rho != nullptr);
+        rc = launch_gather_density(*t, t->d_rho, d_io, grad_rho != nullptr);
         hipError_t e = hipSuccess;
         if (rc == PDFXC_OK)
-            e = hipMemcpyAsync(rho, io.p, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost, t->stream);
+            e = hipMemcpyAsync(rho, d_io, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost, t->stream);
         if (rc == PDFXC_OK && e == hipSuccess && grad_rho)
-            e = hipMemcpyAsync(grad_rho, io.as<double>() + n, sizeof(double) * 3 * (size_t)n, hipMemcpyDeviceToHost,
+            e = hipMemcpyAsync(grad_rho, d_io + n, sizeof(double) * 3 * (size_t)n, hipMemcpyDeviceToHost,
                                t->stream);
         if (rc == PDFXC_OK && e == hipSuccess) e = hipStreamSynchronize(t->stream);
         if (e != hipSuccess) rc = hip_fail(e, "pdfxc_density_at_points: download");
     }
+    if (rc == PDFXC_OK && keep) {
+        gfree(*t, d_io);
+        reset_grid(*t);  // its buffers wait for the next call, up to kPoolKeep
+        c->probe = t;
+        return PDFXC_OK;
+    }
+    (void)hipStreamSynchronize(t->stream);
+    gfree(*t, d_io);
+    const std::string msg = g_last_error;
     pdfxc_ctx_destroy(th);
+    if (rc) set_error(msg);
     return rc;
 }
 
