@@ -484,10 +484,18 @@ __device__ inline double group_prod(double v) {
 // not negligible contribute, so a group of GW lanes takes one point:
 //   1. a cell per lane against the kNear atoms nearest to A, which ends every
 //      cell with two zero factors (then P_i and every G_ij are 0) or a product
-//      below 1e-24 (s is 0 or above 5e-17, where ds/dmu is at most 4e4 s, so
-//      G_ij R_ij / Z stays below 1e-19; A's own cell, whose terms are divided
-//      by P_A, keeps any product).  16 near atoms leave 8 cells of 24 and 13 of
-//      59 on average, 8 atoms leave 10 and 18;
+//      below 1e-22 of Z (A's own cell, whose terms are divided by P_A, keeps
+//      any).  Such a cell's share K omega G_ij of the point's term is e / R_ij
+//      times (P_i / Z) (ds/dmu / s): s is 0 or at least 5.5e-17, where
+//      ds/dmu / s is at most 5e3 (Becke) or 3.5e5 (Stratmann-Scuseria, whose s
+//      is rounding alone there), so the share stays below 5e-19 or 4e-17 of e.
+//      Z is not known yet, so the first cut is at 1e-24, which serves every
+//      Z >= 1e-2; the few points below (1 in 2,000 on the grids of 8 waters and
+//      a helix of 8 residues, but all those inside a hollow cage, where n atoms
+//      as far as one another leave Z = n 2^-(n - 1)) go through 1. and 2. once
+//      more with the cut at 1e-24 of the Z found.
+//      16 near atoms leave 8 cells of 24 and 13 of 59 on average, 8 atoms
+//      leave 10 and 18;
 //   2. a neighbour per lane for each cell left: P_i without its zero factors;
 //   3. the same again for G_ij: lane j adds the term of atom j, the group's
 //      sum of the rest goes to atom i.
@@ -503,7 +511,7 @@ __device__ inline double group_prod(double v) {
 // ss: the grid's partition is Stratmann-Scuseria (else Becke).
 // LDS: xyz [3 na] | per group: r, product [na], unit vectors, sums [3 na] | per group: cells [na]
 // ---------------------------------------------------------------------------
-constexpr double kCellMin = 1e-24;
+constexpr double kCellMin = 1e-24, kCellZ = 1e-2;
 
 // 1 / x to the last bit or two, for x away from the ends of the exponent range:
 // the hardware's estimate and two Newton steps (a full division is twice that)
@@ -560,63 +568,74 @@ __global__ __launch_bounds__(256) void k_grad_w(const double* __restrict__ atoms
         }
         __builtin_amdgcn_wave_barrier();
         __threadfence_block();
-        // 1. cells that survive the nearest atoms of A
+        // twice where some point of the wave has a Z so small that the first cut
+        // may have dropped too much: the second cut is taken from its Z, which
+        // the cells added can only raise
+        double cut = kCellMin, Zs = 0.0, PA = 0.0;
         int ncell = 0;
-        for (int m0 = 0; m0 < na; m0 += GW) {
-            const int m = m0 + gl;
-            bool live = valid && m < na;
-            if (live) {
-                const double rm = r[m];
+#pragma unroll 1
+        for (int pass = 0;; ++pass) {
+            // 1. cells that survive the nearest atoms of A
+            ncell = 0;
+            for (int m0 = 0; m0 < na; m0 += GW) {
+                const int m = m0 + gl;
+                bool live = valid && m < na;
+                if (live) {
+                    const double rm = r[m];
+                    double p = 1.0;
+                    int nz = 0;
+                    for (int q = 0; q < kNear && live; ++q) {
+                        const int k = nbr[A * kNear + q];
+                        if (k < 0) break;
+                        if (k == m) continue;
+                        const double mu = (rm - r[k]) * invd[(size_t)m * na + k];
+                        double s, ds;
+                        cell_step(ss, mu, amat[(size_t)m * na + k], s, ds);
+                        if (s > 0.0)
+                            p *= s;
+                        else
+                            ++nz;
+                        live = nz < 2 && (p >= cut || m == A);
+                    }
+                }
+                const unsigned long long b = __ballot(live);
+                if (live) cell[ncell + __popcll(b & below)] = m;
+                ncell += __popcll(b & gmask);
+            }
+            __builtin_amdgcn_wave_barrier();
+            __threadfence_block();
+            // 2. P_i of the cells left: the product of the factors that are not 0,
+            // negated when one is 0 (P_i = 0), 0 when more are
+            Zs = PA = 0.0;
+            for (int c = 0; c < ncell; ++c) {
+                const int i = cell[c];
+                const double ri = r[i];
                 double p = 1.0;
                 int nz = 0;
-                for (int q = 0; q < kNear && live; ++q) {
-                    const int k = nbr[A * kNear + q];
-                    if (k < 0) break;
-                    if (k == m) continue;
-                    const double mu = (rm - r[k]) * invd[(size_t)m * na + k];
-                    double s, ds;
-                    cell_step(ss, mu, amat[(size_t)m * na + k], s, ds);
-                    if (s > 0.0)
-                        p *= s;
-                    else
-                        ++nz;
-                    live = nz < 2 && (p >= kCellMin || m == A);
+                for (int j0 = 0; j0 < na; j0 += GW) {
+                    const int j = j0 + gl;
+                    bool zero = false;
+                    if (j < na && j != i) {
+                        double s, ds;
+                        cell_step(ss, (ri - r[j]) * invd[(size_t)i * na + j], amat[(size_t)i * na + j], s, ds);
+                        zero = !(s > 0.0);
+                        if (!zero) p *= s;
+                    }
+                    nz += __popcll(__ballot(zero) & gmask);
                 }
-            }
-            const unsigned long long b = __ballot(live);
-            if (live) cell[ncell + __popcll(b & below)] = m;
-            ncell += __popcll(b & gmask);
-        }
-        __builtin_amdgcn_wave_barrier();
-        __threadfence_block();
-        // 2. P_i of the cells left: the product of the factors that are not 0,
-        // negated when one is 0 (P_i = 0), 0 when more are
-        double Zs = 0.0, PA = 0.0;
-        for (int c = 0; c < ncell; ++c) {
-            const int i = cell[c];
-            const double ri = r[i];
-            double p = 1.0;
-            int nz = 0;
-            for (int j0 = 0; j0 < na; j0 += GW) {
-                const int j = j0 + gl;
-                bool zero = false;
-                if (j < na && j != i) {
-                    double s, ds;
-                    cell_step(ss, (ri - r[j]) * invd[(size_t)i * na + j], amat[(size_t)i * na + j], s, ds);
-                    zero = !(s > 0.0);
-                    if (!zero) p *= s;
+                p = group_prod<GW>(p);
+                if (nz == 0) {
+                    Zs += p;
+                    if (i == A) PA = p;
                 }
-                nz += __popcll(__ballot(zero) & gmask);
+                if (gl == 0) Pv[c] = nz > 1 ? 0.0 : nz == 1 ? -p : p;
             }
-            p = group_prod<GW>(p);
-            if (nz == 0) {
-                Zs += p;
-                if (i == A) PA = p;
-            }
-            if (gl == 0) Pv[c] = (nz > 1 || (p < kCellMin && i != A)) ? 0.0 : nz == 1 ? -p : p;
+            __builtin_amdgcn_wave_barrier();
+            __threadfence_block();
+            const bool again = pass == 0 && PA > 0.0 && Zs < kCellZ;
+            if (__ballot(again) == 0ull) break;
+            if (again) cut = kCellMin * Zs;
         }
-        __builtin_amdgcn_wave_barrier();
-        __threadfence_block();
         // 3. the pair terms (none where omega = 0)
         const double om = PA > 0.0 ? PA / Zs : 0.0;
         if (om > 0.0) {
@@ -625,7 +644,7 @@ __global__ __launch_bounds__(256) void k_grad_w(const double* __restrict__ atoms
             for (int c = 0; c < ncell; ++c) {
                 const int i = cell[c];
                 const double Pc = Pv[c];
-                if (Pc == 0.0) continue;
+                if (Pc == 0.0 || (i != A && fabs(Pc) < kCellMin * Zs)) continue;
                 const double f = K * ((i == A ? 1.0 : 0.0) - om) * fabs(Pc);
                 const double ri = r[i];
                 const double xi = s_xyz[3 * i], yi = s_xyz[3 * i + 1], zi = s_xyz[3 * i + 2];
