@@ -222,9 +222,11 @@ int pdfxc_get_grid(pdfxc_ctx* ctx, double* x, double* y, double* z, double* w);
 /* The same as rows (x, y, z, w), 4 n_pts values. */
 int pdfxc_get_grid_rows(pdfxc_ctx* ctx, double* xyzw);
 
-/* getWholeDensity (DfCalcGridX.cpp:2502-2537): the integrated rho_alpha (and,
- * after a UKS build, rho_beta; n_beta may be null) of the context's last build
- * through a host entry point. */
+/* getWholeDensity (DfCalcGridX.cpp:2502-2537): the integrated rho_alpha and
+ * rho_beta (0 after an RKS build; n_beta may be null) of the context's last
+ * build through a host entry point; both are 0 after an HF build, which forms
+ * no density.  PDFXC_ERR_ARGUMENT before such a build, after one that failed
+ * and after the grid was set anew. */
 int pdfxc_whole_density(pdfxc_ctx* ctx, double* n_alpha, double* n_beta);
 
 /* calcXCIntegForFockAndEnergy, RKS (DfCalcGridX.cpp:2280-2289 LDA, :2305-2315 GGA):

@@ -503,6 +503,7 @@ static void reset_grid(Context& c) {
     free_grid_buffers(&c);
     gfree(c, c.d_grid);
     c.pool.trim(kPoolKeep);
+    c.whole_spins = 0;
     c.n_pts = 0;
     c.n_slots = 0;
     c.gx.clear();
@@ -2020,11 +2021,14 @@ int pdfxc_build_rks(pdfxc_ctx* ctx, int functional, const double* P_packed, doub
 
 static int build_host(Context* c, int xc, int nspin, const double* const* P_packed, double* const* K_packed,
                       double* E_xc, double* rho_out, int accumulate_rho) {
+    c->whole_spins = 0;  // n_whole is this build's, once it has succeeded
+    c->n_whole[0] = c->n_whole[1] = 0.0;
     if (c->n_pts == 0 || c->blocks.empty()) {
         set_error("build: no grid set");
         return PDFXC_ERR_NO_GRID;
     }
     if (xc == kHF) {
+        c->whole_spins = nspin;  // no density is formed: both integrals are 0
         // no grid term: E_xc = 0, K and rho_out untouched (DfXCFunctional.h:141-143)
         *E_xc = 0.0;
         for (double& t : c->last_kernel_ms) t = 0.0;
@@ -2072,6 +2076,7 @@ static int build_host(Context* c, int xc, int nspin, const double* const* P_pack
         PDFXC_HIP(hipMemcpyAsync(rho_out, c->d_rho_out, sizeof(double) * n_out, hipMemcpyDeviceToHost, c->stream));
         PDFXC_HIP(hipStreamSynchronize(c->stream));
     }
+    c->whole_spins = nspin;
     return PDFXC_OK;
 }
 
@@ -2094,6 +2099,7 @@ static int uks_args(Context* c, int functional, const void* a, const void* b, co
 int pdfxc_whole_density(pdfxc_ctx* ctx, double* n_alpha, double* n_beta) {
     Context* c = reinterpret_cast<Context*>(ctx);
     if (!c || !n_alpha) return arg_error("pdfxc_whole_density: bad arguments");
+    if (c->whole_spins == 0) return arg_error("pdfxc_whole_density: no host build has succeeded on this grid");
     *n_alpha = c->n_whole[0];
     if (n_beta) *n_beta = c->n_whole[1];
     return PDFXC_OK;

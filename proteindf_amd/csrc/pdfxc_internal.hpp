@@ -296,7 +296,8 @@ struct Context {
     double* d_packed = nullptr;   // host entry points: packed P in, packed K and E, integrated densities out
     double* h_pinned = nullptr;   // its pinned staging (packed_doubles(N) values)
     int whole_density = 0;        // spins whose integrated density the running build sums (0: none)
-    double n_whole[2] = {0.0, 0.0};  // integrated rho_alpha (and rho_beta) of the last host build
+    int whole_spins = 0;         // spins of the last host build on this grid, 0 when there is none
+    double n_whole[2] = {0.0, 0.0};  // its integrated rho_alpha and rho_beta (0 after an RKS build)
 
     // split precision (opts.precision != PDFXC_FP64)
     int split_nc = 0;                   // N rounded up to 8: row length of the P slices

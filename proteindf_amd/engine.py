@@ -405,7 +405,7 @@ class XcContext:
         return E.value, K, rho
 
     def whole_density(self, nspin=1):
-        """Integrated rho_alpha (nspin 1) or (rho_alpha, rho_beta) of the last host build."""
+        """Integrated rho_alpha (nspin 1) or (rho_alpha, rho_beta) of the last host build on this grid."""
         n = (ctypes.c_double(), ctypes.c_double())
         check(lib().pdfxc_whole_density(self.h, ctypes.byref(n[0]), ctypes.byref(n[1])))
         return n[0].value if nspin == 1 else (n[0].value, n[1].value)
