@@ -1451,6 +1451,7 @@ static void orientation(int na, const int* Z, const double* xyz, double O[9]) {
 }
 
 int ensure_host_grid(Context& c) {
+    std::lock_guard<std::mutex> lock(c.host_mu);
     if ((int64_t)c.gx.size() == c.n_pts) return PDFXC_OK;
     std::vector<double>* g[4] = {&c.gx, &c.gy, &c.gz, &c.gw};
     for (int q = 3; q >= 0; --q) {
@@ -1463,6 +1464,7 @@ int ensure_host_grid(Context& c) {
 }
 
 int ensure_host_lists(Context& c) {
+    std::lock_guard<std::mutex> lock(c.host_mu);
     if ((int64_t)c.block_cols.size() == c.n_block_cols && (int64_t)c.block_shells.size() == c.n_block_shells)
         return PDFXC_OK;
     auto get = [&](std::vector<int>& v, const int* d, int64_t n) {
@@ -1478,6 +1480,7 @@ int ensure_host_lists(Context& c) {
 }
 
 int ensure_host_slots(Context& c) {
+    std::lock_guard<std::mutex> lock(c.host_mu);
     if ((int64_t)c.slot_of_point.size() == c.n_pts) return PDFXC_OK;
     std::vector<int> s((size_t)c.n_pts);
     PDFXC_HIP(hipMemcpyAsync(s.data(), c.d_slot_of_point, sizeof(int) * (size_t)c.n_pts, hipMemcpyDeviceToHost, c.stream));

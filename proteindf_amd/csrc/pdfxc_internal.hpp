@@ -163,6 +163,8 @@ struct DeviceShell {
 // the next: 18 allocations and as many frees took 4 of the 26 ms of a new
 // FINE grid of a 20-residue helix and half of a small density call.  All use
 // is on the context's stream, whose work ends before a buffer changes hands.
+// Several threads may take and give: a grid may be read (pdfxc_get_grid_rows)
+// while another thread builds.
 // Buffers not in use are bounded by trim and go with the context.
 class DevicePool {
 public:
@@ -170,6 +172,7 @@ public:
         for (const Buf& b : bufs_) (void)hipFree(b.p);
     }
     hipError_t take(void** p, size_t bytes) {
+        std::lock_guard<std::mutex> lock(mu_);
         Buf* best = nullptr;
         for (Buf& b : bufs_)
             if (!b.used && b.cap >= bytes && b.cap <= 2 * bytes + 65536 && (!best || b.cap < best->cap)) best = &b;
@@ -182,7 +185,7 @@ public:
             hipError_t e = hipMalloc(&q, cap);
             if (e != hipSuccess) {
                 (void)hipGetLastError();
-                trim(0);
+                trim_locked(0);
                 e = hipMalloc(&q, cap);
             }
             if (e != hipSuccess) return e;
@@ -194,6 +197,7 @@ public:
         return hipSuccess;
     }
     bool give(void* p) {  // false: not one of this pool's
+        std::lock_guard<std::mutex> lock(mu_);
         for (Buf& b : bufs_)
             if (b.p == p) {
                 b.used = false;
@@ -202,6 +206,12 @@ public:
         return false;
     }
     void trim(size_t keep) {  // frees unused buffers, the largest first, until at most `keep` bytes are left
+        std::lock_guard<std::mutex> lock(mu_);
+        trim_locked(keep);
+    }
+
+private:
+    void trim_locked(size_t keep) {
         std::sort(bufs_.begin(), bufs_.end(), [](const Buf& a, const Buf& b) { return a.cap < b.cap; });
         size_t kept = 0;
         std::vector<Buf> left;
@@ -218,12 +228,12 @@ public:
         bufs_.swap(left);
     }
 
-private:
     struct Buf {
         void* p;
         size_t cap;
         bool used;
     };
+    std::mutex mu_;
     std::vector<Buf> bufs_;
 };
 constexpr size_t kPoolKeep = (size_t)512 << 20;
@@ -242,7 +252,9 @@ struct Context {
     hipEvent_t ev[6] = {};
 
     // grid in caller order: x, y, z, w columns on the device; host copies only
-    // where a caller needs them (ensure_host_grid)
+    // where a caller needs them (ensure_host_grid; host_mu while they are made:
+    // batches on several threads may share contexts)
+    std::mutex host_mu;
     int64_t n_pts = 0;
     double* d_grid = nullptr;
     std::vector<double> gx, gy, gz, gw;
