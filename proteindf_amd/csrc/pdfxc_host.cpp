@@ -580,6 +580,26 @@ struct DeviceBuf {
     }
 };
 
+// For a call that reads a context and has nothing to do with the program's
+// current device or with a graph that some thread is capturing on a stream of
+// its own: the context's device for the scope, and allocations outside the
+// capture's rules (they would be refused and end it).
+class ReadScope {
+public:
+    explicit ReadScope(const Context& c) : device_(c.device) {
+        (void)hipThreadExchangeStreamCaptureMode(&mode_);
+        if (hipGetDevice(&prev_) == hipSuccess && prev_ != device_) (void)hipSetDevice(device_);
+    }
+    ~ReadScope() {
+        if (prev_ != device_) (void)hipSetDevice(prev_);
+        (void)hipThreadExchangeStreamCaptureMode(&mode_);
+    }
+
+private:
+    int device_, prev_ = 0;
+    hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+};
+
 static int build_blocks_impl(Context& c) {
     const int64_t n = c.n_pts;
     const int nb = (int)((n + kBlockPts - 1) / kBlockPts);
@@ -1616,9 +1636,23 @@ int pdfxc_get_grid_rows(pdfxc_ctx* ctx, double* xyzw) {
         set_error("pdfxc_get_grid_rows: no grid");
         return PDFXC_ERR_NO_GRID;
     }
+    const ReadScope scope(*c);
     const int64_t per = std::min<int64_t>(c->n_pts, 1 << 22);  // 128 MiB of rows at a time
     DeviceBuf rows(*c);
-    if (int rc = rows.alloc(4 * sizeof(double) * (size_t)per)) return rc;
+    if (rows.alloc(4 * sizeof(double) * (size_t)per) != PDFXC_OK) {
+        // no device memory left for rows: columns, a stretch at a time
+        const int64_t step = std::min<int64_t>(c->n_pts, 1 << 16);
+        std::vector<double> col((size_t)step);
+        for (int q = 0; q < 4; ++q)
+            for (int64_t at = 0; at < c->n_pts; at += step) {
+                const int64_t n = std::min(step, c->n_pts - at);
+                PDFXC_HIP(hipMemcpyAsync(col.data(), c->d_grid + q * c->n_pts + at, sizeof(double) * (size_t)n,
+                                         hipMemcpyDeviceToHost, c->stream));
+                PDFXC_HIP(hipStreamSynchronize(c->stream));
+                for (int64_t i = 0; i < n; ++i) xyzw[4 * (at + i) + q] = col[i];
+            }
+        return PDFXC_OK;
+    }
     for (int64_t at = 0; at < c->n_pts; at += per) {
         const int64_t n = std::min(per, c->n_pts - at);
         if (int rc = launch_grid_rows(at, n, c->n_pts, c->d_grid, rows.as<double>(), c->stream)) return rc;

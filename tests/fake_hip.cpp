@@ -1,7 +1,7 @@
 // A stand-in for the HIP runtime in host memory, for CPU tests of the engine's
 // host code: device buffers are host allocations, copies are real, kernels are
-// not run.  Allocations and copies can be made to fail, and buffers and streams
-// know the device they were made on.  Loaded with RTLD_GLOBAL before the
+// not run.  Allocations and copies can be made to fail, and streams know the device
+// they were made on.  Loaded with RTLD_GLOBAL before the
 // engine library (or linked into a test program), it takes the place of every
 // runtime call the engine makes after load.
 #include <hip/hip_runtime.h>
@@ -12,18 +12,16 @@
 #include <map>
 #include <mutex>
 #include <thread>
+#include <utility>
 
 namespace {
 
-struct Buf {
-    size_t bytes;
-    int device;
-};
 std::mutex mu;
-std::map<void*, Buf> bufs;
+std::map<void*, size_t> bufs;
 std::map<hipStream_t, int> streams;
 thread_local int device = 0;
 thread_local hipStream_t launch_stream = nullptr;
+thread_local hipStreamCaptureMode capture_mode = hipStreamCaptureModeGlobal;
 size_t live = 0, limit = ~(size_t)0;
 int fail_copy = -1;       // copies to the host until one fails (-1: none does)
 int slow_copy_ms = 0;     // what a copy to the host takes
@@ -49,11 +47,6 @@ void fake_limit(size_t bytes) { limit = bytes; }  // hipMalloc fails beyond this
 void fake_fail_copy(int after) { fail_copy = after; }
 void fake_slow_copy(int ms) { slow_copy_ms = ms; }
 long long fake_misplaced() { return misplaced; }
-int fake_device_of(void* p) {
-    std::lock_guard<std::mutex> g(mu);
-    auto it = bufs.find(p);
-    return it == bufs.end() ? -1 : it->second.device;
-}
 
 hipError_t hipSetDevice(int d) {
     device = d;
@@ -63,12 +56,16 @@ hipError_t hipGetDevice(int* d) {
     *d = device;
     return hipSuccess;
 }
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode* m) {
+    std::swap(*m, capture_mode);
+    return hipSuccess;
+}
 hipError_t hipMalloc(void** p, size_t n) {
     std::lock_guard<std::mutex> g(mu);
     if (live + n > limit) return hipErrorOutOfMemory;
     *p = std::calloc(1, n ? n : 1);
     if (!*p) return hipErrorOutOfMemory;
-    bufs[*p] = Buf{n, device};
+    bufs[*p] = n;
     live += n;
     return hipSuccess;
 }
@@ -77,7 +74,7 @@ hipError_t hipFree(void* p) {
     std::lock_guard<std::mutex> g(mu);
     auto it = bufs.find(p);
     if (it == bufs.end()) return hipErrorInvalidValue;
-    live -= it->second.bytes;
+    live -= it->second;
     std::free(p);
     bufs.erase(it);
     return hipSuccess;

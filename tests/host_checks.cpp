@@ -97,13 +97,37 @@ void host_copy_threads() {
     pdfxc_ctx_destroy(ctx);
 }
 
+// the grid's rows need no device memory that is not there, and no current device
+void grid_rows() {
+    pdfxc_ctx* ctx = context();
+    const int64_t n = 3000;
+    set_grid(ctx, n);
+    int device = -1;
+    CHECK(hipSetDevice(1) == hipSuccess);
+    std::vector<double> rows(4 * n);
+    CHECK(pdfxc_get_grid_rows(ctx, rows.data()) == PDFXC_OK);
+    CHECK(fake_misplaced() == 0);
+    CHECK(hipGetDevice(&device) == hipSuccess && device == 1);
+    CHECK(hipSetDevice(0) == hipSuccess);
+    reinterpret_cast<Context*>(ctx)->pool.trim(0);
+    fake_limit(fake_live_bytes());
+    CHECK(pdfxc_get_grid_rows(ctx, rows.data()) == PDFXC_OK);
+    const Context& c = *reinterpret_cast<Context*>(ctx);
+    CHECK(ensure_host_grid(*reinterpret_cast<Context*>(ctx)) == PDFXC_OK && host_grid_is_right(c));
+    for (int64_t i = 0; i < n; ++i)
+        CHECK(rows[4 * i] == c.gx[i] && rows[4 * i + 1] == c.gy[i] && rows[4 * i + 2] == c.gz[i] &&
+              rows[4 * i + 3] == c.gw[i]);
+    fake_limit(~(size_t)0);
+    pdfxc_ctx_destroy(ctx);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     struct {
         const char* name;
         void (*run)();
-    } const checks[] = {{"pool_threads", pool_threads}, {"host_copy_threads", host_copy_threads}};
+    } const checks[] = {{"pool_threads", pool_threads}, {"host_copy_threads", host_copy_threads}, {"grid_rows", grid_rows}};
     for (const auto& k : checks)
         if (argc == 2 && !std::strcmp(argv[1], k.name)) {
             k.run();
