@@ -49,20 +49,53 @@ static void dfree(T*& p) {
     p = nullptr;
 }
 
+// Memory ran out: what the context keeps in reserve (unused buffers, the
+// context of its densities, for that one its owner's buffers) goes.
+static void release_reserve(Context& c) {
+    (void)hipGetLastError();
+    c.pool.trim(0);
+    if (c.probe_of) c.probe_of->pool.trim(0);
+    std::unique_lock<std::mutex> lock(c.probe_mu, std::try_to_lock);
+    if (lock.owns_lock() && c.probe) {
+        pdfxc_ctx_destroy(reinterpret_cast<pdfxc_ctx*>(c.probe));
+        c.probe = nullptr;
+    }
+}
+
+int context_take(Context& c, void** p, size_t bytes) {
+    *p = nullptr;
+    hipError_t e = c.pool.take(p, bytes);
+    if (e != hipSuccess) {
+        release_reserve(c);
+        e = c.pool.take(p, bytes);
+    }
+    if (e != hipSuccess) {
+        set_error(std::string("hipMalloc of ") + std::to_string(bytes) + " bytes: " + hipGetErrorString(e));
+        return PDFXC_ERR_MEMORY;
+    }
+    return PDFXC_OK;
+}
+
+void context_give(Context& c, void* p) { (void)c.pool.give(p); }
+
+// dalloc of a context's buffer that is not the pool's
+template <typename T>
+static int dalloc(Context& c, T** p, size_t count) {
+    int rc = dalloc(p, count);
+    if (rc == PDFXC_ERR_MEMORY) {
+        release_reserve(c);
+        rc = dalloc(p, count);
+    }
+    return rc;
+}
+
 // the same from a context's pool
 template <typename T>
 static int galloc(Context& c, T** p, size_t count) {
     void* q = nullptr;
-    *p = nullptr;
-    if (count == 0) count = 1;
-    const hipError_t e = c.pool.take(&q, count * sizeof(T));
-    if (e != hipSuccess) {
-        set_error(std::string("hipMalloc of ") + std::to_string(count * sizeof(T)) +
-                  " bytes: " + hipGetErrorString(e));
-        return PDFXC_ERR_MEMORY;
-    }
+    const int rc = context_take(c, &q, std::max<size_t>(count, 1) * sizeof(T));
     *p = static_cast<T*>(q);
-    return PDFXC_OK;
+    return rc;
 }
 
 template <typename T>
@@ -502,7 +535,6 @@ static double shell_cut(const Shell& s, double screen) {
 static void reset_grid(Context& c) {
     free_grid_buffers(&c);
     gfree(c, c.d_grid);
-    c.pool.trim(kPoolKeep);
     c.whole_spins = 0;
     c.n_pts = 0;
     c.n_slots = 0;
@@ -1574,11 +1606,11 @@ static std::vector<int> near_atoms(int n, const double* xyz) {
 int ensure_beta_buffers(Context* c) {
     const size_t n = 4 * (size_t)c->n_slots;
     if (!c->d_rho_b) {
-        if (int rc = dalloc(&c->d_rho_b, n)) return rc;
+        if (int rc = dalloc(*c, &c->d_rho_b, n)) return rc;
         PDFXC_HIP(hipMemset(c->d_rho_b, 0, n * sizeof(double)));
     }
     if (!c->d_coef_b) {
-        if (int rc = dalloc(&c->d_coef_b, n)) return rc;
+        if (int rc = dalloc(*c, &c->d_coef_b, n)) return rc;
         PDFXC_HIP(hipMemset(c->d_coef_b, 0, n * sizeof(double)));
     }
     return PDFXC_OK;
@@ -2075,8 +2107,8 @@ static int build_host(Context* c, int xc, int nspin, const double* const* P_pack
     const int N = c->n_aos;
     const size_t NN = (size_t)N * N;
     if (nspin == 2 && !c->d_P2) {
-        if (int rc = dalloc(&c->d_P2, NN)) return rc;
-        if (int rc = dalloc(&c->d_K2, NN)) return rc;
+        if (int rc = dalloc(*c, &c->d_P2, NN)) return rc;
+        if (int rc = dalloc(*c, &c->d_K2, NN)) return rc;
     }
     double* dP[2] = {c->d_P, c->d_P2};
     double* dK[2] = {c->d_K, c->d_K2};
@@ -2105,7 +2137,7 @@ static int build_host(Context* c, int xc, int nspin, const double* const* P_pack
         if (c->n_rho_out < n_out) {  // kept with the grid: rho is asked for again with every iteration
             dfree(c->d_rho_out);
             c->n_rho_out = 0;
-            if (int e = dalloc(&c->d_rho_out, n_out)) return e;
+            if (int e = dalloc(*c, &c->d_rho_out, n_out)) return e;
             c->n_rho_out = n_out;
         }
         for (int sp = 0; sp < nspin; ++sp)
@@ -2464,7 +2496,8 @@ int pdfxc_density_at_points(pdfxc_ctx* ctx, const double* P_packed, int64_t n, c
     int dev = 0;
     PDFXC_HIP(hipGetDevice(&dev));
     std::unique_lock<std::mutex> lock(c->probe_mu, std::try_to_lock);
-    const bool keep = lock.owns_lock() && dev == c->device;
+    const size_t matrices = sizeof(double) * (2 * (size_t)N * N + packed_doubles(N));
+    const bool keep = lock.owns_lock() && dev == c->device && matrices <= kPoolKeep;
     pdfxc_ctx* th = keep ? reinterpret_cast<pdfxc_ctx*>(c->probe) : nullptr;
     if (keep) c->probe = nullptr;  // back once the call has succeeded
     int rc = PDFXC_OK;
@@ -2485,9 +2518,18 @@ int pdfxc_density_at_points(pdfxc_ctx* ctx, const double* P_packed, int64_t n, c
             }
         pdfxc_opts o = c->opts;
         o.precision = PDFXC_FP64;
-        rc = pdfxc_ctx_create(&th, N, center.data(), type.data(), nprim.data(), exps.data(), coefs.data(), kMaxPrim, &o);
+        auto create = [&] {
+            return pdfxc_ctx_create(&th, N, center.data(), type.data(), nprim.data(), exps.data(), coefs.data(), kMaxPrim, &o);
+        };
+        rc = create();
+        if (rc == PDFXC_ERR_MEMORY) {
+            (void)hipGetLastError();
+            c->pool.trim(0);
+            rc = create();
+        }
         if (rc) return rc;
         reinterpret_cast<Context*>(th)->rho_only = true;
+        reinterpret_cast<Context*>(th)->probe_of = c;
     }
     Context* t = reinterpret_cast<Context*>(th);
     if (n > ((int64_t)1 << 31) - kBlockPts) {
@@ -2577,8 +2619,8 @@ int pdfxc_eval_aos(pdfxc_ctx* ctx, int64_t n, const double* xyz, double* phi, do
     if (n == 0) return PDFXC_OK;
     const size_t plane = (size_t)n * c->n_aos;
     double *dx = nullptr, *dout = nullptr;
-    int rc = dalloc(&dx, 3 * (size_t)n);
-    if (rc == PDFXC_OK) rc = dalloc(&dout, 4 * plane);
+    int rc = dalloc(*c, &dx, 3 * (size_t)n);
+    if (rc == PDFXC_OK) rc = dalloc(*c, &dout, 4 * plane);
     if (rc == PDFXC_OK) {
         hipError_t e = hipMemcpy(dx, xyz, 3 * n * sizeof(double), hipMemcpyHostToDevice);
         if (e != hipSuccess) rc = hip_fail(e, "pdfxc_eval_aos: upload");
@@ -2950,36 +2992,45 @@ int pdfxc_batch_create(pdfxc_batch** out, int n_mol, pdfxc_ctx* const* ctxs) {
         const hipError_t ee = hipMemcpy(d, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice);
         if (ee != hipSuccess) rc = hip_fail(ee, "pdfxc_batch_create: upload");
     };
-    if (rc == PDFXC_OK) rc = dalloc(&m.d_shrec, rec.size());
-    if (rc == PDFXC_OK) rc = dalloc(&m.d_queue, kMaxQueues);
-    if (rc == PDFXC_OK) rc = dalloc(&m.d_pts, soa.size());
-    if (rc == PDFXC_OK) rc = dalloc(&m.d_blocks, m.blocks.size());
-    if (rc == PDFXC_OK) rc = dalloc(&m.d_kblocks, m.kblocks.size());
-    if (rc == PDFXC_OK) rc = dalloc(&m.d_block_shells, std::max<size_t>(1, m.block_shells.size()));
-    if (rc == PDFXC_OK) rc = dalloc(&m.d_block_cols, std::max<size_t>(1, m.block_cols.size()));
-    if (rc == PDFXC_OK) rc = dalloc(&m.d_block_shell_col, std::max<size_t>(1, m.block_shell_col.size()));
-    if (rc == PDFXC_OK) rc = dalloc(&m.d_block_sorder, std::max<size_t>(1, m.block_sorder.size()));
-    if (rc == PDFXC_OK) rc = dalloc(&m.d_rho_work, std::max<size_t>(1, m.h_rho_work.size()));
-    if (rc == PDFXC_OK) rc = dalloc(reinterpret_cast<char**>(&m.d_k_work), std::max<size_t>(1, m.h_k_work.size()) * sizeof(KWork));
-    if (rc == PDFXC_OK) rc = dalloc(&m.d_coef, 4 * (size_t)m.n_slots);
-    if (rc == PDFXC_OK) rc = dalloc(&m.d_rho, 4 * (size_t)m.n_slots);
-    if (rc == PDFXC_OK) rc = dalloc(&m.d_eblock, (size_t)m.n_slots / 256);
-    if (rc == PDFXC_OK) rc = dalloc(&b->d_ebounds, ebounds.size());
+    // buffers that the contexts keep in reserve give way to the batch's
+    auto alloc = [&](auto** p, size_t count) {
+        int r = dalloc(p, count);
+        if (r == PDFXC_ERR_MEMORY) {
+            for (int i = 0; i < n_mol; ++i) release_reserve(*reinterpret_cast<Context*>(ctxs[i]));
+            r = dalloc(p, count);
+        }
+        return r;
+    };
+    if (rc == PDFXC_OK) rc = alloc(&m.d_shrec, rec.size());
+    if (rc == PDFXC_OK) rc = alloc(&m.d_queue, kMaxQueues);
+    if (rc == PDFXC_OK) rc = alloc(&m.d_pts, soa.size());
+    if (rc == PDFXC_OK) rc = alloc(&m.d_blocks, m.blocks.size());
+    if (rc == PDFXC_OK) rc = alloc(&m.d_kblocks, m.kblocks.size());
+    if (rc == PDFXC_OK) rc = alloc(&m.d_block_shells, std::max<size_t>(1, m.block_shells.size()));
+    if (rc == PDFXC_OK) rc = alloc(&m.d_block_cols, std::max<size_t>(1, m.block_cols.size()));
+    if (rc == PDFXC_OK) rc = alloc(&m.d_block_shell_col, std::max<size_t>(1, m.block_shell_col.size()));
+    if (rc == PDFXC_OK) rc = alloc(&m.d_block_sorder, std::max<size_t>(1, m.block_sorder.size()));
+    if (rc == PDFXC_OK) rc = alloc(&m.d_rho_work, std::max<size_t>(1, m.h_rho_work.size()));
+    if (rc == PDFXC_OK) rc = alloc(reinterpret_cast<char**>(&m.d_k_work), std::max<size_t>(1, m.h_k_work.size()) * sizeof(KWork));
+    if (rc == PDFXC_OK) rc = alloc(&m.d_coef, 4 * (size_t)m.n_slots);
+    if (rc == PDFXC_OK) rc = alloc(&m.d_rho, 4 * (size_t)m.n_slots);
+    if (rc == PDFXC_OK) rc = alloc(&m.d_eblock, (size_t)m.n_slots / 256);
+    if (rc == PDFXC_OK) rc = alloc(&b->d_ebounds, ebounds.size());
     if (rc == PDFXC_OK && split) {
-        rc = dalloc(&m.d_sblocks, m.sblocks.size());
-        if (rc == PDFXC_OK) rc = dalloc(&m.d_chunks, std::max<size_t>(1, m.chunks.size()));
-        if (rc == PDFXC_OK) rc = dalloc(&m.d_sshell_col, std::max<size_t>(1, m.sshell_col.size()));
-        if (rc == PDFXC_OK) rc = dalloc(&m.d_srho_work, std::max<size_t>(1, m.h_srho_work.size()));
-        if (rc == PDFXC_OK) rc = dalloc(&m.d_kg_work, std::max<size_t>(1, m.h_kg_work.size()));
-        if (rc == PDFXC_OK) rc = dalloc(&m.d_kgroups, std::max<size_t>(1, m.kgroups.size()));
-        if (rc == PDFXC_OK) rc = dalloc(&m.d_kg_blocks, std::max<size_t>(1, m.kg_blocks.size()));
-        if (rc == PDFXC_OK) rc = dalloc(&m.d_kg_shells, std::max<size_t>(1, m.kg_shells.size()));
-        if (rc == PDFXC_OK) rc = dalloc(&m.d_kg_shell_col, std::max<size_t>(1, m.kg_shell_col.size()));
-        if (rc == PDFXC_OK) rc = dalloc(&m.d_kg_sorder, std::max<size_t>(1, m.kg_sorder.size()));
-        if (rc == PDFXC_OK) rc = dalloc(&m.d_kg_cols, std::max<size_t>(1, m.kg_cols.size()));
-        if (rc == PDFXC_OK) rc = dalloc(&m.d_kg_masks, std::max<size_t>(1, m.kg_masks.size()));
-        if (rc == PDFXC_OK) rc = dalloc(&m.d_perm, perm.size());
-        if (rc == PDFXC_OK) rc = dalloc(&m.d_Ps, (size_t)psoff);
+        rc = alloc(&m.d_sblocks, m.sblocks.size());
+        if (rc == PDFXC_OK) rc = alloc(&m.d_chunks, std::max<size_t>(1, m.chunks.size()));
+        if (rc == PDFXC_OK) rc = alloc(&m.d_sshell_col, std::max<size_t>(1, m.sshell_col.size()));
+        if (rc == PDFXC_OK) rc = alloc(&m.d_srho_work, std::max<size_t>(1, m.h_srho_work.size()));
+        if (rc == PDFXC_OK) rc = alloc(&m.d_kg_work, std::max<size_t>(1, m.h_kg_work.size()));
+        if (rc == PDFXC_OK) rc = alloc(&m.d_kgroups, std::max<size_t>(1, m.kgroups.size()));
+        if (rc == PDFXC_OK) rc = alloc(&m.d_kg_blocks, std::max<size_t>(1, m.kg_blocks.size()));
+        if (rc == PDFXC_OK) rc = alloc(&m.d_kg_shells, std::max<size_t>(1, m.kg_shells.size()));
+        if (rc == PDFXC_OK) rc = alloc(&m.d_kg_shell_col, std::max<size_t>(1, m.kg_shell_col.size()));
+        if (rc == PDFXC_OK) rc = alloc(&m.d_kg_sorder, std::max<size_t>(1, m.kg_sorder.size()));
+        if (rc == PDFXC_OK) rc = alloc(&m.d_kg_cols, std::max<size_t>(1, m.kg_cols.size()));
+        if (rc == PDFXC_OK) rc = alloc(&m.d_kg_masks, std::max<size_t>(1, m.kg_masks.size()));
+        if (rc == PDFXC_OK) rc = alloc(&m.d_perm, perm.size());
+        if (rc == PDFXC_OK) rc = alloc(&m.d_Ps, (size_t)psoff);
     }
     up(m.d_shrec, rec);
     up(m.d_pts, soa);

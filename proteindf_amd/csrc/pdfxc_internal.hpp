@@ -163,9 +163,13 @@ struct DeviceShell {
 // the next: 18 allocations and as many frees took 4 of the 26 ms of a new
 // FINE grid of a 20-residue helix and half of a small density call.  All use
 // is on the context's stream, whose work ends before a buffer changes hands.
+// At most kPoolKeep bytes are ever kept unused (give frees what is over, the
+// largest first), they give way to the context's other allocations
+// (release_reserve) and go with the context.  A buffer serves requests down to
+// four fifths of its size (and 64 KiB less): a grid holds its buffers for long.
 // Several threads may take and give: a grid may be read (pdfxc_get_grid_rows)
 // while another thread builds.
-// Buffers not in use are bounded by trim and go with the context.
+constexpr size_t kPoolKeep = (size_t)512 << 20;
 class DevicePool {
 public:
     ~DevicePool() {
@@ -175,8 +179,11 @@ public:
         std::lock_guard<std::mutex> lock(mu_);
         Buf* best = nullptr;
         for (Buf& b : bufs_)
-            if (!b.used && b.cap >= bytes && b.cap <= 2 * bytes + 65536 && (!best || b.cap < best->cap)) best = &b;
-        if (!best) {
+            if (!b.used && b.cap >= bytes && b.cap <= bytes + bytes / 4 + 65536 && (!best || b.cap < best->cap))
+                best = &b;
+        if (best) {
+            idle_ -= best->cap;
+        } else {
             // up to an eighth more than asked for, so that the next geometry's sizes fit
             size_t step = 256;
             while (step * 16 <= bytes) step *= 2;
@@ -188,7 +195,10 @@ public:
                 trim_locked(0);
                 e = hipMalloc(&q, cap);
             }
-            if (e != hipSuccess) return e;
+            if (e != hipSuccess) {
+                (void)hipGetLastError();  // the caller has the error; the next launch is not to find it
+                return e;
+            }
             bufs_.push_back(Buf{q, cap, false});
             best = &bufs_.back();
         }
@@ -201,6 +211,8 @@ public:
         for (Buf& b : bufs_)
             if (b.p == p) {
                 b.used = false;
+                idle_ += b.cap;
+                if (idle_ > kPoolKeep) trim_locked(kPoolKeep);
                 return true;
             }
         return false;
@@ -211,38 +223,35 @@ public:
     }
 
 private:
-    void trim_locked(size_t keep) {
-        std::sort(bufs_.begin(), bufs_.end(), [](const Buf& a, const Buf& b) { return a.cap < b.cap; });
-        size_t kept = 0;
-        std::vector<Buf> left;
-        for (const Buf& b : bufs_) {
-            if (!b.used) {
-                if (kept + b.cap > keep) {
-                    (void)hipFree(b.p);
-                    continue;
-                }
-                kept += b.cap;
-            }
-            left.push_back(b);
-        }
-        bufs_.swap(left);
-    }
-
     struct Buf {
         void* p;
         size_t cap;
         bool used;
     };
+    void trim_locked(size_t keep) {
+        std::sort(bufs_.begin(), bufs_.end(), [](const Buf& a, const Buf& b) { return a.cap < b.cap; });
+        while (idle_ > keep) {
+            size_t i = bufs_.size();
+            while (bufs_[i - 1].used) --i;
+            (void)hipFree(bufs_[i - 1].p);
+            idle_ -= bufs_[i - 1].cap;
+            bufs_.erase(bufs_.begin() + (i - 1));
+        }
+    }
+
     std::mutex mu_;
     std::vector<Buf> bufs_;
+    size_t idle_ = 0;  // bytes of the buffers not in use
 };
-constexpr size_t kPoolKeep = (size_t)512 << 20;
 
 struct Context {
     pdfxc_opts opts;
     DevicePool pool;
     bool rho_only = false;      // points for densities alone: no K work, no point terms
-    Context* probe = nullptr;   // the points of density_at_points, kept between calls (probe_mu)
+    // the points of density_at_points, kept between calls (probe_mu) while its
+    // matrices take no more than kPoolKeep; its own way back to this context
+    Context* probe = nullptr;
+    Context* probe_of = nullptr;
     std::mutex probe_mu;
     pdfxc_tuning tune{0, 96, 0, 24, 4, 2, 0.0};  // launch shapes (pdfxc_set_tuning / pdfxc_autotune)
     int n_aos = 0;
@@ -379,6 +388,10 @@ int hip_fail(hipError_t e, const char* what);
         hipError_t e_ = (call);                                  \
         if (e_ != hipSuccess) return ::pdfxc::hip_fail(e_, #call); \
     } while (0)
+
+// device memory for the length of a call, from the context's pool
+int context_take(Context& c, void** p, size_t bytes);
+void context_give(Context& c, void* p);
 
 // host copies of a context's grid, block lists and slots (no-ops once made)
 int ensure_host_grid(Context& c);

@@ -120,25 +120,29 @@ static int write_matrix(const char* path, int type, int64_t rows, int64_t cols, 
 // caller-order rho (n_pts x 4) <-> the context's slots
 static int download_rho(Context* c, double* rho, const double* d_src) {
     const size_t bytes = sizeof(double) * 4 * (size_t)c->n_pts;
-    double* d = nullptr;
-    PDFXC_HIP(hipMalloc(reinterpret_cast<void**>(&d), bytes));
+    void* p = nullptr;
+    if (int rc = context_take(*c, &p, bytes)) return rc;
+    double* d = static_cast<double*>(p);
     int rc = launch_gather_points(*c, d_src, d, 4, 0);
     hipError_t e = rc == PDFXC_OK ? hipMemcpyAsync(rho, d, bytes, hipMemcpyDeviceToHost, c->stream) : hipSuccess;
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    (void)hipFree(d);
+    const hipError_t es = hipStreamSynchronize(c->stream);  // also on failure: d changes hands
+    if (e == hipSuccess) e = es;
+    context_give(*c, d);
     return rc != PDFXC_OK ? rc : e == hipSuccess ? PDFXC_OK : hip_fail(e, "rho download");
 }
 
 static int upload_rho(Context* c, const double* rho, double* d_dst) {
     const size_t bytes = sizeof(double) * 4 * (size_t)c->n_pts;
-    double* d = nullptr;
-    PDFXC_HIP(hipMalloc(reinterpret_cast<void**>(&d), bytes));
+    void* p = nullptr;
+    if (int rc = context_take(*c, &p, bytes)) return rc;
+    double* d = static_cast<double*>(p);
     int rc = PDFXC_OK;
     hipError_t e = hipMemsetAsync(d_dst, 0, sizeof(double) * 4 * (size_t)c->n_slots, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(d, rho, bytes, hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) rc = launch_scatter_points(*c, d, d_dst);
-    if (e == hipSuccess && rc == PDFXC_OK) e = hipStreamSynchronize(c->stream);
-    (void)hipFree(d);
+    const hipError_t es = hipStreamSynchronize(c->stream);
+    if (e == hipSuccess) e = es;
+    context_give(*c, d);
     return rc != PDFXC_OK ? rc : e == hipSuccess ? PDFXC_OK : hip_fail(e, "rho upload");
 }
 

@@ -28,13 +28,14 @@ using namespace pdfxc;
         }                                                               \
     } while (0)
 
-pdfxc_ctx* context() {
-    const double centre[3] = {0.0, 0.0, 0.0}, exps[1] = {1.0}, coefs[1] = {1.0};
-    const int type = 0, nprim = 1;
+pdfxc_ctx* context(int n_aos = 1) {
+    const std::vector<double> centre(3 * (size_t)n_aos, 0.0), ones((size_t)n_aos, 1.0);
+    const std::vector<int> type((size_t)n_aos, 0), nprim((size_t)n_aos, 1);
     pdfxc_opts o;
     pdfxc_default_opts(&o);
     pdfxc_ctx* ctx = nullptr;
-    CHECK(pdfxc_ctx_create(&ctx, 1, centre, &type, &nprim, exps, coefs, 1, &o) == PDFXC_OK);
+    CHECK(pdfxc_ctx_create(&ctx, n_aos, centre.data(), type.data(), nprim.data(), ones.data(), ones.data(), 1, &o) ==
+          PDFXC_OK);
     return ctx;
 }
 
@@ -121,13 +122,95 @@ void grid_rows() {
     pdfxc_ctx_destroy(ctx);
 }
 
+// what a pool holds beyond the buffers in use stays bounded at every moment,
+// and a buffer is not given for a quarter of its size
+void pool_bound() {
+    const size_t mib = (size_t)1 << 20;
+    DevicePool pool;
+    std::vector<void*> p(6);
+    size_t used = 0;
+    for (void*& v : p) CHECK(pool.take(&v, 200 * mib) == hipSuccess);
+    used = fake_live_bytes();
+    const size_t each = used / p.size();
+    for (void* v : p) {
+        pool.give(v);
+        used -= each;
+        CHECK(fake_live_bytes() <= used + kPoolKeep);
+    }
+    const size_t before = fake_live_bytes();
+    void* v = nullptr;
+    CHECK(pool.take(&v, 120 * mib) == hipSuccess);
+    CHECK(fake_live_bytes() > before);  // not one of 200 MiB
+    pool.give(v);
+    CHECK(fake_live_bytes() <= kPoolKeep);
+}
+
+// buffers in reserve give way to every allocation of the context: the second
+// spin's, rho in the caller's order, a batch's, a file's, a density's
+void reserve_gives_way() {
+    pdfxc_ctx* ctx = context();
+    Context& c = *reinterpret_cast<Context*>(ctx);
+    const int64_t n = 100000;
+    double P = 1.0, K = 0.0, E = 0.0, x[3] = {0.0, 0.0, 0.0}, rho = 0.0;
+    std::vector<double> out(8 * n);
+    auto full = [&](size_t reserve) {  // nothing free but `reserve` bytes kept by the pool
+        void* v = nullptr;
+        fake_limit(~(size_t)0);
+        c.pool.trim(0);
+        CHECK(c.pool.take(&v, reserve) == hipSuccess);
+        c.pool.give(v);
+        fake_limit(fake_live_bytes());
+    };
+    set_grid(ctx, n);
+    full(2 * 4 * sizeof(double) * (n + kBlockPts) + 4096);
+    CHECK(pdfxc_build_uks(ctx, PDFXC_SVWN, &P, &P, &K, &K, &E, nullptr) == PDFXC_OK);
+    full(8 * sizeof(double) * n);
+    CHECK(pdfxc_build_uks(ctx, PDFXC_SVWN, &P, &P, &K, &K, &E, out.data()) == PDFXC_OK);
+    full(4 * sizeof(double) * n);
+    CHECK(pdfxc_save_grid_matrix(ctx, "/dev/null", 4) == PDFXC_OK);
+    std::vector<double> phi(n);
+    full(sizeof(double) * 7 * n);
+    CHECK(pdfxc_eval_aos(ctx, n, out.data(), phi.data(), nullptr, nullptr, nullptr) == PDFXC_OK);
+    full((size_t)64 << 20);
+    pdfxc_batch* batch = nullptr;
+    CHECK(pdfxc_batch_create(&batch, 1, &ctx) == PDFXC_OK);
+    pdfxc_batch_destroy(batch);
+    full((size_t)8 << 20);
+    CHECK(pdfxc_density_at_points(ctx, &P, 1, x, &rho, nullptr) == PDFXC_OK);
+    // the kept context of the densities gives way too
+    fake_limit(~(size_t)0);
+    CHECK(pdfxc_density_at_points(ctx, &P, n, out.data(), phi.data(), nullptr) == PDFXC_OK);
+    CHECK(c.probe != nullptr);
+    c.pool.trim(0);
+    fake_limit(fake_live_bytes());
+    CHECK(pdfxc_eval_aos(ctx, 1000, out.data(), phi.data(), nullptr, nullptr, nullptr) == PDFXC_OK);
+    fake_limit(~(size_t)0);
+    pdfxc_ctx_destroy(ctx);
+    CHECK(fake_live_bytes() == 0);
+}
+
+// the context that densities keep holds no matrices beyond the pool's bound
+void density_keeps_little() {
+    const int n = 4800;  // three matrices of 4800 x 4800 are 553 MB
+    pdfxc_ctx* ctx = context(n);
+    const std::vector<double> P((size_t)n * (n + 1) / 2, 0.0), x(3000, 0.5);
+    std::vector<double> rho(1000);
+    const size_t before = fake_live_bytes();
+    CHECK(pdfxc_density_at_points(ctx, P.data(), 1000, x.data(), rho.data(), nullptr) == PDFXC_OK);
+    CHECK(fake_live_bytes() <= before + kPoolKeep);
+    pdfxc_ctx_destroy(ctx);
+    CHECK(fake_live_bytes() == 0);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     struct {
         const char* name;
         void (*run)();
-    } const checks[] = {{"pool_threads", pool_threads}, {"host_copy_threads", host_copy_threads}, {"grid_rows", grid_rows}};
+    } const checks[] = {{"pool_threads", pool_threads}, {"host_copy_threads", host_copy_threads}, {"grid_rows", grid_rows},
+                  {"pool_bound", pool_bound},     {"reserve_gives_way", reserve_gives_way},
+                  {"density_keeps_little", density_keeps_little}};
     for (const auto& k : checks)
         if (argc == 2 && !std::strcmp(argv[1], k.name)) {
             k.run();
