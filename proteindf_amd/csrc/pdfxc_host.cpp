@@ -1502,41 +1502,45 @@ static void orientation(int na, const int* Z, const double* xyz, double O[9]) {
     }
 }
 
+// Host copies of n[k] values from each d[k] into *v[k]: all of them or, on
+// failure, none (their sizes say that they are there).
+template <typename T, size_t K>
+static int host_copies(Context& c, std::vector<T>* const (&v)[K], const T* const (&d)[K], const int64_t (&n)[K]) {
+    std::vector<T> got[K];
+    hipError_t e = hipSuccess;
+    for (size_t k = 0; k < K && e == hipSuccess; ++k) {
+        got[k].resize((size_t)n[k]);
+        if (n[k]) e = hipMemcpyAsync(got[k].data(), d[k], sizeof(T) * (size_t)n[k], hipMemcpyDeviceToHost, c.stream);
+    }
+    const hipError_t es = hipStreamSynchronize(c.stream);  // also on failure: the copies end here
+    if (e == hipSuccess) e = es;
+    if (e != hipSuccess) return hip_fail(e, "copy of a grid's lists to the host");
+    for (size_t k = 0; k < K; ++k) v[k]->swap(got[k]);
+    return PDFXC_OK;
+}
+
 int ensure_host_grid(Context& c) {
     std::lock_guard<std::mutex> lock(c.host_mu);
     if ((int64_t)c.gx.size() == c.n_pts) return PDFXC_OK;
-    std::vector<double>* g[4] = {&c.gx, &c.gy, &c.gz, &c.gw};
-    for (int q = 3; q >= 0; --q) {
-        g[q]->resize((size_t)c.n_pts);
-        PDFXC_HIP(hipMemcpyAsync(g[q]->data(), c.d_grid + q * c.n_pts, sizeof(double) * (size_t)c.n_pts,
-                                 hipMemcpyDeviceToHost, c.stream));
-    }
-    PDFXC_HIP(hipStreamSynchronize(c.stream));
-    return PDFXC_OK;
+    const int64_t n = c.n_pts;
+    return host_copies<double, 4>(c, {&c.gx, &c.gy, &c.gz, &c.gw},
+                                  {c.d_grid, c.d_grid + n, c.d_grid + 2 * n, c.d_grid + 3 * n}, {n, n, n, n});
 }
 
 int ensure_host_lists(Context& c) {
     std::lock_guard<std::mutex> lock(c.host_mu);
     if ((int64_t)c.block_cols.size() == c.n_block_cols && (int64_t)c.block_shells.size() == c.n_block_shells)
         return PDFXC_OK;
-    auto get = [&](std::vector<int>& v, const int* d, int64_t n) {
-        v.resize((size_t)n);
-        return n ? hipMemcpyAsync(v.data(), d, sizeof(int) * (size_t)n, hipMemcpyDeviceToHost, c.stream) : hipSuccess;
-    };
-    PDFXC_HIP(get(c.block_shell_col, c.d_block_shell_col, c.n_block_shells));
-    PDFXC_HIP(get(c.block_sorder, c.d_block_sorder, c.n_block_shells));
-    PDFXC_HIP(get(c.block_shells, c.d_block_shells, c.n_block_shells));
-    PDFXC_HIP(get(c.block_cols, c.d_block_cols, c.n_block_cols));
-    PDFXC_HIP(hipStreamSynchronize(c.stream));
-    return PDFXC_OK;
+    return host_copies<int, 4>(c, {&c.block_shell_col, &c.block_sorder, &c.block_shells, &c.block_cols},
+                               {c.d_block_shell_col, c.d_block_sorder, c.d_block_shells, c.d_block_cols},
+                               {c.n_block_shells, c.n_block_shells, c.n_block_shells, c.n_block_cols});
 }
 
 int ensure_host_slots(Context& c) {
     std::lock_guard<std::mutex> lock(c.host_mu);
     if ((int64_t)c.slot_of_point.size() == c.n_pts) return PDFXC_OK;
-    std::vector<int> s((size_t)c.n_pts);
-    PDFXC_HIP(hipMemcpyAsync(s.data(), c.d_slot_of_point, sizeof(int) * (size_t)c.n_pts, hipMemcpyDeviceToHost, c.stream));
-    PDFXC_HIP(hipStreamSynchronize(c.stream));
+    std::vector<int> s;
+    if (int rc = host_copies<int, 1>(c, {&s}, {c.d_slot_of_point}, {c.n_pts})) return rc;
     c.slot_of_point.assign(s.begin(), s.end());
     return PDFXC_OK;
 }

@@ -202,6 +202,35 @@ void density_keeps_little() {
     CHECK(fake_live_bytes() == 0);
 }
 
+// a copy that fails leaves no half-made host copies behind
+void failed_copies() {
+    pdfxc_ctx* ctx = context();
+    Context& c = *reinterpret_cast<Context*>(ctx);
+    for (int k = 0; k < 4; ++k) {
+        set_grid(ctx, 1000 + k);
+        fake_fail_copy(k);
+        CHECK(ensure_host_grid(c) == PDFXC_ERR_HIP);
+        fake_fail_copy(-1);
+        CHECK(ensure_host_grid(c) == PDFXC_OK && host_grid_is_right(c));
+    }
+    const std::vector<int> want{3, 1, 4, 1, 5};
+    int* lists[4] = {c.d_block_shells, c.d_block_cols, c.d_block_shell_col, c.d_block_sorder};
+    for (int* d : lists) CHECK(hipMemcpy(d, want.data(), 5 * sizeof(int), hipMemcpyHostToDevice) == hipSuccess);
+    for (int k = 0; k < 4; ++k) {
+        c.n_block_shells = c.n_block_cols = 5;
+        c.block_shells.clear();
+        c.block_cols.clear();
+        c.block_shell_col.clear();
+        c.block_sorder.clear();
+        fake_fail_copy(k);
+        CHECK(ensure_host_lists(c) == PDFXC_ERR_HIP);
+        fake_fail_copy(-1);
+        CHECK(ensure_host_lists(c) == PDFXC_OK);
+        CHECK(c.block_shells == want && c.block_cols == want && c.block_shell_col == want && c.block_sorder == want);
+    }
+    pdfxc_ctx_destroy(ctx);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -210,7 +239,7 @@ int main(int argc, char** argv) {
         void (*run)();
     } const checks[] = {{"pool_threads", pool_threads}, {"host_copy_threads", host_copy_threads}, {"grid_rows", grid_rows},
                   {"pool_bound", pool_bound},     {"reserve_gives_way", reserve_gives_way},
-                  {"density_keeps_little", density_keeps_little}};
+                  {"density_keeps_little", density_keeps_little}, {"failed_copies", failed_copies}};
     for (const auto& k : checks)
         if (argc == 2 && !std::strcmp(argv[1], k.name)) {
             k.run();
