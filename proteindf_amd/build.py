@@ -19,7 +19,7 @@ ROOT = PKG.parent
 SRC = PKG / "csrc"
 OUT = PKG / "_lib" / "libpdfxc.so"
 SOURCES = [SRC / "pdfxc_host.cpp", SRC / "pdfxc_io.cpp", SRC / "pdfxc_blocks.hip", SRC / "pdfxc_kernels.hip", SRC / "pdfxc_split.hip", SRC / "pdfxc_grad.hip"]
-HEADERS = [SRC / "pdfxc_internal.hpp", SRC / "pdfxc_device.hpp", SRC / "xc_functional.hpp", ROOT / "include" / "pdfxc.h"]
+HEADERS = [SRC / "pdfxc_internal.hpp", SRC / "pdfxc_partition.hpp", SRC / "pdfxc_device.hpp", SRC / "xc_functional.hpp", ROOT / "include" / "pdfxc.h"]
 
 
 def hipcc():

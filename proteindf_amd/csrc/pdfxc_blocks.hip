@@ -31,24 +31,15 @@
 #include <vector>
 
 #include "pdfxc_internal.hpp"
+#include "pdfxc_partition.hpp"
 
 namespace pdfxc {
 
 namespace {
 
-constexpr int kNodeMax = 4096;  // points of a node that one workgroup cuts in LDS (120 KiB)
-constexpr int kChunk = 4096;    // points per workgroup of the level passes
+static_assert(kLeafPts == kBlockPts, "a leaf of the bisection is a block");
 constexpr int kPasses = 12;     // 8-bit digits: 8 of the coordinate's key, 4 of the index
 
-struct PartNode {
-    int lo, hi, mid;
-};
-struct PartChunk {
-    int node, lo, hi;
-};
-struct LeafNode {
-    int lo, hi, buf;
-};
 struct PartState {  // per node
     unsigned long long box[6];  // ordered keys: min of 3 dimensions, then max
     unsigned long long prefix[kPasses + 1];
@@ -116,11 +107,11 @@ __global__ __launch_bounds__(256) void k_part_box(const PartChunk* __restrict__ 
     __syncthreads();
     for (int d = 0; d < 3; ++d) {
         unsigned long long mn = ~0ull, mx = 0ull;
-        for (int i = C.lo + t; i < C.hi; i += 256) {
+        each_point(C, t, [&](int i) {
             const unsigned long long k = key_of(b.v[d][i]);
             mn = k < mn ? k : mn;
             mx = k > mx ? k : mx;
-        }
+        });
         for (int off = 32; off > 0; off >>= 1) {
             const unsigned long long a = __shfl_xor(mn, off), c = __shfl_xor(mx, off);
             mn = a < mn ? a : mn;
@@ -191,7 +182,7 @@ __global__ __launch_bounds__(256) void k_part_hist(int p, const PartChunk* __res
     }
     __syncthreads();
     const double* v = b.v[state_dim(st[C.node])];
-    for (int i = C.lo + t; i < C.hi; i += 256) {
+    each_point(C, t, [&](int i) {
         const unsigned long long k = key_of(v[i]);
         if (p < 8) {
             if (p == 0 || (k >> (64 - 8 * p)) == prefix) atomicAdd(&s_h[(k >> (56 - 8 * p)) & 255u], 1u);
@@ -200,7 +191,7 @@ __global__ __launch_bounds__(256) void k_part_hist(int p, const PartChunk* __res
             const int q = p - 8;
             if (q == 0 || (ix >> (32 - 8 * q)) == iprefix) atomicAdd(&s_h[(ix >> (24 - 8 * q)) & 255u], 1u);
         }
-    }
+    });
     __syncthreads();
     if (s_h[t]) atomicAdd(&nh[p * 256 + t], s_h[t]);
 }
@@ -216,13 +207,15 @@ __global__ __launch_bounds__(256) void k_part_split(const PartChunk* __restrict_
     int rank;
     part_pick(kPasses, st[C.node], hist + (int64_t)C.node * kPasses * 256, &prefix, &iprefix, &rank);
     const double* v = src.v[state_dim(st[C.node])];
+    const int n = C.hi - C.lo;
     // which of this thread's points go left: those below the cut's (coordinate, index)
     unsigned int left = 0u;
     int nleft = 0;
     for (int r = 0; r < kChunk / 256; ++r) {
-        const int i = C.lo + r * 256 + t;
+        const int j = r * 256 + t;  // within the chunk
         bool l = false;
-        if (i < C.hi) {
+        if (j < n) {
+            const int i = C.lo + j;
             const unsigned long long k = key_of(v[i]);
             l = k < prefix || (k == prefix && (unsigned int)src.idx[i] < iprefix);
         }
@@ -234,7 +227,7 @@ __global__ __launch_bounds__(256) void k_part_split(const PartChunk* __restrict_
     if (t == 0) {
         const int tot = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
         s_base[0] = atomicAdd(&st[C.node].cursor[0], tot);
-        s_base[1] = atomicAdd(&st[C.node].cursor[1], (C.hi - C.lo) - tot);
+        s_base[1] = atomicAdd(&st[C.node].cursor[1], n - tot);
     }
     __syncthreads();
     // wave w's share of the two runs
@@ -242,15 +235,16 @@ __global__ __launch_bounds__(256) void k_part_split(const PartChunk* __restrict_
     for (int w = 0; w < wave; ++w) {
         lb += s_cnt[w];
         int mine = 0;  // points of wave w in this chunk
-        for (int r = 0; r < kChunk / 256; ++r) mine += max(0, min(64, C.hi - (C.lo + r * 256 + w * 64)));
+        for (int r = 0; r < kChunk / 256; ++r) mine += max(0, min(64, n - (r * 256 + w * 64)));
         rb += mine - s_cnt[w];
     }
     const unsigned long long below = (1ull << (t & 63)) - 1ull;
     for (int r = 0; r < kChunk / 256; ++r) {
-        const int i = C.lo + r * 256 + t;
-        const bool in = i < C.hi, l = (left >> r) & 1u;
+        const int j = r * 256 + t;
+        const bool in = j < n, l = (left >> r) & 1u;
         const unsigned long long ml = __ballot(in && l), mr = __ballot(in && !l);
         if (in) {
+            const int i = C.lo + j;
             const int o = l ? lb + __popcll(ml & below) : rb + __popcll(mr & below);
             dst.v[0][o] = src.v[0][i];
             dst.v[1][o] = src.v[1][i];
@@ -708,34 +702,8 @@ unsigned blocks256(int64_t n) { return (unsigned)((n + 255) / 256); }
 
 int device_partition(int64_t n64, const double* d_grid, int* d_order, hipStream_t s, DevicePool& pool) {
     const int n = (int)n64;
-    // the tree: every level's large nodes and their chunks, and the nodes left to k_part_leaf
-    std::vector<PartNode> nodes;
-    std::vector<PartChunk> chunks;
-    std::vector<int> node_off{0}, chunk_off{0};
-    std::vector<LeafNode> leaves;
-    std::vector<std::pair<int, int>> cur{{0, n}}, next;
-    size_t most = 0;
-    for (int level = 0; !cur.empty(); ++level) {
-        next.clear();
-        for (const auto& [lo, hi] : cur) {
-            if (hi - lo <= kNodeMax) {
-                leaves.push_back(LeafNode{lo, hi, level & 1});
-                continue;
-            }
-            const int mid = lo + ((hi - lo + kBlockPts - 1) / kBlockPts / 2) * kBlockPts;
-            const int id = (int)nodes.size() - node_off.back();
-            nodes.push_back(PartNode{lo, hi, mid});
-            for (int k = lo; k < hi; k += kChunk) chunks.push_back(PartChunk{id, k, std::min(hi, k + kChunk)});
-            next.push_back({lo, mid});
-            next.push_back({mid, hi});
-        }
-        if ((int)nodes.size() > node_off.back()) {
-            most = std::max(most, nodes.size() - node_off.back());
-            node_off.push_back((int)nodes.size());
-            chunk_off.push_back((int)chunks.size());
-        }
-        cur.swap(next);
-    }
+    const PartTree tree = part_tree(n);
+    const auto& [nodes, chunks, node_off, chunk_off, leaves, most] = tree;
     const int levels = (int)node_off.size() - 1;
     // one workspace: two point buffers | states | histograms | tables
     auto up = [](size_t b) { return (b + 255) / 256 * 256; };

@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "pdfxc_internal.hpp"
+#include "pdfxc_partition.hpp"
 
 extern "C" {
 size_t fake_live_bytes();
@@ -231,6 +232,46 @@ void failed_copies() {
     pdfxc_ctx_destroy(ctx);
 }
 
+// the bisection's tree for every number of points a grid may have: each level's
+// chunks cover its nodes, the leaves cover the points, threads take each once
+void part_tree_sizes() {
+    for (int64_t n : {(int64_t)1, (int64_t)128, (int64_t)4096, (int64_t)4097, (int64_t)8193, (int64_t)1000077,
+                      ((int64_t)1 << 31) - 128}) {
+        const PartTree T = part_tree(n);
+        int64_t covered = 0;
+        std::vector<LeafNode> leaves = T.leaves;
+        std::sort(leaves.begin(), leaves.end(), [](const LeafNode& a, const LeafNode& b) { return a.lo < b.lo; });
+        for (const LeafNode& L : leaves) {
+            CHECK(L.lo == covered && L.hi > L.lo && L.hi - L.lo <= kNodeMax);
+            covered = L.hi;
+        }
+        CHECK(covered == n);
+        for (size_t level = 0; level + 1 < T.node_off.size(); ++level) {
+            int c = T.chunk_off[level];
+            for (int k = T.node_off[level]; k < T.node_off[level + 1]; ++k) {
+                const PartNode& N = T.nodes[k];
+                CHECK(N.lo < N.mid && N.mid < N.hi && (N.mid - N.lo) % kLeafPts == 0);
+                int64_t at = N.lo;
+                for (; c < T.chunk_off[level + 1] && T.chunks[c].node == k - T.node_off[level]; ++c) {
+                    CHECK(T.chunks[c].lo == at && T.chunks[c].hi > at && T.chunks[c].hi - at <= kChunk);
+                    at = T.chunks[c].hi;
+                }
+                CHECK(at == N.hi);
+            }
+            CHECK(c == T.chunk_off[level + 1]);
+        }
+        if (T.chunks.empty()) continue;
+        const PartChunk& last = T.chunks.back();
+        std::vector<int> times((size_t)(last.hi - last.lo), 0);
+        for (int t = 0; t < kPartThreads; ++t)
+            each_point(last, t, [&](int i) {
+                CHECK(i >= last.lo && i < last.hi);
+                ++times[i - last.lo];
+            });
+        for (int k : times) CHECK(k == 1);
+    }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -239,7 +280,8 @@ int main(int argc, char** argv) {
         void (*run)();
     } const checks[] = {{"pool_threads", pool_threads}, {"host_copy_threads", host_copy_threads}, {"grid_rows", grid_rows},
                   {"pool_bound", pool_bound},     {"reserve_gives_way", reserve_gives_way},
-                  {"density_keeps_little", density_keeps_little}, {"failed_copies", failed_copies}};
+                  {"density_keeps_little", density_keeps_little}, {"failed_copies", failed_copies},
+                  {"part_tree_sizes", part_tree_sizes}};
     for (const auto& k : checks)
         if (argc == 2 && !std::strcmp(argv[1], k.name)) {
             k.run();

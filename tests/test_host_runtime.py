@@ -14,9 +14,9 @@ TESTS = ROOT / "tests"
 
 @pytest.fixture(scope="session")
 def program(tmp_path_factory):
-    """host_checks.cpp linked to the stand-in first, the engine library second."""
+    """host_checks.cpp (signed overflow ends it) linked to the stand-in first, the engine library second."""
     out = tmp_path_factory.mktemp("host")
-    cxx = ["g++", "-std=c++17", "-O1", "-g", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", f"-I{ROOT / 'include'}",
+    cxx = ["g++", "-std=c++17", "-O1", "-g", "-ftrapv", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", f"-I{ROOT / 'include'}",
            f"-I{ROOT / 'proteindf_amd' / 'csrc'}"]
     fake, lib = out / "libfake.so", Path(engine.LIB_PATH)
     subprocess.run(cxx + ["-fPIC", "-shared", str(TESTS / "fake_hip.cpp"), "-o", str(fake)], check=True)
@@ -26,7 +26,7 @@ def program(tmp_path_factory):
 
 
 @pytest.mark.parametrize("check", ["pool_threads", "host_copy_threads", "grid_rows", "pool_bound",
-                                   "reserve_gives_way", "density_keeps_little", "failed_copies"])
+                                   "reserve_gives_way", "density_keeps_little", "failed_copies", "part_tree_sizes"])
 def test_host_code(program, check):
     r = subprocess.run([str(program), check], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
