@@ -1,0 +1,63 @@
+"""K units of two blocks in every kind of FP64 build: UKS, update mode and a
+batch that mixes such a context with one of single blocks.  The same sums in
+another order: 1e-12 of the largest value."""
+import numpy as np
+import pytest
+import torch
+
+from proteindf_amd import calc_grid, engine, guess, molecules
+
+pytestmark = pytest.mark.gpu
+
+
+def _context(waters, n, seed):
+    mol = molecules.water_cluster(waters, seed)
+    info = calc_grid.orbital_info(mol)
+    rng = np.random.default_rng(seed)
+    grid = np.concatenate([mol.xyz[rng.integers(0, mol.n_atoms, n)] + rng.normal(0.0, 1.0, (n, 3)),
+                           rng.uniform(0.0, 1.0, (n, 1))], 1)
+    ctx = engine.XcContext(info)
+    ctx.set_grid(grid)
+    return ctx, guess.pack_lower(0.5 * guess.density_guess(mol, info, seed=seed, eps=0.05))
+
+
+def _many():
+    # 10 units of two blocks per CU, an odd block and a ragged one besides
+    return 20 * torch.cuda.get_device_properties(0).multi_processor_count * 128 + 128 + 77
+
+
+def _close(got, want):
+    np.testing.assert_allclose(got, want, rtol=0, atol=1e-12 * np.abs(want).max())
+
+
+def test_uks_and_update_builds():
+    ctx, P = _context(3, _many(), 5)
+    print("[gpu-case] pairs of blocks, UKS and update", flush=True)
+
+    def builds():
+        E, KA, KB, _ = ctx.build_uks(P, 0.6 * P)
+        ctx.build_rks(0.25 * P)
+        Eu, Ku, _ = ctx.build_rks_update(0.75 * P)
+        return E, KA, KB, Eu, Ku
+
+    pairs = builds()
+    ctx.set_tuning(split_k_group=1)
+    single = builds()
+    ctx.close()
+    for got, want in zip(pairs, single):
+        _close(got, want)
+
+
+def test_a_batch_with_pairs_and_single_blocks():
+    made = [_context(2, 3000, 3), _context(3, _many(), 5), _context(1, 50, 7), _context(2, _many() + 128, 9)]
+    print("[gpu-case] a batch with pairs of blocks", flush=True)
+    want = [ctx.build_rks(P)[:2] for ctx, P in made]
+    batch = engine.XcBatch([ctx for ctx, _ in made])
+    for _ in range(3):
+        E, Ks = batch.build_rks([P for _, P in made])
+        for k, (e, K) in enumerate(want):
+            assert E[k] == e
+            _close(Ks[k], K)
+    batch.close()
+    for ctx, _ in made:
+        ctx.close()

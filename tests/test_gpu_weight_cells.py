@@ -59,3 +59,14 @@ def test_generated_ss_grid_of_a_cage():
     one = oracle.generate_grid_ex(np.array([1], dtype=np.int32), np.zeros((1, 3)), o)[0]
     radius = np.unique(np.round(np.linalg.norm(one[:, :3], axis=1), 9))[-2]
     _compare(_cage(100, radius), np.zeros((1, 3)), None, 1)
+
+
+@pytest.mark.parametrize("n", [276, 277])
+def test_four_waves_and_one_per_workgroup(n):
+    # a chain: 276 atoms are the most that leave two workgroups of four waves on a CU
+    rng = np.random.default_rng(n)
+    xyz = np.zeros((n, 3))
+    xyz[:, 0] = 2.1 * np.arange(n)
+    mol = molecules.Molecule(["H"] * n, xyz + rng.uniform(-0.2, 0.2, xyz.shape), f"H{n}")
+    atom = np.sort(rng.integers(0, n, 600)).astype(np.int32)
+    _compare(mol, mol.xyz[atom] + rng.normal(0.0, 0.6, (600, 3)), atom, 0)
