@@ -114,8 +114,8 @@ typedef struct pdfxc_stats {
  * neighbours in the point bisection) whose K contributions the split K pass
  * sums on the union of their AO columns before one scatter into K, i.e.
  * 128 x split_k_group points per K work unit (a group too wide for the
- * kernel's LDS is halved; the FP64 K pass takes pairs of blocks unless this
- * is 1 or the grid is small); persistent (bit mask, 0..3): bit 0 the FP64
+ * kernel's LDS is halved; the FP64 K pass takes pairs of blocks where their
+ * union is hardly wider, unless this is 1 or the grid is small); persistent (bit mask, 0..3): bit 0 the FP64
  * rho-pass kernels of the widest classes (those that run one workgroup per CU:
  * their persistent form loads the next item's set-up data while the current
  * one runs) and the split rho-pass kernels, bit 1 the K-pass kernels run as

@@ -577,6 +577,10 @@ static void reset_grid(Context& c) {
 
 static int build_blocks_impl(Context& c);
 
+// workgroup shape of k_kmat for a unit of ldn padded columns: at most 8, 10 or
+// more tiles of 16
+static int kmat_class(int ldn) { return ldn <= 8 * 16 ? 0 : ldn <= 10 * 16 ? 1 : 2; }
+
 // dynamic LDS of a k_kmat item
 static size_t kmat_lds(int ps, int ncols, int nsh, int rec_stride) {
     return sizeof(double) * (4 * (size_t)ps * ncols + (size_t)nsh * rec_stride) + sizeof(int) * (size_t)(ncols + 2 * nsh);
@@ -675,8 +679,8 @@ static int build_blocks_impl(Context& c) {
         }
     }
     // Blocks per K unit: the FP64 K pass adds N_b^2 / 2 values to K by atomics
-    // per unit, at 53 G/s a longer time than its matrix products, and the
-    // union of two neighbours is only 2 % wider than either
+    // per unit, at 53 G/s a longer time than its matrix products, and two
+    // neighbours keep nearly the same columns (kKUnitsPerCu)
     int kper = c.opts.precision == PDFXC_FP64 && !c.rho_only ? std::min(kKGroupMax, c.tune.split_k_group) : 1;
     while (kper > 1 && nb / kper < kKUnitsPerCu * c.n_cu) kper /= 2;
     const int ng = kper > 1 ? (nb + kper - 1) / kper : 0;
@@ -761,8 +765,9 @@ static int build_blocks_impl(Context& c) {
         c.max_nao = std::max(c.max_nao, B.nao);
     }
     c.mean_nao = nb ? sum_nao / nb : 0.0;
-    // units of k_kmat: the groups, or the blocks of a group whose union would
-    // not fit a workgroup's LDS, in descending order of cost
+    // units of k_kmat: the groups, or the blocks of a group whose union is too
+    // wide for them, is of a class with too few others or would not fit a
+    // workgroup's LDS, in descending order of cost
     const int RS = c.rec_stride;
     c.kblocks.clear();
     auto unit_of = [&](int li) {
@@ -777,6 +782,8 @@ static int build_blocks_impl(Context& c) {
         for (int li = 0; li < nb; ++li) block_of_leaf[lorder[li]] = li;
         std::vector<KBlock> units;
         std::vector<int> ugroup;
+        int of_class[kKmatClasses] = {};  // groups whose union falls in each class
+        for (int g = 0; g < ng; ++g) ++of_class[kmat_class(padded(gcounts[2 * g + 1]))];
         for (int g = 0; g < ng; ++g) {
             const int l0 = g * kper, l1 = std::min(nb, l0 + kper);
             KBlock U{};
@@ -784,7 +791,11 @@ static int build_blocks_impl(Context& c) {
             U.nao = gcounts[2 * g + 1];
             U.ldn = padded(U.nao);
             U.ldp = c.n_aos;
-            if (l1 - l0 == 1 || kmat_lds(8, U.ldn, U.nshell, RS) > kKmatLds[kKmatClasses - 1]) {
+            int64_t own = 0;  // AOs of the blocks, each by itself
+            for (int lf = l0; lf < l1; ++lf) own += counts[2 * lf + 1];
+            if (l1 - l0 == 1 || of_class[kmat_class(U.ldn)] < c.n_cu ||
+                (int64_t)U.nao * (l1 - l0) * 100 > own * (100 + kKWiderPct) ||
+                kmat_lds(8, U.ldn, U.nshell, RS) > kKmatLds[kKmatClasses - 1]) {
                 for (int lf = l0; lf < l1; ++lf) {
                     units.push_back(unit_of(block_of_leaf[lf]));
                     ugroup.push_back(-1);
@@ -888,7 +899,7 @@ static int build_blocks_impl(Context& c) {
         const KBlock& B = c.kblocks[b];
         const int T = B.ldn / 16, Tp = (T + 1) / 2;
         const int np = Tp * (Tp + 1) / 2;
-        const int cls = T <= 8 ? 0 : T <= 10 ? 1 : 2;
+        const int cls = kmat_class(B.ldn);
         const int per = cls < 2 ? np : c.tune.k_tiles * 36 / 96;
         for (int t0 = 0; t0 < np; t0 += per) {
             KWork w;

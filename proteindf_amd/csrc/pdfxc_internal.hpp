@@ -74,12 +74,27 @@ struct SplitBlock {
 // K pass work unit of k_kmat: 1 to kKGroupMax blocks, neighbours in the point
 // bisection, on the union of their shells; all of them but the last full.
 constexpr int kKGroupMax = 2;
-// Units of two blocks where that leaves this many per CU.  K pass with one and
-// two blocks a unit: 37.0 and 28.1 ms (79,000 blocks, a 30-residue helix), 4.0
-// and 3.4 ms (10,600 blocks, 10 residues), but 0.234 and 0.240 ms (3,200
-// blocks, 8 waters) and 0.42 and 0.75 ms (2,800 blocks, UKS, 12 waters), whose
-// last round of workgroups is then nearly empty.
-constexpr int kKUnitsPerCu = 10;
+// Units of two blocks: on grids with at least kKUnitsPerCu of them per CU;
+// where the union has at most kKWiderPct % more AOs than the two have on
+// average (phi and V of the union are evaluated at the points of both); and
+// where its workgroup shape has a unit for every CU (a shape is a launch of its
+// own, and one of a few units takes as long as its longest).  K pass, ms, of
+// single blocks, all pairs, pairs up to 15 % wider, and those of shapes with a
+// unit per CU:
+//   blocks (units of two per CU)          single    all    15 %   15 %, filled
+//   14,000 (27.4)   10-residue helix       5.50    4.48    4.57      4.58
+//    8,500 (16.7)   10 residues            3.51    2.88    2.85      2.84
+//    5,300 (10.3)   10 residues            2.29    2.01    1.93      1.90
+//    5,200 (10.1)    5 residues            1.66    1.44    1.43      1.42
+//   14,000 (27.3)   23 waters              1.16    1.18    1.06      1.02
+//    8,400 (16.5)   23 waters              0.76    0.85    0.73      0.68
+//    5,200 (10.2)   23 waters              0.52    0.68    0.64      0.48
+//    5,200 (10.2)    8 waters              0.256   0.257   0.245     0.243
+//    3,200           8 waters              0.234   0.240
+//    2,800 (UKS)    12 waters              0.42    0.75
+// (79,000 blocks of 30 residues: 37.0 single, 28.1 all pairs; limits of 10 %
+// and 30 % are within 2 % of this, two or more units per CU up to 8 % slower).
+constexpr int kKUnitsPerCu = 10, kKWiderPct = 15;
 struct KBlock {
     int slot[kKGroupMax];  // first slot of every block
     int npts;              // real points of all of them

@@ -61,3 +61,20 @@ def test_a_batch_with_pairs_and_single_blocks():
     batch.close()
     for ctx, _ in made:
         ctx.close()
+
+
+def test_a_grid_of_pairs_and_single_blocks():
+    # blocks of a large cluster: some neighbours' unions are too wide for a unit of two
+    mol = molecules.water_cluster(23, 0)
+    info = calc_grid.orbital_info(mol)
+    P = guess.pack_lower(0.5 * guess.density_guess(mol, info, seed=1, eps=0.05))
+    ctx = engine.XcContext(info)
+    ctx.generate_grid(mol.Z, mol.xyz, 50, 302)
+    assert ctx.stats().n_blocks >= 20 * torch.cuda.get_device_properties(0).multi_processor_count
+    print("[gpu-case] pairs and single blocks of one grid", flush=True)
+    both = ctx.build_rks(P)
+    ctx.set_tuning(split_k_group=1)
+    single = ctx.build_rks(P)
+    ctx.close()
+    assert both[0] == single[0]
+    _close(both[1], single[1])
