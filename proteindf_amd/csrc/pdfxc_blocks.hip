@@ -834,8 +834,8 @@ int launch_item_shells(Context& c, int n, const KWork* d_work, int* d_nsh) {
     return check("k_item_shells");
 }
 
-int launch_gather_points(Context& c, const double* d_slots, double* d_pts, int stride, int off) {
-    hipLaunchKernelGGL(k_gather_points, dim3(blocks256(4 * c.n_pts)), dim3(256), 0, c.stream, c.n_pts, c.d_slot_of_point,
+int launch_gather_points(Context& c, int64_t first, int64_t n, const double* d_slots, double* d_pts, int stride, int off) {
+    hipLaunchKernelGGL(k_gather_points, dim3(blocks256(4 * n)), dim3(256), 0, c.stream, n, c.d_slot_of_point + first,
                        d_slots, d_pts, stride, off);
     return check("k_gather_points");
 }
@@ -846,8 +846,8 @@ int launch_gather_density(Context& c, const double* d_slots, double* d_out, bool
     return check("k_gather_density");
 }
 
-int launch_scatter_points(Context& c, const double* d_pts, double* d_slots) {
-    hipLaunchKernelGGL(k_scatter_points, dim3(blocks256(4 * c.n_pts)), dim3(256), 0, c.stream, c.n_pts, c.d_slot_of_point,
+int launch_scatter_points(Context& c, int64_t first, int64_t n, const double* d_pts, double* d_slots) {
+    hipLaunchKernelGGL(k_scatter_points, dim3(blocks256(4 * n)), dim3(256), 0, c.stream, n, c.d_slot_of_point + first,
                        d_pts, d_slots);
     return check("k_scatter_points");
 }

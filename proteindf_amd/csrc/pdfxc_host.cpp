@@ -402,8 +402,6 @@ static void free_grid_buffers(Context* c) {
     gfree(*c, c->d_rho);
     gfree(*c, c->d_coef_b);
     gfree(*c, c->d_rho_b);
-    gfree(*c, c->d_rho_out);
-    c->n_rho_out = 0;
     gfree(*c, c->d_eblock);
     gfree(*c, c->d_sblocks);
     gfree(*c, c->d_chunks);
@@ -1556,6 +1554,69 @@ int ensure_host_slots(Context& c) {
     return PDFXC_OK;
 }
 
+// Points at a time: 128 MiB of rows per spin, a buffer that the pool keeps.
+constexpr int64_t kRhoPts = 1 << 22;
+
+int rho_to_host(Context& c, int nspin, const double* const* d_slots, double* rows) {
+    const int stride = 4 * nspin;
+    const int64_t per = std::min(c.n_pts, kRhoPts);
+    void* buf = nullptr;
+    if (context_take(c, &buf, sizeof(double) * (size_t)(stride * per)) != PDFXC_OK) {
+        // no device memory left: the slots as they are, put in order here
+        if (int rc = ensure_host_slots(c)) return rc;
+        std::vector<double> s(4 * (size_t)c.n_slots);
+        for (int sp = 0; sp < nspin; ++sp) {
+            PDFXC_HIP(hipMemcpyAsync(s.data(), d_slots[sp], sizeof(double) * s.size(), hipMemcpyDeviceToHost, c.stream));
+            PDFXC_HIP(hipStreamSynchronize(c.stream));
+            for (int64_t p = 0; p < c.n_pts; ++p)
+                for (int q = 0; q < 4; ++q) rows[stride * p + 4 * sp + q] = s[4 * c.slot_of_point[p] + q];
+        }
+        return PDFXC_OK;
+    }
+    double* d = static_cast<double*>(buf);
+    int rc = PDFXC_OK;
+    hipError_t e = hipSuccess;
+    for (int64_t at = 0; at < c.n_pts && rc == PDFXC_OK && e == hipSuccess; at += per) {
+        const int64_t n = std::min(per, c.n_pts - at);
+        for (int sp = 0; sp < nspin && rc == PDFXC_OK; ++sp)
+            rc = launch_gather_points(c, at, n, d_slots[sp], d, stride, 4 * sp);
+        if (rc == PDFXC_OK)
+            e = hipMemcpyAsync(rows + stride * at, d, sizeof(double) * (size_t)(stride * n), hipMemcpyDeviceToHost, c.stream);
+    }
+    const hipError_t es = hipStreamSynchronize(c.stream);  // also on failure: the buffer changes hands
+    context_give(c, buf);
+    if (rc) return rc;
+    if (e == hipSuccess) e = es;
+    return e == hipSuccess ? PDFXC_OK : hip_fail(e, "rho download");
+}
+
+int rho_from_host(Context& c, const double* rows, double* d_slots) {
+    const int64_t per = std::min(c.n_pts, kRhoPts);
+    void* buf = nullptr;
+    if (context_take(c, &buf, sizeof(double) * 4 * (size_t)per) != PDFXC_OK) {
+        if (int rc = ensure_host_slots(c)) return rc;
+        std::vector<double> s(4 * (size_t)c.n_slots, 0.0);
+        for (int64_t p = 0; p < c.n_pts; ++p)
+            for (int q = 0; q < 4; ++q) s[4 * c.slot_of_point[p] + q] = rows[4 * p + q];
+        PDFXC_HIP(hipMemcpyAsync(d_slots, s.data(), sizeof(double) * s.size(), hipMemcpyHostToDevice, c.stream));
+        PDFXC_HIP(hipStreamSynchronize(c.stream));
+        return PDFXC_OK;
+    }
+    double* d = static_cast<double*>(buf);
+    int rc = PDFXC_OK;
+    hipError_t e = hipMemsetAsync(d_slots, 0, sizeof(double) * 4 * (size_t)c.n_slots, c.stream);
+    for (int64_t at = 0; at < c.n_pts && rc == PDFXC_OK && e == hipSuccess; at += per) {
+        const int64_t n = std::min(per, c.n_pts - at);
+        e = hipMemcpyAsync(d, rows + 4 * at, sizeof(double) * 4 * (size_t)n, hipMemcpyHostToDevice, c.stream);
+        if (e == hipSuccess) rc = launch_scatter_points(c, at, n, d, d_slots);
+    }
+    const hipError_t es = hipStreamSynchronize(c.stream);
+    context_give(c, buf);
+    if (rc) return rc;
+    if (e == hipSuccess) e = es;
+    return e == hipSuccess ? PDFXC_OK : hip_fail(e, "rho upload");
+}
+
 // A buffer for a new grid's columns; the old grid and its buffers go first.
 static int alloc_grid(Context& c, int64_t n, double** d_grid) {
     reset_grid(c);
@@ -2147,18 +2208,8 @@ static int build_host(Context* c, int xc, int nspin, const double* const* P_pack
     *E_xc = H[nspin * NP];
     for (int sp = 0; sp < nspin; ++sp) c->n_whole[sp] = H[nspin * NP + 1 + sp];
     if (rho_out) {
-        const int stride = 4 * nspin;
-        const size_t n_out = (size_t)stride * (size_t)c->n_pts;
-        if (c->n_rho_out < n_out) {  // kept with the grid: rho is asked for again with every iteration
-            dfree(c->d_rho_out);
-            c->n_rho_out = 0;
-            if (int e = dalloc(*c, &c->d_rho_out, n_out)) return e;
-            c->n_rho_out = n_out;
-        }
-        for (int sp = 0; sp < nspin; ++sp)
-            if (int e = launch_gather_points(*c, sp ? c->d_rho_b : c->d_rho, c->d_rho_out, stride, 4 * sp)) return e;
-        PDFXC_HIP(hipMemcpyAsync(rho_out, c->d_rho_out, sizeof(double) * n_out, hipMemcpyDeviceToHost, c->stream));
-        PDFXC_HIP(hipStreamSynchronize(c->stream));
+        const double* d_rho[2] = {c->d_rho, c->d_rho_b};
+        if ((rc = rho_to_host(*c, nspin, d_rho, rho_out))) return rc;
     }
     c->whole_spins = nspin;
     return PDFXC_OK;

@@ -321,8 +321,6 @@ struct Context {
     double* d_rho = nullptr;      // per slot: rho, grad rho (4)
     double* d_rho_b = nullptr;    // UKS: beta rho, grad rho per slot (allocated by the first UKS build)
     double* d_coef_b = nullptr;   // UKS: beta point terms
-    double* d_rho_out = nullptr;  // rho in the caller's order (allocated by the first build that returns it)
-    size_t n_rho_out = 0;
     double* d_eblock = nullptr;   // per 256 slots: energy, then w rho of each spin (k_xc_points partial sums)
     double* d_P = nullptr;        // dense N x N
     double* d_K = nullptr;        // dense N x N
@@ -413,6 +411,11 @@ int ensure_host_grid(Context& c);
 int ensure_host_lists(Context& c);
 int ensure_host_slots(Context& c);
 
+// (rho, grad rho) of nspin spins from their slots to rows of 4 nspin in the
+// caller's order, and of one spin from such rows of 4 to its slots
+int rho_to_host(Context& c, int nspin, const double* const* d_slots, double* rows);
+int rho_from_host(Context& c, const double* rows, double* d_slots);
+
 // grid blocks (pdfxc_blocks.hip)
 // d_order: the points of block b are d_order[128 b ..); synchronises s
 int device_partition(int64_t n, const double* d_grid, int* d_order, hipStream_t s, DevicePool& pool);
@@ -437,10 +440,10 @@ int launch_group_masks(int nb, int per, int nsh, const ScreenShell* d_shells, in
 int launch_fill_groups(Context& c, int n, const int* d_group, int nw, int ncls, const ScreenShell* d_shells,
                        const unsigned long long* d_gmasks);
 int launch_item_shells(Context& c, int n, const KWork* d_work, int* d_nsh);
-// four values per point between the slots and the caller's order (row stride and offset of the latter)
-int launch_gather_points(Context& c, const double* d_slots, double* d_pts, int stride, int off);
+// four values per point between the slots and n points of the caller's order from `first` on (its row stride and offset)
+int launch_gather_points(Context& c, int64_t first, int64_t n, const double* d_slots, double* d_pts, int stride, int off);
 int launch_gather_density(Context& c, const double* d_slots, double* d_out, bool grad);  // rho [n] | grad [n][3]
-int launch_scatter_points(Context& c, const double* d_pts, double* d_slots);
+int launch_scatter_points(Context& c, int64_t first, int64_t n, const double* d_pts, double* d_slots);
 int launch_scatter_atoms(Context& c, const int* d_atom, int* d_slot_atom);
 int launch_points_to_grid(int64_t n, const double* d_xyz, double* d_grid, hipStream_t s);
 

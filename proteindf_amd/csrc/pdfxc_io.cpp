@@ -117,35 +117,6 @@ static int write_matrix(const char* path, int type, int64_t rows, int64_t cols, 
     return ok ? PDFXC_OK : io_error(std::string("write failed: ") + path);
 }
 
-// caller-order rho (n_pts x 4) <-> the context's slots
-static int download_rho(Context* c, double* rho, const double* d_src) {
-    const size_t bytes = sizeof(double) * 4 * (size_t)c->n_pts;
-    void* p = nullptr;
-    if (int rc = context_take(*c, &p, bytes)) return rc;
-    double* d = static_cast<double*>(p);
-    int rc = launch_gather_points(*c, d_src, d, 4, 0);
-    hipError_t e = rc == PDFXC_OK ? hipMemcpyAsync(rho, d, bytes, hipMemcpyDeviceToHost, c->stream) : hipSuccess;
-    const hipError_t es = hipStreamSynchronize(c->stream);  // also on failure: d changes hands
-    if (e == hipSuccess) e = es;
-    context_give(*c, d);
-    return rc != PDFXC_OK ? rc : e == hipSuccess ? PDFXC_OK : hip_fail(e, "rho download");
-}
-
-static int upload_rho(Context* c, const double* rho, double* d_dst) {
-    const size_t bytes = sizeof(double) * 4 * (size_t)c->n_pts;
-    void* p = nullptr;
-    if (int rc = context_take(*c, &p, bytes)) return rc;
-    double* d = static_cast<double*>(p);
-    int rc = PDFXC_OK;
-    hipError_t e = hipMemsetAsync(d_dst, 0, sizeof(double) * 4 * (size_t)c->n_slots, c->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(d, rho, bytes, hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess) rc = launch_scatter_points(*c, d, d_dst);
-    const hipError_t es = hipStreamSynchronize(c->stream);
-    if (e == hipSuccess) e = es;
-    context_give(*c, d);
-    return rc != PDFXC_OK ? rc : e == hipSuccess ? PDFXC_OK : hip_fail(e, "rho upload");
-}
-
 }  // namespace pdfxc
 
 using namespace pdfxc;
@@ -256,7 +227,7 @@ int pdfxc_load_grid_matrix(pdfxc_ctx* ctx, const char* path, int64_t* n_pts_out,
             for (int q = 0; q < per_spin; ++q) rho[4 * p + q] = col[(5 + per_spin * sp + q) * n + p];
         if (sp == 1)
             if (int rc = ensure_beta_buffers(c)) return rc;
-        if (int rc = upload_rho(c, rho.data(), sp ? c->d_rho_b : c->d_rho)) return rc;
+        if (int rc = rho_from_host(*c, rho.data(), sp ? c->d_rho_b : c->d_rho)) return rc;
     }
     if (n_pts_out) *n_pts_out = n;
     if (n_cols_out) *n_cols_out = (int)nc;
@@ -284,7 +255,8 @@ int pdfxc_save_grid_matrix(pdfxc_ctx* ctx, const char* path, int n_rho_cols) {
     const int per_spin = n_rho_cols / nspin;
     for (int sp = 0; per_spin > 0 && sp < nspin; ++sp) {
         std::vector<double> rho(4 * (size_t)n);
-        if (int rc = download_rho(c, rho.data(), sp ? c->d_rho_b : c->d_rho)) return rc;
+        const double* d_rho = sp ? c->d_rho_b : c->d_rho;
+        if (int rc = rho_to_host(*c, 1, &d_rho, rho.data())) return rc;
         for (int64_t p = 0; p < n; ++p)
             for (int q = 0; q < per_spin; ++q) m[(5 + per_spin * sp + q) * n + p] = rho[4 * p + q];
     }

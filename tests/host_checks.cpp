@@ -1,5 +1,7 @@
 // Checks of the engine's host code against the stand-in HIP runtime, one per
 // argument; exit status 0 when it holds.
+#include <unistd.h>
+
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -190,6 +192,50 @@ void reserve_gives_way() {
     CHECK(fake_live_bytes() == 0);
 }
 
+// rho goes to the host and back without device memory of its own
+void rho_without_memory() {
+    pdfxc_ctx* ctx = context();
+    Context& c = *reinterpret_cast<Context*>(ctx);
+    const int64_t n = 1000;
+    double P = 1.0, K = 0.0, E = 0.0;
+    std::vector<double> out(8 * n), mat(13 * n);
+    set_grid(ctx, n);
+    CHECK(pdfxc_build_uks(ctx, PDFXC_SVWN, &P, &P, &K, &K, &E, nullptr) == PDFXC_OK);
+    // point p in slot n - 1 - p; rho of slot s: 8 s + 0 .. 3 and, beta, + 4 .. 7
+    std::vector<int> slots((size_t)n);
+    for (int64_t i = 0; i < n; ++i) slots[i] = (int)(n - 1 - i);
+    CHECK(hipMemcpy(c.d_slot_of_point, slots.data(), n * sizeof(int), hipMemcpyHostToDevice) == hipSuccess);
+    for (int64_t s = 0; s < n; ++s)
+        for (int q = 0; q < 4; ++q) {
+            c.d_rho[4 * s + q] = 8 * s + q;
+            c.d_rho_b[4 * s + q] = 8 * s + 4 + q;
+        }
+    c.pool.trim(0);
+    fake_limit(fake_live_bytes());
+    CHECK(pdfxc_build_uks(ctx, PDFXC_SVWN, &P, &P, &K, &K, &E, out.data()) == PDFXC_OK);
+    for (int64_t i = 0; i < n; ++i)
+        for (int q = 0; q < 8; ++q) CHECK(out[8 * i + q] == 8 * (n - 1 - i) + q);
+    char path[] = "/tmp/pdfxc_rho_XXXXXX";
+    const int fd = mkstemp(path);
+    CHECK(fd >= 0);
+    close(fd);
+    CHECK(pdfxc_save_grid_matrix(ctx, path, 8) == PDFXC_OK);
+    CHECK(pdfxc_load_general_matrix(path, n, 13, mat.data()) == PDFXC_OK);
+    unlink(path);
+    for (int64_t i = 0; i < n; ++i)
+        for (int q = 0; q < 8; ++q) CHECK(mat[(5 + q) * n + i] == out[8 * i + q]);
+    std::fill(c.d_rho, c.d_rho + 4 * c.n_slots, -1.0);
+    std::vector<double> alpha(4 * n);
+    for (int64_t i = 0; i < n; ++i)
+        for (int q = 0; q < 4; ++q) alpha[4 * i + q] = out[8 * i + q];
+    CHECK(rho_from_host(c, alpha.data(), c.d_rho) == PDFXC_OK);
+    for (int64_t s = 0; s < c.n_slots; ++s)
+        for (int q = 0; q < 4; ++q) CHECK(c.d_rho[4 * s + q] == (s < n ? 8 * s + q : 0.0));
+    fake_limit(~(size_t)0);
+    pdfxc_ctx_destroy(ctx);
+    CHECK(fake_live_bytes() == 0);
+}
+
 // the context that densities keep holds no matrices beyond the pool's bound
 void density_keeps_little() {
     const int n = 4800;  // three matrices of 4800 x 4800 are 553 MB
@@ -281,7 +327,7 @@ int main(int argc, char** argv) {
     } const checks[] = {{"pool_threads", pool_threads}, {"host_copy_threads", host_copy_threads}, {"grid_rows", grid_rows},
                   {"pool_bound", pool_bound},     {"reserve_gives_way", reserve_gives_way},
                   {"density_keeps_little", density_keeps_little}, {"failed_copies", failed_copies},
-                  {"part_tree_sizes", part_tree_sizes}};
+                  {"part_tree_sizes", part_tree_sizes}, {"rho_without_memory", rho_without_memory}};
     for (const auto& k : checks)
         if (argc == 2 && !std::strcmp(argv[1], k.name)) {
             k.run();
