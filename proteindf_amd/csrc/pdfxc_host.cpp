@@ -453,15 +453,19 @@ void* pdfxc_stream(pdfxc_ctx* ctx) {
 namespace pdfxc {
 
 // ---------------------------------------------------------------------------
-// Grid blocks of the split precision modes: recursive bisection of the point
-// set along its widest extent, cutting at a multiple of 128 so that every block
-// but the last is full.  The device's bisection makes the same cuts (12 times
-// as fast at 1.5 million points) but leaves the points of a block in another
-// order, and the FP32 sums of the split kernels, taken over runs of 16 points,
-// round to other values (4e-9 of K, as much as their error): these modes keep
-// the order, and so the results, that std::nth_element leaves.
+// Grid blocks of small grids and of the split precision modes: recursive
+// bisection of the point set along its widest extent, cutting at a multiple of
+// 128 so that every block but the last is full.  The device's bisection makes
+// the same cuts but leaves the points of a block in another order.  For few
+// points it is slower, its workgroup of 4096 points alone taking 0.3 ms:
+// set_grid of 3,000 points takes 305 us with these cuts and 449 with the
+// device's, 5,000 points 442 and 580, 8,000 points 705 and 623, 12,000 points
+// 977 and 730 (1.5 million: a twelfth of the
+// time).  The FP32 sums of the split kernels, taken over runs of 16 points,
+// round to other values in another order (4e-9 of K, as much as their error):
+// these modes keep the order, and so the results, that std::nth_element leaves.
 // ---------------------------------------------------------------------------
-static void partition_points(const Context& c, std::vector<int>& order) {
+void partition_points(const Context& c, std::vector<int>& order) {
     order.resize((size_t)c.n_pts);
     std::iota(order.begin(), order.end(), 0);
     std::vector<std::pair<int64_t, int64_t>> stack;
@@ -701,7 +705,17 @@ static int build_blocks_impl(Context& c) {
     int* d_gcounts = reinterpret_cast<int*>(reinterpret_cast<char*>(d_gmasks) + b_gmask);
     int* d_group = reinterpret_cast<int*>(reinterpret_cast<char*>(d_gcounts) + b_gcnt);
     std::vector<int> order;
-    if (c.opts.precision == PDFXC_FP64) {
+    // (the end of everything queued, before the host's lists of this function go)
+    struct StreamEnd {
+        hipStream_t s;
+        ~StreamEnd() { (void)hipStreamSynchronize(s); }
+    };
+    std::vector<int> lorder(nb), unit_group;  // leaf of every block; mask of a K unit of several blocks, else -1
+    std::vector<int> rho_work, srho_work;
+    std::vector<KGWork> skw;
+    std::vector<KWork> kall;
+    const StreamEnd end{c.stream};
+    if (c.opts.precision == PDFXC_FP64 && n > kHostCut) {
         rc = device_partition(n, c.d_grid, d_order, c.stream, c.pool);
         if (rc) return rc;
     } else {
@@ -724,7 +738,6 @@ static int build_blocks_impl(Context& c) {
     // launch order: descending cost (longest blocks first)
     auto padded = [](int nao) { return std::max(kColPad, (nao + kColPad - 1) / kColPad * kColPad); };
     auto npts_of = [&](int leaf) { return (int)std::min<int64_t>(kBlockPts, n - (int64_t)leaf * kBlockPts); };
-    std::vector<int> lorder(nb);
     std::vector<int64_t> cost(nb);
     for (int b = 0; b < nb; ++b) {
         const int64_t ldn = padded(counts[2 * b + 1]);
@@ -772,7 +785,6 @@ static int build_blocks_impl(Context& c) {
         const BlockDesc& B = c.blocks[li];
         return KBlock{{B.pt_begin}, B.npts, B.shell_begin, B.nshell, B.nao, B.ldn, B.col_begin, B.ldp, 0, B.poff};
     };
-    std::vector<int> unit_group;  // mask of a unit of several blocks, else -1
     if (!ng) {
         for (int li = 0; li < nb; ++li) c.kblocks.push_back(unit_of(li));
     } else {
@@ -845,13 +857,17 @@ static int build_blocks_impl(Context& c) {
         rc = launch_fill_groups(c, nu, d_group, nw, ncls, d_sc, d_gmasks);
         if (rc) return rc;
     }
-    PDFXC_HIP(hipStreamSynchronize(c.stream));
+    if (!order.empty() && n <= kHostPts) {
+        c.slot_of_point.resize((size_t)n);
+        for (int li = 0; li < nb; ++li)
+            for (int k = 0; k < c.blocks[li].npts; ++k)
+                c.slot_of_point[order[lorder[li] * kBlockPts + k]] = (int64_t)li * kBlockPts + k;
+    }
 
     // k_rho work lists by template class: ldn <= 128 (64 points per
     // workgroup), <= 256 (64 when the plane fits in LDS: class 4, else 32),
     // <= 512, <= 1024 (16); the tuning may move every block up by rho_shift
     // classes (fewer points per workgroup; ldn <= 256 then takes 16)
-    std::vector<int> rho_work;
     c.rho_launches.clear();
     auto rho_lds = [&](const BlockDesc& B, size_t pb) {
         return sizeof(double) * (std::max<size_t>((size_t)B.ldn * pb, 4 * 512) + (size_t)B.nshell * RS) +
@@ -911,11 +927,19 @@ static int build_blocks_impl(Context& c) {
             kw[cls].push_back(w);
         }
     }
-    // the shells of every item, counted where the block lists are
+    // the shells of every item: all of its unit's, or, for an item that leaves
+    // out the unit's last columns, counted where the block lists are
     size_t n_items = 0;
-    for (const auto& w : kw) n_items += w.size();
-    std::vector<int> item_nsh(n_items);
-    if (n_items > 0) {
+    bool partial = false;
+    for (auto& list : kw) {
+        n_items += list.size();
+        for (KWork& w : list) {
+            w.nsh = c.kblocks[w.block].nshell;
+            partial = partial || w.ncols < c.kblocks[w.block].ldn;
+        }
+    }
+    if (partial) {
+        std::vector<int> item_nsh(n_items);
         DeviceBuf items(c);
         if (int e = items.alloc((sizeof(KWork) + sizeof(int)) * n_items)) return e;
         KWork* d_items = items.as<KWork>();
@@ -927,12 +951,14 @@ static int build_blocks_impl(Context& c) {
         if (int e = launch_item_shells(c, (int)n_items, d_items, d_nsh)) return e;
         PDFXC_HIP(hipMemcpyAsync(item_nsh.data(), d_nsh, sizeof(int) * n_items, hipMemcpyDeviceToHost, c.stream));
         PDFXC_HIP(hipStreamSynchronize(c.stream));
+        size_t at = 0;
+        for (auto& list : kw)
+            for (KWork& w : list) w.nsh = item_nsh[at++];
     }
     // points per slab: 16, or 8 where 16 would cost the class its workgroups
     // per CU (3, 2 and 1 by its registers), or what one workgroup can have
-    for (int cls = 0, at = 0; cls < kKmatClasses; ++cls)
+    for (int cls = 0; cls < kKmatClasses; ++cls)
         for (KWork& w : kw[cls]) {
-            w.nsh = item_nsh[at++];
             auto lds_of = [&](int ps) { return kmat_lds(ps, w.ncols, w.nsh, RS); };
             w.ps = 16;
             if (lds_of(16) > kKmatLds[cls]) w.ps = lds_of(8) <= kKmatLds[kKmatClasses - 1] ? 8 : 4;
@@ -943,7 +969,6 @@ static int build_blocks_impl(Context& c) {
             }
             klds[cls] = std::max(klds[cls], lds);
         }
-    std::vector<KWork> kall;
     c.kmat_launches.clear();
     for (int cls = 0; cls < kKmatClasses; ++cls) {
         if (kw[cls].empty()) continue;
@@ -953,8 +978,6 @@ static int build_blocks_impl(Context& c) {
 
     // split precision: chunked column layout and k_rho_split classes (ldnp <=
     // 256: 64 points per workgroup, <= 512: 32, <= 1024: 16); k_kmat_split items
-    std::vector<int> srho_work;
-    std::vector<KGWork> skw;
     size_t sk_lds = 0;
     c.sblocks.clear();
     c.chunks.clear();
@@ -1263,7 +1286,7 @@ static int build_blocks_impl(Context& c) {
         if (rc == PDFXC_OK) rc = galloc(c, &c.d_kg_masks, c.kg_masks.size());
     }
     if (rc != PDFXC_OK) return rc;
-    auto up = [](void* d, const void* h, size_t n) { return hipMemcpy(d, h, n, hipMemcpyHostToDevice); };
+    auto up = [&](void* d, const void* h, size_t bytes) { return hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, c.stream); };
     PDFXC_HIP(up(c.d_rho_work, rho_work.data(), rho_work.size() * sizeof(int)));
     if (!kall.empty()) PDFXC_HIP(up(c.d_k_work, kall.data(), kall.size() * sizeof(KWork)));
     if (c.opts.precision != PDFXC_FP64) {
@@ -1532,6 +1555,13 @@ int ensure_host_grid(Context& c) {
     std::lock_guard<std::mutex> lock(c.host_mu);
     if ((int64_t)c.gx.size() == c.n_pts) return PDFXC_OK;
     const int64_t n = c.n_pts;
+    if (n <= kHostPts) {  // one copy of all columns
+        std::vector<double> flat;
+        if (int rc = host_copies<double, 1>(c, {&flat}, {c.d_grid}, {4 * n})) return rc;
+        std::vector<double>* own[4] = {&c.gx, &c.gy, &c.gz, &c.gw};
+        for (int q = 3; q >= 0; --q) own[q]->assign(flat.begin() + q * n, flat.begin() + (q + 1) * n);
+        return PDFXC_OK;
+    }
     return host_copies<double, 4>(c, {&c.gx, &c.gy, &c.gz, &c.gw},
                                   {c.d_grid, c.d_grid + n, c.d_grid + 2 * n, c.d_grid + 3 * n}, {n, n, n, n});
 }
@@ -1561,13 +1591,13 @@ int rho_to_host(Context& c, int nspin, const double* const* d_slots, double* row
     const int stride = 4 * nspin;
     const int64_t per = std::min(c.n_pts, kRhoPts);
     void* buf = nullptr;
-    if (context_take(c, &buf, sizeof(double) * (size_t)(stride * per)) != PDFXC_OK) {
-        // no device memory left: the slots as they are, put in order here
+    if (c.n_pts <= kHostRho || context_take(c, &buf, sizeof(double) * (size_t)(stride * per)) != PDFXC_OK) {
+        // few points, or no device memory left: the slots as they are, put in order here
         if (int rc = ensure_host_slots(c)) return rc;
         std::vector<double> s(4 * (size_t)c.n_slots);
         for (int sp = 0; sp < nspin; ++sp) {
-            PDFXC_HIP(hipMemcpyAsync(s.data(), d_slots[sp], sizeof(double) * s.size(), hipMemcpyDeviceToHost, c.stream));
             PDFXC_HIP(hipStreamSynchronize(c.stream));
+            PDFXC_HIP(hipMemcpy(s.data(), d_slots[sp], sizeof(double) * s.size(), hipMemcpyDeviceToHost));
             for (int64_t p = 0; p < c.n_pts; ++p)
                 for (int q = 0; q < 4; ++q) rows[stride * p + 4 * sp + q] = s[4 * c.slot_of_point[p] + q];
         }
@@ -1593,13 +1623,13 @@ int rho_to_host(Context& c, int nspin, const double* const* d_slots, double* row
 int rho_from_host(Context& c, const double* rows, double* d_slots) {
     const int64_t per = std::min(c.n_pts, kRhoPts);
     void* buf = nullptr;
-    if (context_take(c, &buf, sizeof(double) * 4 * (size_t)per) != PDFXC_OK) {
+    if (c.n_pts <= kHostRho || context_take(c, &buf, sizeof(double) * 4 * (size_t)per) != PDFXC_OK) {
         if (int rc = ensure_host_slots(c)) return rc;
         std::vector<double> s(4 * (size_t)c.n_slots, 0.0);
         for (int64_t p = 0; p < c.n_pts; ++p)
             for (int q = 0; q < 4; ++q) s[4 * c.slot_of_point[p] + q] = rows[4 * p + q];
-        PDFXC_HIP(hipMemcpyAsync(d_slots, s.data(), sizeof(double) * s.size(), hipMemcpyHostToDevice, c.stream));
         PDFXC_HIP(hipStreamSynchronize(c.stream));
+        PDFXC_HIP(hipMemcpy(d_slots, s.data(), sizeof(double) * s.size(), hipMemcpyHostToDevice));
         return PDFXC_OK;
     }
     double* d = static_cast<double*>(buf);
@@ -1623,39 +1653,56 @@ static int alloc_grid(Context& c, int64_t n, double** d_grid) {
     return galloc(c, d_grid, 4 * (size_t)n);
 }
 
+// First point with a value that is not finite (n when there is none), by the
+// device.
+static int first_not_finite(Context& c, int64_t n, const double* d_grid, const char* who, int64_t* first) {
+    unsigned long long f = (unsigned long long)n;
+    // the energy accumulator's 8 bytes hold the answer
+    unsigned long long* d_first = reinterpret_cast<unsigned long long*>(c.d_E);
+    hipError_t e = hipMemcpyAsync(d_first, &f, sizeof(f), hipMemcpyHostToDevice, c.stream);
+    if (e == hipSuccess)
+        if (int rc = device_check_finite(n, d_grid, d_first, c.stream)) return rc;
+    if (e == hipSuccess) e = hipMemcpyAsync(&f, d_first, sizeof(f), hipMemcpyDeviceToHost, c.stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
+    if (e != hipSuccess) return hip_fail(e, who);
+    *first = (int64_t)f;
+    return PDFXC_OK;
+}
+
 // Takes over d_grid (n x 4 columns, written on c.stream) as the context's grid
 // and builds its blocks; a grid with a value that is not finite is refused and
-// leaves the context without one.
-static int set_device_grid(Context& c, int64_t n, double* d_grid, const char* who) {
+// leaves the context without one.  Up to kHostPts points the context has the
+// columns on the host as well: col if given, else copied back.
+static int set_device_grid(Context& c, int64_t n, double* d_grid, const char* who, const double* const* col = nullptr) {
     gfree(c, c.d_grid);
     c.d_grid = d_grid;
-    c.gx.clear();
-    c.gy.clear();
-    c.gz.clear();
-    c.gw.clear();
+    std::vector<double>* own[4] = {&c.gx, &c.gy, &c.gz, &c.gw};
+    for (std::vector<double>* v : own) v->clear();
     c.n_pts = n;
     c.gen_atom.clear();
     c.grid_partition = PDFXC_PARTITION_BECKE;
     c.grid_size_adjust = 1;
-    unsigned long long first = (unsigned long long)n;
-    {
-        // the energy accumulator's 8 bytes hold the answer
-        unsigned long long* d_first = reinterpret_cast<unsigned long long*>(c.d_E);
-        hipError_t e = hipMemcpyAsync(d_first, &first, sizeof(first), hipMemcpyHostToDevice, c.stream);
-        int rc = e == hipSuccess ? device_check_finite(n, d_grid, d_first, c.stream) : hip_fail(e, who);
-        if (rc == PDFXC_OK) {
-            e = hipMemcpyAsync(&first, d_first, sizeof(first), hipMemcpyDeviceToHost, c.stream);
-            if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
-            if (e != hipSuccess) rc = hip_fail(e, who);
-        }
-        if (rc != PDFXC_OK) {
-            const std::string msg = g_last_error;
-            reset_grid(c);
-            set_error(msg);
-            return rc;
-        }
+    int64_t first = n;
+    int rc = PDFXC_OK;
+    if (n <= (c.rho_only ? kHostCut : kHostPts)) {
+        if (col)
+            for (int q = 0; q < 4; ++q) own[q]->assign(col[q], col[q] + n);
+        else
+            rc = ensure_host_grid(c);
+        for (int q = 0; q < 4 && rc == PDFXC_OK; ++q)
+            first = std::min<int64_t>(first, std::find_if(own[q]->begin(), own[q]->begin() + first,
+                                                          [](double v) { return !std::isfinite(v); }) -
+                                                 own[q]->begin());
+    } else {
+        rc = first_not_finite(c, n, d_grid, who, &first);
     }
-    if (first < (unsigned long long)n) {
+    if (rc != PDFXC_OK) {
+        const std::string msg = g_last_error;
+        reset_grid(c);
+        set_error(msg);
+        return rc;
+    }
+    if (first < n) {
         reset_grid(c);
         return arg_error(std::string(who) + ": non-finite grid value at point " + std::to_string(first));
     }
@@ -1710,15 +1757,23 @@ int pdfxc_set_grid(pdfxc_ctx* ctx, int64_t n_pts, const double* x, const double*
     double* d_grid = nullptr;
     if (int rc = alloc_grid(*c, n_pts, &d_grid)) return rc;
     const double* col[4] = {x, y, z, w};
-    for (int q = 0; q < 4; ++q) {
-        const hipError_t e = hipMemcpyAsync(d_grid + q * n_pts, col[q], sizeof(double) * (size_t)n_pts,
-                                            hipMemcpyHostToDevice, c->stream);
-        if (e != hipSuccess) {
-            gfree(*c, d_grid);
-            return hip_fail(e, "pdfxc_set_grid: upload");
-        }
+    std::vector<double> flat;  // a small grid crosses in one copy
+    if (n_pts <= kHostPts)
+        for (const double* v : col) flat.insert(flat.end(), v, v + n_pts);
+    hipError_t e = hipSuccess;
+    if (!flat.empty())
+        e = hipMemcpyAsync(d_grid, flat.data(), sizeof(double) * flat.size(), hipMemcpyHostToDevice, c->stream);
+    else
+        for (int q = 0; q < 4 && e == hipSuccess; ++q)
+            e = hipMemcpyAsync(d_grid + q * n_pts, col[q], sizeof(double) * (size_t)n_pts, hipMemcpyHostToDevice, c->stream);
+    if (e != hipSuccess) {
+        (void)hipStreamSynchronize(c->stream);
+        gfree(*c, d_grid);
+        return hip_fail(e, "pdfxc_set_grid: upload");
     }
-    return set_device_grid(*c, n_pts, d_grid, "pdfxc_set_grid");
+    const int rc = set_device_grid(*c, n_pts, d_grid, "pdfxc_set_grid", col);
+    if (rc != PDFXC_OK) (void)hipStreamSynchronize(c->stream);  // flat goes
+    return rc;
 }
 
 int pdfxc_get_grid(pdfxc_ctx* ctx, double* x, double* y, double* z, double* w) {
@@ -1729,6 +1784,12 @@ int pdfxc_get_grid(pdfxc_ctx* ctx, double* x, double* y, double* z, double* w) {
         return PDFXC_ERR_NO_GRID;
     }
     double* col[4] = {x, y, z, w};
+    if (c->n_pts <= kHostPts) {
+        const std::vector<double>* own[4] = {&c->gx, &c->gy, &c->gz, &c->gw};
+        for (int q = 0; q < 4; ++q)
+            if (col[q]) std::copy(own[q]->begin(), own[q]->end(), col[q]);
+        return PDFXC_OK;
+    }
     for (int q = 0; q < 4; ++q)
         if (col[q])
             PDFXC_HIP(hipMemcpyAsync(col[q], c->d_grid + q * c->n_pts, sizeof(double) * (size_t)c->n_pts,
@@ -1743,6 +1804,15 @@ int pdfxc_get_grid_rows(pdfxc_ctx* ctx, double* xyzw) {
     if (c->n_pts == 0) {
         set_error("pdfxc_get_grid_rows: no grid");
         return PDFXC_ERR_NO_GRID;
+    }
+    if (c->n_pts <= kHostPts) {
+        for (int64_t i = 0; i < c->n_pts; ++i) {
+            xyzw[4 * i] = c->gx[i];
+            xyzw[4 * i + 1] = c->gy[i];
+            xyzw[4 * i + 2] = c->gz[i];
+            xyzw[4 * i + 3] = c->gw[i];
+        }
+        return PDFXC_OK;
     }
     const ReadScope scope(*c);
     const int64_t per = std::min<int64_t>(c->n_pts, 1 << 22);  // 128 MiB of rows at a time

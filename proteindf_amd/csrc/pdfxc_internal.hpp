@@ -411,6 +411,14 @@ int ensure_host_grid(Context& c);
 int ensure_host_lists(Context& c);
 int ensure_host_slots(Context& c);
 
+// Grids of up to kHostPts points stay on the host as well, and are read there
+// (60,000 points: 34 us from the host, about 150 by rows from the device); up to
+// kHostCut points the host cuts them into blocks, and up to kHostRho points it
+// puts rho in order (a build of 8 waters with rho: 11 us more than without for
+// 1,000 points, 60 for 20,000, either way, against 47 and 55 by the device).
+constexpr int64_t kHostPts = 65536, kHostCut = 6144, kHostRho = 16384;
+void partition_points(const Context& c, std::vector<int>& order);
+
 // (rho, grad rho) of nspin spins from their slots to rows of 4 nspin in the
 // caller's order, and of one spin from such rows of 4 to its slots
 int rho_to_host(Context& c, int nspin, const double* const* d_slots, double* rows);

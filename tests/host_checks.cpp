@@ -87,7 +87,7 @@ void pool_threads() {
 void host_copy_threads() {
     pdfxc_ctx* ctx = context();
     Context& c = *reinterpret_cast<Context*>(ctx);
-    set_grid(ctx, 1000);
+    set_grid(ctx, 70000);
     fake_slow_copy(50);
     bool ok[2] = {};
     auto work = [&](int k) { ok[k] = ensure_host_grid(c) == PDFXC_OK && host_grid_is_right(c); };
@@ -104,7 +104,7 @@ void host_copy_threads() {
 // the grid's rows need no device memory that is not there, and no current device
 void grid_rows() {
     pdfxc_ctx* ctx = context();
-    const int64_t n = 3000;
+    const int64_t n = 70000;
     set_grid(ctx, n);
     int device = -1;
     CHECK(hipSetDevice(1) == hipSuccess);
@@ -196,7 +196,7 @@ void reserve_gives_way() {
 void rho_without_memory() {
     pdfxc_ctx* ctx = context();
     Context& c = *reinterpret_cast<Context*>(ctx);
-    const int64_t n = 1000;
+    const int64_t n = 70000;
     double P = 1.0, K = 0.0, E = 0.0;
     std::vector<double> out(8 * n), mat(13 * n);
     set_grid(ctx, n);
@@ -236,6 +236,69 @@ void rho_without_memory() {
     CHECK(fake_live_bytes() == 0);
 }
 
+// a small grid is read from the host alone, and its blocks are those of the cuts'
+// definition: every node sorted along its widest extent by (coordinate, index)
+void small_grids() {
+    unsigned seed = 1;
+    for (int64_t n : {(int64_t)1, (int64_t)128, (int64_t)129, (int64_t)300, (int64_t)2049, kHostCut}) {
+        pdfxc_ctx* ctx = context();  // its buffers are new: no kernel writes the block counts
+        Context& c = *reinterpret_cast<Context*>(ctx);
+        std::vector<double> col[4];
+        for (auto& v : col)
+            for (int64_t i = 0; i < n; ++i) {
+                seed = seed * 1664525u + 1013904223u;
+                v.push_back((double)((int)(seed >> 24) - 128) * 0.25);  // many equal coordinates
+            }
+        CHECK(pdfxc_set_grid(ctx, n, col[0].data(), col[1].data(), col[2].data(), col[3].data()) == PDFXC_OK);
+        fake_fail_copy(0);
+        std::vector<double> rows(4 * n), x((size_t)n);
+        CHECK(pdfxc_get_grid_rows(ctx, rows.data()) == PDFXC_OK);
+        CHECK(pdfxc_get_grid(ctx, x.data(), nullptr, nullptr, nullptr) == PDFXC_OK && x == col[0]);
+        fake_fail_copy(-1);
+        for (int64_t i = 0; i < n; ++i)
+            for (int q = 0; q < 4; ++q) CHECK(rows[4 * i + q] == col[q][i]);
+        std::vector<int> order, want((size_t)n);
+        partition_points(c, order);
+        for (int64_t i = 0; i < n; ++i) want[i] = (int)i;
+        std::vector<std::pair<int, int>> nodes{{0, (int)n}};
+        while (!nodes.empty()) {
+            const auto [lo, hi] = nodes.back();
+            nodes.pop_back();
+            if (hi - lo <= kBlockPts) continue;
+            int dim = 0;
+            double widest = -1.0;
+            for (int d = 0; d < 3; ++d) {
+                double mn = 1e300, mx = -1e300;
+                for (int k = lo; k < hi; ++k) {
+                    mn = std::min(mn, col[d][want[k]]);
+                    mx = std::max(mx, col[d][want[k]]);
+                }
+                if (mx - mn > widest) {
+                    widest = mx - mn;
+                    dim = d;
+                }
+            }
+            std::sort(want.begin() + lo, want.begin() + hi, [&](int p, int q) {
+                return col[dim][p] < col[dim][q] || (col[dim][p] == col[dim][q] && p < q);
+            });
+            const int mid = lo + ((hi - lo + kBlockPts - 1) / kBlockPts / 2) * kBlockPts;
+            nodes.push_back({lo, mid});
+            nodes.push_back({mid, hi});
+        }
+        for (int64_t b = 0; b < n; b += kBlockPts) {  // a block's points, in any order
+            const int64_t e = std::min<int64_t>(n, b + kBlockPts);
+            std::sort(order.begin() + b, order.begin() + e);
+            std::sort(want.begin() + b, want.begin() + e);
+        }
+        CHECK(order == want);
+        std::vector<int> seen((size_t)c.n_slots, 0);
+        CHECK((int64_t)c.slot_of_point.size() == n);
+        for (int64_t s : c.slot_of_point) CHECK(s >= 0 && s < c.n_slots && seen[s]++ == 0);
+        pdfxc_ctx_destroy(ctx);
+    }
+    CHECK(fake_live_bytes() == 0);
+}
+
 // the context that densities keep holds no matrices beyond the pool's bound
 void density_keeps_little() {
     const int n = 4800;  // three matrices of 4800 x 4800 are 553 MB
@@ -254,7 +317,7 @@ void failed_copies() {
     pdfxc_ctx* ctx = context();
     Context& c = *reinterpret_cast<Context*>(ctx);
     for (int k = 0; k < 4; ++k) {
-        set_grid(ctx, 1000 + k);
+        set_grid(ctx, 70000 + k);
         fake_fail_copy(k);
         CHECK(ensure_host_grid(c) == PDFXC_ERR_HIP);
         fake_fail_copy(-1);
@@ -327,7 +390,8 @@ int main(int argc, char** argv) {
     } const checks[] = {{"pool_threads", pool_threads}, {"host_copy_threads", host_copy_threads}, {"grid_rows", grid_rows},
                   {"pool_bound", pool_bound},     {"reserve_gives_way", reserve_gives_way},
                   {"density_keeps_little", density_keeps_little}, {"failed_copies", failed_copies},
-                  {"part_tree_sizes", part_tree_sizes}, {"rho_without_memory", rho_without_memory}};
+                  {"part_tree_sizes", part_tree_sizes}, {"rho_without_memory", rho_without_memory},
+                  {"small_grids", small_grids}};
     for (const auto& k : checks)
         if (argc == 2 && !std::strcmp(argv[1], k.name)) {
             k.run();

@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 def test_grid_is_read_during_a_capture():
     mol = molecules.water_cluster(1, 6)
     rng = np.random.default_rng(1)
-    grid = rng.normal(size=(4000, 4))  # rows larger than any workspace its set-up has left behind
+    grid = rng.normal(size=(70000, 4))  # rows larger than any workspace its set-up has left behind
     ctx = engine.XcContext(calc_grid.orbital_info(mol))
     ctx.set_grid(grid)
     x = torch.zeros(64, device="cuda")

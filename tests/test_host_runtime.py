@@ -27,7 +27,7 @@ def program(tmp_path_factory):
 
 @pytest.mark.parametrize("check", ["pool_threads", "host_copy_threads", "grid_rows", "pool_bound",
                                    "reserve_gives_way", "density_keeps_little", "failed_copies", "part_tree_sizes",
-                                   "rho_without_memory"])
+                                   "rho_without_memory", "small_grids"])
 def test_host_code(program, check):
     r = subprocess.run([str(program), check], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
