@@ -332,10 +332,11 @@ int pdfxc_ctx_create(pdfxc_ctx** out, int n_aos, const double* ao_center, const 
     }
     if (rc == PDFXC_OK) rc = dalloc(&c->d_P, (size_t)n_aos * n_aos);
     if (rc == PDFXC_OK) rc = dalloc(&c->d_K, (size_t)n_aos * n_aos);
-    if (rc == PDFXC_OK) rc = dalloc(&c->d_E, 1);
-    if (rc == PDFXC_OK) rc = dalloc(&c->d_packed, packed_doubles(n_aos));
-    if (rc == PDFXC_OK) rc = dalloc(&c->d_queue, kMaxQueues);
+    // one allocation: packed values | E | work-queue counters
+    if (rc == PDFXC_OK) rc = dalloc(&c->d_packed, packed_doubles(n_aos) + 1 + kMaxQueues);
     if (rc == PDFXC_OK) {
+        c->d_E = c->d_packed + packed_doubles(n_aos);
+        c->d_queue = reinterpret_cast<int*>(c->d_E + 1);
         e = hipDeviceGetAttribute(&c->n_cu, hipDeviceAttributeMultiprocessorCount, c->device);
         if (e != hipSuccess) rc = hip_fail(e, "pdfxc_ctx_create: compute unit count");
     }
@@ -428,10 +429,8 @@ int pdfxc_ctx_destroy(pdfxc_ctx* ctx) {
     dfree(c->d_shrec);
     dfree(c->d_P);
     dfree(c->d_K);
-    dfree(c->d_queue);
     dfree(c->d_P2);
     dfree(c->d_K2);
-    dfree(c->d_E);
     dfree(c->d_packed);
     dfree(c->d_Ps);
     dfree(c->d_perm);
@@ -2861,6 +2860,7 @@ static void batch_free(Batch* b) {
     if (b->m.stream) (void)hipStreamSynchronize(b->m.stream);
     if (b->exec) (void)hipGraphExecDestroy(b->exec);
     if (b->graph) (void)hipGraphDestroy(b->graph);
+    b->m.d_kblocks = nullptr;  // in d_k_work's allocation
     free_grid_buffers(&b->m);
     dfree(b->m.d_shrec);
     dfree(b->m.d_queue);
@@ -2923,9 +2923,29 @@ int pdfxc_batch_create(pdfxc_batch** out, int n_mol, pdfxc_ctx* const* ctxs) {
     for (int i = 0; i < n_mol; ++i) RS = std::max(RS, reinterpret_cast<const Context*>(ctxs[i])->rec_stride);
     m.rec_stride = RS;
     std::vector<double> rec;
-    std::vector<double> pts;
     std::vector<int> perm;
     std::vector<int> ebounds{0};
+    // every molecule's slots from a multiple of 256; SoA layout x | y | z | w as
+    // the kernels read it, zero weights in the padding
+    for (int i = 0; i < n_mol; ++i)
+        m.n_slots += (reinterpret_cast<const Context*>(ctxs[i])->n_slots + 255) / 256 * 256;
+    std::vector<double> soa(4 * (size_t)m.n_slots, 0.0);
+    {
+        size_t nb = 0, nk = 0, nsh = 0, nco = 0;
+        for (int i = 0; i < n_mol; ++i) {
+            const Context& c = *reinterpret_cast<const Context*>(ctxs[i]);
+            nb += c.blocks.size();
+            nk += c.kblocks.size();
+            nsh += c.block_shells.size();
+            nco += c.block_cols.size();
+        }
+        m.blocks.reserve(nb);
+        m.kblocks.reserve(nk);
+        m.block_shells.reserve(nsh);
+        m.block_shell_col.reserve(nsh);
+        m.block_sorder.reserve(nsh);
+        m.block_cols.reserve(nco);
+    }
     std::vector<int> kw_cls;  // class of every FP64 KWork in m.h_k_work order (built per class below)
     b->doff.assign(1, 0);
     b->poff.assign(1, 0);
@@ -3011,15 +3031,11 @@ int pdfxc_batch_create(pdfxc_batch** out, int n_mol, pdfxc_ctx* const* ctxs) {
             perm.insert(perm.end(), c.split_perm.begin(), c.split_perm.end());
             psoff += psplit_elems(m.opts.precision, N);
         }
-        pts.resize(4 * (size_t)(slot_base + c.n_slots), 0.0);
-        for (int64_t p = 0; p < c.n_pts; ++p) {
-            const int64_t sl = slot_base + c.slot_of_point[p];
-            const int64_t ns = slot_base + c.n_slots;  // provisional column stride, fixed below
-            (void)ns;
-            pts[4 * sl + 0] = c.gx[p];
-            pts[4 * sl + 1] = c.gy[p];
-            pts[4 * sl + 2] = c.gz[p];
-            pts[4 * sl + 3] = c.gw[p];
+        const std::vector<double>* col[4] = {&c.gx, &c.gy, &c.gz, &c.gw};
+        for (int q = 0; q < 4; ++q) {
+            const double* from = col[q]->data();
+            double* to = soa.data() + q * m.n_slots + slot_base;
+            for (int64_t p = 0; p < c.n_pts; ++p) to[c.slot_of_point[p]] = from[p];
         }
         slot_base += c.n_slots;
         slot_base = (slot_base + 255) / 256 * 256;  // zero-weight padding slots
@@ -3032,14 +3048,6 @@ int pdfxc_batch_create(pdfxc_batch** out, int n_mol, pdfxc_ctx* const* ctxs) {
         m.flops += c.flops;
         m.max_nao = std::max(m.max_nao, c.max_nao);
     }
-    m.n_slots = slot_base;
-    pts.resize(4 * (size_t)m.n_slots, 0.0);
-    // SoA layout x | y | z | w as the kernels read it
-    std::vector<double> soa(4 * (size_t)m.n_slots);
-    for (int64_t sl = 0; sl < m.n_slots; ++sl)
-        for (int q = 0; q < 4; ++q) soa[q * m.n_slots + sl] = pts[4 * sl + q];
-    pts.clear();
-    pts.shrink_to_fit();
     {
         double sum = 0.0;
         for (int i = 0; i < n_mol; ++i) {
@@ -3141,13 +3149,16 @@ int pdfxc_batch_create(pdfxc_batch** out, int n_mol, pdfxc_ctx* const* ctxs) {
     if (rc == PDFXC_OK) rc = alloc(&m.d_queue, kMaxQueues);
     if (rc == PDFXC_OK) rc = alloc(&m.d_pts, soa.size());
     if (rc == PDFXC_OK) rc = alloc(&m.d_blocks, m.blocks.size());
-    if (rc == PDFXC_OK) rc = alloc(&m.d_kblocks, m.kblocks.size());
     if (rc == PDFXC_OK) rc = alloc(&m.d_block_shells, std::max<size_t>(1, m.block_shells.size()));
     if (rc == PDFXC_OK) rc = alloc(&m.d_block_cols, std::max<size_t>(1, m.block_cols.size()));
     if (rc == PDFXC_OK) rc = alloc(&m.d_block_shell_col, std::max<size_t>(1, m.block_shell_col.size()));
     if (rc == PDFXC_OK) rc = alloc(&m.d_block_sorder, std::max<size_t>(1, m.block_sorder.size()));
     if (rc == PDFXC_OK) rc = alloc(&m.d_rho_work, std::max<size_t>(1, m.h_rho_work.size()));
-    if (rc == PDFXC_OK) rc = alloc(reinterpret_cast<char**>(&m.d_k_work), std::max<size_t>(1, m.h_k_work.size()) * sizeof(KWork));
+    // the K items and, in the same allocation, their units
+    const size_t k_units = (m.h_k_work.size() * sizeof(KWork) + 255) / 256 * 256;
+    if (rc == PDFXC_OK)
+        rc = alloc(reinterpret_cast<char**>(&m.d_k_work), k_units + std::max<size_t>(1, m.kblocks.size()) * sizeof(KBlock));
+    if (rc == PDFXC_OK) m.d_kblocks = reinterpret_cast<KBlock*>(reinterpret_cast<char*>(m.d_k_work) + k_units);
     if (rc == PDFXC_OK) rc = alloc(&m.d_coef, 4 * (size_t)m.n_slots);
     if (rc == PDFXC_OK) rc = alloc(&m.d_rho, 4 * (size_t)m.n_slots);
     if (rc == PDFXC_OK) rc = alloc(&m.d_eblock, (size_t)m.n_slots / 256);
@@ -3171,13 +3182,17 @@ int pdfxc_batch_create(pdfxc_batch** out, int n_mol, pdfxc_ctx* const* ctxs) {
     up(m.d_shrec, rec);
     up(m.d_pts, soa);
     up(m.d_blocks, m.blocks);
-    up(m.d_kblocks, m.kblocks);
     up(m.d_block_shells, m.block_shells);
     up(m.d_block_cols, m.block_cols);
     up(m.d_block_shell_col, m.block_shell_col);
     up(m.d_block_sorder, m.block_sorder);
     up(m.d_rho_work, m.h_rho_work);
-    up(reinterpret_cast<KWork*>(m.d_k_work), m.h_k_work);
+    {
+        std::vector<char> both(k_units + m.kblocks.size() * sizeof(KBlock));
+        std::memcpy(both.data(), m.h_k_work.data(), m.h_k_work.size() * sizeof(KWork));
+        std::memcpy(both.data() + k_units, m.kblocks.data(), m.kblocks.size() * sizeof(KBlock));
+        up(static_cast<char*>(m.d_k_work), both);
+    }
     up(b->d_ebounds, ebounds);
     if (split) {
         up(m.d_sblocks, m.sblocks);
