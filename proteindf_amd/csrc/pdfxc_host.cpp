@@ -587,6 +587,91 @@ static size_t kmat_lds(int ps, int ncols, int nsh, int rec_stride) {
     return sizeof(double) * (4 * (size_t)ps * ncols + (size_t)nsh * rec_stride) + sizeof(int) * (size_t)(ncols + 2 * nsh);
 }
 
+// k_kmat work: the lower 2 x 2 tile patches of a unit, row-major, in one item
+// where a workgroup shape holds them (10 of 12, 15 of 16 or 36 patches: at most
+// 8, 10 or 16 tiles a side), else in items of at most 36, or of most[unit] where
+// the tuning cuts them smaller.  kw: items by shape, without shells and points.
+static void kmat_items(const std::vector<KBlock>& units, const std::vector<int>& most, int n_cu,
+                       std::vector<KWork> (&kw)[kKmatClasses]) {
+    auto each_item = [&](int b, int per, auto f) {
+        const int ldn = units[b].ldn, Tp = (ldn / 16 + 1) / 2, np = Tp * (Tp + 1) / 2;
+        for (int t0 = 0, P = 0; t0 < np; t0 += per) {
+            KWork w{b, t0, std::min(np, t0 + per), 0, 0, 0};
+            while ((P + 1) * (P + 2) / 2 <= w.t1 - 1) ++P;
+            w.ncols = std::min(ldn, 32 * (P + 1));
+            f(w);
+        }
+    };
+    bool tuned = false;
+    for (int b = 0; b < (int)units.size(); ++b) {
+        const int cls = kmat_class(units[b].ldn);
+        tuned = tuned || most[b] != kKPatches;
+        each_item(b, cls < 2 ? kKPatches : most[b], [&](const KWork& w) { kw[cls].push_back(w); });
+    }
+    // a shape is a launch of its own, which takes as long as its longest item: one
+    // with few items joins the next wider shape (kKJoinPerCu, kKWidenPerCu)
+    for (int cls = 0; cls + 1 < kKmatClasses; ++cls) {
+        size_t wider = 0;
+        for (int k = cls + 1; k < kKmatClasses; ++k) wider += kw[k].size();
+        if ((int64_t)kw[cls].size() >= (int64_t)(wider ? kKJoinPerCu : kKWidenPerCu) * n_cu) continue;
+        kw[cls + 1].insert(kw[cls + 1].begin(), kw[cls].begin(), kw[cls].end());
+        std::stable_sort(kw[cls + 1].begin(), kw[cls + 1].end(), [](const KWork& a, const KWork& b) { return a.block < b.block; });
+        kw[cls].clear();
+    }
+    // few items of the widest shape: the size that gives the shortest sum over
+    // rounds of one item per CU of the round's longest (kKCostPerCol)
+    std::vector<KWork>& wide = kw[kKmatClasses - 1];
+    if (tuned || wide.empty() || (int64_t)wide.size() >= (int64_t)kKSizePerCu * n_cu) return;
+    std::vector<int> blocks;
+    for (const KWork& w : wide)
+        if (blocks.empty() || blocks.back() != w.block) blocks.push_back(w.block);
+    int best = kKPatches;
+    double best_cost = HUGE_VAL;
+    for (int per : {kKPatches, 30, 24, 18, 15, 12, 9, 6}) {
+        int count[256] = {};  // items by cost
+        for (int b : blocks)
+            each_item(b, per, [&](const KWork& w) {
+                ++count[std::min(255, w.t1 - w.t0 + (int)(kKCostPerCol * w.ncols))];
+            });
+        double cost = 0.0;
+        int64_t seen = 0, next = 0;  // items of larger cost; the first item of the next round
+        for (int k = 255; k >= 0; --k)
+            for (seen += count[k]; next < seen; next += n_cu) cost += k;
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = per;
+        }
+    }
+    if (best == kKPatches) return;
+    wide.clear();
+    for (int b : blocks) each_item(b, best, [&](const KWork& w) { wide.push_back(w); });
+}
+
+// Points per slab of every item (its shells known): 16, or 8 where 16 would cost
+// the shape its workgroups per CU (3, 2 and 1 by its registers), or what one
+// workgroup can have; the items in launch order and their launches.
+static int kmat_launches(std::vector<KWork> (&kw)[kKmatClasses], int RS, size_t (&klds)[kKmatClasses],
+                         std::vector<KWork>& out, std::vector<LaunchRange>& launches) {
+    launches.clear();
+    for (int cls = 0; cls < kKmatClasses; ++cls) {
+        for (KWork& w : kw[cls]) {
+            auto lds_of = [&](int ps) { return kmat_lds(ps, w.ncols, w.nsh, RS); };
+            w.ps = 16;
+            if (lds_of(16) > kKmatLds[cls]) w.ps = lds_of(8) <= kKmatLds[kKmatClasses - 1] ? 8 : 4;
+            const size_t lds = lds_of(w.ps);
+            if (lds > kKmatLds[kKmatClasses - 1]) {
+                set_error("set_grid: block too wide for the K kernel's LDS");
+                return PDFXC_ERR_UNSUPPORTED;
+            }
+            klds[cls] = std::max(klds[cls], lds);
+        }
+        if (kw[cls].empty()) continue;
+        launches.push_back(LaunchRange{cls, (int)out.size(), (int)kw[cls].size(), klds[cls]});
+        out.insert(out.end(), kw[cls].begin(), kw[cls].end());
+    }
+    return PDFXC_OK;
+}
+
 // Blocks, work lists and device buffers of the context's grid; on failure the
 // context is left with no grid (nothing half-built stays reachable).
 static int build_blocks(Context& c) {
@@ -902,30 +987,10 @@ static int build_blocks_impl(Context& c) {
         r.lds = maxdyn;
         if (r.count) c.rho_launches.push_back(r);
     }
-    // k_kmat work: the lower 2 x 2 tile patches of a unit, row-major, in one
-    // item where a workgroup shape holds them (10 of 12, 15 of 16 or 36
-    // patches: at most 8, 10 or 16 tiles a side), else in items of at most 36
-    // (k_tiles = 96; the tuning may cut those smaller)
+    // k_kmat work
     std::vector<KWork> kw[kKmatClasses];
     size_t klds[kKmatClasses] = {};
-    for (int b = 0; b < nu && !c.rho_only; ++b) {
-        const KBlock& B = c.kblocks[b];
-        const int T = B.ldn / 16, Tp = (T + 1) / 2;
-        const int np = Tp * (Tp + 1) / 2;
-        const int cls = kmat_class(B.ldn);
-        const int per = cls < 2 ? np : c.tune.k_tiles * 36 / 96;
-        for (int t0 = 0; t0 < np; t0 += per) {
-            KWork w;
-            w.block = b;
-            w.t0 = t0;
-            w.t1 = std::min(np, t0 + per);
-            int P = 0;
-            while ((P + 1) * (P + 2) / 2 <= w.t1 - 1) ++P;
-            w.ncols = std::min(B.ldn, 32 * (P + 1));
-            w.nsh = w.ps = 0;
-            kw[cls].push_back(w);
-        }
-    }
+    if (!c.rho_only) kmat_items(c.kblocks, std::vector<int>((size_t)nu, c.tune.k_tiles * kKPatches / 96), c.n_cu, kw);
     // the shells of every item: all of its unit's, or, for an item that leaves
     // out the unit's last columns, counted where the block lists are
     size_t n_items = 0;
@@ -954,26 +1019,7 @@ static int build_blocks_impl(Context& c) {
         for (auto& list : kw)
             for (KWork& w : list) w.nsh = item_nsh[at++];
     }
-    // points per slab: 16, or 8 where 16 would cost the class its workgroups
-    // per CU (3, 2 and 1 by its registers), or what one workgroup can have
-    for (int cls = 0; cls < kKmatClasses; ++cls)
-        for (KWork& w : kw[cls]) {
-            auto lds_of = [&](int ps) { return kmat_lds(ps, w.ncols, w.nsh, RS); };
-            w.ps = 16;
-            if (lds_of(16) > kKmatLds[cls]) w.ps = lds_of(8) <= kKmatLds[kKmatClasses - 1] ? 8 : 4;
-            const size_t lds = lds_of(w.ps);
-            if (lds > kKmatLds[kKmatClasses - 1]) {
-                set_error("set_grid: block too wide for the K kernel's LDS");
-                return PDFXC_ERR_UNSUPPORTED;
-            }
-            klds[cls] = std::max(klds[cls], lds);
-        }
-    c.kmat_launches.clear();
-    for (int cls = 0; cls < kKmatClasses; ++cls) {
-        if (kw[cls].empty()) continue;
-        c.kmat_launches.push_back(LaunchRange{cls, (int)kall.size(), (int)kw[cls].size(), klds[cls]});
-        kall.insert(kall.end(), kw[cls].begin(), kw[cls].end());
-    }
+    if (int e = kmat_launches(kw, RS, klds, kall, c.kmat_launches)) return e;
 
     // split precision: chunked column layout and k_rho_split classes (ldnp <=
     // 256: 64 points per workgroup, <= 512: 32, <= 1024: 16); k_kmat_split items
@@ -3095,8 +3141,30 @@ int pdfxc_batch_create(pdfxc_batch** out, int n_mol, pdfxc_ctx* const* ctxs) {
     };
     merge_int([](const Context& c) -> const std::vector<LaunchRange>& { return c.rho_launches; },
               [](const Context& c) -> const std::vector<int>& { return c.h_rho_work; }, m.h_rho_work, m.rho_launches);
-    merge_kw([](const Context& c) -> const std::vector<LaunchRange>& { return c.kmat_launches; },
-             [](const Context& c) -> const std::vector<KWork>& { return c.h_k_work; }, m.h_k_work, m.kmat_launches);
+    if (!split) {
+        // FP64 K items of the batch's own count of units (a context's are sized for it alone)
+        std::vector<int> most;
+        for (int i = 0; i < n_mol; ++i) {
+            const Context& c = *reinterpret_cast<const Context*>(ctxs[i]);
+            most.insert(most.end(), c.kblocks.size(), c.tune.k_tiles * kKPatches / 96);
+        }
+        std::vector<KWork> kw[kKmatClasses];
+        size_t klds[kKmatClasses] = {};
+        kmat_items(m.kblocks, most, c0->n_cu, kw);
+        for (auto& list : kw)
+            for (KWork& w : list) {
+                const KBlock& U = m.kblocks[w.block];
+                const int* col = m.block_shell_col.data() + U.shell_begin;
+                w.nsh = (int)(std::lower_bound(col, col + U.nshell, w.ncols) - col);
+            }
+        if (int rc = kmat_launches(kw, RS, klds, m.h_k_work, m.kmat_launches)) {
+            batch_free(b);
+            return rc;
+        }
+    } else {
+        merge_kw([](const Context& c) -> const std::vector<LaunchRange>& { return c.kmat_launches; },
+                 [](const Context& c) -> const std::vector<KWork>& { return c.h_k_work; }, m.h_k_work, m.kmat_launches);
+    }
     if (split) {
         merge_kw([](const Context& c) -> const std::vector<LaunchRange>& { return c.k_fp64_launches; },
                  [](const Context& c) -> const std::vector<KWork>& { return c.h_k_work; }, m.h_k_work,

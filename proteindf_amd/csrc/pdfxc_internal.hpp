@@ -95,6 +95,24 @@ constexpr int kKGroupMax = 2;
 // (79,000 blocks of 30 residues: 37.0 single, 28.1 all pairs; limits of 10 %
 // and 30 % are within 2 % of this, two or more units per CU up to 8 % slower).
 constexpr int kKUnitsPerCu = 10, kKWiderPct = 15;
+// An item has at most kKPatches patches of tiles.
+// K items of a workgroup shape join the next wider one below kKJoinPerCu items
+// per CU where that has items, and below kKWidenPerCu where it has none (12
+// waves take a narrow unit in less time than 4, and CUs are idle).  K pass, us,
+// with a launch for every shape, and joined:
+//     40 blocks, 187 AOs at most     202     67      235 blocks, 8 waters (13 AOs)  34   34
+//     40 blocks, 304                 232    103       40 blocks, 8 waters           66   37
+//    313 blocks, 294                 277    207       40 blocks, 96 AOs             59   34
+//  2,344 blocks, 185                 657    468    4,688 blocks, 23 waters         562  504
+//  4,688 blocks, 284                1477   1297    7,813 blocks, 23 waters         686  682
+// (joined at any number: 562 -> 543 and 686 -> 592 in the last two; at 4 items
+// per CU: 657 -> 597, 1477 -> 1380.  Widened at 4: 36 -> 50 for 313 blocks.)
+constexpr int kKPatches = 36, kKJoinPerCu = 16, kKWidenPerCu = 1;
+// Size of the widest shape's items below kKSizePerCu items per CU: an item
+// takes about 1.8 us a patch, and for the production of phi and V that every
+// item of a block repeats as much as kKCostPerCol patches a column.
+constexpr int kKSizePerCu = 4;
+constexpr double kKCostPerCol = 0.09;
 struct KBlock {
     int slot[kKGroupMax];  // first slot of every block
     int npts;              // real points of all of them
