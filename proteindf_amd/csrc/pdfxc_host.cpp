@@ -593,8 +593,8 @@ static size_t kmat_lds(int ps, int ncols, int nsh, int rec_stride) {
 // the tuning cuts them smaller.  kw: items by shape, without shells and points.
 static void kmat_items(const std::vector<KBlock>& units, const std::vector<int>& most, int n_cu,
                        std::vector<KWork> (&kw)[kKmatClasses]) {
-    auto each_item = [&](int b, int per, auto f) {
-        const int ldn = units[b].ldn, Tp = (ldn / 16 + 1) / 2, np = Tp * (Tp + 1) / 2;
+    auto each_item = [](int b, int ldn, int per, auto f) {
+        const int Tp = (ldn / 16 + 1) / 2, np = Tp * (Tp + 1) / 2;
         for (int t0 = 0, P = 0; t0 < np; t0 += per) {
             KWork w{b, t0, std::min(np, t0 + per), 0, 0, 0};
             while ((P + 1) * (P + 2) / 2 <= w.t1 - 1) ++P;
@@ -606,7 +606,7 @@ static void kmat_items(const std::vector<KBlock>& units, const std::vector<int>&
     for (int b = 0; b < (int)units.size(); ++b) {
         const int cls = kmat_class(units[b].ldn);
         tuned = tuned || most[b] != kKPatches;
-        each_item(b, cls < 2 ? kKPatches : most[b], [&](const KWork& w) { kw[cls].push_back(w); });
+        each_item(b, units[b].ldn, cls < 2 ? kKPatches : most[b], [&](const KWork& w) { kw[cls].push_back(w); });
     }
     // a shape is a launch of its own, which takes as long as its longest item: one
     // with few items joins the next wider shape (kKJoinPerCu, kKWidenPerCu)
@@ -623,15 +623,22 @@ static void kmat_items(const std::vector<KBlock>& units, const std::vector<int>&
     std::vector<KWork>& wide = kw[kKmatClasses - 1];
     if (tuned || wide.empty() || (int64_t)wide.size() >= (int64_t)kKSizePerCu * n_cu) return;
     std::vector<int> blocks;
-    for (const KWork& w : wide)
-        if (blocks.empty() || blocks.back() != w.block) blocks.push_back(w.block);
+    std::vector<std::pair<int, int>> widths;  // columns, units of that width
+    for (const KWork& w : wide) {
+        if (!blocks.empty() && blocks.back() == w.block) continue;
+        blocks.push_back(w.block);
+        const int ldn = units[w.block].ldn;
+        auto at = std::find_if(widths.begin(), widths.end(), [&](const auto& v) { return v.first == ldn; });
+        if (at == widths.end()) widths.push_back({ldn, 1});
+        else ++at->second;
+    }
     int best = kKPatches;
     double best_cost = HUGE_VAL;
     for (int per : {kKPatches, 30, 24, 18, 15, 12, 9, 6}) {
         int count[256] = {};  // items by cost
-        for (int b : blocks)
-            each_item(b, per, [&](const KWork& w) {
-                ++count[std::min(255, w.t1 - w.t0 + (int)(kKCostPerCol * w.ncols))];
+        for (const auto& [ldn, n] : widths)
+            each_item(0, ldn, per, [&, k = n](const KWork& w) {
+                count[std::min(255, w.t1 - w.t0 + (int)(kKCostPerCol * w.ncols))] += k;
             });
         double cost = 0.0;
         int64_t seen = 0, next = 0;  // items of larger cost; the first item of the next round
@@ -644,7 +651,7 @@ static void kmat_items(const std::vector<KBlock>& units, const std::vector<int>&
     }
     if (best == kKPatches) return;
     wide.clear();
-    for (int b : blocks) each_item(b, best, [&](const KWork& w) { wide.push_back(w); });
+    for (int b : blocks) each_item(b, units[b].ldn, best, [&](const KWork& w) { wide.push_back(w); });
 }
 
 // Points per slab of every item (its shells known): 16, or 8 where 16 would cost
@@ -1716,8 +1723,8 @@ static int first_not_finite(Context& c, int64_t n, const double* d_grid, const c
 
 // Takes over d_grid (n x 4 columns, written on c.stream) as the context's grid
 // and builds its blocks; a grid with a value that is not finite is refused and
-// leaves the context without one.  Up to kHostPts points the context has the
-// columns on the host as well: col if given, else copied back.
+// leaves the context without one.  Up to kHostPts points that came from the host
+// (col), and up to kHostCut made on the device, the host has the columns as well.
 static int set_device_grid(Context& c, int64_t n, double* d_grid, const char* who, const double* const* col = nullptr) {
     gfree(c, c.d_grid);
     c.d_grid = d_grid;
@@ -1729,7 +1736,7 @@ static int set_device_grid(Context& c, int64_t n, double* d_grid, const char* wh
     c.grid_size_adjust = 1;
     int64_t first = n;
     int rc = PDFXC_OK;
-    if (n <= (c.rho_only ? kHostCut : kHostPts)) {
+    if (n <= (col ? kHostPts : kHostCut)) {
         if (col)
             for (int q = 0; q < 4; ++q) own[q]->assign(col[q], col[q] + n);
         else
@@ -1830,10 +1837,13 @@ int pdfxc_get_grid(pdfxc_ctx* ctx, double* x, double* y, double* z, double* w) {
     }
     double* col[4] = {x, y, z, w};
     if (c->n_pts <= kHostPts) {
+        std::lock_guard<std::mutex> lock(c->host_mu);
         const std::vector<double>* own[4] = {&c->gx, &c->gy, &c->gz, &c->gw};
-        for (int q = 0; q < 4; ++q)
-            if (col[q]) std::copy(own[q]->begin(), own[q]->end(), col[q]);
-        return PDFXC_OK;
+        if ((int64_t)own[0]->size() == c->n_pts) {
+            for (int q = 0; q < 4; ++q)
+                if (col[q]) std::copy(own[q]->begin(), own[q]->end(), col[q]);
+            return PDFXC_OK;
+        }
     }
     for (int q = 0; q < 4; ++q)
         if (col[q])
@@ -1851,13 +1861,16 @@ int pdfxc_get_grid_rows(pdfxc_ctx* ctx, double* xyzw) {
         return PDFXC_ERR_NO_GRID;
     }
     if (c->n_pts <= kHostPts) {
-        for (int64_t i = 0; i < c->n_pts; ++i) {
-            xyzw[4 * i] = c->gx[i];
-            xyzw[4 * i + 1] = c->gy[i];
-            xyzw[4 * i + 2] = c->gz[i];
-            xyzw[4 * i + 3] = c->gw[i];
+        std::lock_guard<std::mutex> lock(c->host_mu);
+        if ((int64_t)c->gx.size() == c->n_pts) {
+            for (int64_t i = 0; i < c->n_pts; ++i) {
+                xyzw[4 * i] = c->gx[i];
+                xyzw[4 * i + 1] = c->gy[i];
+                xyzw[4 * i + 2] = c->gz[i];
+                xyzw[4 * i + 3] = c->gw[i];
+            }
+            return PDFXC_OK;
         }
-        return PDFXC_OK;
     }
     const ReadScope scope(*c);
     const int64_t per = std::min<int64_t>(c->n_pts, 1 << 22);  // 128 MiB of rows at a time

@@ -429,8 +429,8 @@ int ensure_host_grid(Context& c);
 int ensure_host_lists(Context& c);
 int ensure_host_slots(Context& c);
 
-// Grids of up to kHostPts points stay on the host as well, and are read there
-// (60,000 points: 34 us from the host, about 150 by rows from the device); up to
+// Grids of up to kHostPts points that came from the host stay there as well, and
+// are read there (60,000 points: 34 us, about 150 by rows from the device); up to
 // kHostCut points the host cuts them into blocks, and up to kHostRho points it
 // puts rho in order (a build of 8 waters with rho: 11 us more than without for
 // 1,000 points, 60 for 20,000, either way, against 47 and 55 by the device).
