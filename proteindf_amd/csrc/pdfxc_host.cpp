@@ -3115,6 +3115,15 @@ int pdfxc_batch_create(pdfxc_batch** out, int n_mol, pdfxc_ctx* const* ctxs) {
         }
         m.mean_nao = sum / (double)nblocks;
     }
+    // LDS that a context's items need beyond what it reckoned: its shell records
+    // have the batch's length here, that of the context with most primitives
+    auto longer = [&](const Context& c) {
+        int most = 0;
+        for (const BlockDesc& B : c.blocks) most = std::max(most, B.nshell);
+        for (const KBlock& U : c.kblocks) most = std::max(most, U.nshell);
+        for (const KGroup& G : c.kgroups) most = std::max(most, G.nshell);
+        return sizeof(double) * (size_t)(RS - c.rec_stride) * (size_t)most;
+    };
     // work lists: every launch class over all molecules
     auto merge_int = [&](auto get_ranges, auto get_list, std::vector<int>& out_list, std::vector<LaunchRange>& out_r) {
         for (int cls = 0; cls < kRhoFp64Class + 8; ++cls) {
@@ -3125,7 +3134,7 @@ int pdfxc_batch_create(pdfxc_batch** out, int n_mol, pdfxc_ctx* const* ctxs) {
                     if (q.cls != cls) continue;
                     const std::vector<int>& L = get_list(c);
                     for (int k = 0; k < q.count; ++k) out_list.push_back(L[q.offset + k] + block_base[i]);
-                    r.lds = std::max(r.lds, q.lds);
+                    r.lds = std::max(r.lds, q.lds + longer(c));
                 }
             }
             r.count = (int)out_list.size() - r.offset;
@@ -3145,7 +3154,7 @@ int pdfxc_batch_create(pdfxc_batch** out, int n_mol, pdfxc_ctx* const* ctxs) {
                         w.block += kblock_base[i];
                         out_list.push_back(w);
                     }
-                    r.lds = std::max(r.lds, q.lds);
+                    r.lds = std::max(r.lds, q.lds + longer(c));
                 }
             }
             r.count = (int)out_list.size() - r.offset;
@@ -3196,7 +3205,7 @@ int pdfxc_batch_create(pdfxc_batch** out, int n_mol, pdfxc_ctx* const* ctxs) {
                         w.group += group_base[i];
                         m.h_kg_work.push_back(w);
                     }
-                    r.lds = std::max(r.lds, q.lds);
+                    r.lds = std::max(r.lds, q.lds + longer(c));
                 }
             }
             r.count = (int)m.h_kg_work.size() - r.offset;
