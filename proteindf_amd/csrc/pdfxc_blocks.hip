@@ -23,8 +23,8 @@
 // points take 9 levels.  On the host the same cuts (std::nth_element over an
 // index array), the screening and the lists took 185, 104 and 78 ms for those
 // 1.5 million points in 11,900 blocks, against 1.9, 0.06 and 0.16 ms here.
-// (The split precision modes keep the host's cuts for their order within a
-// block, see partition_points.)
+// (Grids of few points and the split precision modes take the host's cuts, see
+// partition_points.)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

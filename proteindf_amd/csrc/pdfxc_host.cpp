@@ -1845,6 +1845,7 @@ int pdfxc_get_grid(pdfxc_ctx* ctx, double* x, double* y, double* z, double* w) {
             return PDFXC_OK;
         }
     }
+    const ReadScope scope(*c);
     for (int q = 0; q < 4; ++q)
         if (col[q])
             PDFXC_HIP(hipMemcpyAsync(col[q], c->d_grid + q * c->n_pts, sizeof(double) * (size_t)c->n_pts,

@@ -689,7 +689,8 @@ __global__ __launch_bounds__(256) void k_xc_points_uks(int64_t n_slots, const do
 // 4.6 -> 4.0 ms, of a 30-residue helix 43.1 -> 36.9 ms, there bound by the
 // scatter's atomics (26.6 ms without them); with two blocks a unit 3.4 and
 // 28.1 ms, 26.9 without the scatter, 22.5 without the production and 18.4
-// without the products, whose MFMAs alone take 17.
+// without the products, whose MFMAs alone take 17; with the narrow shapes'
+// few items in the widest shape's launch 3.1 and 27.8 ms.
 // Slab element (point p, column c) is at p LD + (c ^ (p & 15)): the 16 lanes
 // of an operand read stay on one 256-byte run, and a producer's 16 points of
 // one column fall on 16 different 16-byte slots.
@@ -900,7 +901,8 @@ __device__ __forceinline__ void k_kmat_item(int item, const KWork* __restrict__ 
 }
 
 // Workgroup shapes by the unit's tile count T: up to 8 tiles (10
-// patches) 4 waves, up to 10 (15 patches) 8, wider 12 (36 patches are T = 16).
+// patches) 4 waves, up to 10 (15 patches) 8, wider 12 (36 patches are T = 16);
+// a shape of few items joins the next one, which takes narrower units as well.
 template <int NW, int NPW, bool PERSIST>
 __global__ __launch_bounds__(NW * 64, NW == 8 ? 4 : 3) void k_kmat(const KWork* __restrict__ work, const KBlock* __restrict__ units,
                                               const double* __restrict__ pts, int64_t n_slots,
@@ -1073,7 +1075,7 @@ __global__ __launch_bounds__(256) void k_becke(const double* __restrict__ atoms,
 // atom is 0 leaves with one test, and of a cell that stays the lanes take the
 // neighbours, only the factors that are not 1 being multiplied (own atom
 // first, then in index order).  One lane per cell with all neighbours in turn
-// (k_becke) took 23.2 ms for the 2.6 million points of a 142-atom helix,
+// (k_becke) took 23.2 ms for the 2.15 million points of a 143-atom helix,
 // bound by the few lanes whose cells stay; this takes 8.1 ms.
 __device__ __forceinline__ double ss_factor(double rm, double rk, double inv) {
     const double u = (rm - rk) * inv;
