@@ -9,6 +9,7 @@
 #include <cstring>
 #include <numeric>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "pdfxc_internal.hpp"
@@ -330,11 +331,13 @@ int pdfxc_ctx_create(pdfxc_ctx** out, int n_aos, const double* ao_center, const 
         e = hipMemcpy(c->d_shrec, rec.data(), rec.size() * sizeof(double), hipMemcpyHostToDevice);
         if (e != hipSuccess) rc = hip_fail(e, "pdfxc_ctx_create: shell records upload");
     }
-    if (rc == PDFXC_OK) rc = dalloc(&c->d_P, (size_t)n_aos * n_aos);
-    if (rc == PDFXC_OK) rc = dalloc(&c->d_K, (size_t)n_aos * n_aos);
-    // one allocation: packed values | E | work-queue counters
-    if (rc == PDFXC_OK) rc = dalloc(&c->d_packed, packed_doubles(n_aos) + 1 + kMaxQueues);
+    // one allocation: P | K | packed values | E | work-queue counters (P and K
+    // from multiples of 256 bytes)
+    const size_t nn = ((size_t)n_aos * n_aos + 31) / 32 * 32;
+    if (rc == PDFXC_OK) rc = dalloc(&c->d_P, 2 * nn + packed_doubles(n_aos) + 1 + kMaxQueues);
     if (rc == PDFXC_OK) {
+        c->d_K = c->d_P + nn;
+        c->d_packed = c->d_K + nn;
         c->d_E = c->d_packed + packed_doubles(n_aos);
         c->d_queue = reinterpret_cast<int*>(c->d_E + 1);
         e = hipDeviceGetAttribute(&c->n_cu, hipDeviceAttributeMultiprocessorCount, c->device);
@@ -389,6 +392,21 @@ int pdfxc_ctx_create(pdfxc_ctx** out, int n_aos, const double* ao_center, const 
 }
 
 static void free_grid_buffers(Context* c) {
+    if (c->d_lists) {  // one buffer for all of these
+        c->d_slot_of_point = nullptr;
+        c->d_blocks = nullptr;
+        c->d_kblocks = nullptr;
+        c->d_block_shells = nullptr;
+        c->d_block_cols = nullptr;
+        c->d_block_shell_col = nullptr;
+        c->d_block_sorder = nullptr;
+        gfree(*c, c->d_lists);
+    }
+    if (c->d_work) {
+        c->d_rho_work = nullptr;
+        c->d_k_work = nullptr;
+        gfree(*c, c->d_work);
+    }
     gfree(*c, c->d_pts);
     gfree(*c, c->d_slot_of_point);
     gfree(*c, c->d_blocks);
@@ -428,10 +446,8 @@ int pdfxc_ctx_destroy(pdfxc_ctx* ctx) {
     dfree(c->d_shells);
     dfree(c->d_shrec);
     dfree(c->d_P);
-    dfree(c->d_K);
     dfree(c->d_P2);
     dfree(c->d_K2);
-    dfree(c->d_packed);
     dfree(c->d_Ps);
     dfree(c->d_perm);
     if (c->h_pinned) (void)hipHostFree(c->h_pinned);
@@ -930,13 +946,27 @@ static int build_blocks_impl(Context& c) {
     c.n_block_shells = sh0;
     c.n_block_cols = col0;
     rc = galloc(c, &c.d_pts, 4 * (size_t)c.n_slots);
-    if (rc == PDFXC_OK) rc = galloc(c, &c.d_slot_of_point, (size_t)n);
-    if (rc == PDFXC_OK) rc = galloc(c, &c.d_blocks, c.blocks.size());
-    if (rc == PDFXC_OK) rc = galloc(c, &c.d_kblocks, c.kblocks.size());
-    if (rc == PDFXC_OK) rc = galloc(c, &c.d_block_shells, (size_t)sh0);
-    if (rc == PDFXC_OK) rc = galloc(c, &c.d_block_cols, (size_t)col0);
-    if (rc == PDFXC_OK) rc = galloc(c, &c.d_block_shell_col, (size_t)sh0);
-    if (rc == PDFXC_OK) rc = galloc(c, &c.d_block_sorder, (size_t)sh0);
+    if (rc == PDFXC_OK) {
+        // blocks | units | slots | shells | columns | first columns | order
+        const size_t b_b = align(sizeof(BlockDesc) * c.blocks.size()), b_k = align(sizeof(KBlock) * c.kblocks.size()),
+                     b_s = align(sizeof(int) * (size_t)n), b_sh = align(sizeof(int) * (size_t)sh0),
+                     b_c = align(sizeof(int) * (size_t)col0);
+        rc = galloc(c, &c.d_lists, b_b + b_k + b_s + 3 * b_sh + b_c);
+        char* q = c.d_lists;
+        auto part = [&](auto*& p, size_t bytes) {
+            p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(q);
+            q += bytes;
+        };
+        if (rc == PDFXC_OK) {
+            part(c.d_blocks, b_b);
+            part(c.d_kblocks, b_k);
+            part(c.d_slot_of_point, b_s);
+            part(c.d_block_shells, b_sh);
+            part(c.d_block_cols, b_c);
+            part(c.d_block_shell_col, b_sh);
+            part(c.d_block_sorder, b_sh);
+        }
+    }
     if (rc) return rc;
     PDFXC_HIP(hipMemcpyAsync(c.d_blocks, c.blocks.data(), sizeof(BlockDesc) * (size_t)nb, hipMemcpyHostToDevice, c.stream));
     PDFXC_HIP(hipMemcpyAsync(d_leaf, lorder.data(), sizeof(int) * (size_t)nb, hipMemcpyHostToDevice, c.stream));
@@ -1318,8 +1348,14 @@ static int build_blocks_impl(Context& c) {
     }
 
     // device buffers
-    if (rc == PDFXC_OK) rc = galloc(c, &c.d_rho_work, rho_work.size());
-    if (rc == PDFXC_OK) rc = galloc(c, reinterpret_cast<char**>(&c.d_k_work), kall.size() * sizeof(KWork));
+    if (rc == PDFXC_OK) {
+        const size_t b_r = align(sizeof(int) * rho_work.size());
+        rc = galloc(c, &c.d_work, b_r + sizeof(KWork) * kall.size());
+        if (rc == PDFXC_OK) {
+            c.d_rho_work = reinterpret_cast<int*>(c.d_work);
+            c.d_k_work = c.d_work + b_r;
+        }
+    }
     if (rc == PDFXC_OK && !c.rho_only) rc = galloc(c, &c.d_coef, 4 * (size_t)c.n_slots);
     if (rc == PDFXC_OK) rc = galloc(c, &c.d_rho, 4 * (size_t)c.n_slots);
     if (rc == PDFXC_OK) rc = galloc(c, &c.d_eblock, 3 * (size_t)((c.n_slots + 255) / 256));

@@ -326,6 +326,8 @@ struct Context {
     int rec_stride = 0;
     double* d_pts = nullptr;  // 4 x n_slots SoA: x, y, z, w
     int64_t n_slots = 0;
+    char* d_lists = nullptr;  // a context's slots, blocks, units and their lists (a batch has a buffer for each)
+    char* d_work = nullptr;   // its rho and K work lists
     int* d_slot_of_point = nullptr;
     BlockDesc* d_blocks = nullptr;
     KBlock* d_kblocks = nullptr;
